@@ -46,6 +46,7 @@ SIGNATURES = {
     "apx_col2im_s2": (ctypes.c_int, [_p, _i32, _i32, _i32, _i32, _i32, _p, _p]),
     "apx_cast_gate_bf16": (ctypes.c_int, [_p, _p, _i64, _p, _p, _p]),
     "apx_colsum": (ctypes.c_int, [_p, _i32, _i32, _p, _p]),
+    "apx_gate_colsum_bf16": (ctypes.c_int, [_p, _p, _i32, _i32, _p, _p, _p, _i64, _p]),
     "apx_adam": (ctypes.c_int, [_p, _p, _p, _p, _i64, _f32, _f32, _f32, _f32, _i32, _p, _p]),
     "apx_asinh_input": (ctypes.c_int, [_p, _p, _i32, _i32, _p, _p]),
 }
@@ -80,6 +81,12 @@ def gemm(A, sam, sak, B, sbk, sbn, C, M, N, K, ldc=None, bias=None, relu=False, 
 def cast_bf16(src, dst, mask=None, dstf=None):
     L.check(L.load().apx_cast_gate_bf16(src.data_ptr(), _ptr(mask), src.numel(), dst.data_ptr(), _ptr(dstf),
                                         L.stream()))
+
+
+def gate_colsum(src, M, N, dst, out, ws, mask=None):
+    """dst = bf16 of src (M, N), zeroed where mask <= 0; out = the column sums of the gated float32 values."""
+    L.check(L.load().apx_gate_colsum_bf16(src.data_ptr(), _ptr(mask), M, N, dst.data_ptr(), out.data_ptr(),
+                                          ws.data_ptr(), ws.numel(), L.stream()))
 
 
 # ---------------------------------------------------------------------------
@@ -266,32 +273,26 @@ class InitNet:
         ws = buf["ws"]
         f1, f2 = self.layers[4], self.layers[5]
         db = buf["gbf"][:dout.numel()]
-        cast_bf16(dout, db)
+        gate_colsum(dout, B, f2.cout, db, f2.gb, ws)
         # fc2
         gemm(buf["hb"], 1, f2.cin, db, f2.cout, 1, f2.gw, f2.cin, f2.cout, B, ws=ws)
-        L.check(lib.apx_colsum(dout.data_ptr(), B, f2.cout, f2.gb.data_ptr(), L.stream()))
         dh = buf["g32"][:B * f2.cin]
         gemm(db, f2.cout, 1, f2.wb, 1, f2.cout, dh, B, f2.cin, f2.cout)
         dz = buf["gbf2"][:B * f2.cin]
-        dzf = buf["g32b"][:B * f2.cin]
-        cast_bf16(dh, dz, mask=buf["h"], dstf=dzf)
+        gate_colsum(dh, B, f1.cout, dz, f1.gb, ws, mask=buf["h"])
         # fc1
         y4b = buf["yb"][3]
         gemm(y4b, 1, f1.cin, dz, f1.cout, 1, f1.gw, f1.cin, f1.cout, B, ws=ws)
-        L.check(lib.apx_colsum(dzf.data_ptr(), B, f1.cout, f1.gb.data_ptr(), L.stream()))
         dy = buf["g32"][:B * f1.cin]
         gemm(dz, f1.cout, 1, f1.wb, 1, f1.cout, dy, B, f1.cin, f1.cout)
         # convolutions, last to first: dz_l = dy_l * (y_l > 0).  dy of the
-        # last convolution is in g32; col2im leaves the others in g32b, where
-        # the (element-wise) gate then writes its float32 copy in place.
+        # last convolution is in g32, of the others in g32b.
         for i in range(len(CONV) - 1, -1, -1):
             H, cin, cout, M, K = buf["dims"][i]
             lay = self.layers[i]
             dzb = buf["gbf"][:M * cout]
-            dzf = buf["g32b"][:M * cout]
-            cast_bf16(dy, dzb, mask=buf["y"][i], dstf=dzf)
+            gate_colsum(dy, M, cout, dzb, lay.gb, ws, mask=buf["y"][i])
             gemm(buf["col"][i], 1, K, dzb, cout, 1, lay.gw, K, cout, M, ws=ws)
-            L.check(lib.apx_colsum(dzf.data_ptr(), M, cout, lay.gb.data_ptr(), L.stream()))
             if i == 0:
                 break
             dcol = buf["g32"][:M * K]

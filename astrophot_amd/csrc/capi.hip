@@ -234,6 +234,11 @@ int apx_cast_gate_bf16(const float* src, const float* mask, int64_t n, uint16_t*
   return apx::cast_gate(src, mask, n, dst, dstf, static_cast<hipStream_t>(stream));
 }
 
+int apx_gate_colsum_bf16(const float* src, const float* mask, int32_t M, int32_t N, uint16_t* dst, float* out,
+                         float* ws, int64_t ws_floats, void* stream) {
+  return apx::gate_colsum(src, mask, M, N, dst, out, ws, ws_floats, static_cast<hipStream_t>(stream));
+}
+
 int apx_colsum(const float* X, int32_t M, int32_t N, float* out, void* stream) {
   return apx::colsum(X, M, N, out, static_cast<hipStream_t>(stream));
 }

@@ -83,6 +83,8 @@ int col2im_s2(const float* dcol, int Bn, int H, int W, int Cin, int Kp, float* d
 int cast_gate(const float* src, const float* mask, int64_t n, uint16_t* dst, float* dstf,
               hipStream_t stream);
 int colsum(const float* X, int M, int N, float* out, hipStream_t stream);
+int gate_colsum(const float* src, const float* mask, int M, int N, uint16_t* dst, float* out, float* ws,
+                int64_t ws_floats, hipStream_t stream);
 int adam(float* w, const float* g, float* m, float* v, int64_t n, float lr, float b1, float b2,
          float eps, int step, uint16_t* wb, hipStream_t stream);
 int asinh_input(const float* x, const float* sigma, int Bn, int npx, uint16_t* out, hipStream_t stream);

@@ -546,6 +546,12 @@ int apx_cast_gate_bf16(const float* src, const float* mask, int64_t n, uint16_t*
 /* out[n] = sum_m X[m,n] (bias gradients). */
 int apx_colsum(const float* X, int32_t M, int32_t N, float* out, void* stream);
 
+/* apx_cast_gate_bf16 of src (M, N) into dst, and out[n] = sum_m of the gated
+ * float32 values, in one pass.  ws: at least N floats, one partial sum row a
+ * workgroup (512 N floats let every workgroup have its own). */
+int apx_gate_colsum_bf16(const float* src, const float* mask, int32_t M, int32_t N, uint16_t* dst,
+                         float* out, float* ws, int64_t ws_floats, void* stream);
+
 /* One Adam step (bias-corrected, step >= 1) on float32 weights w with
  * gradient g and moments m, v; w_bf16 (optional) receives bf16(w). */
 int apx_adam(float* w, const float* g, float* m, float* v, int64_t n, float lr, float beta1,

@@ -49,6 +49,26 @@ def test_gemm_bf16_matches_float32(M, N, K, ta, tb, split):
     assert torch.equal(Cb.cpu(), C.cpu().to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("M,N,masked,off", [(1, 8, False, 0), (257, 8, True, 0), (1000, 32, True, 0), (4099, 64, False, 0),
+                                            (2050, 128, True, 0), (1000, 32, True, 1), (77, 12, True, 0), (300, 37, False, 0),
+                                            (5, 1028, True, 0)])
+def test_gate_colsum(M, N, masked, off):
+    """Gate, bf16 copy and column sums in one pass: 4-column and general
+    paths (``off``: a source not on 16 bytes), remainders of the row steps.
+    A sum adds at most 64 terms in a chain (rows of a thread, rows of a step,
+    workgroups of a lane): 64 rounding errors of the column's sum of |v|."""
+    g = torch.Generator().manual_seed(M + N)
+    src = torch.randn(M * N + off, generator=g).to(DEV)[off:].view(M, N)
+    mask = torch.randn(M, N, generator=g).to(DEV) if masked else None
+    dst = torch.zeros((M, N), dtype=torch.bfloat16, device=DEV)
+    out, ws = torch.zeros(N, device=DEV), torch.zeros(1 << 18, device=DEV)
+    cnn.gate_colsum(src, M, N, dst, out, ws, mask=mask)
+    ref = src if mask is None else torch.where(mask > 0, src, torch.zeros_like(src))
+    assert torch.equal(dst, ref.to(torch.bfloat16))
+    err = (out.double() - ref.double().sum(0)).abs()
+    assert bool((err <= 64 * 2.0 ** -24 * ref.double().abs().sum(0)).all())
+
+
 def torch_reference(net, x, dout_seed=3):
     """The same network in torch on the CPU (float32), bf16 rounding where the kernels round."""
     params = []
