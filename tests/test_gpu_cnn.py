@@ -49,6 +49,26 @@ def test_gemm_bf16_matches_float32(M, N, K, ta, tb, split):
     assert torch.equal(Cb.cpu(), C.cpu().to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K", [(8, 8, 8), (72, 40, 104), (64, 128, 32), (136, 64, 40), (65, 33, 31), (64, 64, 65)])
+def test_gemm_wide_loads_equal_the_general_path(M, N, K, ta, tb):
+    """Operands on 16 bytes (wide loads where the strides allow them) and the
+    same operands 2 bytes off (the general path) give the same bits."""
+    g = torch.Generator().manual_seed(M + N + K)
+    out = []
+    a = torch.randn(M * K, generator=g).to(torch.bfloat16).to(DEV)
+    b = torch.randn(K * N, generator=g).to(torch.bfloat16).to(DEV)
+    sam, sak = (1, M) if ta else (K, 1)
+    sbk, sbn = (1, K) if tb else (N, 1)
+    for off in (0, 1):
+        A, B = (torch.cat([x.new_zeros(off), x])[off:] for x in (a, b))
+        assert (A.data_ptr() % 16 == 0) == (off == 0)
+        C = torch.zeros((M, N), device=DEV)
+        cnn.gemm(A, sam, sak, B, sbk, sbn, C, M, N, K)
+        out.append(C)
+    assert torch.equal(out[0], out[1])
+
+
 @pytest.mark.parametrize("M,N,masked,off", [(1, 8, False, 0), (257, 8, True, 0), (1000, 32, True, 0), (4099, 64, False, 0),
                                             (2050, 128, True, 0), (1000, 32, True, 1), (77, 12, True, 0), (300, 37, False, 0),
                                             (5, 1028, True, 0)])
