@@ -49,20 +49,32 @@ __global__ __launch_bounds__(256) void chi2_partial_kernel(const float* __restri
   if (threadIdx.x == 0) partial[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
 
-// out[k] = sum_b partial[b * stride + k] for k < n
-__global__ __launch_bounds__(256) void sum_partials_kernel(const double* partial, int nblocks,
+// out[k] = sum_b partial[b * stride + k] for k < n, one wave an output: 64
+// partials in flight a step and the lanes' sums folded in a fixed order.  A
+// thread an output read its up to 512 partials one after another: 81 us each
+// for chi2 and rpp, now 4.7 us.
+__device__ __forceinline__ double partial_sum(const double* __restrict__ partial, int nblocks, int stride, int k) {
+  double t = 0.0;
+  for (int b = threadIdx.x & 63; b < nblocks; b += 64) t += partial[(int64_t)b * stride + k];
+  return wave_sum(t);
+}
+
+__global__ __launch_bounds__(256) void sum_partials_kernel(const double* __restrict__ partial, int nblocks,
                                                            int stride, int n, double* out,
                                                            double scale) {
-  for (int k = threadIdx.x; k < n; k += 256) {
-    double t = 0.0;
-    for (int b = 0; b < nblocks; ++b) t += partial[(int64_t)b * stride + k];
-    out[k] = t * scale;
-  }
+  const int k = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+  if (k >= n) return;
+  const double t = partial_sum(partial, nblocks, stride, k);
+  if ((threadIdx.x & 63) == 0) out[k] = t * scale;
 }
 
 // J^T W J and J^T W (Y - m): one 16x16x4 MFMA per 4 pixels per wavefront.
 // Lane l holds parameter r = l % 16 of pixel base + l / 16:
 //   A[r][k] = J[p_k][r], B[k][c] = W_p J[p_k][c], D[4(l/16)+i][l%16] (reg i).
+// Bound by HBM (J, model, data and weight read once).  A wave has the loads of
+// kStep steps in flight: with one step's it waited out a memory round trip
+// every 4 pixels, 308 us for 2048^2 x 13 (268 MB), 102 us now.
+constexpr int kStep = 8;  // divides 64, the steps between two flushes
 __global__ __launch_bounds__(256) void normal_eq_kernel(const float* __restrict__ J,
                                                         const float* __restrict__ model,
                                                         const float* __restrict__ data,
@@ -80,17 +92,35 @@ __global__ __launch_bounds__(256) void normal_eq_kernel(const float* __restrict_
   double gacc = 0.0;
   float gpart = 0.0f;
   int since = 0;
-  for (int64_t base = gwave * 4; base < npix; base += nwave * 4) {
-    const int64_t p = base + k;
-    float a = 0.0f, w = 0.0f, res = 0.0f;
-    if (p < npix && r < np && !(mask && mask[p])) {
-      a = J[p * np + r];
-      w = weight ? weight[p] : 1.0f;
-      res = data[p] - model[p];
+  for (int64_t base = gwave * 4; base < npix; base += kStep * nwave * 4) {
+    // the loads of kStep steps (unconditional, at pixel 0 and column 0 where
+    // there is nothing to read, so that none waits for another), then their
+    // products in step order; what is not kept is zero and adds nothing
+    float a[kStep], w[kStep], res[kStep], y[kStep], m[kStep];
+    uint8_t drop[kStep];
+#pragma unroll
+    for (int u = 0; u < kStep; ++u) {
+      const int64_t p = base + u * nwave * 4 + k, q = p < npix ? p : 0;
+      drop[u] = mask ? mask[q] : (uint8_t)0;
+      a[u] = J[q * np + (r < np ? r : 0)];
+      w[u] = weight ? weight[q] : 1.0f;
+      y[u] = data[q];
+      m[u] = model[q];
     }
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a, w * a, acc, 0, 0, 0);
-    gpart = fmaf(a * w, res, gpart);
-    if (++since == 64) {
+#pragma unroll
+    for (int u = 0; u < kStep; ++u) {
+      const bool keep = base + u * nwave * 4 + k < npix && r < np && !drop[u];
+      a[u] = keep ? a[u] : 0.0f;
+      w[u] = keep ? w[u] : 0.0f;
+      res[u] = keep ? y[u] - m[u] : 0.0f;
+    }
+#pragma unroll
+    for (int u = 0; u < kStep; ++u) {
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], w[u] * a[u], acc, 0, 0, 0);
+      gpart = fmaf(a[u] * w[u], res[u], gpart);
+    }
+    since += kStep;
+    if (since == 64) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         accd[i] += (double)acc[i];
@@ -120,14 +150,15 @@ __global__ __launch_bounds__(256) void normal_eq_kernel(const float* __restrict_
                              redg[3][threadIdx.x];
 }
 
-// unpack 16x16 padded partial sums into np x np hess and np grad
-__global__ __launch_bounds__(256) void normal_eq_final_kernel(const double* partial, int nblocks,
+// unpack 16x16 padded partial sums into np x np hess and np grad (one wave an
+// entry, as sum_partials_kernel; 125 us with a thread an entry, 4.8 us now)
+__global__ __launch_bounds__(256) void normal_eq_final_kernel(const double* __restrict__ partial, int nblocks,
                                                               int np, double* hess, double* grad) {
   const int stride = kMaxNp * kMaxNp + kMaxNp;
-  for (int e = threadIdx.x; e < np * np + np; e += 256) {
-    const int src = e < np * np ? (e / np) * kMaxNp + (e % np) : 256 + (e - np * np);
-    double t = 0.0;
-    for (int b = 0; b < nblocks; ++b) t += partial[(int64_t)b * stride + src];
+  const int e = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+  if (e >= np * np + np) return;
+  const double t = partial_sum(partial, nblocks, stride, e < np * np ? (e / np) * kMaxNp + (e % np) : 256 + (e - np * np));
+  if ((threadIdx.x & 63) == 0) {
     if (e < np * np)
       hess[e] = t;
     else
@@ -135,6 +166,11 @@ __global__ __launch_bounds__(256) void normal_eq_final_kernel(const double* part
   }
 }
 
+// One pixel a thread, 256 pixels a workgroup step.  Their rows of J are one
+// contiguous run: it is read coalesced, a float a thread at a time, and passed
+// through LDS, and the next step's run is requested before this one's sums.
+// Bound by HBM.  Each thread reading its own row (13 floats, 52 bytes apart
+// from its neighbour's) took 116 us for 2048^2 x 13, this 86 us.
 __global__ __launch_bounds__(256) void rpp_kernel(const float* __restrict__ J,
                                                   const float* __restrict__ m0,
                                                   const float* __restrict__ m1,
@@ -142,21 +178,39 @@ __global__ __launch_bounds__(256) void rpp_kernel(const float* __restrict__ J,
                                                   const uint8_t* __restrict__ mask, int64_t npix,
                                                   int np, const double* __restrict__ h, double d,
                                                   double* partial) {
+  __shared__ float rows[256 * kMaxNp];
   __shared__ double red[4][kMaxNp];
+  const int t = threadIdx.x;
   double hv[kMaxNp], acc[kMaxNp];
 #pragma unroll
   for (int r = 0; r < kMaxNp; ++r) {
     hv[r] = r < np ? h[r] : 0.0;
     acc[r] = 0.0;
   }
-  for (int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x; p < npix;
-       p += (int64_t)gridDim.x * 256) {
-    if (mask && mask[p]) continue;
+  const int64_t step = (int64_t)gridDim.x * 256, total = npix * np;
+  float next[kMaxNp];  // floats t, t + 256, ... of the step's run
+  auto request = [&](int64_t base) {
+#pragma unroll
+    for (int r = 0; r < kMaxNp; ++r) {
+      const int64_t e = base * np + r * 256 + t;
+      next[r] = (r < np && e < total) ? J[e] : 0.0f;
+    }
+  };
+  request((int64_t)blockIdx.x * 256);
+  for (int64_t base = (int64_t)blockIdx.x * 256; base < npix; base += step) {
+    __syncthreads();  // the previous step's rows are read
+#pragma unroll
+    for (int r = 0; r < kMaxNp; ++r)
+      if (r < np) rows[r * 256 + t] = next[r];
+    __syncthreads();
+    if (base + step < npix) request(base + step);
+    const int64_t p = base + t;
+    if (p >= npix || (mask && mask[p])) continue;
     float jr[kMaxNp];
     double jh = 0.0;
 #pragma unroll
     for (int r = 0; r < kMaxNp; ++r) {
-      jr[r] = r < np ? J[p * np + r] : 0.0f;
+      jr[r] = r < np ? rows[t * np + r] : 0.0f;
       jh += (double)jr[r] * hv[r];
     }
     const double w = weight ? (double)weight[p] : 1.0;
@@ -167,8 +221,8 @@ __global__ __launch_bounds__(256) void rpp_kernel(const float* __restrict__ J,
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
 #pragma unroll
   for (int r = 0; r < kMaxNp; ++r) {
-    const double t = wave_sum(acc[r]);
-    if (lane == 0) red[wv][r] = t;
+    const double s = wave_sum(acc[r]);
+    if (lane == 0) red[wv][r] = s;
   }
   __syncthreads();
   if (threadIdx.x < kMaxNp)
@@ -249,7 +303,7 @@ int normal_equations(const float* J, const float* model, const float* data, cons
   double* partial = static_cast<double*>(ws);
   hipLaunchKernelGGL(normal_eq_kernel, dim3(nb), dim3(256), 0, stream, J, model, data, weight,
                      mask, npix, np, partial);
-  hipLaunchKernelGGL(normal_eq_final_kernel, dim3(1), dim3(256), 0, stream, partial, nb, np, hess,
+  hipLaunchKernelGGL(normal_eq_final_kernel, dim3((np * np + np + 3) / 4), dim3(256), 0, stream, partial, nb, np, hess,
                      grad);
   return check_launch("normal_equations");
 }
@@ -265,7 +319,7 @@ int rpp(const float* J, const float* m0, const float* m1, const float* weight, c
   double* partial = static_cast<double*>(ws);
   hipLaunchKernelGGL(rpp_kernel, dim3(nb), dim3(256), 0, stream, J, m0, m1, weight, mask, npix, np,
                      h, d, partial);
-  hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(256), 0, stream, partial, nb, kMaxNp, np,
+  hipLaunchKernelGGL(sum_partials_kernel, dim3((np + 3) / 4), dim3(256), 0, stream, partial, nb, kMaxNp, np,
                      out, 1.0);
   return check_launch("rpp");
 }
@@ -290,7 +344,7 @@ int normal_equations_noalloc(const float* J, const float* model, const float* da
   // every workgroup overwrites its whole partial block, so nothing is cleared
   hipLaunchKernelGGL(normal_eq_kernel, dim3(nb), dim3(256), 0, stream, J, model, data, weight,
                      mask, npix, np, partial);
-  hipLaunchKernelGGL(normal_eq_final_kernel, dim3(1), dim3(256), 0, stream, partial, nb, np, hess,
+  hipLaunchKernelGGL(normal_eq_final_kernel, dim3((np * np + np + 3) / 4), dim3(256), 0, stream, partial, nb, np, hess,
                      grad);
   return check_launch("normal_equations_noalloc");
 }

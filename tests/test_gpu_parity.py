@@ -287,6 +287,61 @@ def test_lm_solve_matches_reference_formula():
         assert torch.allclose(h.cpu(), ref, rtol=1e-9, atol=1e-12)
 
 
+@pytest.mark.parametrize("npar", [1, 2, 13, 15, 16, 17, 64])
+def test_lm_solve_sizes_and_bad_pivots(npar):
+    """The one-wave solve (up to 16) and the workgroup one at the edges of
+    their ranges; with an indefinite matrix both report the first bad pivot and
+    solve by elimination.  1e-9 relative: condition below 1e5, float64."""
+    lib = ap._lib.load()
+    g = torch.Generator().manual_seed(npar)
+    A = torch.randn(4 * npar + 8, npar, dtype=torch.float64, generator=g)
+    grad = torch.randn(npar, dtype=torch.float64, generator=g)
+    for bad in (None, npar // 2):
+        hess = A.T @ A
+        if bad is not None:
+            hess[bad, bad] = -50.0
+        h = torch.empty(npar, dtype=torch.float64, device="cuda")
+        st = torch.full((1,), 7, dtype=torch.int32, device="cuda")
+        hd, gd = hess.cuda(), grad.cuda()
+        ap._lib.check(lib.apx_lm_solve(hd.data_ptr(), gd.data_ptr(), npar, 0.5, h.data_ptr(), st.data_ptr(), ap._lib.stream()))
+        ref = H.lm_damped_solve(0.5, grad, hess)
+        assert st.item() == (0 if bad is None else bad + 1)
+        assert float((h.cpu() - ref).norm() / ref.norm()) < 1e-9
+
+
+@pytest.mark.parametrize("npix,npar", [(1, 1), (3, 16), (255, 13), (1023, 7), (4097, 16), (70001, 5), (600000, 13)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_lm_products_sizes(npix, npar, masked):
+    """chi^2, the normal equations and rpp at ragged sizes, from one pixel to
+    more than one step of every workgroup.  float64 sums of float64 products
+    (chi^2, rpp): 1e-11; J^T W J sums at most 256 float32 products in a chain:
+    1e-5 of the largest entry, as test_chi2_and_normal_equations."""
+    lib = ap._lib.load()
+    g = torch.Generator(device="cuda").manual_seed(npix + npar)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    J, m, y, m1 = rnd(npix, npar), rnd(npix), rnd(npix), rnd(npix)
+    w = torch.rand(npix, generator=g, device="cuda") + 0.1
+    mask = (rnd(npix) > 1).to(torch.uint8) if masked else None
+    keep = torch.ones(npix, device="cuda", dtype=torch.float64) if mask is None else (mask == 0).double()
+    wsb = lib.apx_reduce_workspace_bytes(npix, npar)
+    ws = torch.empty(wsb, dtype=torch.uint8, device="cuda")
+    chi2, hess, grad, rpp = (torch.empty(s, dtype=torch.float64, device="cuda") for s in ((1,), (npar, npar), (npar,), (npar,)))
+    h = rnd(npar).double()
+    p, st = ap._lib.ptr, ap._lib.stream()
+    ap._lib.check(lib.apx_chi2(p(m), p(y), p(w), p(mask), npix, p(chi2), p(ws), wsb, st))
+    ap._lib.check(lib.apx_normal_equations(p(J), p(m), p(y), p(w), p(mask), npix, npar, p(hess), p(grad), p(ws), wsb, st))
+    ap._lib.check(lib.apx_rpp(p(J), p(m), p(m1), p(w), p(mask), npix, npar, p(h), 0.1, p(rpp), p(ws), wsb, st))
+    Jd, wd = J.double(), w.double() * keep
+    r = y.double() - m.double()
+    ref = (wd * r * r).sum()
+    assert abs(float(chi2 - ref)) <= 1e-11 * float(ref) + 1e-300
+    Href, gref = Jd.T @ (wd[:, None] * Jd), Jd.T @ (wd * r)
+    v = 20.0 * (wd * (m1 - m).double() / 0.1 - wd * (Jd @ h))
+    assert float((hess - Href).abs().max()) <= 1e-5 * float(Href.abs().max())
+    assert float((grad - gref).abs().max()) <= 1e-5 * float((Jd.abs().T @ (wd * r.abs())).max())
+    assert float((rpp - Jd.T @ v).abs().max()) <= 1e-11 * float((Jd.abs().T @ v.abs()).max())
+
+
 @pytest.mark.parametrize("kind", ["sersic", "exponential", "gaussian", "moffat", "flat_sky"])
 @pytest.mark.parametrize("psf_mode", ["none", "full"])
 def test_adjoint_vjp(kind, psf_mode):
