@@ -45,7 +45,7 @@ constexpr int kConvChan = kNChan - 1;
 constexpr int kTR = 16;      // output rows of a batch tile (64 x kTR pixels)
 // separable-convolution tap vectors are zero-padded to a multiple of 4 taps
 __host__ __device__ inline int sp_k4(int k) { return (k + 3) & ~3; }
-constexpr int kMfmaMax = kMfmaWide;  // widest kernel the MFMA convolution takes (67, up to 128 KiB LDS)
+constexpr int kMfmaMax = kMfmaWide;  // widest kernel the MFMA convolution takes (67, up to 73 KiB LDS)
 
 enum : int32_t { PH_INIT = 0, PH_NEEDJ = 1, PH_SUB = 2, PH_DONE = 3 };
 enum : int32_t { ST_JAC = 0, ST_PROBE = 1, ST_TRIAL = 2, ST_ALL = 3, ST_ALL_JAC = 4 };
@@ -1224,6 +1224,8 @@ __host__ __device__ inline int conv_stage_floats(int kmax) {
 }
 __host__ inline size_t conv_lds_bytes(int kmax) { return sizeof(float) * (size_t)conv_stage_floats(kmax); }
 constexpr size_t kConvStaticLds = sizeof(double) * 4 * 8;
+// MFMA passes a tile: 3 kernels of the value plane and the partial planes, or the value alone
+__host__ __device__ constexpr int mfma_passes(bool jac) { return jac ? kConvChan + 2 : 1; }
 
 // The probe (rpp) and trial (chi2) epilogues of one output pixel, summed into
 // rd[] in float64 (lm.py:276-292)
@@ -1439,43 +1441,42 @@ __global__ __launch_bounds__(256) void conv_kernel(apx_batch b, Scratch s, float
 // ---------------------------------------------------------------------------
 // MFMA convolution (kernels up to kMfmaMax): the Toeplitz formulation of
 // conv_common.h (mfma_columns), one 16 x 16 output block per wave of the
-// 64 x kTR tile.
+// 64 x kTR tile.  A work item is one (tile, plane, kernel) pass: its LDS is one
+// staged plane and one tap table, so at least two workgroups share a CU and one
+// loads while the other multiplies.  Both arrive by stage_rows.  Bound by the
+// FP32 matrix pipe.  With a tile's 7 passes in one workgroup (three tap tables:
+// one workgroup a CU for 67-px kernels) and rows copied through registers one
+// wait at a time, 125 sources on 1024 x 1024 took 5.83 ms; so @@ ms.
 template <int MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void conv_mfma_kernel(apx_batch b, Scratch s, float* out) {
   extern __shared__ float smem[];
   __shared__ double redd[4][8];  // kConvStaticLds
   constexpr bool JAC = MODE == EPI_NORMAL;
-  constexpr int nchan = JAC ? kConvChan : 1;
-  constexpr int nkt = JAC ? 3 : 1;
   constexpr int W = MODE == EPI_RPP ? NP : 1;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int lm = lane & 15, lk = lane >> 4;
-  for (int base = 0; base < s.cnt[2]; base += gridDim.x) {
-    const int k = xcd_tile(base, s.cnt[2]);
-    if (k < 0) continue;
-    const int2 e = s.tile_list[k];
+  const int total = s.cnt[2] * mfma_passes(JAC);
+  for (int base = 0; base < total; base += gridDim.x) {
+    const int item = xcd_tile(base, total);
+    if (item < 0) continue;
+    // passes 0 .. 2: the value plane with K, dK/dcx, dK/dcy; 3 ..: a partial plane with K
+    const int pass = item % mfma_passes(JAC), c = pass < 3 ? 0 : pass - 2, kk = pass < 3 ? pass : 0;
+    const int2 e = s.tile_list[item / mfma_passes(JAC)];
     const int g = __builtin_amdgcn_readfirstlane(e.x);
     const apx_batch_galaxy G = b.gal[g];
     const GalState* st = st_of(b, g);
-    const float ie_scale = JAC ? (float)(kLn10 * s.ev[g].dvdr[NP - 1]) : 0.0f;
     const int nxw = G.nx + G.pw + 1, nyw = G.ny + G.ph + 1;  // cutout + 2 * border
     const int ntx = (G.nx + 63) / 64;
     const int ox0 = (e.y % ntx) * 64, oy0 = (e.y / ntx) * kTR;
     const int kh = G.ph + 2, kw = G.pw + 2;
     const int nks = mf_nks(kh), LW = mf_lw(kw), DD = mf_dd(kh), kts = fast_kts(kh);
     const int rows = mf_rows(kh), cols = 64 + kw - 1;
-    const int64_t tile = G.tile_off + e.y;
     float* tin = smem;             // rows x LW
-    float* tab = smem + rows * LW; // [kk][kx][dd]
-    const float* kt = b.taps + G.tap_off;
-    __syncthreads();  // the previous tile's readers are done with LDS
-    for (int r = w; r < nkt * kw; r += 4) {  // tap-table row (kk, kx) per wave, dd across lanes
-      const float* src = kt + (int64_t)r * kts + 7;  // KT[kk][kx][u] = Kf[u - 7][kx]
-      for (int dd = lane; dd < DD; dd += 64) {
-        const int a = dd - 15;  // Kf row
-        tab[r * DD + dd] = (a >= 0 && a < kh) ? src[a] : 0.0f;
-      }
-    }
+    float* tab = smem + rows * LW; // [kx][dd]
+    __syncthreads();  // the previous item's readers are done with LDS
+    stage_rows(b.planes + (int64_t)c * b.nwork + G.work_off, nxw, nxw, nyw, ox0, oy0, rows, cols, tin, LW);
+    // tap-table row kx: dd -> Kf[dd - 15][kx] = KT[kk][kx][dd - 8], zero outside KT's row
+    stage_rows(b.taps + G.tap_off + (int64_t)kk * kw * kts, kts, kts, kw, -8, 0, kw, DD, tab, DD);
     // this lane's 4 output pixels: x = 16 w + 4 lk + i, row lm
     const int oy = oy0 + lm;
     bool valid[4];
@@ -1489,40 +1490,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
     double rd[W];
 #pragma unroll
     for (int i = 0; i < W; ++i) rd[i] = 0.0;
-    for (int c = 0; c < nchan; ++c) {
-      const float* plane = b.planes + (int64_t)c * b.nwork + G.work_off;
-      __syncthreads();
-      for (int q = threadIdx.x; q < rows * cols; q += 256) {
-        const int t = q / cols, u = q % cols;
-        const int gy = oy0 + t, gx = ox0 + u;
-        tin[t * LW + u] = (gy < nyw && gx < nxw) ? plane[(int64_t)gy * nxw + gx] : 0.0f;
-      }
-      __syncthreads();
-      const int nk = (JAC && c == 0) ? 3 : 1;
-      for (int kk = 0; kk < nk; ++kk) {
-        const float* ta = tin + lk * LW + 16 * w + lm;
-        const float* tb = tab + kk * kw * DD + lk - lm + 15;
-        const v4f acc = mfma_block(nks, ta, tb, kw, LW, DD);
-        const int col = c == 0 ? kk - 1 : c + 1;  // J column, -1 for the value
+    __builtin_amdgcn_s_waitcnt(0);  // this wave's rows have landed in LDS
+    __syncthreads();
+    const v4f acc = mfma_block(nks, tin + lk * LW + 16 * w + lm, tab + lk - lm + 15, kw, LW, DD);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (!valid[i]) continue;
-          if (JAC) {
-            if (col < 0) {
-              out[pp[i]] = acc[i];
-              b.jac[(int64_t)(NP - 1) * b.npix + pp[i]] = ie_scale * acc[i];
-            } else {
-              b.jac[(int64_t)col * b.npix + pp[i]] = acc[i];
-            }
-          } else if (MODE == EPI_OUT) {
-            out[pp[i]] = acc[i];
-          } else {
-            epilogue_pixel<MODE>(b, st, pp[i], acc[i], rd);
-          }
+    for (int i = 0; i < 4; ++i) {
+      if (!valid[i]) continue;
+      if (JAC) {
+        const int col = c == 0 ? kk - 1 : c + 1;  // J column, -1 for the value
+        if (col < 0) {
+          out[pp[i]] = acc[i];
+          b.jac[(int64_t)(NP - 1) * b.npix + pp[i]] = (float)(kLn10 * s.ev[g].dvdr[NP - 1]) * acc[i];
+        } else {
+          b.jac[(int64_t)col * b.npix + pp[i]] = acc[i];
         }
+      } else if (MODE == EPI_OUT) {
+        out[pp[i]] = acc[i];
+      } else {
+        epilogue_pixel<MODE>(b, st, pp[i], acc[i], rd);
       }
     }
-    if (MODE == EPI_RPP || MODE == EPI_CHI2) tile_partial<W>(redd, rd, s.part + tile * kPart, lane, w);
+    if (MODE == EPI_RPP || MODE == EPI_CHI2) tile_partial<W>(redd, rd, s.part + (G.tile_off + e.y) * kPart, lane, w);
   }
 }
 
@@ -1553,10 +1541,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
 // Staged columns past the plane's width hold the next row's values (or 0 past
 // the plane's end): they reach only outputs past the cutout's width.
 typedef const __attribute__((address_space(4))) float* ctaps;
-typedef __attribute__((address_space(3))) void* lds_ptr;
 
 constexpr int kSepMax = 61;  // widest kernel the separable convolution takes (LDS)
-constexpr int kBufWord3 = 0x00020000;  // buffer resource word 3 on gfx9: 32-bit data
 __host__ __device__ inline int sp_pitch(int cols) { return cols + ((1 - cols) & 3); }  // >= cols, 1 mod 4
 // staged-row pitch for kernels up to kmax columns: 64 + kw4 - 1 columns fit
 __host__ inline int sp_stage_pitch(int kmax) { return 63 + sp_k4(kmax) <= 96 ? 96 : 128; }
@@ -2472,9 +2458,10 @@ void conv_part(const apx_batch& b, const Scratch& s, int mode, float* out, hipSt
   const bool sep = b.conv_impl == 3;
   const bool mf = !sep && b.conv_impl != 1 && b.max_kernel <= kMfmaMax;
   const size_t lds = sep  ? sep_lds_bytes(b.max_kernel, mode == EPI_NORMAL)
-                     : mf ? mfma_lds_bytes(b.max_kernel, mode == EPI_NORMAL ? 3 : 1)
+                     : mf ? mfma_lds_bytes(b.max_kernel)
                           : conv_lds_bytes(b.max_kernel);
-  const int tc = (int)std::min<int64_t>(b.ntile, b.conv_blocks > 0 ? b.conv_blocks : 2 * kPersist);
+  const int64_t items = b.ntile * (mf ? mfma_passes(mode == EPI_NORMAL) : 1);
+  const int tc = (int)std::min<int64_t>(items, b.conv_blocks > 0 ? b.conv_blocks : 2 * kPersist);
 #define APX_CONV(M)                                                                                \
   do {                                                                                             \
     if (sep) {                                                                                     \
@@ -2558,9 +2545,9 @@ int batch_plan(apx_batch_galaxy* gal, int32_t ngal, apx_batch* b) {
     kmax = std::max(kmax, std::max(G.ph, G.pw) + 2);
   }
   // the VALU convolution is every batch's fallback and must fit 64 KiB; the MFMA
-  // one (kmax <= kMfmaMax) takes up to 128 KiB of the 160 KiB a workgroup has
+  // one (kmax <= kMfmaMax) takes up to 73 KiB of the 160 KiB a workgroup has
   if (conv_lds_bytes(kmax) + kConvStaticLds > 65536 ||
-      (kmax <= kMfmaMax && mfma_lds_bytes(kmax, 3) + kConvStaticLds > 160 * 1024))
+      (kmax <= kMfmaMax && mfma_lds_bytes(kmax) + kConvStaticLds > 160 * 1024))
     return set_error(APX_E_LIMIT, "batch_plan: psf too large for the batched Jacobian convolution");
   if (work > (int64_t)INT32_MAX || chunk > (int64_t)INT32_MAX || tile > (int64_t)INT32_MAX)
     return set_error(APX_E_LIMIT, "batch_plan: batch too large");

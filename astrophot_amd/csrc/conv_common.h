@@ -73,6 +73,34 @@ __device__ __forceinline__ void conv_accumulate(const float* smem, int LW, int l
 
 
 // ---------------------------------------------------------------------------
+// Rows from HBM straight into LDS: row t of dst (rows x cols, pitch dpitch) gets
+// src[(gy0 + t) * pitch + gx0 ..], zero where that lies outside nx x ny.  The
+// workgroup's waves take the rows in turn, 64 floats a load, through a buffer
+// resource of one source row: its range check gives the zeros (a column before
+// the row is a huge unsigned offset, a row outside has an empty resource), so no
+// register holds the data, nothing is divided and every load of the tile is in
+// flight at once.  Completion: vmcnt, then a barrier.
+typedef __attribute__((address_space(3))) void* lds_ptr;
+constexpr int kBufWord3 = 0x00020000;  // buffer resource word 3 on gfx9: 32-bit data
+
+__device__ __forceinline__ void stage_rows(const float* src, int64_t pitch, int nx, int ny, int gx0, int gy0, int rows,
+                                           int cols, float* dst, int dpitch) {
+  const int lane = threadIdx.x & 63;
+  for (int t = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); t < rows; t += 4) {
+    const int gy = gy0 + t;
+    const bool in = gy >= 0 && gy < ny;
+    // every field of the resource is uniform: read from lane 0 so that it stays in SGPRs
+    const uint64_t a = (uint64_t)(src + (int64_t)(in ? gy : 0) * pitch);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+        reinterpret_cast<void*>(((uint64_t)hi << 32) | lo), (short)0, __builtin_amdgcn_readfirstlane(in ? nx * 4 : 0), kBufWord3);
+    for (int c = 0; c < cols; c += 64)
+      if (c + lane < cols)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr)(dst + t * dpitch + c), 4, (gx0 + c + lane) * 4, 0, 0, 0);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // MFMA convolution by v_mfma_f32_16x16x4f32.  A wave computes a 16 x 16
 // output block (16 columns x, kMfR rows r) as
 //   out[r][x] = sum_kx sum_j A_kx[x][j] B_kx[j][r],
@@ -94,9 +122,11 @@ __host__ __device__ inline int mf_rows(int kh) { return 4 * mf_nks(kh); }
 // of an A operand (lanes l / 16, l % 16) fall in distinct LDS banks
 __host__ __device__ inline int mf_lw(int kw) { return 16 + 32 * ((64 + kw - 1 - 16 + 31) / 32); }
 __host__ __device__ inline int mf_dd(int kh) { return mf_rows(kh) + 15; }
-__host__ inline size_t mfma_lds_bytes(int kmax, int nk) {
-  return sizeof(float) * ((size_t)mf_rows(kmax) * mf_lw(kmax) + (size_t)nk * kmax * mf_dd(kmax));
+// LDS of one pass: the staged input and one tap table
+__host__ inline size_t mfma_lds_bytes(int kh, int kw) {
+  return sizeof(float) * ((size_t)mf_rows(kh) * mf_lw(kw) + (size_t)kw * mf_dd(kh));
 }
+__host__ inline size_t mfma_lds_bytes(int kmax) { return mfma_lds_bytes(kmax, kmax); }
 
 // All kernel columns of one output block: column kx needs NKS k-steps; the
 // operands of the next column are loaded while the MFMAs of the current one

@@ -31,7 +31,6 @@ constexpr int kTX = 64;   // output tile width = one wavefront
 constexpr int kRY = 4;    // outputs per thread (vertical)
 constexpr int kTY = 16;   // output tile height (4 waves x kRY)
 constexpr int kKR = 32;   // kernel rows staged per pass
-constexpr size_t kMaxLds = 160 * 1024;  // LDS a gfx950 workgroup may use
 
 __device__ __forceinline__ double block_sum256(double v, double* red) {
 #pragma unroll
@@ -294,67 +293,68 @@ __global__ __launch_bounds__(256) void convolve_fast_kernel(apx_conv_job job,
 
 // MFMA convolution of one job (kernels of kMfmaMin .. kMfmaWide rows): a
 // 64 x kMfR output tile per workgroup, each wave one 16 x 16 block
-// (mfma_block, conv_common.h).  The tap table of every kernel of the job is
-// built in LDS once per workgroup; per render plane the input tile is staged
-// and each of its kernels accumulated; outputs are added into the image or the
-// Jacobian column as convolve_fast_kernel does.
+// (mfma_block, conv_common.h).  A workgroup does one pass, one render plane
+// with one kernel: its staged rows (stage_rows) and its tap table leave room for
+// a second workgroup on the CU, which multiplies while this one loads, and a
+// small image's passes spread over the CUs instead of following one another.
+// The tiles of a pass are padded to a multiple of 8, so that every pass of a
+// tile, which adds to the same lines of the Jacobian, lands on one XCD (they
+// take the workgroups round robin).  Bound by the FP32 matrix pipe.  With all
+// passes of a tile in one workgroup, rows copied through registers a load at a
+// time, 512^2 with 53 x 53 kernels took 41 us (value) and 244 us (Jacobian of 7
+// columns); so @@ and @@ us.
 constexpr int kMfmaMin = 21;  // shorter kernels waste over half of each MFMA on the band's zeros
+constexpr int kMaxPass = APX_MAX_CHAN + 2;
 
-__host__ inline size_t conv_mfma_lds_bytes(int kh, int kw, int nk) {
-  return sizeof(float) * ((size_t)mf_rows(kh) * mf_lw(kw) + (size_t)nk * kw * mf_dd(kh));
-}
+struct ConvPasses {
+  int n;
+  int8_t plane[kMaxPass], kernel[kMaxPass];
+};
 
-template <int NK0>
 __global__ __launch_bounds__(256) void convolve_mfma_kernel(apx_conv_job job, const float* __restrict__ planes,
-                                                            const float* __restrict__ kernels) {
+                                                            const float* __restrict__ kernels, ConvPasses passes,
+                                                            int ntx, int ntile) {
   extern __shared__ float smem[];
+  const int padded = (ntile + 7) & ~7;
+  const int pass = blockIdx.x / padded, tile = blockIdx.x - pass * padded;
+  if (tile >= ntile) return;
+  const int c = passes.plane[pass], k = passes.kernel[pass];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int lm = lane & 15, lk = lane >> 4;
-  const int ox0 = blockIdx.x * 64, oy0 = blockIdx.y * kMfR;
+  const int ox0 = (tile % ntx) * 64, oy0 = (tile / ntx) * kMfR;
   const int kh = job.kh, kw = job.kw, ch = (kh - 1) / 2, cw = (kw - 1) / 2;
-  const int nks = mf_nks(kh), rows = mf_rows(kh), LW = mf_lw(kw), DD = mf_dd(kh);
-  const int cols = 64 + kw - 1;
-  const int gx0 = job.x0 + ox0 - cw, gy0 = job.y0 + oy0 - ch;
-  const int64_t npl = (int64_t)job.nx * job.ny;
+  const int rows = mf_rows(kh), LW = mf_lw(kw), DD = mf_dd(kh);
   float* tin = smem;             // rows x LW
-  float* tab = smem + rows * LW; // [k][kx][dd] = Kf_k[dd - 15][kx]
-  for (int e = threadIdx.x; e < NK0 * kw * DD; e += 256) {
-    const int dd = e % DD, kx = (e / DD) % kw, k = e / (DD * kw);
-    const int a = dd - 15;
-    tab[e] = (a >= 0 && a < kh) ? kernels[((int64_t)k * kh + a) * kw + kx] : 0.0f;
+  float* tab = smem + rows * LW; // [kx][dd] = Kf[dd - 15][kx]
+  stage_rows(planes + (int64_t)c * job.nx * job.ny, job.nx, job.nx, job.ny, job.x0 + ox0 - cw, job.y0 + oy0 - ch, rows,
+             64 + kw - 1, tin, LW);
+  // the tap table: kernel rows read coalesced, stored DD (odd) apart; its first
+  // 15 and last columns stay zero
+  const float* K = kernels + (int64_t)k * kh * kw;
+  for (int kx = lane; kx < kw; kx += 64) {
+#pragma unroll 6
+    for (int a = w; a < kh; a += 4) tab[kx * DD + 15 + a] = K[a * kw + kx];
+    for (int dd = w; dd < DD; dd += 4)
+      if (dd < 15 || dd >= 15 + kh) tab[kx * DD + dd] = 0.0f;
   }
+  __builtin_amdgcn_s_waitcnt(0);  // this wave's rows have landed in LDS
+  __syncthreads();
+  const v4f acc = mfma_block(mf_nks(kh), tin + lk * LW + 16 * w + lm, tab + lk - lm + 15, kw, LW, DD);
   // this lane's 4 outputs: x = 16 w + 4 lk + i, row lm
-  const int oy = oy0 + lm;
-  const int c_first = (job.img || NK0 > 1) ? 0 : 1;
-  for (int c = c_first; c < job.nchan; ++c) {
-    const float* plane = planes + c * npl;
-    __syncthreads();
-    for (int e = threadIdx.x; e < rows * cols; e += 256) {
-      const int t = e / cols, u = e - t * cols;
-      const int gy = gy0 + t, gx = gx0 + u;
-      tin[t * LW + u] = (gy >= 0 && gy < job.ny && gx >= 0 && gx < job.nx) ? plane[(int64_t)gy * job.nx + gx]
-                                                                          : 0.0f;
-    }
-    __syncthreads();
-    const int nk = (c == 0) ? NK0 : 1;
-    for (int k = 0; k < nk; ++k) {
-      const float* ta = tin + lk * LW + 16 * w + lm;
-      const float* tb = tab + k * kw * DD + lk - lm + 15;
-      const v4f acc = mfma_block(nks, ta, tb, kw, LW, DD);
-      if (oy >= job.oh) continue;
+  const int oy = oy0 + lm, ox = ox0 + 16 * w + 4 * lk;
+  if (oy >= job.oh) return;
+  const int n = min(4, job.ow - ox);
+  if (c == 0 && k == 0) {
+    float* d = job.img + (int64_t)(job.img_y0 + oy) * job.img_row + (job.img_x0 + ox);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int ox = ox0 + 16 * w + 4 * lk + i;
-        if (ox >= job.ow) continue;
-        if (c == 0 && k == 0) {
-          if (job.img) job.img[(int64_t)(job.img_y0 + oy) * job.img_row + (job.img_x0 + ox)] += acc[i];
-        } else if (job.jac) {
-          float* d = job.jac + (int64_t)(job.jac_y0 + oy) * job.jac_row + (int64_t)(job.jac_x0 + ox) * job.jac_np;
-          const int col = (c == 0) ? job.dk_col[k - 1] : job.chan_col[c];
-          if (col >= 0) d[col] += acc[i];
-        }
-      }
-    }
+    for (int i = 0; i < 4; ++i)
+      if (i < n) d[i] += acc[i];
+  } else {
+    float* d = job.jac + (int64_t)(job.jac_y0 + oy) * job.jac_row + (int64_t)(job.jac_x0 + ox) * job.jac_np +
+               (c == 0 ? job.dk_col[k - 1] : job.chan_col[c]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (i < n) d[i * job.jac_np] += acc[i];
   }
 }
 
@@ -474,19 +474,33 @@ int convolve(const apx_conv_job* jp, const float* planes, const float* kernels, 
   }
   const int nk0 = dk ? 3 : 1;
   if (job.kh >= kMfmaMin && job.kh <= kMfmaWide && job.kw >= kMfmaMin && job.kw <= kMfmaWide &&
-      conv_mfma_lds_bytes(job.kh, job.kw, nk0) <= kMaxLds) {
-    const size_t lds = conv_mfma_lds_bytes(job.kh, job.kw, nk0);
-    const dim3 grid((unsigned)((job.ow + 63) / 64), (unsigned)((job.oh + kMfR - 1) / kMfR));
-    if (dk) {
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&convolve_mfma_kernel<3>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      hipLaunchKernelGGL(convolve_mfma_kernel<3>, grid, dim3(256), lds, stream, job, planes, kernels);
-    } else {
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&convolve_mfma_kernel<1>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      hipLaunchKernelGGL(convolve_mfma_kernel<1>, grid, dim3(256), lds, stream, job, planes, kernels);
+      job.nx < (1 << 29) /* a row's bytes fit the range check of its buffer resource */) {
+    const size_t lds = mfma_lds_bytes(job.kh, job.kw);
+    ConvPasses ps = {};
+    auto add = [&](int plane, int kernel) {
+      ps.plane[ps.n] = (int8_t)plane;
+      ps.kernel[ps.n++] = (int8_t)kernel;
+    };
+    if (job.img) add(0, 0);
+    for (int k = 0; k < 2; ++k)
+      if (job.dk_col[k] >= 0) add(0, 1 + k);
+    for (int c = 1; c < job.nchan; ++c) add(c, 0);
+    if (ps.n == 0) return APX_OK;
+    // the passes run side by side, so each needs a column of its own
+    bool own = true;
+    auto column = [&](int p) { return ps.plane[p] == 0 ? job.dk_col[ps.kernel[p] - 1] : job.chan_col[ps.plane[p]]; };
+    for (int p = job.img ? 1 : 0; p < ps.n; ++p)
+      for (int q = job.img ? 1 : 0; q < p; ++q) own = own && column(p) != column(q);
+    const int ntx = (job.ow + 63) / 64;
+    const int64_t ntile = (int64_t)ntx * ((job.oh + kMfR - 1) / kMfR), blocks = ((ntile + 7) & ~(int64_t)7) * ps.n;
+    if (own && blocks <= (int64_t)INT32_MAX / 256) {
+      if (lds > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(&convolve_mfma_kernel),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+        return set_error(APX_E_HIP, "convolve: LDS size refused");
+      hipLaunchKernelGGL(convolve_mfma_kernel, dim3((unsigned)blocks), dim3(256), lds, stream, job, planes, kernels, ps, ntx,
+                         (int)ntile);
+      return check_launch("convolve (MFMA)");
     }
-    return check_launch("convolve (MFMA)");
   }
   if (job.kh <= kFastMax && job.kw <= kFastMax) {
     if (!workspace || ws_bytes < convolve_workspace_bytes(job.kh, job.kw))
