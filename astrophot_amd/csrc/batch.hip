@@ -1446,7 +1446,7 @@ __global__ __launch_bounds__(256) void conv_kernel(apx_batch b, Scratch s, float
 // loads while the other multiplies.  Both arrive by stage_rows.  Bound by the
 // FP32 matrix pipe.  With a tile's 7 passes in one workgroup (three tap tables:
 // one workgroup a CU for 67-px kernels) and rows copied through registers one
-// wait at a time, 125 sources on 1024 x 1024 took 5.83 ms; so @@ ms.
+// wait at a time, 125 sources on 1024 x 1024 took 5.83 ms; 2.78 ms so.
 template <int MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void conv_mfma_kernel(apx_batch b, Scratch s, float* out) {
   extern __shared__ float smem[];
@@ -1469,12 +1469,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
     const int ntx = (G.nx + 63) / 64;
     const int ox0 = (e.y % ntx) * 64, oy0 = (e.y / ntx) * kTR;
     const int kh = G.ph + 2, kw = G.pw + 2;
-    const int nks = mf_nks(kh), LW = mf_lw(kw), DD = mf_dd(kh), kts = fast_kts(kh);
+    const int nks = mf_nks(kh), DD = mf_dd(kh), kts = fast_kts(kh);
     const int rows = mf_rows(kh), cols = 64 + kw - 1;
-    float* tin = smem;             // rows x LW
-    float* tab = smem + rows * LW; // [kx][dd]
+    float* tin = smem;             // rows x kMfLW
+    float* tab = smem + rows * kMfLW; // [kx][dd]
     __syncthreads();  // the previous item's readers are done with LDS
-    stage_rows(b.planes + (int64_t)c * b.nwork + G.work_off, nxw, nxw, nyw, ox0, oy0, rows, cols, tin, LW);
+    stage_rows(b.planes + (int64_t)c * b.nwork + G.work_off, nxw, nxw, nyw, ox0, oy0, rows, cols, tin, kMfLW);
     // tap-table row kx: dd -> Kf[dd - 15][kx] = KT[kk][kx][dd - 8], zero outside KT's row
     stage_rows(b.taps + G.tap_off + (int64_t)kk * kw * kts, kts, kts, kw, -8, 0, kw, DD, tab, DD);
     // this lane's 4 output pixels: x = 16 w + 4 lk + i, row lm
@@ -1492,7 +1492,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
     for (int i = 0; i < W; ++i) rd[i] = 0.0;
     __builtin_amdgcn_s_waitcnt(0);  // this wave's rows have landed in LDS
     __syncthreads();
-    const v4f acc = mfma_block(nks, tin + lk * LW + 16 * w + lm, tab + lk - lm + 15, kw, LW, DD);
+    v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (ox0 + 16 * w < G.nx)  // a wave past the cutout's right edge has no output
+      acc = mfma_block(nks, tin + lk * kMfLW + 16 * w + lm, tab + lk - lm + 15, kw, DD);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       if (!valid[i]) continue;

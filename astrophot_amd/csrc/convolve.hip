@@ -302,7 +302,8 @@ __global__ __launch_bounds__(256) void convolve_fast_kernel(apx_conv_job job,
 // take the workgroups round robin).  Bound by the FP32 matrix pipe.  With all
 // passes of a tile in one workgroup, rows copied through registers a load at a
 // time, 512^2 with 53 x 53 kernels took 41 us (value) and 244 us (Jacobian of 7
-// columns); so @@ and @@ us.
+// columns); so 24.5 and 122 us
+// (100^2 with 27 x 27: 19 and 110 us, 12 and 14 us).
 constexpr int kMfmaMin = 21;  // shorter kernels waste over half of each MFMA on the band's zeros
 constexpr int kMaxPass = APX_MAX_CHAN + 2;
 
@@ -323,11 +324,11 @@ __global__ __launch_bounds__(256) void convolve_mfma_kernel(apx_conv_job job, co
   const int lm = lane & 15, lk = lane >> 4;
   const int ox0 = (tile % ntx) * 64, oy0 = (tile / ntx) * kMfR;
   const int kh = job.kh, kw = job.kw, ch = (kh - 1) / 2, cw = (kw - 1) / 2;
-  const int rows = mf_rows(kh), LW = mf_lw(kw), DD = mf_dd(kh);
-  float* tin = smem;             // rows x LW
-  float* tab = smem + rows * LW; // [kx][dd] = Kf[dd - 15][kx]
+  const int rows = mf_rows(kh), DD = mf_dd(kh);
+  float* tin = smem;             // rows x kMfLW
+  float* tab = smem + rows * kMfLW; // [kx][dd] = Kf[dd - 15][kx]
   stage_rows(planes + (int64_t)c * job.nx * job.ny, job.nx, job.nx, job.ny, job.x0 + ox0 - cw, job.y0 + oy0 - ch, rows,
-             64 + kw - 1, tin, LW);
+             64 + kw - 1, tin, kMfLW);
   // the tap table: kernel rows read coalesced, stored DD (odd) apart; its first
   // 15 and last columns stay zero
   const float* K = kernels + (int64_t)k * kh * kw;
@@ -339,7 +340,8 @@ __global__ __launch_bounds__(256) void convolve_mfma_kernel(apx_conv_job job, co
   }
   __builtin_amdgcn_s_waitcnt(0);  // this wave's rows have landed in LDS
   __syncthreads();
-  const v4f acc = mfma_block(mf_nks(kh), tin + lk * LW + 16 * w + lm, tab + lk - lm + 15, kw, LW, DD);
+  if (ox0 + 16 * w >= job.ow) return;
+  const v4f acc = mfma_block(mf_nks(kh), tin + lk * kMfLW + 16 * w + lm, tab + lk - lm + 15, kw, DD);
   // this lane's 4 outputs: x = 16 w + 4 lk + i, row lm
   const int oy = oy0 + lm, ox = ox0 + 16 * w + 4 * lk;
   if (oy >= job.oh) return;

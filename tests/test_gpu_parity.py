@@ -5,6 +5,7 @@ Tolerances (max-norm relative to the oracle's max):
   Jacobian     2e-4 per column (float32 analytic partials vs float64 forward AD)
 """
 
+import ctypes
 import math
 
 import numpy as np
@@ -285,6 +286,50 @@ def test_lm_solve_matches_reference_formula():
         ref = H.lm_damped_solve(Lval, grad.cpu(), hess.cpu())
         assert st.item() == 0
         assert torch.allclose(h.cpu(), ref, rtol=1e-9, atol=1e-12)
+
+
+@pytest.mark.parametrize("kh,kw,ow,oh,nchan,zero,shared", [
+    (1, 1, 70, 33, 1, 0, False), (19, 19, 64, 16, 2, 0, False), (21, 21, 65, 17, 3, 0, False), (53, 21, 130, 31, 2, 0, False),
+    (23, 67, 63, 48, 2, 1, False), (67, 67, 100, 40, 4, 1, False), (69, 69, 64, 24, 2, 0, False), (27, 27, 66, 20, 3, 0, True),
+    (91, 91, 40, 20, 2, 0, False)])
+def test_convolve_shapes(kh, kw, ow, oh, nchan, zero, shared):
+    """apx_convolve at the edges of its three kernels and their tiles: value,
+    centre and channel columns at an offset in the destinations, added to what
+    is there; ``zero``: taps that reach outside the planes read 0; ``shared``:
+    two channels added to one column.  float32 sums of kh kw products in a
+    fixed order against float64: 1e-5 of the sum of their magnitudes."""
+    lib = ap._lib.load()
+    g = torch.Generator().manual_seed(kh + ow)
+    rnd = lambda *s: torch.randn(s, generator=g).cuda()  # noqa: E731
+    m = 0 if zero else 1
+    nx, ny = ow + m * (kw - 1) + 3, oh + m * (kh - 1) + 2
+    x0, y0 = (1, 1) if zero else ((kw - 1) // 2 + 2, (kh - 1) // 2 + 1)
+    planes, kern = rnd(nchan, ny, nx), rnd(3, kh, kw)
+    img, jac = rnd(oh + 3, ow + 5), rnd(oh + 3, ow + 5, nchan + 3)
+    ref_i, ref_j = img.double(), jac.double()
+    job = ap._lib.ConvJob()
+    job.nx, job.ny, job.nchan, job.kh, job.kw, job.x0, job.y0, job.ow, job.oh = nx, ny, nchan, kh, kw, x0, y0, ow, oh
+    job.img, job.img_row, job.img_w, job.img_h, job.img_x0, job.img_y0 = img.data_ptr(), ow + 5, ow + 5, oh + 3, 4, 2
+    job.jac, job.jac_np, job.jac_row = jac.data_ptr(), nchan + 3, (ow + 5) * (nchan + 3)
+    job.jac_w, job.jac_h, job.jac_x0, job.jac_y0 = ow + 5, oh + 3, 4, 2
+    job.dk_col[0], job.dk_col[1] = nchan + 1, 0
+    col = [0] + [1 if shared else c for c in range(1, nchan)]
+    job.chan_col[:nchan] = col
+    job.zero_outside = zero
+    wsb = lib.apx_convolve_workspace_bytes(kh, kw)
+    ws = torch.empty(wsb, dtype=torch.uint8, device="cuda")
+    pad = torch.nn.functional.pad(planes.double().cpu(), (kw, kw, kh, kh))
+    box = pad[:, kh + y0 - (kh - 1) // 2:kh + y0 + oh + (kh - 1) // 2, kw + x0 - (kw - 1) // 2:kw + x0 + ow + (kw - 1) // 2]
+    conv = lambda p, k: torch.nn.functional.conv2d(p[None, None], k.double().cpu()[None, None])[0, 0].cuda()  # noqa: E731
+    tol = 1e-5 * float(conv(box.abs().max(0).values, kern.abs().max(0).values).max())
+    ref_i[2:2 + oh, 4:4 + ow] += conv(box[0], kern[0])
+    for k, c in ((1, nchan + 1), (2, 0)):
+        ref_j[2:2 + oh, 4:4 + ow, c] += conv(box[0], kern[k])
+    for c in range(1, nchan):
+        ref_j[2:2 + oh, 4:4 + ow, col[c]] += conv(box[c], kern[0])
+    ap._lib.check(lib.apx_convolve(ctypes.byref(job), planes.data_ptr(), kern.data_ptr(), ws.data_ptr(), wsb, ap._lib.stream()))
+    assert float((img.double() - ref_i).abs().max()) <= tol
+    assert float((jac.double() - ref_j).abs().max()) <= tol
 
 
 @pytest.mark.parametrize("npar", [1, 2, 13, 15, 16, 17, 64])
