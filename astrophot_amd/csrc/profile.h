@@ -52,7 +52,7 @@ struct Prof {
 };
 
 template <typename T>
-__device__ inline Prof<T> make_prof(int profile, const double* P, double fx, double fy,
+__host__ __device__ inline Prof<T> make_prof(int profile, const double* P, double fx, double fy,
                                     double pixel_area, double softening, double q, double pa,
                                     const double* prm) {
   Prof<T> p;
@@ -111,10 +111,17 @@ __device__ inline Prof<T> make_prof(int profile, const double* P, double fx, dou
   return p;
 }
 
-template <typename T>
-__device__ inline Prof<T> make_prof(const apx_component& cp) {
-  return make_prof<T>(cp.profile, cp.P, cp.frac[0], cp.frac[1], cp.pixel_area, cp.softening, cp.q,
-                      cp.pa, cp.prm);
+// The constants of one component in both types, made once on the host and
+// passed to the kernels by value (their float64 pow, cos, sin and log2 cost a
+// thread more than the sample it then takes).
+struct RenderConst {
+  Prof<float> f;
+  Prof<double> d;
+};
+
+inline RenderConst render_const(const apx_component& cp) {
+  return {make_prof<float>(cp.profile, cp.P, cp.frac[0], cp.frac[1], cp.pixel_area, cp.softening, cp.q, cp.pa, cp.prm),
+          make_prof<double>(cp.profile, cp.P, cp.frac[0], cp.frac[1], cp.pixel_area, cp.softening, cp.q, cp.pa, cp.prm)};
 }
 
 // Value (times `scale`, the pixel-area ratio of the sampling level) and, when

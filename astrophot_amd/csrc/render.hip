@@ -3,7 +3,7 @@
 //
 // Restates models/_model_methods.py:82-184 (_sample_init midpoint / quad:N,
 // _sample_integrate threshold) and utils/operations.py:94-247
-// (single_quad_integrate, grid_integrate) as three launches:
+// (single_quad_integrate, grid_integrate) as four launches:
 //   1. init     : one thread per working pixel, float32 profile value and
 //                 Jacobian channels; a float64 per-block partial sum when the
 //                 integrate reference is the mean sample.
@@ -13,10 +13,12 @@
 //                 threshold are re-decided in float64, so the selected set is
 //                 the float64 one.  Selected pixels are appended to a list with
 //                 one atomic per wavefront.
-//   3. integrate: one wavefront per listed pixel; the recursive quadrature
-//                 (levels 1..max_depth, threshold x gridding^2 per level as in
-//                 operations.py:241) runs in float64 and overwrites the
-//                 pixel's value and Jacobian channels.
+//   3. level 1  : float64 Gauss-Legendre of the selected pixels, one lane a
+//                 node; a pixel that needs refining goes to a second list.
+//   4. deep     : levels 2 and 3 of those (threshold x gridding^2 per level as
+//                 in operations.py:241), a workgroup a pixel; float32 samples
+//                 summed in float64.
+// The adjoint runs 3 and 4 again, reducing against its weights.
 #include <hip/hip_runtime.h>
 
 #include "capi_internal.h"
@@ -28,17 +30,19 @@ namespace apx {
 namespace {
 
 constexpr int kInitBlock = 256;
-constexpr int kIntegrateWaves = 2048;
+constexpr int kLevelBlocks = 512;  // workgroups of the level-1 pass
+constexpr int kDeepBlocks = 1024;  // workgroups of the deep pass
 
 // workspace layout (bytes)
 struct RenderWs {
-  int32_t* count;     // [0]: selected pixels
+  int32_t* count;     // [0]: selected pixels, [1]: those refined past level 1
   double* reference;  // mean-sample reference (when mean_reference)
   double* partial;    // per-init-block sums
   int32_t* list;      // selected pixel indices
   float* centre;      // quad:N centre-node samples
-  uint8_t* flags;     // 1 = pixel selected for integration
-  double* vpart;      // per-integrate-block adjoint sums (8 per block)
+  int32_t* deep;      // refined pixel indices (in place of centre once the selection is made)
+  uint8_t* flags;     // 1 = pixel selected for integration, 2 = refined past level 1
+  double* vpart;      // adjoint sums of the level-1 and deep workgroups (8 per block)
 };
 
 __host__ __device__ inline int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
@@ -58,6 +62,7 @@ __host__ inline RenderWs carve(void* ws, int64_t npix) {
   w.list = reinterpret_cast<int32_t*>(b + off);
   off += align256(4 * npix);
   w.centre = reinterpret_cast<float*>(b + off);
+  w.deep = reinterpret_cast<int32_t*>(b + off);
   off += align256(4 * npix);
   w.flags = reinterpret_cast<uint8_t*>(b + off);
   off += align256(npix);
@@ -66,11 +71,12 @@ __host__ inline RenderWs carve(void* ws, int64_t npix) {
 }
 
 template <bool GRAD>
-__global__ __launch_bounds__(kInitBlock) void render_init_kernel(apx_component cp, float* planes,
+__global__ __launch_bounds__(kInitBlock) void render_init_kernel(apx_component cp, RenderConst rc, float* planes,
                                                                  RenderWs ws) {
   const int64_t npix = (int64_t)cp.nx * cp.ny;
   const int64_t pix = (int64_t)blockIdx.x * kInitBlock + threadIdx.x;
-  const Prof<float> p = make_prof<float>(cp);
+  const Prof<float>& p = rc.f;
+  if (blockIdx.x == 0 && threadIdx.x < 2) ws.count[threadIdx.x] = 0;
   float value = 0.0f;
   if (pix < npix) {
     const int i = (int)(pix % cp.nx), j = (int)(pix / cp.nx);
@@ -94,7 +100,7 @@ __global__ __launch_bounds__(kInitBlock) void render_init_kernel(apx_component c
       }
     }
   }
-  if (cp.mean_reference) {
+  if (cp.mean_reference && cp.integrate) {
     // deterministic float64 block sum of the initial samples
     __shared__ double red[kInitBlock / 64];
     double v = wave_sum((double)value);
@@ -118,7 +124,6 @@ __global__ __launch_bounds__(256) void mean_reference_kernel(RenderWs ws, int64_
   __syncthreads();
   if (threadIdx.x == 0) {
     ws.reference[0] = (red[0] + red[1] + red[2] + red[3]) / (double)npix;
-    ws.count[0] = 0;
   }
 }
 
@@ -153,7 +158,7 @@ __device__ bool select_f64(const apx_component& cp, const Prof<double>& p, int i
   return fabs(mid - (mid + curv)) > thr;  // |deep - reference| (_model_methods.py:164-165)
 }
 
-__global__ __launch_bounds__(256) void render_select_kernel(apx_component cp, const float* planes,
+__global__ __launch_bounds__(256) void render_select_kernel(apx_component cp, RenderConst rc, const float* planes,
                                                             RenderWs ws) {
   const int64_t npix = (int64_t)cp.nx * cp.ny;
   const int64_t pix = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -162,9 +167,8 @@ __global__ __launch_bounds__(256) void render_select_kernel(apx_component cp, co
   if (cp.integrate == APX_INTEGRATE_RADIUS) {
     // pixels whose centre lies within the radius of the model centre
     if (pix < npix) {
-      const Prof<double> p = make_prof<double>(cp);
       double X, Y;
-      pixel_xy(p, cp, (int)(pix % cp.nx), (int)(pix / cp.nx), X, Y);
+      pixel_xy(rc.d, cp, (int)(pix % cp.nx), (int)(pix / cp.nx), X, Y);
       // inclusive, with a 1e-9 relative margin: with the centre on a pixel
       // centre (psf_mode "full") lattice points lie exactly on the circle
       sel = X * X + Y * Y <= cp.integrate_radius * cp.integrate_radius * (1.0 + 1e-9);
@@ -190,8 +194,7 @@ __global__ __launch_bounds__(256) void render_select_kernel(apx_component cp, co
     if (dm > thr + band) {
       sel = true;
     } else if (dm >= thr - band) {
-      const Prof<double> p = make_prof<double>(cp);
-      sel = select_f64(cp, p, i, j, thr);
+      sel = select_f64(cp, rc.d, i, j, thr);
     }
   }
   if (pix < npix) ws.flags[pix] = sel ? 1 : 0;
@@ -208,39 +211,274 @@ __global__ __launch_bounds__(256) void render_select_kernel(apx_component cp, co
   }
 }
 
-// float64 adaptive quadrature of listed pixels, one wavefront per pixel
-template <bool GRAD>
-__global__ __launch_bounds__(256) void render_integrate_kernel(apx_component cp, float* planes,
-                                                               RenderWs ws) {
+// What the quadrature passes do with a pixel's sums: write the value, the value
+// and the channels, or (adjoint) add them, weighted, to the workgroup's sums.
+enum : int { Q_VALUE = 0, Q_GRAD = 1, Q_VJP = 2 };
+
+// the workgroup's adjoint sums of slots chan_slot[1 .. nchan-1] into part[0 .. 7]
+__device__ __forceinline__ void vjp_part(const apx_component& cp, const double* acc, double* part) {
+  __shared__ double red[4][8];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+#pragma unroll
+  for (int s = 0; s < APX_NSLOT; ++s) {
+    const double t = wave_sum(acc[s]);
+    if (lane == 0) red[wv][s] = t;
+  }
+  __syncthreads();
+  const int c = threadIdx.x;
+  if (c >= 1 && c < cp.nchan) {
+    const int s = cp.chan_slot[c];
+    part[c] = red[0][s] + red[1][s] + red[2][s] + red[3][s];
+  }
+}
+
+// Level 1 of the listed pixels (operations.py:210-228, area 1, float64, which
+// is the value of every selected pixel that is not refined further): one lane a
+// node, 64 / quad_level^2 pixels a wave (7 for the 3 x 3 rule), the nodes'
+// terms added in node order by lane reads.  Bound by the latency of one float64
+// sample and its sum.  A wave a pixel kept 9 lanes of 64 busy, and carried the
+// pixel's deeper levels in the same wave (render_deep_kernel): 51 us for a 100^2
+// cutout, 71 us for 1537 x 1201 (adjoint 114); 17 and 35 us (42) the two passes.
+template <int MODE>
+__global__ __launch_bounds__(256) void render_level1_kernel(apx_component cp, RenderConst rc, float* planes,
+                                                            const float* __restrict__ B, RenderWs ws) {
+  constexpr bool GRAD = MODE != Q_VALUE;
   const int lane = threadIdx.x & 63;
-  const int wave = (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
-  const int nwaves = (int)(gridDim.x * 4);
+  const int n = cp.quad_level, nn = n * n, per = 64 / nn;
+  const int grp = lane / nn, node = lane - grp * nn, first = grp * nn;
+  const int wave = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), nwaves = (int)(gridDim.x * 4);
   const int count = ws.count[0];
   const int64_t npix = (int64_t)cp.nx * cp.ny;
-  const Prof<double> p = make_prof<double>(cp);
-  const Prof<float> pf = make_prof<float>(cp);
+  const Prof<double>& p = rc.d;
   const double thr1 = cp.tolerance * (cp.mean_reference ? ws.reference[0] : cp.reference);
-  for (int k = wave; k < count; k += nwaves) {
-    const int32_t pix = ws.list[k];
-    double out[1 + APX_NSLOT];
-    integrate_pixel<GRAD>(cp, p, pf, cp.nx, cp.ci, cp.cj, pix, thr1, lane, out);
-    if (lane == 0) {
-      planes[pix] = (float)out[0];
-      if (GRAD) {
+  const double u = cp.gl_node[node % n], v = cp.gl_node[node / n];
+  const double w = cp.gl_weight[node % n] * cp.gl_weight[node / n] * 0.25;
+  const double ox = 0.5 * (p.P00 * u + p.P01 * v), oy = 0.5 * (p.P10 * u + p.P11 * v);
+  double adj[APX_NSLOT];
+#pragma unroll
+  for (int s = 0; s < APX_NSLOT; ++s) adj[s] = 0.0;
+  for (int k0 = wave * per; k0 < count; k0 += nwaves * per) {
+    const int k = k0 + grp;
+    const bool on = grp < per && k < count;
+    const int32_t pix = on ? ws.list[k] : 0;
+    if (MODE == Q_VJP && (!on || ws.flags[pix] == 2)) continue;  // no lane reads below
+    double X0, Y0, gl[APX_NSLOT];
+    pixel_xy(p, cp, pix % cp.nx, pix / cp.nx, X0, Y0);
+    const double v1 = eval_profile<double, GRAD>(p, X0 + ox, Y0 + oy, 1.0, gl);
+    if (MODE == Q_VJP) {
+      const double wb = w * (double)B[pix];
+#pragma unroll
+      for (int s = 0; s < APX_NSLOT; ++s) adj[s] += wb * gl[s];
+      continue;
+    }
+    const double t = w * v1;
+    double res = 0.0;
+    for (int j = 0; j < nn; ++j) res += __shfl(t, first + j, 64);
+    const double centre = __shfl(v1, first + nn / 2, 64);
+    const bool refine = on && cp.max_depth > 1 && fabs(res - centre) > thr1;
+    double gs[APX_NSLOT];
+    if (GRAD) {
+#pragma unroll
+      for (int s = 0; s < APX_NSLOT; ++s) {
+        const double tg = w * gl[s];
+        gs[s] = 0.0;
+        for (int j = 0; j < nn; ++j) gs[s] += __shfl(tg, first + j, 64);
+      }
+    }
+    const bool lead = on && node == 0;
+    if (lead && !refine) {
+      planes[pix] = (float)res;
+      if (GRAD)
         for (int c = 1; c < cp.nchan; ++c) {
           const int s = cp.chan_slot[c];
-          planes[c * npix + pix] = (float)(out[1 + s] * cp.dvdr[s]);
+          planes[c * npix + pix] = (float)(gs[s] * cp.dvdr[s]);
         }
+    }
+    const uint64_t ballot = __ballot(lead && refine);
+    if (ballot) {
+      int base = 0;
+      if (lane == 0) base = atomicAdd(ws.count + 1, (int)__popcll(ballot));
+      base = __shfl(base, 0, 64);
+      if (lead && refine) {
+        ws.deep[base + (int)__popcll(ballot & ((lane == 0) ? 0ull : (~0ull >> (64 - lane))))] = pix;
+        ws.flags[pix] = 2;
       }
     }
   }
+  if (MODE == Q_VJP) vjp_part(cp, adj, ws.vpart + 8 * blockIdx.x);
+}
+
+// Levels 2 and 3 of the refined pixels (operations.py:229-247), a workgroup a
+// pixel.  Samples are float32, sums float64; a level-2 test whose float32 value
+// lies within kSampleBand of its threshold is taken again from float64 samples,
+// so the sub-pixels refined are the ones float64 arithmetic picks.  The samples
+// of every flagged sub-pixel form one run that the 256 threads share, so that a
+// cuspy centre pixel, up to 25 x 225 samples, is not one wave's serial chain.
+// FAST: the default 3 x 3 rule on 5 x 5 sub-pixels, whose 225 level-2 samples
+// take a thread each (summed per sub-pixel in node order); else a thread a
+// sub-pixel.
+template <int MODE, bool FAST>
+__global__ __launch_bounds__(256) void render_deep_kernel(apx_component cp, RenderConst rc, float* planes,
+                                                          const float* __restrict__ B, RenderWs ws, int voff) {
+  constexpr bool GRAD = MODE != Q_VALUE;
+  constexpr int NV = GRAD ? 1 + APX_NSLOT : 1;
+  constexpr int NS = FAST ? 225 : 1;
+  __shared__ float sample[NV][NS];
+  __shared__ double sx[64], sy[64];   // flagged sub-pixels
+  __shared__ double ox3[NS], oy3[NS], w3[NS];
+  __shared__ double red[4][NV];
+  __shared__ int nflag;
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int n = FAST ? 3 : cp.quad_level, nn = n * n, g = FAST ? 5 : cp.gridding, gg = g * g;
+  const int64_t npix = (int64_t)cp.nx * cp.ny;
+  const Prof<double>& p = rc.d;
+  const Prof<float>& pf = rc.f;
+  const double thr1 = cp.tolerance * (cp.mean_reference ? ws.reference[0] : cp.reference);
+  const double ig = 1.0 / (double)g, sub0 = -(double)(g - 1) / (2.0 * g), subd = ig;
+  const double sc2 = ig * ig, thr2 = thr1 * (double)gg, sc3 = sc2 * ig * ig;
+  const float h = (float)(0.5 * ig);
+  // offset and weight of level-3 sample e of a sub-pixel: sub-sub-pixel e / nn, node e % nn
+  auto offset3 = [&](int e, double& x, double& y, double& w) {
+    const int q = e / nn, kk = e - q * nn;
+    const double a = (sub0 + subd * (q % g)) * ig, b = (sub0 + subd * (q / g)) * ig;
+    const double hu = a + 0.5 * ig * ig * cp.gl_node[kk % n], hv = b + 0.5 * ig * ig * cp.gl_node[kk / n];
+    x = p.P00 * hu + p.P01 * hv;
+    y = p.P10 * hu + p.P11 * hv;
+    w = cp.gl_weight[kk % n] * cp.gl_weight[kk / n] * 0.25;
+  };
+  if (FAST && t < NS) offset3(t, ox3[t], oy3[t], w3[t]);
+  // sub-pixel and node of this thread at level 2
+  const int sub = FAST ? t / 9 : t, k2 = FAST ? t - 9 * sub : 0;
+  const double sa = sub0 + subd * (sub % g), sb = sub0 + subd * (sub / g);
+  const double sdx = p.P00 * sa + p.P01 * sb, sdy = p.P10 * sa + p.P11 * sb;
+  const float nu = (float)cp.gl_node[k2 % n], nv = (float)cp.gl_node[k2 / n];
+  auto weight2 = [&](int q) { return (float)(cp.gl_weight[q % 3] * cp.gl_weight[q / 3] * 0.25); };
+  const int count = ws.count[1];
+  double adj[APX_NSLOT];
+#pragma unroll
+  for (int s = 0; s < APX_NSLOT; ++s) adj[s] = 0.0;
+  for (int k = blockIdx.x; k < count; k += gridDim.x) {
+    const int32_t pix = ws.deep[k];
+    double X0, Y0;
+    pixel_xy(p, cp, pix % cp.nx, pix / cp.nx, X0, Y0);
+    double acc[NV];
+#pragma unroll
+    for (int s = 0; s < NV; ++s) acc[s] = 0.0;
+    if (FAST) {
+      if (t < NS) {
+        float gl[APX_NSLOT];
+        const float val = eval_profile<float, GRAD>(pf, (float)(X0 + sdx) + h * pf.P00 * nu + h * pf.P01 * nv,
+                                                    (float)(Y0 + sdy) + h * pf.P10 * nu + h * pf.P11 * nv, (float)sc2, gl);
+        sample[0][t] = val;
+        if (GRAD) {
+#pragma unroll
+          for (int s = 0; s < APX_NSLOT; ++s) sample[1 + s][t] = gl[s];
+        }
+      }
+      __syncthreads();
+    }
+    // level 2: thread t < gg sums sub-pixel t and tests it
+    if (t < 64) {
+      bool deeper = false;
+      double x2 = 0.0, y2 = 0.0;
+      if (t < gg) {
+        const double a = sub0 + subd * (t % g), b = sub0 + subd * (t / g);
+        x2 = X0 + p.P00 * a + p.P01 * b;
+        y2 = Y0 + p.P10 * a + p.P11 * b;
+        float gs[APX_NSLOT], centre = 0.0f, r2 = 0.0f;
+        if (FAST) {
+#pragma unroll
+          for (int q = 0; q < 9; ++q) r2 += weight2(q) * sample[0][9 * t + q];
+          centre = sample[0][9 * t + 4];
+          if (GRAD) {
+#pragma unroll
+            for (int s = 0; s < APX_NSLOT; ++s) {
+              gs[s] = 0.0f;
+#pragma unroll
+              for (int q = 0; q < 9; ++q) gs[s] += weight2(q) * sample[1 + s][9 * t + q];
+            }
+          }
+        } else {
+          r2 = quad_sample<float, GRAD>(pf, cp, (float)x2, (float)y2, n, cp.gl_node, cp.gl_weight, (float)sc2, h * pf.P00,
+                                        h * pf.P01, h * pf.P10, h * pf.P11, gs, centre);
+        }
+        if (cp.max_depth > 2) {
+          const double D = fabs((double)r2 - (double)centre);
+          const double band = kSampleBand * (fabs((double)r2) + fabs((double)centre)) + 1e-7 * thr2;
+          if (D > thr2 + band) {
+            deeper = true;
+          } else if (D >= thr2 - band) {
+            double cd = 0.0;
+            const double rd = quad_sample<double, false>(p, cp, x2, y2, n, cp.gl_node, cp.gl_weight, sc2,
+                                                         0.5 * ig * p.P00, 0.5 * ig * p.P01, 0.5 * ig * p.P10,
+                                                         0.5 * ig * p.P11, nullptr, cd);
+            deeper = fabs(rd - cd) > thr2;
+          }
+        }
+        if (!deeper) {
+          acc[0] = (double)r2;
+          if (GRAD) {
+#pragma unroll
+            for (int s = 0; s < APX_NSLOT; ++s) acc[1 + s] = (double)gs[s];
+          }
+        }
+      }
+      const uint64_t flags = __ballot(deeper);
+      if (deeper) {
+        const int at = (int)__popcll(flags & ((lane == 0) ? 0ull : (~0ull >> (64 - lane))));
+        sx[at] = x2;
+        sy[at] = y2;
+      }
+      if (t == 0) nflag = (int)__popcll(flags);
+    }
+    __syncthreads();
+    // level 3: the samples of the flagged sub-pixels, one run over the workgroup
+    const int per3 = gg * nn, total3 = nflag * per3;
+    for (int e = t; e < total3; e += 256) {
+      const int f = e / per3, q = e - f * per3;
+      double dx, dy, w;
+      if (FAST) {
+        dx = ox3[q];
+        dy = oy3[q];
+        w = w3[q];
+      } else {
+        offset3(q, dx, dy, w);
+      }
+      float gl[APX_NSLOT];
+      const float val = eval_profile<float, GRAD>(pf, (float)(sx[f] + dx), (float)(sy[f] + dy), (float)sc3, gl);
+      acc[0] += w * (double)val;
+      if (GRAD) {
+#pragma unroll
+        for (int s = 0; s < APX_NSLOT; ++s) acc[1 + s] += w * (double)gl[s];
+      }
+    }
+    if (MODE == Q_VJP) {
+      const double wb = (double)B[pix];
+#pragma unroll
+      for (int s = 0; s < APX_NSLOT; ++s) adj[s] += wb * acc[1 + s];
+    } else {
+#pragma unroll
+      for (int s = 0; s < NV; ++s) {
+        const double a = wave_sum(acc[s]);
+        if (lane == 0) red[wv][s] = a;
+      }
+      __syncthreads();
+      if (t < cp.nchan && (GRAD || t == 0)) {
+        const int s = t == 0 ? 0 : 1 + cp.chan_slot[t];
+        const double a = red[0][s] + red[1][s] + red[2][s] + red[3][s];
+        planes[t * npix + pix] = (float)(t == 0 ? a : a * cp.dvdr[s - 1]);
+      }
+    }
+    __syncthreads();  // the next pixel writes sample, sx, sy and red again
+  }
+  if (MODE == Q_VJP) vjp_part(cp, adj, ws.vpart + 8 * (voff + blockIdx.x));
 }
 
 // Adjoint of the render: sum over working pixels of B[q] * d deep[q] / d slot
 // for the slots chan_slot[1 .. nchan-1].  Unselected pixels use the float32
 // analytic partials (what the Jacobian channels hold); selected pixels
-// recompute the forward quadrature (render_vjp_integrate_kernel).
-__global__ __launch_bounds__(256) void render_vjp_kernel(apx_component cp,
+// recompute the forward quadrature (the level-1 and deep passes).
+__global__ __launch_bounds__(256) void render_vjp_kernel(apx_component cp, RenderConst rc,
                                                          const float* __restrict__ B, RenderWs ws,
                                                          int use_flags) {
   __shared__ double red[4][8];
@@ -250,7 +488,7 @@ __global__ __launch_bounds__(256) void render_vjp_kernel(apx_component cp,
 #pragma unroll
   for (int c = 0; c < 8; ++c) acc[c] = 0.0;
   if (pix < npix && !(use_flags && ws.flags[pix])) {
-    const Prof<float> p = make_prof<float>(cp);
+    const Prof<float>& p = rc.f;
     const int i = (int)(pix % cp.nx), j = (int)(pix / cp.nx);
     float X, Y, g[APX_NSLOT];
     pixel_xy(p, cp, i, j, X, Y);
@@ -276,35 +514,6 @@ __global__ __launch_bounds__(256) void render_vjp_kernel(apx_component cp,
         red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
 }
 
-__global__ __launch_bounds__(256) void render_vjp_integrate_kernel(apx_component cp,
-                                                                   const float* __restrict__ B,
-                                                                   RenderWs ws) {
-  __shared__ double red[4][8];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int wave = (int)(blockIdx.x * 4 + wv);
-  const int nwaves = (int)(gridDim.x * 4);
-  const int count = ws.count[0];
-  const Prof<double> p = make_prof<double>(cp);
-  const Prof<float> pf = make_prof<float>(cp);
-  const double thr1 = cp.tolerance * (cp.mean_reference ? ws.reference[0] : cp.reference);
-  double acc[8];
-#pragma unroll
-  for (int c = 0; c < 8; ++c) acc[c] = 0.0;
-  for (int k = wave; k < count; k += nwaves) {
-    const int32_t pix = ws.list[k];
-    double out[1 + APX_NSLOT];
-    integrate_pixel<true>(cp, p, pf, cp.nx, cp.ci, cp.cj, pix, thr1, lane, out);
-    const double w = (double)B[pix];
-    for (int c = 1; c < cp.nchan; ++c) acc[c] += w * out[1 + cp.chan_slot[c]];
-  }
-  if (lane == 0)
-    for (int c = 0; c < 8; ++c) red[wv][c] = acc[c];
-  __syncthreads();
-  if (threadIdx.x >= 1 && threadIdx.x < 8)
-    ws.vpart[blockIdx.x * 8 + threadIdx.x] =
-        red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
-}
-
 // One workgroup a slot, 256 partials in flight a step (a thread a slot read the
 // 7,900 partials of a 1537 x 1201 image one after another: 1.24 ms; now 14 us).
 __global__ __launch_bounds__(256) void render_vjp_final_kernel(apx_component cp, RenderWs ws,
@@ -320,7 +529,28 @@ __global__ __launch_bounds__(256) void render_vjp_final_kernel(apx_component cp,
   if (threadIdx.x == 0) grad[c - 1] = (red[0] + red[1] + red[2] + red[3]) * cp.dvdr[cp.chan_slot[c]];
 }
 
-__global__ void zero_count_kernel(RenderWs ws) { ws.count[0] = 0; }
+// workgroups of the two passes over npix pixels: no more than could find work
+int level_blocks(const apx_component& cp, int64_t npix) {
+  const int per = 4 * (64 / (cp.quad_level * cp.quad_level));
+  return (int)std::min<int64_t>(kLevelBlocks, (npix + per - 1) / per);
+}
+int deep_blocks(const apx_component& cp, int64_t npix) {
+  return cp.max_depth < 2 ? 0 : (int)std::min<int64_t>(kDeepBlocks, npix);
+}
+
+// the level-1 and deep passes of a component
+template <int MODE>
+void integrate(const apx_component& cp, const RenderConst& rc, float* planes, const float* B, const RenderWs& ws,
+               hipStream_t stream) {
+  const int64_t npix = (int64_t)cp.nx * cp.ny;
+  const int nl = level_blocks(cp, npix), nd = deep_blocks(cp, npix);
+  hipLaunchKernelGGL((render_level1_kernel<MODE>), dim3(nl), dim3(256), 0, stream, cp, rc, planes, B, ws);
+  if (nd == 0) return;
+  if (cp.quad_level == 3 && cp.gridding == 5)
+    hipLaunchKernelGGL((render_deep_kernel<MODE, true>), dim3(nd), dim3(256), 0, stream, cp, rc, planes, B, ws, nl);
+  else
+    hipLaunchKernelGGL((render_deep_kernel<MODE, false>), dim3(nd), dim3(256), 0, stream, cp, rc, planes, B, ws, nl);
+}
 
 // PSF_Model.sample's normalisation to unit sum (psf_model_object.py:255-257)
 // applied to render planes: plane 0 becomes P / S with S = sum P, and each
@@ -375,7 +605,7 @@ int normalize_planes(float* planes, int32_t nchan, int64_t npix, hipStream_t str
 
 int64_t render_workspace_bytes(int64_t npix) {
   return 256 + align256(8 * 8 * init_blocks(npix)) + align256(4 * npix) + align256(4 * npix) +
-         align256(npix) + align256(8 * 8 * (kIntegrateWaves / 4));
+         align256(npix) + align256(8 * 8 * (kLevelBlocks + kDeepBlocks));
 }
 
 int render_component(const apx_component* cp_in, float* planes, void* workspace, int64_t ws_bytes,
@@ -418,26 +648,20 @@ int render_component(const apx_component* cp_in, float* planes, void* workspace,
   const RenderWs ws = carve(workspace, npix);
   const bool grad = cp.nchan > 1;
   const int64_t nb = init_blocks(npix);
+  const RenderConst rc = render_const(cp);
   if (grad)
     hipLaunchKernelGGL(render_init_kernel<true>, dim3((unsigned)nb), dim3(kInitBlock), 0, stream,
-                       cp, planes, ws);
+                       cp, rc, planes, ws);
   else
     hipLaunchKernelGGL(render_init_kernel<false>, dim3((unsigned)nb), dim3(kInitBlock), 0, stream,
-                       cp, planes, ws);
-  if (cp.mean_reference)
-    hipLaunchKernelGGL(mean_reference_kernel, dim3(1), dim3(256), 0, stream, ws, nb, npix);
-  else
-    hipLaunchKernelGGL(zero_count_kernel, dim3(1), dim3(1), 0, stream, ws);
+                       cp, rc, planes, ws);
   if (cp.integrate) {
+    if (cp.mean_reference)
+      hipLaunchKernelGGL(mean_reference_kernel, dim3(1), dim3(256), 0, stream, ws, nb, npix);
     hipLaunchKernelGGL(render_select_kernel, dim3((unsigned)((npix + 255) / 256)), dim3(256), 0,
-                       stream, cp, planes, ws);
-    const int blocks = (int)std::min<int64_t>((npix + 3) / 4, kIntegrateWaves / 4);
-    if (grad)
-      hipLaunchKernelGGL(render_integrate_kernel<true>, dim3(blocks), dim3(256), 0, stream, cp,
-                         planes, ws);
-    else
-      hipLaunchKernelGGL(render_integrate_kernel<false>, dim3(blocks), dim3(256), 0, stream, cp,
-                         planes, ws);
+                       stream, cp, rc, planes, ws);
+    if (grad) integrate<Q_GRAD>(cp, rc, planes, nullptr, ws, stream);
+    else integrate<Q_VALUE>(cp, rc, planes, nullptr, ws, stream);
   }
   return check_launch("render");
 }
@@ -460,12 +684,13 @@ int render_vjp(const apx_component* cp_in, const float* weights, float* value_pl
   const int64_t npix = (int64_t)cp.nx * cp.ny;
   const RenderWs ws = carve(workspace, npix);
   const int64_t nb = init_blocks(npix);
-  hipLaunchKernelGGL(render_vjp_kernel, dim3((unsigned)nb), dim3(kInitBlock), 0, stream, cp, weights,
+  const RenderConst rcst = render_const(cp);
+  hipLaunchKernelGGL(render_vjp_kernel, dim3((unsigned)nb), dim3(kInitBlock), 0, stream, cp, rcst, weights,
                      ws, cp.integrate);
   int nb2 = 0;
   if (cp.integrate) {
-    nb2 = (int)std::min<int64_t>((npix + 3) / 4, kIntegrateWaves / 4);
-    hipLaunchKernelGGL(render_vjp_integrate_kernel, dim3(nb2), dim3(256), 0, stream, cp, weights, ws);
+    nb2 = level_blocks(cp, npix) + deep_blocks(cp, npix);  // the value render left the lists
+    integrate<Q_VJP>(cp, rcst, nullptr, weights, ws, stream);
   }
   hipLaunchKernelGGL(render_vjp_final_kernel, dim3(cp.nchan - 1), dim3(256), 0, stream, cp, ws, (int)nb, nb2,
                      grad);

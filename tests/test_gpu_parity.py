@@ -288,6 +288,28 @@ def test_lm_solve_matches_reference_formula():
         assert torch.allclose(h.cpu(), ref, rtol=1e-9, atol=1e-12)
 
 
+@pytest.mark.parametrize("level,gridding,depth", [(3, 5, 3), (3, 5, 2), (3, 5, 1), (3, 4, 3), (5, 3, 3), (7, 8, 2), (1, 2, 3)])
+def test_integration_settings(level, gridding, depth):
+    """The level-1 and deep passes at other Gauss-Legendre orders, griddings
+    and depths than the default's (a cuspy, well resolved Sersic refines at
+    every level): image, Jacobian and adjoint against the oracle, at the
+    repository's bars (1e-5 of the image's max; 2e-4 of a column's)."""
+    p = dict(GAL["sersic"], n=4.5, Re=5.0)
+    om, m = single("sersic", p, psf=PSF11, psf_mode="full", integrate_quad_level=level, integrate_gridding=gridding,
+                   integrate_max_depth=depth, sampling_tolerance=1e-3)
+    rep = om.vector_representation()
+    assert rel_err(m().data, om.forward(rep).reshape(36, 40)) < 1e-5
+    J = m.jacobian(parameters=rep.clone(), as_representation=True).data
+    ref = om.jacobian(rep).reshape(36, 40, -1)
+    for k in range(7):
+        assert rel_err(J[..., k], ref[..., k]) < 2e-4, k
+    G = torch.randn(36, 40, generator=torch.Generator().manual_seed(level), dtype=torch.float64)
+    g = m.vjp(G, parameters=rep.clone())
+    gref = (ref * G[..., None]).sum(dim=(0, 1))
+    scale = (ref * G[..., None]).abs().sum(dim=(0, 1))
+    assert bool(((g.cpu() - gref).abs() <= 2e-4 * scale).all())
+
+
 @pytest.mark.parametrize("kh,kw,ow,oh,nchan,zero,shared", [
     (1, 1, 70, 33, 1, 0, False), (19, 19, 64, 16, 2, 0, False), (21, 21, 65, 17, 3, 0, False), (53, 21, 130, 31, 2, 0, False),
     (23, 67, 63, 48, 2, 1, False), (67, 67, 100, 40, 4, 1, False), (69, 69, 64, 24, 2, 0, False), (27, 27, 66, 20, 3, 0, True),
