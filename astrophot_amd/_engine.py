@@ -115,12 +115,29 @@ def _gl(n):
     return tuple(float(v) for v in x), tuple(float(v) for v in w)
 
 
+@functools.lru_cache(maxsize=8)
+def _device(device):
+    return torch.device(device)
+
+
+@functools.lru_cache(maxsize=256)
+def _render_bytes(npix):
+    return int(L.load().apx_render_workspace_bytes(npix))
+
+
+@functools.lru_cache(maxsize=256)
+def _convolve_bytes(kh, kw):
+    return int(L.load().apx_convolve_workspace_bytes(kh, kw))
+
+
 def _buffer(owner, name, nbytes, device):
     """A device byte buffer of at least ``nbytes`` kept on ``owner`` between
     calls (work on one stream is ordered, so reuse is safe)."""
-    cache = owner.__dict__.setdefault("_apx_buffers", {})
+    cache = owner.__dict__.get("_apx_buffers")
+    if cache is None:
+        cache = owner.__dict__["_apx_buffers"] = {}
     b = cache.get(name)
-    if b is None or b.numel() < nbytes or b.device != torch.device(device):
+    if b is None or b.numel() < nbytes or b.device != _device(device):
         b = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)
         cache[name] = b
     return b
@@ -151,19 +168,12 @@ class Plan:
     out_window: object = None  # where the convolved output lands (after the block sum)
 
 
-def plan(model, values, window, slot_cols=None, dvdr=None, channels=False, ref_npix=None) -> Plan:
-    """Fill the apx_component of ``model`` for sampling ``window``.
-    ``ref_npix`` (Sersic): the working-grid pixel count of the window the
-    model is nominally sampled on, when only a part of it is rendered."""
-    kind = model._profile
-    psf_full = "full" in model.psf_mode and kind != "flat_sky"
-    window = window.copy()
-    cx, cy = (float(v) for v in values["center"].reshape(-1).tolist())
-    P = window._P
+@functools.lru_cache(maxsize=256)
+def _template(kind, sm, im, quad_level, gridding, max_depth, radius, softening, tolerance) -> bytes:
+    """The fields of an apx_component that the model's knobs alone decide."""
     cp = L.Component()
     cp.profile = PROFILE_CODE[kind]
     # sampling mode (_model_methods.py:82-148)
-    sm = model.sampling_mode
     if sm == "midpoint":
         cp.sampling = L.APX_SAMPLE_MIDPOINT
     elif sm == "simpsons":
@@ -189,25 +199,44 @@ def plan(model, values, window, slot_cols=None, dvdr=None, channels=False, ref_n
         cp.sq_weight[:2] = (1.0, 1.0)
     else:
         raise SpecificationConflict(
-            f"{model.name} has unknown sampling mode: {sm}. Should be one of: midpoint, simpsons, quad:level, trapezoid")
-    im = model.integrate_mode if kind != "flat_sky" else "none"
+            f"{{name}} has unknown sampling mode: {sm}. Should be one of: midpoint, simpsons, quad:level, trapezoid")
     if im not in ("none", "threshold", "radius"):
         raise SpecificationConflict(
-            f"{model.name} has unknown integration mode: {im}. Should be one of: none, threshold, radius")
+            f"{{name}} has unknown integration mode: {im}. Should be one of: none, threshold, radius")
     cp.integrate = {"none": L.APX_INTEGRATE_NONE, "threshold": L.APX_INTEGRATE_THRESHOLD,
                     "radius": L.APX_INTEGRATE_RADIUS}[im]
     if cp.integrate:
-        cp.quad_level = int(model.integrate_quad_level)
-        cp.gridding = int(model.integrate_gridding)
-        cp.max_depth = int(model.integrate_max_depth)
+        cp.quad_level, cp.gridding, cp.max_depth = quad_level, gridding, max_depth
         if im == "radius":
-            # integrate_radius is in pixels of the model's own window
-            cp.integrate_radius = float(model.integrate_radius) * math.sqrt(abs(window._area))
+            cp.integrate_radius = radius
             cp.gridding, cp.max_depth = 1, 1
         if not 1 <= cp.quad_level <= L.APX_MAX_QUAD_LEVEL:
             raise SpecificationConflict(f"integrate_quad_level must be 1..{L.APX_MAX_QUAD_LEVEL}")
         x, w = _gl(cp.quad_level)
         cp.gl_node[:cp.quad_level], cp.gl_weight[:cp.quad_level] = x, w
+    cp.softening, cp.tolerance = softening, tolerance
+    return bytes(cp)
+
+
+def plan(model, values, window, slot_cols=None, dvdr=None, channels=False, ref_npix=None) -> Plan:
+    """Fill the apx_component of ``model`` for sampling ``window``.
+    ``ref_npix`` (Sersic): the working-grid pixel count of the window the
+    model is nominally sampled on, when only a part of it is rendered."""
+    kind = model._profile
+    psf_full = "full" in model.psf_mode and kind != "flat_sky"
+    window = window.copy()
+    cx, cy = values["center"].reshape(-1).tolist()
+    P = window._P
+    im = model.integrate_mode if kind != "flat_sky" else "none"
+    # integrate_radius is in pixels of the model's own window
+    radius = float(model.integrate_radius) * math.sqrt(abs(window._area)) if im == "radius" else 0.0
+    quad = (int(model.integrate_quad_level), int(model.integrate_gridding), int(model.integrate_max_depth)) if im != "none" \
+        else (0, 0, 0)
+    try:
+        cp = L.Component.from_buffer_copy(_template(kind, model.sampling_mode, im, *quad, radius, float(model.softening),
+                                                    float(model.sampling_tolerance)))
+    except SpecificationConflict as e:
+        raise SpecificationConflict(str(e).replace("{name}", str(model.name))) from None
 
     shift = None
     upscale = 1
@@ -247,8 +276,6 @@ def plan(model, values, window, slot_cols=None, dvdr=None, channels=False, ref_n
     cp.P[:] = P
     cp.frac[0], cp.frac[1] = fx, fy
     cp.pixel_area = window._area
-    cp.softening = float(model.softening)
-    cp.tolerance = float(model.sampling_tolerance)
     if kind == "flat_sky":
         cp.q, cp.pa = 1.0, 0.0
     elif getattr(model, "_is_psf", False):
@@ -283,7 +310,7 @@ def plan(model, values, window, slot_cols=None, dvdr=None, channels=False, ref_n
 
 def psf_upscale(window, psf) -> int:
     """model_object.py:313: round(window pixel length / PSF pixel length)."""
-    U = round(float(window.pixel_length) / float(psf.window.pixel_length))
+    U = round(math.sqrt(window._area) / math.sqrt(psf.window._area))
     if U < 1:
         raise SpecificationConflict("PSF pixels must not be larger than the image pixels")
     return U
@@ -312,7 +339,7 @@ def psf_render(psf_model, dev, st, slots=(), dvdr=None):
     cp = pl.cp
     n = cp.nx * cp.ny
     planes = _buffer(psf_model, "planes", 4 * cp.nchan * n, dev)
-    wsb = lib.apx_render_workspace_bytes(n)
+    wsb = _render_bytes(n)
     ws = _buffer(psf_model, "render_ws", wsb, dev)
     L.check(lib.apx_render_component(ctypes.byref(cp), L.ptr(planes), L.ptr(ws), wsb, st))
     if psf_model.normalize_psf:
@@ -374,11 +401,14 @@ def _dk_pairs(kern: Kernels, psf_cols):
     return out
 
 
+_NO_CHAN, _NO_DK = (-1,) * L.APX_MAX_CHAN, (-1, -1)
+
+
 def _new_job(pl, kh, kw):
     job = L.ConvJob()
     job.nx, job.ny, job.nchan, job.kh, job.kw = pl.cp.nx, pl.cp.ny, pl.cp.nchan, kh, kw
-    job.chan_col[:] = [-1] * L.APX_MAX_CHAN
-    job.dk_col[0] = job.dk_col[1] = -1
+    job.chan_col[:] = _NO_CHAN
+    job.dk_col[:] = _NO_DK
     return job
 
 
@@ -427,7 +457,7 @@ def render(model, values: Dict[str, torch.Tensor], req: RenderRequest):
     cp, nx, ny = pl.cp, pl.cp.nx, pl.cp.ny
     dev = AP_config.ap_device
     planes = _buffer(model, "planes", 4 * cp.nchan * ny * nx, dev)
-    wsb = lib.apx_render_workspace_bytes(nx * ny)
+    wsb = _render_bytes(nx * ny)
     ws = _buffer(model, "render_ws", wsb, dev)
     st = L.stream()
     _launch("render", nx * ny, lambda: L.check(
@@ -437,7 +467,7 @@ def render(model, values: Dict[str, torch.Tensor], req: RenderRequest):
     kern = _kernels(model, pl, dvdr, dev, st, sorted(psf_cols) if req.jac is not None else ())
     kptr, kh, kw = kern.ptr, kern.kh, kern.kw
     # crop back to the sampling window, then window-aware accumulation
-    cwsb = lib.apx_convolve_workspace_bytes(kh, kw)
+    cwsb = _convolve_bytes(kh, kw)
     cws = _buffer(model, "conv_ws", cwsb, dev)
     job = _new_job(pl, kh, kw)
     bx, by, U, out_w = pl.bx, pl.by, pl.upscale, pl.out_window
@@ -448,7 +478,7 @@ def render(model, values: Dict[str, torch.Tensor], req: RenderRequest):
         img = req.image.data
         if img.dtype != torch.float32 or not img.is_contiguous():
             raise SpecificationConflict("model image must be contiguous float32")
-        j1 = _job_copy(job)
+        j1 = job if req.jac is None else _job_copy(job)
         j1.nchan = 1
         j1.x0, j1.y0, j1.ow, j1.oh = bx + U * sx, by + U * sy, U * w, U * h
         if U == 1:
@@ -548,7 +578,7 @@ def vjp(model, values, window, G, G_window, slot_cols, dvdr, region=None):
     Gw[by + sy:by + sy + h, bx + sx:bx + sx + w] = Gc
     kern = _kernels(model, pl, dvdr, dev, st, sorted(psf_cols))
     kh, kw = kern.kh, kern.kw
-    cwsb = lib.apx_convolve_workspace_bytes(kh, kw)
+    cwsb = _convolve_bytes(kh, kw)
     cws = _buffer(model, "conv_ws", cwsb, dev)
     if pl.psf_full:
         # B = adjoint of the convolution: correlation with the unflipped taps
@@ -563,7 +593,7 @@ def vjp(model, values, window, G, G_window, slot_cols, dvdr, region=None):
     else:
         B = Gw
     value = _buffer(model, "planes", 4 * ny * nx, dev)
-    wsb = lib.apx_render_workspace_bytes(nx * ny)
+    wsb = _render_bytes(nx * ny)
     ws = _buffer(model, "render_ws", wsb, dev)
     centre_dk = pl.psf_full and pl.shift is not None and (L.APX_P_CX in slot_cols or L.APX_P_CY in slot_cols)
     psf_dk = pl.psf_full and bool(kern.dk_slots) and bool(psf_cols)

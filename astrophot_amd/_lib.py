@@ -114,6 +114,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_gpu_seen = False
 
 
 def _apply(lib, signatures) -> None:
@@ -134,9 +135,13 @@ def register(signatures) -> None:
 def load(require_gpu: bool = True):
     """Open the library (once).  Raises APXError if it is missing, or if
     ``require_gpu`` and torch sees no GPU."""
-    global _lib
-    if require_gpu and not torch.cuda.is_available():
-        raise APXError("astrophot_amd needs a HIP GPU: torch.cuda.is_available() is False")
+    global _lib, _gpu_seen
+    if _lib is not None and (_gpu_seen or not require_gpu):
+        return _lib
+    if require_gpu:
+        if not torch.cuda.is_available():
+            raise APXError("astrophot_amd needs a HIP GPU: torch.cuda.is_available() is False")
+        _gpu_seen = True
     if _lib is None:
         if not LIB_PATH.exists():
             raise APXError(f"{LIB_PATH.name} is not built; run `python -m astrophot_amd._build`")
@@ -158,4 +163,6 @@ def ptr(t) -> int:
 
 
 def stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream of the current device (its handle alone: a Stream object costs 3 us)."""
+    torch.cuda._lazy_init()
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())

@@ -258,7 +258,7 @@ class Window:
         p = self._pix(pixels)
         lo = p[:2]
         hi = p[:2] if len(p) == 2 else p[2:]
-        self.pixel_shape = (self._nx + lo[0] + hi[0], self._ny + lo[1] + hi[1])
+        self._nx, self._ny = round(self._nx + lo[0] + hi[0]), round(self._ny + lo[1] + hi[1])
         self._rij = (self._rij[0] + lo[0], self._rij[1] + lo[1])
         return self
 
@@ -309,7 +309,10 @@ class Window:
         else:  # window_object.py:483-495
             lo = (min(-0.5, o[0]), min(-0.5, o[1]))
             hi = (max(float(self._nx), e[0]), max(float(self._ny), e[1]))
-        return self.copy(origin=self._p2x(*lo), pixel_shape=(hi[0] - lo[0], hi[1] - lo[1]))
+        w = self.copy()
+        w._nx, w._ny = round(hi[0] - lo[0]), round(hi[1] - lo[1])
+        w._rij, w._rxy = (-0.5, -0.5), self._p2x(*lo)
+        return w
 
     def __and__(self, other):
         return self._box(other, "and")

@@ -26,7 +26,7 @@ from . import _engine
 from . import _lib as L
 from .errors import InvalidTarget, SpecificationConflict, UnrecognizedModel
 from .image import Jacobian_Image, Model_Image, PSF_Image, Target_Image, Window
-from .param import Param_Mask, Parameter_Node
+from .param import Param_Mask, Parameter_Node, _dval_drep1, _val_to_rep1
 
 __all__ = ["AstroPhot_Model", "Component_Model", "Galaxy_Model", "Sersic_Galaxy", "Exponential_Galaxy",
            "Gaussian_Galaxy", "Moffat_Galaxy", "Sky_Model", "Flat_Sky", "PSF_Model", "Moffat_PSF",
@@ -110,6 +110,8 @@ class AstroPhot_Model:
     def make_model_image(self, window: Optional[Window] = None):
         """core_model.py:193-204."""
         w = self.window if window is None else (self.window & window)
+        if type(self.target) is Target_Image:  # the window of target[w], without slicing its data
+            return Model_Image(window=self.target.window & w)
         return self.target[w].model_image()
 
     def fit_mask(self):
@@ -282,14 +284,16 @@ class Component_Model(AstroPhot_Model):
         aux_ids = set() if aux is None else {id(n) for n in aux.parameters._leaves()}
         out = []
         for leaf in self.parameters._leaves():
-            rep = leaf._leaf_val_to_rep(leaf.value)
-            d = leaf._leaf_dval_drep(rep).reshape(-1)
-            for e in range(leaf.size):
-                if bool(leaf.mask.reshape(-1)[e]):
+            values = leaf.value.reshape(-1).tolist()
+            keep = None if leaf._mask is None else leaf._mask.reshape(-1).tolist()
+            for e, v in enumerate(values):
+                if keep is None or keep[e]:
+                    rep = _val_to_rep1(v, *leaf.limits, leaf.cyclic)
+                    d = _dval_drep1(rep, *leaf.limits, leaf.cyclic)
                     if id(leaf) in aux_ids:
-                        out.append((_engine.PSF_SLOT0 + aux._slot_of(leaf.name, e), float(d[e])))
+                        out.append((_engine.PSF_SLOT0 + aux._slot_of(leaf.name, e), d))
                     else:
-                        out.append((self._slot_of(leaf.name, e), float(d[e])))
+                        out.append((self._slot_of(leaf.name, e), d))
         return out
 
     # -- sampling (model_object.py:258-375) ---------------------------------
@@ -350,9 +354,9 @@ class Component_Model(AstroPhot_Model):
                 self.parameters.vector_set_representation(parameters)
             else:
                 self.parameters.vector_set_values(parameters)
-        ids = list(self.parameters.vector_identities())
+        ids = self.parameters._identities()
         if pass_jacobian is None:
-            jac = self.target[window].jacobian_image(parameters=ids)
+            jac = self.target[window].jacobian_image(parameters=list(self.parameters.vector_identities()))
         else:
             jac = pass_jacobian
             for pid in ids:

@@ -66,6 +66,56 @@ def cyclic_boundaries(v, lo, hi):
     return lo + torch.remainder(_t(v) - lo, hi - lo)
 
 
+# The same maps on Python floats.  A parameter has one or two elements, so a
+# torch operation on it costs a microsecond of dispatch for a nanosecond of
+# arithmetic, and a Jacobian of two components ran several hundred of them.
+# They follow the tensor operations on infinities and NaN, where Python's own
+# would raise.
+def _inv(x):
+    return 1.0 / x if x != 0.0 else math.copysign(math.inf, x)
+
+
+def _val_to_rep1(v, lo, hi, cyclic):
+    if cyclic:
+        return lo + (v - lo) % (hi - lo)
+    if lo is None:
+        return v if hi is None else v - _inv(v - hi)
+    if hi is None:
+        return v - _inv(v - lo)
+    x = (v - lo) * math.pi / (hi - lo) - math.pi / 2
+    return math.tan(x) if math.isfinite(x) else math.nan
+
+
+def _rep_to_val1(r, lo, hi, cyclic):
+    if cyclic:
+        return lo + (r - lo) % (hi - lo)
+    if lo is None:
+        return r if hi is None else (r + hi - math.sqrt((r - hi) * (r - hi) + 4)) * 0.5
+    if hi is None:
+        return (r + lo + math.sqrt((r - lo) * (r - lo) + 4)) * 0.5
+    return (math.atan(r) + math.pi / 2) * (hi - lo) / math.pi + lo
+
+
+def _dval_drep1(r, lo, hi, cyclic):
+    if cyclic or (lo is None and hi is None):
+        return 1.0
+    if lo is None:
+        return 0.5 - 0.5 * (r - hi) / math.sqrt((r - hi) * (r - hi) + 4)
+    if hi is None:
+        return 0.5 + 0.5 * (r - lo) / math.sqrt((r - lo) * (r - lo) + 4)
+    return (hi - lo) / (math.pi * (r * r + 1))
+
+
+def _floats(v):
+    """The elements of a plain tensor as Python floats; None for one that
+    carries a graph, a tangent or a transform, which the tensor operations keep."""
+    if type(v) is not torch.Tensor or v.requires_grad or torch._C._are_functorch_transforms_active():
+        return None
+    if torch.autograd.forward_ad._current_level >= 0 or v.dtype.is_complex:
+        return None
+    return v.to(AP_config.ap_dtype).reshape(-1).tolist()
+
+
 class Parameter_Node:
     """A leaf parameter or a group of nodes (param/parameter.py:18-742)."""
 
@@ -205,10 +255,40 @@ class Parameter_Node:
             return 0 if self._value is None else int(self._value.numel())
         return sum(n.size for n in self._leaves())
 
+    def _free_leaves(self):
+        """(leaf, its number of free elements) in the order of the flat vector."""
+        return [(n, n._value.numel() if n._mask is None else int(n._mask.sum())) for n in self._leaves()]
+
+    def _plain_values(self):
+        """The flat vector as Python floats (None when a tensor has to be kept)."""
+        out = []
+        for n in self._leaves():
+            v = None if n._mask is not None else _floats(n._value)
+            if v is None:
+                return None
+            out += v
+        return out
+
+    def _plain_set(self, vec, to_value):
+        """Set every free element from a plain vector, each mapped by
+        ``to_value(leaf, element)``; False when the tensor path has to do it."""
+        v = _floats(vec)
+        leaves = None if v is None else self._free_leaves()
+        if v is None or sum(m for _, m in leaves) != len(v) or any(n._mask is not None for n, _ in leaves):
+            return False
+        k = 0
+        for n, m in leaves:
+            n._value = torch.tensor([to_value(n, x) for x in v[k:k + m]], dtype=AP_config.ap_dtype).reshape(n._value.shape)
+            k += m
+        return True
+
     # -- vector API (param/parameter.py:169-420) ---------------------------
     def vector_values(self):
         if self.leaf:
             return self._value.reshape(-1)[self.mask]
+        plain = self._plain_values()
+        if plain is not None:
+            return torch.tensor(plain, dtype=AP_config.ap_dtype)
         vec = [n.vector_values() for n in self._leaves()]
         return torch.cat(vec) if vec else torch.zeros(0, dtype=AP_config.ap_dtype)
 
@@ -226,11 +306,15 @@ class Parameter_Node:
         return np.concatenate(vec) if vec else np.array(())
 
     def vector_identities(self):
-        if self.leaf:
-            ids = [str(self.identity)] if self.size == 1 else [f"{self.identity}:{i}" for i in range(self.size)]
-            return np.array(ids)[self.mask.numpy()]
-        vec = [n.vector_identities() for n in self._leaves()]
-        return np.concatenate(vec) if vec else np.array(())
+        ids = self._identities()
+        return np.array(ids) if ids or self.leaf else np.array(())
+
+    def _identities(self):
+        """``vector_identities`` as a list."""
+        if not self.leaf:
+            return [i for n in self._leaves() for i in n._identities()]
+        ids = [str(self.identity)] if self.size == 1 else [f"{self.identity}:{i}" for i in range(self.size)]
+        return ids if self._mask is None else [i for i, keep in zip(ids, self._mask.tolist()) if keep]
 
     def vector_uncertainty(self):
         if self.leaf:
@@ -244,8 +328,7 @@ class Parameter_Node:
         """Yield (leaf, slice of vec) pairs following the masked flat order."""
         vec = _t(vec).reshape(-1)
         k = 0
-        for n in self._leaves():
-            m = int(n.vector_mask().sum())
+        for n, m in self._free_leaves():
             yield n, vec[k:k + m]
             k += m
         if k != len(vec):
@@ -256,6 +339,8 @@ class Parameter_Node:
             v = self._value.reshape(-1).clone()
             v[self.mask] = _t(values).reshape(-1)
             self._value = v.reshape(self._value.shape)
+            return
+        if self._plain_set(values, lambda n, x: x):
             return
         for n, v in self._split(values):
             n.vector_set_values(v)
@@ -323,6 +408,8 @@ class Parameter_Node:
         return self.vector_transform_val_to_rep(self.vector_values())
 
     def vector_set_representation(self, rep):
+        if not self.leaf and self._plain_set(rep, lambda n, x: _rep_to_val1(x, *n.limits, n.cyclic)):
+            return
         self.vector_set_values(self.vector_transform_rep_to_val(rep))
 
     # -- state --------------------------------------------------------------

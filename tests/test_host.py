@@ -315,3 +315,51 @@ def test_device_decode_matches_the_host_decode():
     r = values_to_rep(v)
     rd = values_to_rep_device(torch.as_tensor(v)).numpy()
     np.testing.assert_allclose(rd, r, rtol=1e-12, atol=1e-9)
+
+
+LIMITS = [((None, None), False), ((0.0, None), False), ((None, 3.0), False), ((0.36, 8.0), False), ((0.0, math.pi), True)]
+
+
+@pytest.mark.parametrize("limits,cyclic", LIMITS)
+def test_float_parameter_maps_equal_the_tensor_maps(limits, cyclic):
+    """The maps on Python floats against the tensor ones, at ordinary values,
+    at the limits, at infinities and NaN: equal to the last bits of the two
+    math libraries (4 ulp)."""
+    from astrophot_amd import param as PM
+    n = PM.Parameter_Node("p", limits=limits, cyclic=cyclic)
+    for x in (0.5, 1.3, 2.7, -4.0, 1e300, math.inf, -math.inf, math.nan, 0.36, 0.0, 3.0, 8.0):
+        t = torch.tensor(x, dtype=torch.float64)
+        for tensor_map, float_map in ((n._leaf_rep_to_val, PM._rep_to_val1), (n._leaf_val_to_rep, PM._val_to_rep1),
+                                      (n._leaf_dval_drep, PM._dval_drep1)):
+            a, b = float(tensor_map(t)), float_map(x, *limits, cyclic)
+            assert (math.isnan(a) and math.isnan(b)) or a == b or abs(a - b) <= 4 * 2.3e-16 * abs(a), (x, a, b)
+
+
+def test_plain_vectors_equal_the_tensor_path():
+    """Reading and setting the flat vector of a tree: a plain vector (Python
+    floats) and one that carries a graph (tensor operations) leave the same
+    values; a masked tree and a wrong length take the tensor path as before."""
+    from astrophot_amd.errors import InvalidParameter
+    from astrophot_amd.param import Param_Mask, Parameter_Node
+
+    def tree():
+        top = Parameter_Node("top")
+        for k, (lim, cyc) in enumerate(LIMITS):
+            top.link(Parameter_Node(f"p{k}", value=[1.1, 2.1] if k == 0 else 1.3 + 0.1 * k, limits=lim, cyclic=cyc))
+        return top
+
+    a, b = tree(), tree()
+    rep = a.vector_representation() * 1.01 + 0.01
+    a.vector_set_representation(rep)
+    b.vector_set_representation(rep.clone().requires_grad_(True))
+    assert not a["p0"].value.requires_grad and b["p0"].value.requires_grad
+    assert torch.allclose(a.vector_values(), b.vector_values().detach(), rtol=1e-15, atol=0)
+    assert [n.value.shape for n in a._leaves()] == [n.value.shape for n in b._leaves()]
+    assert list(a.vector_identities()) == a._identities() and len(a._identities()) == 6
+    a.vector_set_values(b.vector_values().detach())
+    assert torch.equal(a.vector_values(), b.vector_values().detach())
+    with Param_Mask(a, torch.tensor([True, False, True, True, False, True])):
+        assert len(a.vector_values()) == len(a._identities()) == len(a.vector_identities()) == 4
+        a.vector_set_values(a.vector_values() * 1.001)
+    with pytest.raises((InvalidParameter, RuntimeError)):
+        a.vector_set_values(torch.ones(9, dtype=torch.float64))
