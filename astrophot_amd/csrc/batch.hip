@@ -83,20 +83,15 @@ struct Scratch {
   int2* chunk_list;   // nchunk
   int2* tile_list;    // ntile
   int32_t* gal_cnt;   // ngal: pixels each fit sends to the level-2 quadrature
-  int32_t* gal_off;   // ngal + 1: exclusive prefix of gal_cnt
   int32_t* deep;      // nwork: per-fit segments (at work_off) of those pixels
-  int2* dq;           // nwork: the same list after the scan, (fit, pixel) in global order
-  int2* rq;           // nwork: the scanned redo list in the same form
+  int2* dq;           // nwork: the same pixels as one list of (fit, pixel)
+  int2* rq;           // nwork: the redo list in the same form
   int32_t* gal_rcnt;  // ngal: pixels each fit sends to a float64 redo pass
-  int32_t* gal_roff;  // ngal + 1: exclusive prefix of gal_rcnt
   int32_t* redo;      // nwork: per-fit segments of those pixels
   float* mid;         // nwork: midpoint samples
   double* part;       // ntile * kPart: per-tile partial sums of the reductions
   GalEval* ev;        // ngal
-  int32_t* bsum;      // ceil(ngal / kScanBlock): block totals of the count scans
 };
-
-constexpr int kScanBlock = 1024;  // counts per workgroup of the two-pass scan
 
 constexpr int kPart = 64;  // doubles per tile partial (49 H + 7 g + 1 chi2 fit the largest)
 
@@ -126,17 +121,14 @@ __host__ inline int64_t scratch_layout(const apx_batch& b, Scratch* s, TrialBran
   t.chunk_list = reinterpret_cast<int2*>(take(8 * b.nchunk));
   t.tile_list = reinterpret_cast<int2*>(take(8 * b.ntile));
   t.gal_cnt = reinterpret_cast<int32_t*>(take(4 * (int64_t)b.ngal));
-  t.gal_off = reinterpret_cast<int32_t*>(take(4 * ((int64_t)b.ngal + 1)));
   t.deep = reinterpret_cast<int32_t*>(take(4 * b.nwork));
   t.dq = reinterpret_cast<int2*>(take(8 * b.nwork));
   t.rq = reinterpret_cast<int2*>(take(8 * b.nwork));
   t.gal_rcnt = reinterpret_cast<int32_t*>(take(4 * (int64_t)b.ngal));
-  t.gal_roff = reinterpret_cast<int32_t*>(take(4 * ((int64_t)b.ngal + 1)));
   t.redo = reinterpret_cast<int32_t*>(take(4 * b.nwork));
   t.mid = reinterpret_cast<float*>(take(4 * b.nwork));
   t.part = reinterpret_cast<double*>(take(8 * kPart * b.ntile));
   t.ev = reinterpret_cast<GalEval*>(take((int64_t)sizeof(GalEval) * b.ngal));
-  t.bsum = reinterpret_cast<int32_t*>(take(4 * (((int64_t)b.ngal + kScanBlock - 1) / kScanBlock)));
   if (copy == 0 && s) *s = t;
   if (copy == 1 && tb) tb->s = t;
   }
@@ -163,12 +155,6 @@ __host__ int64_t scratch_bytes(const apx_batch& b) {
 
 __device__ __forceinline__ GalState* st_of(const apx_batch& b, int g) {
   return reinterpret_cast<GalState*>(b.state) + g;
-}
-
-__device__ __forceinline__ double wsum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
 }
 
 // ---------------------------------------------------------------------------
@@ -316,8 +302,8 @@ __device__ void prepare_separable_axis(const apx_batch& b, const apx_batch_galax
     S += v;
     Sd += d;
   }
-  S = wsum(S);
-  Sd = wsum(Sd);
+  S = wave_sum(S);
+  Sd = wave_sum(Sd);
   const double iS = 1.0 / S;
   float* kt = b.taps + G.tap_off;
   float* o = kt + (w == 0 ? 0 : H4);
@@ -367,7 +353,7 @@ __global__ __launch_bounds__(256) void prepare_kernel(apx_batch b, Scratch s, in
       Sy += ddy;
     }
     auto bsum = [&](double x) {
-      x = wsum(x);
+      x = wave_sum(x);
       __syncthreads();
       if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
       __syncthreads();
@@ -441,6 +427,18 @@ __device__ __forceinline__ float sersic_f(const Prof<float>& p, float X, float Y
     g[APX_P_C] = I * (float)kLn10;
   }
   return I;
+}
+
+// sersic_f's value with every multiply-add written out.  Which of two products
+// the compiler folds into an addition depends on the code around it, and with it
+// the sample's last bit; the level-3 pass keeps this one whatever its shape.
+__device__ __forceinline__ float sersic_value_f(const Prof<float>& p, float X, float Y, float scale) {
+  const float Xr = fmaf(p.c, X, -(p.s * Y));
+  const float Yr = fmaf(p.s, X, p.c * Y) * p.invq;
+  const float R2 = fmaf(Xr, Xr, Yr * Yr) + p.soft2;
+  const float l2 = fmaf(0.5f, __builtin_amdgcn_logf(R2), p.l2s);
+  const float pw = __builtin_amdgcn_exp2f(l2 * p.inva);
+  return p.amp * scale * __builtin_amdgcn_exp2f(p.nbl2e * (pw - 1.0f));
 }
 
 struct QuadTab {
@@ -765,6 +763,56 @@ __global__ __launch_bounds__(256) void select_kernel(apx_batch b, Scratch s, Qua
   }
 }
 
+// The per-fit segments of pixels (a count and a run at work_off each) as one list
+// of (fit, pixel), so that the passes over it take any fit's pixels evenly: a
+// workgroup takes `fits` of the listed fits (at most kPackFits) and one place in
+// the list (one atomic on its length).  The order of the workgroups' runs in the
+// list does not matter: every pixel is taken by itself.  One launch a list in
+// place of two for a scan and a compaction, with three lists a stage:
+// 56 -> 38 launches a tick (4,096 fits to convergence, with the level-3 pass by
+// waves below: 117.5 -> 102.4 ms).
+// `clear`: the counts start from zero again.
+constexpr int kPackFits = 8;
+
+__global__ __launch_bounds__(256) void pack_kernel(apx_batch b, Scratch s, int fits, int32_t* __restrict__ cnt,
+                                                   const int32_t* __restrict__ seg, int2* __restrict__ out,
+                                                   int32_t* len, int clear) {
+  __shared__ int pre[kPackFits + 1], fit[kPackFits], base;
+  __shared__ int64_t off[kPackFits];
+  for (int first = blockIdx.x * fits; first < s.cnt[0]; first += gridDim.x * fits) {
+    __syncthreads();  // the previous run is read
+    if (threadIdx.x < kPackFits) {
+      const int i = first + (int)threadIdx.x;
+      int n = 0, g = 0;
+      if ((int)threadIdx.x < fits && i < s.cnt[0]) {
+        g = s.gal_list[i];
+        n = cnt[g];
+        if (clear) cnt[g] = 0;
+      }
+      fit[threadIdx.x] = g;
+      off[threadIdx.x] = b.gal[g].work_off;
+      int x = n;
+#pragma unroll
+      for (int o = 1; o < kPackFits; o <<= 1) {
+        const int y = __shfl_up(x, o, 64);
+        if ((int)threadIdx.x >= o) x += y;
+      }
+      pre[threadIdx.x + 1] = x;
+      if (threadIdx.x == 0) pre[0] = 0;
+      if (threadIdx.x == kPackFits - 1 && x > 0) base = atomicAdd(len, x);
+    }
+    __syncthreads();
+    const int total = pre[kPackFits];
+    for (int e = threadIdx.x; e < total; e += 256) {
+      int f = 0;
+#pragma unroll
+      for (int o = kPackFits / 2; o > 0; o >>= 1)
+        if (e >= pre[f + o]) f += o;
+      out[base + e] = make_int2(fit[f], seg[off[f] + (e - pre[f])]);
+    }
+  }
+}
+
 // the pixels select_kernel left undecided, with float64 decisions
 template <bool GRAD, int QN>
 __global__ __launch_bounds__(256) void select_redo_kernel(apx_batch b, Scratch s, QuadTab t) {
@@ -776,92 +824,6 @@ __global__ __launch_bounds__(256) void select_redo_kernel(apx_batch b, Scratch s
     if (select_pixel<GRAD, true, QN>(b, s, G, s.ev[g], t, pix) == PX_DEEPER)
       s.deep[G.work_off + atomicAdd(&s.gal_cnt[g], 1)] = pix;
   }
-}
-
-// exclusive prefix of n per-fit counts: off[0..n], *total = off[n]; the
-// counts are cleared after reading when `clear`.  Two passes over blocks of
-// kScanBlock counts, both coalesced: the block totals, then each block adds
-// the totals of the blocks before it (read in index order) to its own scan.
-__global__ __launch_bounds__(256) void scan_totals_kernel(int n, const int32_t* __restrict__ cnt,
-                                                          int32_t* __restrict__ bsum) {
-  __shared__ int32_t red[4];
-  const int base = blockIdx.x * kScanBlock;
-  int v = 0;
-#pragma unroll
-  for (int k = 0; k < kScanBlock / 256; ++k) {
-    const int g = base + k * 256 + (int)threadIdx.x;
-    v += g < n ? cnt[g] : 0;
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) bsum[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
-}
-
-__global__ __launch_bounds__(256) void scan_apply_kernel(int n, int32_t* __restrict__ cnt,
-                                                         int32_t* __restrict__ off,
-                                                         int32_t* __restrict__ total,
-                                                         const int32_t* __restrict__ bsum, int clear) {
-  __shared__ __align__(16) int32_t vals[kScanBlock];
-  __shared__ int32_t wsums[4];
-  __shared__ int32_t pre_s;
-  const int nb = gridDim.x, base = blockIdx.x * kScanBlock;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  // totals of the blocks before this one, summed in index order
-  if (wv == 0) {
-    int p = 0;
-    for (int q = lane; q < (int)blockIdx.x; q += 64) p += bsum[q];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) p += __shfl_xor(p, o, 64);
-    if (lane == 0) pre_s = p;
-  }
-#pragma unroll
-  for (int k = 0; k < kScanBlock / 256; ++k) {
-    const int e = k * 256 + (int)threadIdx.x, g = base + e;
-    vals[e] = g < n ? cnt[g] : 0;
-    if (clear && g < n) cnt[g] = 0;
-  }
-  __syncthreads();
-  // each thread scans 4 consecutive counts; the thread totals scan across the block
-  int4 q4 = *reinterpret_cast<const int4*>(vals + 4 * threadIdx.x);
-  const int tsum = q4.x + q4.y + q4.z + q4.w;
-  int x = tsum;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_up(x, o, 64);
-    if (lane >= o) x += y;
-  }
-  if (lane == 63) wsums[wv] = x;
-  __syncthreads();
-  int pw = 0;
-  for (int w = 0; w < wv; ++w) pw += wsums[w];
-  int acc = pre_s + pw + x - tsum;
-  int4 o4;
-  o4.x = acc; acc += q4.x;
-  o4.y = acc; acc += q4.y;
-  o4.z = acc; acc += q4.z;
-  o4.w = acc; acc += q4.w;
-  __syncthreads();
-  *reinterpret_cast<int4*>(vals + 4 * threadIdx.x) = o4;
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < kScanBlock / 256; ++k) {
-    const int e = k * 256 + (int)threadIdx.x, g = base + e;
-    if (g < n) off[g] = vals[e];
-  }
-  if (blockIdx.x == nb - 1 && threadIdx.x == 255) {
-    off[n] = acc;  // the last thread's running sum is the grand total
-    *total = acc;
-  }
-}
-
-// the scan of n counts (two launches)
-inline void scan_counts(int n, int32_t* cnt, int32_t* off, int32_t* total, int32_t* bsum, int clear,
-                        hipStream_t stream) {
-  const int nb = (n + kScanBlock - 1) / kScanBlock;
-  hipLaunchKernelGGL(scan_totals_kernel, dim3(nb), dim3(256), 0, stream, n, cnt, bsum);
-  hipLaunchKernelGGL(scan_apply_kernel, dim3(nb), dim3(256), 0, stream, n, cnt, off, total, bsum, clear);
 }
 
 // levels 2 and 3 of the quadrature (operations.py:229-247): a group of GS
@@ -1015,8 +977,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void i
 #pragma unroll
     for (int q = 0; q <= APX_NSLOT; ++q) {
       if (!GRAD && q > 0) break;
-#pragma unroll
-      for (int o = GS / 2; o > 0; o >>= 1) acc[q] += __shfl_xor(acc[q], o, 64);
+      acc[q] = GS == 64 ? wave_sum(acc[q]) : half_sum(acc[q]);
     }
     if (active && gl == 0) {
       const int64_t wo = b.gal[gal].work_off;
@@ -1041,9 +1002,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void i
 // refined pixels at a time (250 of its 256 lanes; a 32-lane group per pixel
 // keeps only 25 busy).  Each lane integrates its sub-pixel with the 3 x 3
 // Gauss-Legendre rule; the sub-pixels the level-2 test flags are collected in
-// workgroup order and integrated one after another by the whole workgroup (225
-// level-3 samples over 256 lanes); the 25 sub-pixel sums of a pixel are added
-// in float64 in sub-pixel order.  Same decisions and outputs as
+// workgroup order and integrated a wave each (225 level-3 samples); the 25
+// sub-pixel sums of a pixel are added in float64 in sub-pixel order.  Same decisions and outputs as
 // integrate_kernel<..., F64 = false, 3, 5>; a pixel with an undecided test goes
 // to the redo list unwritten.
 //
@@ -1059,7 +1019,6 @@ template <bool GRAD>
 __global__ __launch_bounds__(256) void integrate_wg_kernel(apx_batch b, Scratch s, QuadTab t) {
   constexpr int NV = GRAD ? 1 + APX_NSLOT : 1;
   __shared__ double sums[NV][256];     // per-lane sub-pixel totals (level 2 or 3)
-  __shared__ float red[NV][4];         // per-wave level-3 partials
   __shared__ int flagged[256];         // slots whose sub-pixel goes to level 3, in slot order
   __shared__ int wcnt[4], undec[kWgPix], nflag;
   __shared__ float fx[256], fy[256];   // level-2 sub-pixel centres (plane offsets)
@@ -1074,22 +1033,30 @@ __global__ __launch_bounds__(256) void integrate_wg_kernel(apx_batch b, Scratch 
   // log2 of the level-2 scale ig^2 times the corner, edge and centre weights
   const float l2sc = 2.0f * __builtin_amdgcn_logf(ig);
   const float lwc = l2sc + t.lw[0], lwe = l2sc + t.lw[1], lw0 = l2sc + t.lw[4];
-  // level-3 sample of this lane (225 of 256): sub-sub-pixel tt, node kk
-  float l3x = 0.0f, l3y = 0.0f, l3w = 0.0f;
-  if (slot < 225) {
-    const int tt = slot / 9, kk = slot % 9;
+  // level-3 samples of this lane, 64 rd + lane (225 in all): sub-sub-pixel tt, node kk
+  float l3x[4], l3y[4], l3w[4];
+#pragma unroll
+  for (int rd = 0; rd < 4; ++rd) {
+    const int e = 64 * rd + lane;
+    l3x[rd] = l3y[rd] = l3w[rd] = 0.0f;
+    if (e >= 225) continue;
+    const int tt = e / 9, kk = e % 9;
     const float h3 = 0.5f * ig * ig;
-    const float a = (sub0 + subd * (float)(tt % 5)) * ig, c = (sub0 + subd * (float)(tt / 5)) * ig;
-    const float u = a + h3 * t.node[kk % 3], v = c + h3 * t.node[kk / 3];
-    l3x = P00 * u + P01 * v;
-    l3y = P10 * u + P11 * v;
-    l3w = t.w2[kk];
+    // written out: the last round's tt / 5 is a constant, and the compiler would fold it differently
+    const float nu = h3 * t.node[kk % 3], nv = h3 * t.node[kk / 3];
+    const float u = fmaf(ig, fmaf(subd, (float)(tt % 5), sub0), nu), v = fmaf(ig, fmaf(subd, (float)(tt / 5), sub0), nv);
+    l3x[rd] = fmaf(P00, u, P01 * v);
+    l3y[rd] = fmaf(P10, u, P11 * v);
+    l3w[rd] = t.w2[kk];
   }
   const float sc3 = ig * ig * ig * ig;
   int nsub3 = 0;
-  for (int k0 = blockIdx.x * kWgPix; k0 < total; k0 += gridDim.x * kWgPix) {
+  // pixels a workgroup takes at once: fewer than kWgPix where the list is short,
+  // so that it spreads over the CUs
+  const int np = max(1, min(kWgPix, (total + (int)gridDim.x - 1) / (int)gridDim.x));
+  for (int k0 = blockIdx.x * np; k0 < total; k0 += gridDim.x * np) {
     const int k = k0 + px;
-    const bool active = px < kWgPix && k < total;
+    const bool active = px < np && k < total;
     int gal = 0, pix = 0;
     if (active) {
       const int2 q = s.dq[k];
@@ -1146,38 +1113,50 @@ __global__ __launch_bounds__(256) void integrate_wg_kernel(apx_batch b, Scratch 
     __syncthreads();
     const int nf = nflag;
     nsub3 += nf;
-    // level 3: the whole workgroup on each flagged sub-pixel in turn
-    for (int f = 0; f < nf; ++f) {
+    // level 3: a wave a flagged sub-pixel, its 225 samples as 4 rounds of 64 lanes,
+    // each round summed over the wave.  (The whole workgroup on one sub-pixel after
+    // another took two barriers and an LDS round trip each; here the flagged
+    // sub-pixels of ten pixels run four abreast.)
+    for (int f = w; f < nf; f += 4) {
       const int fs = flagged[f];
       const GalEval* F = s.ev + fgal[fs / kWgSub];
       const Prof<float> pg = F->pf;
-      float v[NV];
+      const float cx = fx[fs], cy = fy[fs];
+      double tot[NV];
 #pragma unroll
-      for (int q = 0; q < NV; ++q) v[q] = 0.0f;
-      if (slot < 225) {
-        float gv[APX_NSLOT];
-        const float val = sersic_f<GRAD>(pg, fx[fs] + l3x, fy[fs] + l3y, sc3, gv);
-        v[0] = l3w * val;
-        if (GRAD) {
+      for (int rd = 0; rd < 4; ++rd) {
+        float v[NV];
 #pragma unroll
-          for (int q = 0; q < APX_NSLOT; ++q) v[1 + q] = l3w * gv[q];
+        for (int q = 0; q < NV; ++q) v[q] = 0.0f;
+        if (rd < 3 || lane < 225 - 192) {
+          float gv[APX_NSLOT];
+          const float X = cx + l3x[rd], Y = cy + l3y[rd];
+          const float val = GRAD ? sersic_f<true>(pg, X, Y, sc3, gv) : sersic_value_f(pg, X, Y, sc3);
+          {
+            // the weighted sample is rounded before the sum over the wave (not
+            // folded into its first addition), whether the round is full or not
+#pragma clang fp contract(off)
+            v[0] = l3w[rd] * val;
+            if (GRAD) {
+#pragma unroll
+              for (int q = 0; q < APX_NSLOT; ++q) v[1 + q] = l3w[rd] * gv[q];
+            }
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < NV; ++q) {
+          const double r = (double)wave_sum(v[q]);
+          tot[q] = rd == 0 ? r : tot[q] + r;
         }
       }
+      if (lane == 0) {
 #pragma unroll
-      for (int q = 0; q < NV; ++q) {
-        float x = v[q];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-        if (lane == 0) red[q][w] = x;
+        for (int q = 0; q < NV; ++q) sums[q][fs] = tot[q];
       }
-      __syncthreads();
-      if (slot < NV) {
-        sums[slot][fs] = (double)red[slot][0] + (double)red[slot][1] + (double)red[slot][2] + (double)red[slot][3];
-      }
-      __syncthreads();
     }
+    __syncthreads();
     // per pixel and channel: the 25 sub-pixel totals in order
-    if (slot < kWgPix * NV) {
+    if (slot < np * NV) {
       const int p = slot / NV, q = slot % NV;
       const int kk = k0 + p;
       if (kk < total && !undec[p]) {
@@ -1319,7 +1298,7 @@ __device__ __forceinline__ void tile_partial(double (&redd)[4][8], const double*
                                              int lane, int w) {
 #pragma unroll
   for (int i = 0; i < W; ++i) {
-    const double v = wsum(rd[i]);
+    const double v = wave_sum(rd[i]);
     if (lane == 0) redd[w][i] = v;
   }
   __syncthreads();
@@ -1875,10 +1854,10 @@ __global__ __launch_bounds__(256) void normal_kernel(apx_batch b, Scratch s) {
     for (int i = 0; i < 4; ++i) redH[wv][(4 * kq + i) * 16 + r16] = (double)acc[i];
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
-      const double gd = wsum((double)gl[i]);
+      const double gd = wave_sum((double)gl[i]);
       if (lane == 0) redg[wv][i] = gd;
     }
-    cacc = wsum(cacc);
+    cacc = wave_sum(cacc);
     if (lane == 0) redc[wv] = cacc;
     __syncthreads();
     double* part = s.part + (G.tile_off + e.y) * kPart;  // H row-major, g, chi2
@@ -2338,26 +2317,13 @@ QuadTab quad_table(const apx_batch& b) {
   return t;
 }
 
-// a scanned per-fit list (segments at work_off, exclusive prefix off) as
-// (fit, pixel) pairs in global order, one wave per fit, so the passes over it
-// read each entry's fit instead of searching the offsets
-__global__ __launch_bounds__(256) void compact_list_kernel(apx_batch b, Scratch s, const int32_t* off,
-                                                           const int32_t* list, int2* out) {
-  const int lane = threadIdx.x & 63;
-  // only the fits listed for the stage have entries (build_kernel clears every count)
-  for (int i = blockIdx.x * 4 + (int)(threadIdx.x >> 6); i < s.cnt[0]; i += gridDim.x * 4) {
-    const int g = s.gal_list[i];
-    const int a = off[g], n = off[g + 1] - a;
-    if (n == 0) continue;
-    const int32_t* src = list + b.gal[g].work_off;
-    for (int j = lane; j < n; j += 64) out[a + j] = make_int2(g, src[j]);
-  }
-}
-
-inline void compact_list(const apx_batch& b, const Scratch& s, const int32_t* off, const int32_t* list,
-                         int2* out, hipStream_t stream) {
-  hipLaunchKernelGGL(compact_list_kernel, dim3(std::min((b.ngal + 3) / 4, 16384)), dim3(256), 0, stream, b, s,
-                     off, list, out);
+// the packed list of the segments `seg` with counts `cnt`; few fits go a workgroup
+// each, their runs are the longer for it (125 scene sources: 100^2 to 420^2 pixels)
+inline void pack_list(const apx_batch& b, const Scratch& s, int32_t* cnt, const int32_t* seg, int2* out, int32_t* len,
+                      int clear, hipStream_t stream) {
+  const int fits = std::max(1, std::min(kPackFits, b.ngal / 512));
+  hipLaunchKernelGGL(pack_kernel, dim3(std::min((b.ngal + fits - 1) / fits, 8192)), dim3(256), 0, stream, b, s, fits,
+                     cnt, seg, out, len, clear);
 }
 
 // the lane grouping of a stage's level-2/3 pass: the Jacobian stage takes
@@ -2379,8 +2345,7 @@ void launch_integrate(const apx_batch& b, const Scratch& s, const QuadTab& t, bo
     else hipLaunchKernelGGL((integrate_kernel<false, GS, false, QN, QG>), ig, dim3(256), 0, stream, b, s, t);
   }
   if (float_pass_only) return;
-  scan_counts(b.ngal, s.gal_rcnt, s.gal_roff, s.cnt + 5, s.bsum, 0, stream);
-  compact_list(b, s, s.gal_roff, s.redo, s.rq, stream);
+  pack_list(b, s, s.gal_rcnt, s.redo, s.rq, s.cnt + 5, 0, stream);
   if (jac) hipLaunchKernelGGL((integrate_kernel<true, GS, true, QN, QG>), ig, dim3(256), 0, stream, b, s, t);
   else hipLaunchKernelGGL((integrate_kernel<false, GS, true, QN, QG>), ig, dim3(256), 0, stream, b, s, t);
 }
@@ -2402,12 +2367,10 @@ void render_launches(const apx_batch& b, const Scratch& s, const QuadTab& t, boo
   // float64 redo of undecided selections, then the level-2/3 quadrature of
   // the deep list, then its undecided pixels in float64
   const dim3 ig(b.quad_blocks > 0 ? b.quad_blocks : kPersist / 2);
-  scan_counts(b.ngal, s.gal_rcnt, s.gal_roff, s.cnt + 4, s.bsum, 1, stream);
-  compact_list(b, s, s.gal_roff, s.redo, s.rq, stream);
+  pack_list(b, s, s.gal_rcnt, s.redo, s.rq, s.cnt + 4, 1, stream);
   if (jac) hipLaunchKernelGGL((select_redo_kernel<true, QN>), ig, dim3(256), 0, stream, b, s, t);
   else hipLaunchKernelGGL((select_redo_kernel<false, QN>), ig, dim3(256), 0, stream, b, s, t);
-  scan_counts(b.ngal, s.gal_cnt, s.gal_off, s.cnt + 3, s.bsum, 0, stream);
-  compact_list(b, s, s.gal_off, s.deep, s.dq, stream);
+  pack_list(b, s, s.gal_cnt, s.deep, s.dq, s.cnt + 3, 0, stream);
   if (t.gg <= 32 && stage_group(b, jac) != 64) launch_integrate<32, QN, QG>(b, s, t, jac, stream);
   else launch_integrate<64, QN, QG>(b, s, t, jac, stream);
 }

@@ -22,6 +22,7 @@
 
 #include "capi_internal.h"
 #include "conv_common.h"
+#include "wave.h"
 
 namespace apx {
 
@@ -33,8 +34,7 @@ constexpr int kTY = 16;   // output tile height (4 waves x kRY)
 constexpr int kKR = 32;   // kernel rows staged per pass
 
 __device__ __forceinline__ double block_sum256(double v, double* red) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  v = wave_sum(v);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
@@ -43,8 +43,7 @@ __device__ __forceinline__ double block_sum256(double v, double* red) {
 
 // sum over a 1024-thread workgroup (every thread gets it)
 __device__ __forceinline__ double block_sum1024(double v, double* red) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  v = wave_sum(v);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();

@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include "capi_internal.h"
+#include "wave.h"
 
 namespace apx {
 
@@ -26,12 +27,6 @@ namespace {
 constexpr int kTW = 64, kTH = 16;  // image tile
 constexpr int kNB = 32;            // Cholesky panel
 constexpr int kUT = 64;            // trailing-update tile
-
-__device__ __forceinline__ double wsum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
 
 // lane `src`'s v to every lane (src uniform): two v_readlane_b32 into SGPRs,
 // no LDS round trip
@@ -126,7 +121,7 @@ __global__ __launch_bounds__(256) void group_jtv_kernel(apx_group g, const float
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
 #pragma unroll
   for (int k = 0; k < APX_BATCH_NP; ++k) {
-    const double t = wsum(acc[k]);
+    const double t = wave_sum(acc[k]);
     if (lane == 0) red[wv][k] = t;
   }
   __syncthreads();
@@ -158,8 +153,8 @@ __global__ __launch_bounds__(256) void group_image_sums_kernel(int64_t npix, int
     a += w;
     b += w * ((double)data[p] - (double)model[p]);
   }
-  a = wsum(a);
-  b = wsum(b);
+  a = wave_sum(a);
+  b = wave_sum(b);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   if (lane == 0) {
     red[0][wv] = a;
@@ -226,7 +221,7 @@ __global__ __launch_bounds__(256) void group_source_kernel(apx_group g, const fl
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
 #pragma unroll
   for (int k = 0; k < APX_BATCH_NP; ++k) {
-    const double t0 = wsum(ag[k]), t1 = wsum(ah[k]);
+    const double t0 = wave_sum(ag[k]), t1 = wave_sum(ah[k]);
     if (lane == 0) {
       red[wv][k] = t0;
       red[wv][APX_BATCH_NP + k] = t1;
@@ -286,7 +281,7 @@ __global__ __launch_bounds__(256) void group_pair_kernel(apx_group g, const floa
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
 #pragma unroll
   for (int k = 0; k < NN; ++k) {
-    const double t = wsum(acc[k]);
+    const double t = wave_sum(acc[k]);
     if (lane == 0) red[wv][k] = t;
   }
   __syncthreads();

@@ -12,6 +12,7 @@
 #include <mutex>
 
 #include "capi_internal.h"
+#include "wave.h"
 
 namespace apx {
 
@@ -23,12 +24,6 @@ constexpr int kBlocks = 512;
 constexpr int kMaxNp = 16;
 
 __host__ __device__ inline int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
-
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
 
 __global__ __launch_bounds__(256) void chi2_partial_kernel(const float* __restrict__ model,
                                                            const float* __restrict__ data,

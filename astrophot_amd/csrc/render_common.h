@@ -7,14 +7,9 @@
 
 #include "../../include/astrophot_hip.h"
 #include "profile.h"
+#include "wave.h"
 
 namespace apx {
-
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
 
 // offsets of a working pixel from the centre
 template <typename T>

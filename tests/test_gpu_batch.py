@@ -82,6 +82,34 @@ def test_batch_render_matches_oracle(quad_group):
         assert float(((got - ref).abs() / ref)[bright].max()) < 1e-5, k
 
 
+@pytest.mark.parametrize("quad_group", [32, 25])
+@pytest.mark.parametrize("n", [2, 9, 513, 1100, 4099])
+def test_refined_pixel_lists_of_any_fit_count(n, quad_group):
+    """The lists of refined and undecided pixels are packed several fits a
+    workgroup, by their number: below 1,024 fits one, from 4,096 eight.  A fit's
+    render and Jacobian have the same bits whichever others share the lists, so
+    the first, a middle and the last fit equal a batch of that fit alone."""
+    truths, shapes, _ = make_cutouts(7, seed=11, sizes=(16, 33))
+    which = np.arange(n) % 7
+    cut = [Cutout(np.zeros((s, s)), np.ones((s, s)), psf) for s, psf in shapes]
+
+    def images(idx):
+        bf = BatchFit([cut[i] for i in idx])
+        bf.b.quad_group = quad_group
+        rep = values_to_rep(np.stack([truths[i] for i in idx]))
+        img, J = bf.jacobian(rep)
+        cols = [bf.split(J[:, c].contiguous()) for c in range(7)]
+        return bf.split(bf.render(rep)), bf.split(img), cols
+
+    many = images(which)
+    for k in {0, n // 2, n - 1}:
+        one = images(which[k:k + 1])
+        assert torch.equal(many[0][k], one[0][0])
+        assert torch.equal(many[1][k], one[1][0])
+        for jm, jo in zip(many[2], one[2]):
+            assert torch.equal(jm[k], jo[0])
+
+
 def test_batch_jacobian_matches_single_model():
     """apx_batch_jacobian: every cutout's model and its 7 representation-space
     Jacobian columns equal the single-model jacobian(as_representation=True)
