@@ -100,35 +100,85 @@ __global__ __launch_bounds__(256) void group_rpp_weights_kernel(apx_group g, con
   }
 }
 
-// out[col0 + k] = sum over the window of J_k * v (v a double image)
+// A window (or an overlap of two) of n pixels goes to several workgroups: at
+// most S pieces, of at least kPiece pixels, so that the largest (400 x 400 beside
+// a median overlap of 4,500 pixels) does not set the pass's time.  One workgroup
+// a window: pairs, sources and J^T v of 500 sources on 2048^2 (3,051 pairs, 35 M
+// pair pixels) took 0.94, 0.73 and 0.43 ms; in pieces 0.33, 0.16 and 0.12 ms.
+constexpr int kPiece = 4096;
+
+struct Piece {
+  int x, y, dx, dy, w;  // this thread's pixel, and the step of 256 pixels
+  int64_t e, e1;        // its index, and the end of the piece
+  // piece s of at most S of a w x h rectangle; false: no such piece
+  __device__ __forceinline__ bool open(int w_, int h, int s, int S) {
+    const int64_t n = (int64_t)w_ * h;
+    const int64_t np = min((int64_t)S, max((int64_t)1, (n + kPiece - 1) / kPiece)), len = (n + np - 1) / np;
+    if (s >= np) return false;
+    w = w_;
+    e = s * len + threadIdx.x;
+    e1 = min(n, (s + 1) * len);
+    if (w > 0) {
+      y = (int)(e / w);
+      x = (int)(e - (int64_t)y * w);
+      dy = 256 / w;
+      dx = 256 - dy * w;
+    }
+    return true;
+  }
+  __device__ __forceinline__ void next() {
+    e += 256;
+    x += dx;
+    y += dy;
+    if (x >= w) {
+      x -= w;
+      ++y;
+    }
+  }
+};
+__device__ __forceinline__ int pieces_of(int64_t n, int S) {
+  return (int)min((int64_t)S, max((int64_t)1, (n + kPiece - 1) / kPiece));
+}
+// the most pieces a window gets when `count` of them share the chip
+inline int max_pieces(int count) { return std::max(1, std::min(16, 32768 / std::max(1, count))); }
+
+// part[s S + piece][k] = sum over the piece of the window of J_k * v (v a double image)
 __global__ __launch_bounds__(256) void group_jtv_kernel(apx_group g, const float* __restrict__ J,
-                                                        const double* __restrict__ v,
-                                                        double* __restrict__ out) {
+                                                        const double* __restrict__ v, int S,
+                                                        double* __restrict__ part) {
   __shared__ double red[4][APX_BATCH_NP];
-  const int s = blockIdx.x;
+  const int s = blockIdx.x / S;
   const int* w = g.win + 4 * s;
-  const int64_t n = (int64_t)w[2] * w[3];
+  const int w0 = w[0], w1 = w[1];
+  Piece t;
+  if (!t.open(w[2], w[3], blockIdx.x % S, S)) return;
   double acc[APX_BATCH_NP];
 #pragma unroll
   for (int k = 0; k < APX_BATCH_NP; ++k) acc[k] = 0.0;
-  for (int64_t e = threadIdx.x; e < n; e += 256) {
-    const int dy = (int)(e / w[2]), dx = (int)(e % w[2]);
-    const double vv = v[(int64_t)(w[1] + dy) * g.nx + (w[0] + dx)];
-    const int64_t q = g.pix_off[s] + e;
+  const float* Js = J + g.pix_off[s];
+  for (; t.e < t.e1; t.next()) {
+    const double vv = v[(int64_t)(w1 + t.y) * g.nx + (w0 + t.x)];
 #pragma unroll
-    for (int k = 0; k < APX_BATCH_NP; ++k) acc[k] += (double)J[(int64_t)k * g.nsrcpix + q] * vv;
+    for (int k = 0; k < APX_BATCH_NP; ++k) acc[k] += (double)Js[(int64_t)k * g.nsrcpix + t.e] * vv;
   }
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-  for (int k = 0; k < APX_BATCH_NP; ++k) {
-    const double t = wave_sum(acc[k]);
-    if (lane == 0) red[wv][k] = t;
-  }
+  wave_sums(acc, red[threadIdx.x >> 6]);
   __syncthreads();
   if (threadIdx.x < APX_BATCH_NP) {
     const int k = threadIdx.x;
-    out[g.col0[s] + k] = red[0][k] + red[1][k] + red[2][k] + red[3][k];
+    part[(int64_t)blockIdx.x * APX_BATCH_NP + k] = red[0][k] + red[1][k] + red[2][k] + red[3][k];
   }
+}
+
+// out[col0 + k] = the sum of the source's pieces, in order
+__global__ __launch_bounds__(256) void group_jtv_final_kernel(apx_group g, int S, const double* __restrict__ part,
+                                                              double* __restrict__ out) {
+  const int e = blockIdx.x * 256 + threadIdx.x;
+  if (e >= g.nsrc * APX_BATCH_NP) return;
+  const int s = e / APX_BATCH_NP, k = e % APX_BATCH_NP;
+  const int np = pieces_of((int64_t)g.win[4 * s + 2] * g.win[4 * s + 3], S);
+  double v = 0.0;
+  for (int q = 0; q < np; ++q) v += part[((int64_t)s * S + q) * APX_BATCH_NP + k];
+  out[g.col0[s] + k] = v;
 }
 
 // Image-wide float64 sums, one partial per workgroup (fixed order):
@@ -168,15 +218,20 @@ __global__ __launch_bounds__(256) void group_image_sums_kernel(int64_t npix, int
 
 // the sky entries from the image partials:
 //   mode 0: H[sky][sky] = c^2 sum w, grad[sky] = c sum w r;  mode 1: out[sky] = c sum v
-__global__ void group_sky_final_kernel(int nblocks, int mode, int np, int sky, double c,
-                                       const double* __restrict__ part, double* __restrict__ H,
-                                       double* __restrict__ vec) {
-  if (threadIdx.x != 0) return;
-  double a = 0.0, b = 0.0;
-  for (int k = 0; k < nblocks; ++k) {
-    a += part[2 * k];
-    b += part[2 * k + 1];
+__global__ __launch_bounds__(256) void group_sky_final_kernel(int nblocks, int mode, int np, int sky, double c,
+                                                              const double* __restrict__ part,
+                                                              double* __restrict__ H, double* __restrict__ vec) {
+  __shared__ double red[4][2];
+  double ab[2] = {0.0, 0.0};
+  for (int k = threadIdx.x; k < nblocks; k += 256) {
+    ab[0] += part[2 * k];
+    ab[1] += part[2 * k + 1];
   }
+  wave_sums(ab, red[threadIdx.x >> 6]);
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  const double a = red[0][0] + red[1][0] + red[2][0] + red[3][0];
+  const double b = red[0][1] + red[1][1] + red[2][1] + red[3][1];
   if (mode == 0) {
     H[(int64_t)sky * np + sky] = c * c * a;
     vec[sky] = c * b;
@@ -189,109 +244,158 @@ __global__ __launch_bounds__(256) void fill_kernel(double* __restrict__ a, int64
   for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) a[e] = v;
 }
 
-// Per source: grad[col0 + k] = sum J_k w (data - model) over the window, and
-// the sky column H[col0 + k][sky] = H[sky][col0 + k] = c sum J_k w.
+// Per piece of a source's window: the sums of J_k w (data - model) and J_k w.
 __global__ __launch_bounds__(256) void group_source_kernel(apx_group g, const float* __restrict__ J,
                                                            const float* __restrict__ model,
                                                            const float* __restrict__ data,
                                                            const float* __restrict__ weight,
-                                                           const uint8_t* __restrict__ mask, double c,
-                                                           double* __restrict__ H, double* __restrict__ grad) {
-  __shared__ double red[4][2 * APX_BATCH_NP];
-  const int s = blockIdx.x;
+                                                           const uint8_t* __restrict__ mask, int S,
+                                                           double* __restrict__ part) {
+  constexpr int NP = APX_BATCH_NP;
+  __shared__ double red[4][2 * NP];
+  const int s = blockIdx.x / S;
   const int* w = g.win + 4 * s;
-  const int64_t n = (int64_t)w[2] * w[3];
-  double ag[APX_BATCH_NP], ah[APX_BATCH_NP];
+  const int w0 = w[0], w1 = w[1];
+  Piece t;
+  if (!t.open(w[2], w[3], blockIdx.x % S, S)) return;
+  double acc[2 * NP];
 #pragma unroll
-  for (int k = 0; k < APX_BATCH_NP; ++k) ag[k] = ah[k] = 0.0;
-  for (int64_t e = threadIdx.x; e < n; e += 256) {
-    const int dy = (int)(e / w[2]), dx = (int)(e % w[2]);
-    const int64_t p = (int64_t)(w[1] + dy) * g.nx + (w[0] + dx);
+  for (int k = 0; k < 2 * NP; ++k) acc[k] = 0.0;
+  const float* Js = J + g.pix_off[s];
+  for (; t.e < t.e1; t.next()) {
+    const int64_t p = (int64_t)(w1 + t.y) * g.nx + (w0 + t.x);
     if (mask && mask[p]) continue;
     const double ww = weight ? (double)weight[p] : 1.0;
     const double wr = ww * ((double)data[p] - (double)model[p]);
-    const int64_t q = g.pix_off[s] + e;
 #pragma unroll
-    for (int k = 0; k < APX_BATCH_NP; ++k) {
-      const double j = (double)J[(int64_t)k * g.nsrcpix + q];
-      ag[k] += j * wr;
-      ah[k] += j * ww;
+    for (int k = 0; k < NP; ++k) {
+      const double j = (double)Js[(int64_t)k * g.nsrcpix + t.e];
+      acc[k] += j * wr;
+      acc[NP + k] += j * ww;
     }
   }
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-  for (int k = 0; k < APX_BATCH_NP; ++k) {
-    const double t0 = wave_sum(ag[k]), t1 = wave_sum(ah[k]);
-    if (lane == 0) {
-      red[wv][k] = t0;
-      red[wv][APX_BATCH_NP + k] = t1;
-    }
-  }
+  wave_sums(acc, red[threadIdx.x >> 6]);
   __syncthreads();
-  if (threadIdx.x < APX_BATCH_NP) {
-    const int k = threadIdx.x, col = g.col0[s] + k;
-    grad[col] = red[0][k] + red[1][k] + red[2][k] + red[3][k];
-    if (g.sky_col >= 0) {
-      const int m = APX_BATCH_NP + k;
-      const double hs = c * (red[0][m] + red[1][m] + red[2][m] + red[3][m]);
-      H[(int64_t)col * g.np + g.sky_col] = hs;
-      H[(int64_t)g.sky_col * g.np + col] = hs;
-    }
+  if (threadIdx.x < 2 * NP) {
+    const int k = threadIdx.x;
+    part[(int64_t)blockIdx.x * 2 * NP + k] = red[0][k] + red[1][k] + red[2][k] + red[3][k];
   }
 }
 
+// grad[col0 + k] = sum J_k w (data - model) over the window, and the sky column
+// H[col0 + k][sky] = H[sky][col0 + k] = c sum J_k w: the source's pieces in order.
+__global__ __launch_bounds__(256) void group_source_final_kernel(apx_group g, int S, double c,
+                                                                 const double* __restrict__ part,
+                                                                 double* __restrict__ H,
+                                                                 double* __restrict__ grad) {
+  constexpr int NP = APX_BATCH_NP;
+  const int e = blockIdx.x * 256 + threadIdx.x;
+  if (e >= g.nsrc * 2 * NP) return;
+  const int s = e / (2 * NP), k = e % (2 * NP);
+  if (k >= NP && g.sky_col < 0) return;
+  const int np = pieces_of((int64_t)g.win[4 * s + 2] * g.win[4 * s + 3], S);
+  double v = 0.0;
+  for (int q = 0; q < np; ++q) v += part[((int64_t)s * S + q) * 2 * NP + k];
+  if (k < NP) {
+    grad[g.col0[s] + k] = v;
+  } else {
+    const int col = g.col0[s] + k - NP;
+    H[(int64_t)col * g.np + g.sky_col] = c * v;
+    H[(int64_t)g.sky_col * g.np + col] = c * v;
+  }
+}
+
+// the overlap of windows a and b: corner (x0, y0), size ow x oh (not positive: none)
+struct Overlap {
+  int x0, y0, ow, oh;
+  __device__ __forceinline__ Overlap(const int* wa, const int* wb) {
+    x0 = max(wa[0], wb[0]);
+    y0 = max(wa[1], wb[1]);
+    ow = max(0, min(wa[0] + wa[2], wb[0] + wb[2]) - x0);
+    oh = max(0, min(wa[1] + wa[3], wb[1] + wb[3]) - y0);
+  }
+};
+
 // One 7 x 7 block of J^T W J per pair of overlapping windows (a <= b): sum
-// over the overlap of w J_a J_b^T; written at (a, b) and (b, a).
+// over the overlap of w J_a J_b^T, a piece a workgroup.  Bound by the J values of
+// the pair pixels (56 bytes a pixel, most of them from the caches): the next
+// pixel's loads are issued before the 49 multiply-adds of the current one.
 __global__ __launch_bounds__(256) void group_pair_kernel(apx_group g, const float* __restrict__ J,
                                                          const float* __restrict__ weight,
-                                                         const uint8_t* __restrict__ mask,
-                                                         double* __restrict__ H) {
+                                                         const uint8_t* __restrict__ mask, int S,
+                                                         double* __restrict__ part) {
   constexpr int NP = APX_BATCH_NP, NN = NP * NP;
   __shared__ double red[4][NN];
-  const int a = g.pair[2 * blockIdx.x], b = g.pair[2 * blockIdx.x + 1];
+  const int pr = blockIdx.x / S;
+  const int a = g.pair[2 * pr], b = g.pair[2 * pr + 1];
   const int* wa = g.win + 4 * a;
   const int* wb = g.win + 4 * b;
-  const int x0 = max(wa[0], wb[0]), x1 = min(wa[0] + wa[2], wb[0] + wb[2]);
-  const int y0 = max(wa[1], wb[1]), y1 = min(wa[1] + wa[3], wb[1] + wb[3]);
-  const int ow = x1 - x0, oh = y1 - y0;
+  const Overlap o(wa, wb);
+  const int sa = wa[2], sb = wb[2];
+  Piece t;
+  if (!t.open(o.ow, o.oh, blockIdx.x % S, S)) return;
   double acc[NN];
 #pragma unroll
   for (int k = 0; k < NN; ++k) acc[k] = 0.0;
-  if (ow > 0 && oh > 0) {
-    const int64_t n = (int64_t)ow * oh;
-    for (int64_t e = threadIdx.x; e < n; e += 256) {
-      const int y = y0 + (int)(e / ow), x = x0 + (int)(e % ow);
-      const int64_t p = (int64_t)y * g.nx + x;
-      if (mask && mask[p]) continue;
-      const double ww = weight ? (double)weight[p] : 1.0;
-      const int64_t qa = g.pix_off[a] + (int64_t)(y - wa[1]) * wa[2] + (x - wa[0]);
-      const int64_t qb = g.pix_off[b] + (int64_t)(y - wb[1]) * wb[2] + (x - wb[0]);
-      double ja[NP], jb[NP];
+  const float* Ja = J + g.pix_off[a] + (int64_t)(o.y0 - wa[1]) * sa + (o.x0 - wa[0]);
+  const float* Jb = J + g.pix_off[b] + (int64_t)(o.y0 - wb[1]) * sb + (o.x0 - wb[0]);
+  const int64_t p0 = (int64_t)o.y0 * g.nx + o.x0;
+  struct Px {
+    float ja[NP], jb[NP], w;
+    bool keep;
+  };
+  auto load = [&](Px& v) {
+    v.keep = t.e < t.e1;
+    const int x = v.keep ? t.x : 0, y = v.keep ? t.y : 0;  // past the end: the corner, read and not used
+    const int64_t p = p0 + (int64_t)y * g.nx + x;
+    const float* pa = Ja + (int64_t)y * sa + x;
+    const float* pb = Jb + (int64_t)y * sb + x;
+    v.w = weight ? weight[p] : 1.0f;
+    if (mask) v.keep &= mask[p] == 0;
 #pragma unroll
-      for (int k = 0; k < NP; ++k) {
-        ja[k] = ww * (double)J[(int64_t)k * g.nsrcpix + qa];
-        jb[k] = (double)J[(int64_t)k * g.nsrcpix + qb];
+    for (int k = 0; k < NP; ++k) v.ja[k] = pa[(int64_t)k * g.nsrcpix];
+#pragma unroll
+    for (int k = 0; k < NP; ++k) v.jb[k] = pb[(int64_t)k * g.nsrcpix];
+  };
+  if (t.e1 > 0) {
+    Px cur;
+    load(cur);
+    for (int64_t left = t.e1 - (t.e - threadIdx.x); left > 0; left -= 256) {
+      t.next();
+      Px nxt;
+      load(nxt);
+      if (cur.keep) {
+#pragma unroll
+        for (int k = 0; k < NP; ++k) {
+          const double ja = (double)cur.w * (double)cur.ja[k];
+#pragma unroll
+          for (int l = 0; l < NP; ++l) acc[k * NP + l] += ja * (double)cur.jb[l];
+        }
       }
-#pragma unroll
-      for (int k = 0; k < NP; ++k)
-#pragma unroll
-        for (int l = 0; l < NP; ++l) acc[k * NP + l] += ja[k] * jb[l];
+      cur = nxt;
     }
   }
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-  for (int k = 0; k < NN; ++k) {
-    const double t = wave_sum(acc[k]);
-    if (lane == 0) red[wv][k] = t;
-  }
+  wave_sums(acc, red[threadIdx.x >> 6]);
   __syncthreads();
-  if (threadIdx.x < NN) {
-    const int k = threadIdx.x / NP, l = threadIdx.x % NP;
-    const double v = red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
-    const int ca = g.col0[a], cb = g.col0[b];
-    H[(int64_t)(ca + k) * g.np + (cb + l)] = v;
-    H[(int64_t)(cb + l) * g.np + (ca + k)] = v;
-  }
+  if (threadIdx.x < NN)
+    part[(int64_t)blockIdx.x * NN + threadIdx.x] =
+        red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
+}
+
+// the pair's pieces in order, written at (a, b) and (b, a)
+__global__ __launch_bounds__(64) void group_pair_final_kernel(apx_group g, int S, const double* __restrict__ part,
+                                                              double* __restrict__ H) {
+  constexpr int NP = APX_BATCH_NP, NN = NP * NP;
+  if (threadIdx.x >= NN) return;
+  const int a = g.pair[2 * blockIdx.x], b = g.pair[2 * blockIdx.x + 1];
+  const Overlap o(g.win + 4 * a, g.win + 4 * b);
+  const int np = pieces_of((int64_t)o.ow * o.oh, S);
+  double v = 0.0;
+  for (int q = 0; q < np; ++q) v += part[((int64_t)blockIdx.x * S + q) * NN + threadIdx.x];
+  const int k = threadIdx.x / NP, l = threadIdx.x % NP;
+  const int ca = g.col0[a], cb = g.col0[b];
+  H[(int64_t)(ca + k) * g.np + (cb + l)] = v;
+  H[(int64_t)(cb + l) * g.np + (ca + k)] = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -767,10 +871,15 @@ int group_image(const apx_group* g, const float* src, double sky, float* out, hi
   return check_launch("group_image");
 }
 
+static int64_t group_part_bytes(const apx_group* g) {
+  const int64_t npix = (int64_t)g->nx * g->ny;
+  return 8 * std::max(npix, (int64_t)g->npair * max_pieces(g->npair) * APX_BATCH_NP * APX_BATCH_NP);
+}
+
 int64_t group_workspace_bytes(const apx_group* g) {
   if (!g) return 0;
-  const int64_t npix = (int64_t)g->nx * g->ny;
-  return 8 * npix + 8 * 2 * 4096 + 256;
+  // [u of group_rpp, or the pair partials | image partials | source partials]
+  return group_part_bytes(g) + 8 * 2 * 4096 + 8 * 2 * APX_BATCH_NP * (int64_t)g->nsrc * max_pieces(g->nsrc) + 256;
 }
 
 int group_normal(const apx_group* g, const float* J, const float* model, const float* data,
@@ -782,17 +891,27 @@ int group_normal(const apx_group* g, const float* J, const float* model, const f
   const int64_t np2 = (int64_t)g->np * g->np;
   hipLaunchKernelGGL(fill_kernel, dim3(grid_for(np2)), dim3(256), 0, stream, H, np2, 0.0);
   hipLaunchKernelGGL(fill_kernel, dim3(grid_for(g->np)), dim3(256), 0, stream, grad, (int64_t)g->np, 0.0);
-  if (g->npair > 0)
-    hipLaunchKernelGGL(group_pair_kernel, dim3((unsigned)g->npair), dim3(256), 0, stream, *g, J, weight, mask, H);
-  hipLaunchKernelGGL(group_source_kernel, dim3((unsigned)g->nsrc), dim3(256), 0, stream, *g, J, model, data,
-                     weight, mask, sky_dcol, H, grad);
+  double* part = reinterpret_cast<double*>(static_cast<char*>(ws) + group_part_bytes(g));
+  double* spart = part + 2 * 4096;
+  if (g->npair > 0) {
+    const int S = max_pieces(g->npair);
+    double* pp = static_cast<double*>(ws);
+    hipLaunchKernelGGL(group_pair_kernel, dim3((unsigned)g->npair * S), dim3(256), 0, stream, *g, J, weight, mask, S,
+                       pp);
+    hipLaunchKernelGGL(group_pair_final_kernel, dim3((unsigned)g->npair), dim3(64), 0, stream, *g, S,
+                       (const double*)pp, H);
+  }
+  const int S = max_pieces(g->nsrc);
+  hipLaunchKernelGGL(group_source_kernel, dim3((unsigned)g->nsrc * S), dim3(256), 0, stream, *g, J, model, data,
+                     weight, mask, S, spart);
+  hipLaunchKernelGGL(group_source_final_kernel, dim3((unsigned)((2 * APX_BATCH_NP * g->nsrc + 255) / 256)), dim3(256),
+                     0, stream, *g, S, sky_dcol, (const double*)spart, H, grad);
   if (g->sky_col >= 0) {
     const int64_t npix = (int64_t)g->nx * g->ny;
-    double* part = reinterpret_cast<double*>(static_cast<char*>(ws) + 8 * npix);
     const int nb = std::min(grid_for(npix), 512);
     hipLaunchKernelGGL(group_image_sums_kernel, dim3(nb), dim3(256), 0, stream, npix, 0, model, data, weight,
                        mask, (const double*)nullptr, part);
-    hipLaunchKernelGGL(group_sky_final_kernel, dim3(1), dim3(64), 0, stream, nb, 0, g->np, g->sky_col, sky_dcol,
+    hipLaunchKernelGGL(group_sky_final_kernel, dim3(1), dim3(256), 0, stream, nb, 0, g->np, g->sky_col, sky_dcol,
                        part, H, grad);
   }
   return check_launch("group_normal");
@@ -806,17 +925,21 @@ int group_rpp(const apx_group* g, const float* J, const float* m0, const float* 
   if (ws_bytes < group_workspace_bytes(g)) return set_error(APX_E_INVALID, "group_rpp: workspace too small");
   const int64_t npix = (int64_t)g->nx * g->ny;
   double* u = static_cast<double*>(ws);
-  double* part = reinterpret_cast<double*>(static_cast<char*>(ws) + 8 * npix);
+  double* part = reinterpret_cast<double*>(static_cast<char*>(ws) + group_part_bytes(g));
+  double* spart = part + 2 * 4096;
   hipLaunchKernelGGL(group_rpp_weights_kernel, dim3((unsigned)(g->ntx * g->nty)), dim3(256), 0, stream, *g, J,
                      m0, m1, weight, mask, h, d, sky_dcol, u);
-  hipLaunchKernelGGL(group_jtv_kernel, dim3((unsigned)g->nsrc), dim3(256), 0, stream, *g, J, (const double*)u,
-                     out);
+  const int S = max_pieces(g->nsrc);
+  hipLaunchKernelGGL(group_jtv_kernel, dim3((unsigned)g->nsrc * S), dim3(256), 0, stream, *g, J, (const double*)u,
+                     S, spart);
+  hipLaunchKernelGGL(group_jtv_final_kernel, dim3((unsigned)((APX_BATCH_NP * g->nsrc + 255) / 256)), dim3(256), 0,
+                     stream, *g, S, (const double*)spart, out);
   if (g->sky_col >= 0) {
     const int nb = std::min(grid_for(npix), 512);
     hipLaunchKernelGGL(group_image_sums_kernel, dim3(nb), dim3(256), 0, stream, npix, 1, (const float*)nullptr,
                        (const float*)nullptr, (const float*)nullptr, (const uint8_t*)nullptr, (const double*)u,
                        part);
-    hipLaunchKernelGGL(group_sky_final_kernel, dim3(1), dim3(64), 0, stream, nb, 1, g->np, g->sky_col, sky_dcol,
+    hipLaunchKernelGGL(group_sky_final_kernel, dim3(1), dim3(256), 0, stream, nb, 1, g->np, g->sky_col, sky_dcol,
                        part, (double*)nullptr, out);
   }
   return check_launch("group_rpp");

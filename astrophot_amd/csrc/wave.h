@@ -66,4 +66,31 @@ __device__ __forceinline__ T wave_sum(T v) {
   return half_sum(butterfly_add32(v));
 }
 
+// The wave sums of N values at once, to out[0 .. N) (LDS or global): the two
+// widest steps halve the number of values in flight, as a swap of two registers'
+// halves leaves one value's partial sums in one half and the other's in the
+// other, so N values take about 3 N / 2 + 3 N instructions, not 18 N.
+template <int N>
+__device__ __forceinline__ void wave_sums(const double (&v)[N], double* out) {
+  constexpr int H = (N + 1) / 2, Q = (H + 1) / 2;
+  const int lane = threadIdx.x & 63, row = lane >> 4;
+  double u[2 * Q];
+#pragma unroll
+  for (int j = 0; j < 2 * Q; ++j) {  // lanes 0-31: v[2 j], lanes 32-63: v[2 j + 1]
+    const double a = 2 * j < N ? v[2 * j] : 0.0, b = 2 * j + 1 < N ? v[2 * j + 1] : 0.0;
+    const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)__double2loint(a), (uint32_t)__double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)__double2hiint(a), (uint32_t)__double2hiint(b), false, false);
+    u[j] = __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+  }
+#pragma unroll
+  for (int m = 0; m < Q; ++m) {  // rows 0..3: v[4 m], v[4 m + 2], v[4 m + 1], v[4 m + 3]
+    const double a = u[2 * m], b = u[2 * m + 1];
+    const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)__double2loint(a), (uint32_t)__double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)__double2hiint(a), (uint32_t)__double2hiint(b), false, false);
+    const double t = row_sum(__hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]));
+    const int k = 4 * m + ((row & 1) << 1) + (row >> 1);
+    if ((lane & 15) == 0 && k < N) out[k] = t;
+  }
+}
+
 }  // namespace apx

@@ -106,6 +106,74 @@ def test_dense_damped_cholesky_solve():
             assert np.abs(x.cpu().numpy() - ref).max() <= 1e-9 * np.abs(ref).max(), (n, band, Lval)
 
 
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("sky", [False, True])
+@pytest.mark.parametrize("nx,ny,wins", [
+    (70, 40, [(0, 0, 1, 1), (0, 0, 70, 40), (69, 39, 1, 1), (3, 5, 17, 31)]),        # one piece a window
+    (300, 300, [(0, 0, 300, 300), (10, 20, 257, 255), (299, 0, 1, 300)]),            # up to 22 x 4096 pixels: 16 pieces
+    (130, 200, [(5, 7, 63, 65), (30, 7, 64, 64), (60, 40, 64, 129), (0, 199, 130, 1)]),  # 4095, 4096, 8256 pixels
+])
+def test_normal_equations_and_rpp_of_any_window_sizes(nx, ny, wins, sky, masked):
+    """Windows and overlaps go to workgroups in pieces of 4,096 pixels or more, at
+    most 16: the products against the dense float64 ones.  Sums of n terms of
+    float64 round to at most n 2^-53 of the sum of their magnitudes; 1e-12 of it
+    covers the largest here (90,000 pixels: 1e-11 worst case, 3e-14 typical)."""
+    import ctypes
+    from astrophot_amd.group_fit import plan_tiles
+    gen = torch.Generator(device="cuda").manual_seed(nx)
+    rnd = lambda *n: torch.randn(n, generator=gen, device="cuda")  # noqa: E731
+    W = np.array(wins, dtype=np.int32)
+    n, lib = len(wins), L.load()
+    sizes = (W[:, 2].astype(np.int64) * W[:, 3])
+    off = np.concatenate([[0], np.cumsum(sizes)[:-1]])
+    ntx, nty, tile_ptr, tile_src, pairs = plan_tiles(W, nx, ny)
+    dev = lambda x, dt: torch.as_tensor(np.ascontiguousarray(x), dtype=dt, device="cuda")  # noqa: E731
+    arrays = dict(win=dev(W.reshape(-1), torch.int32), pix_off=dev(off, torch.int64),
+                  col0=dev(np.arange(n) * 7, torch.int32), tile_ptr=dev(tile_ptr, torch.int32),
+                  tile_src=dev(tile_src, torch.int32), pair=dev(pairs, torch.int32))
+    g = L.Group()
+    g.nx, g.ny, g.nsrc, g.np = nx, ny, n, 7 * n + sky
+    g.sky_col, g.sky_after = (7 * n, n) if sky else (-1, -1)
+    g.ntx, g.nty, g.npair, g.nsrcpix = ntx, nty, len(pairs) // 2, int(sizes.sum())
+    for k, t in arrays.items():
+        setattr(g, k, t.data_ptr())
+    npix = nx * ny
+    J, model, data = rnd(7, int(sizes.sum())), rnd(npix), rnd(npix)
+    probe, weight = rnd(npix), 0.5 + rnd(npix).abs()
+    mask = (rnd(npix) > 1).to(torch.uint8) if masked else None
+    if masked:
+        data[mask.bool()] = float("nan")  # a masked pixel takes no part, whatever it holds
+    wsb = lib.apx_group_workspace_bytes(ctypes.byref(g))
+    ws = torch.empty(wsb, dtype=torch.uint8, device="cuda")
+    H = torch.empty((g.np, g.np), dtype=torch.float64, device="cuda")
+    grad, rpp = torch.empty(g.np, dtype=torch.float64, device="cuda"), torch.empty(g.np, dtype=torch.float64, device="cuda")
+    h = rnd(g.np).double()
+    dcol, d = 0.7, 0.1
+    L.check(lib.apx_group_normal(ctypes.byref(g), L.ptr(J), L.ptr(model), L.ptr(data), L.ptr(weight), L.ptr(mask), dcol,
+                                 L.ptr(H), L.ptr(grad), L.ptr(ws), wsb, L.stream()))
+    L.check(lib.apx_group_rpp(ctypes.byref(g), L.ptr(J), L.ptr(model), L.ptr(probe), L.ptr(weight), L.ptr(mask),
+                              L.ptr(h), d, dcol, L.ptr(rpp), L.ptr(ws), wsb, L.stream()))
+    # the dense Jacobian on the CPU
+    D = torch.zeros((npix, g.np), dtype=torch.float64)
+    for s, (x0, y0, w, hh) in enumerate(wins):
+        idx = (torch.arange(y0, y0 + hh)[:, None] * nx + torch.arange(x0, x0 + w)[None, :]).reshape(-1)
+        D[idx, 7 * s:7 * s + 7] = J[:, off[s]:off[s] + sizes[s]].t().double().cpu()
+    if sky:
+        D[:, -1] = dcol
+    keep = torch.ones(npix, dtype=torch.bool) if mask is None else ~mask.bool().cpu()
+    wk = torch.where(keep, weight.double().cpu(), torch.zeros(npix, dtype=torch.float64))
+    r = torch.where(keep, data.double().cpu() - model.double().cpu(), torch.zeros(npix, dtype=torch.float64))
+    m0, m1 = model.cpu(), probe.cpu()
+    u = torch.where(keep, 2 / d * (wk * (m1 - m0).double() / d - wk * (D @ h.cpu())), torch.zeros(npix, dtype=torch.float64))
+    Da = D.abs()
+    assert ((H.cpu() - D.T @ (wk[:, None] * D)).abs() <= 1e-12 * (Da.T @ (wk[:, None] * Da))).all()
+    assert ((grad.cpu() - D.T @ (wk * r)).abs() <= 1e-12 * (Da.T @ (wk * r.abs()))).all()
+    # u itself is a difference of float64 terms of this size
+    ua = torch.where(keep, 2 / d * (wk * (m1 - m0).double().abs() / d + wk * (Da @ h.cpu().abs())),
+                     torch.zeros(npix, dtype=torch.float64))
+    assert ((rpp.cpu() - D.T @ u).abs() <= 1e-12 * (Da.T @ ua)).all()
+
+
 def test_forward_matches_dense_group_and_oracle(scene):
     s, om, data, var, tgt = scene
     g = scene_group(s, tgt)
