@@ -414,23 +414,68 @@ __global__ __launch_bounds__(256) void damp_kernel(const double* __restrict__ H,
   }
 }
 
-// Factor of the diagonal block [k0, k0 + nb) on one wave: lane i holds row i of
-// the block in registers; column j's pivot and entries go lane to lane by
-// lane reads (v_readlane into SGPRs), so the 32 dependent steps wait on no
-// memory.  Every entry takes the same operations in the same order as the
-// textbook right-looking loop:
-//   L_jj = sqrt(A_jj), L_ij = A_ij / L_jj, A_ik -= L_ij L_kj (k > j, i >= k).
-// On return r[k] = L[lane][k] for k <= lane.  A pivot that is not positive
-// and finite gives NaN and sets *status to its 1-based column (first one only,
-// when `report`).  A full block (kFull: nb == kNB) runs as one basic block, so
-// the scheduler can overlap a step's updates with the next step's pivot.
+// One launch a panel of kNB = 32 columns.  A panel's own chain (the diagonal
+// block's factor, then the rows below) is serial, so the update of everything
+// to its right runs beside the next panel: launch k takes panel k - 1 out of
+// block column k and factors it (the first workgroups), and takes panel k - 1
+// out of the block columns after it (the others).  Two launches a panel, with
+// the rows solved after the diagonal factor and a division a step, took 20 + 11 us a
+// panel (n = 3501, a band 658 wide: 3.45 ms a factor); this one 11.8 us (1.29 ms).
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+// 16 x 16 blocks by v_mfma_f64_16x16x4_f64: lane l gives A[l % 16][l / 16] and
+// B[l / 16][l % 16] of a k-step of 4, and holds D[4 r + l / 16][l % 16] in acc[r].
+constexpr int kSteps = kNB / 4;  // k-steps of a panel
+
+// k-step operands of rows r0 .. r0 + 15 of the panel at column p0 (zero past the matrix)
+__device__ __forceinline__ void panel_operand(const double* __restrict__ A, int n, int r0, int p0, double (&o)[kSteps]) {
+  const int lane = threadIdx.x & 63, row = r0 + (lane & 15);
+#pragma unroll
+  for (int t = 0; t < kSteps; ++t) o[t] = row < n ? A[(int64_t)row * n + p0 + 4 * t + (lane >> 4)] : 0.0;
+}
+
+// Rows of block column k0 with panel k0 - kNB taken out, into T: a wave's 16
+// rows r0 .. (T rows 16 w ..) by the block's 32 columns.
+__device__ __forceinline__ void panel_rows(const double* __restrict__ A, int n, int k0, int nb, int r0, int w,
+                                           double (*T)[kNB + 1]) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  v4d c[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = r0 + 4 * r + lk, col = 16 * q + li;
+      c[q][r] = (row < n && col < nb) ? A[(int64_t)row * n + k0 + col] : 0.0;
+    }
+  if (k0 > 0) {
+    double a[kSteps], b[2][kSteps];
+    panel_operand(A, n, r0, k0 - kNB, a);
+    panel_operand(A, n, k0, k0 - kNB, b[0]);
+    panel_operand(A, n, k0 + 16, k0 - kNB, b[1]);
+#pragma unroll
+    for (int t = 0; t < kSteps; ++t)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) c[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[t], b[q][t], c[q], 0, 0, 0);
+  }
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) T[16 * w + 4 * r + lk][16 * q + li] = c[q][r];
+}
+
+// Cholesky of a diagonal block and the solve of rows below it on one wave:
+// lanes 0 .. 31 hold the rows of the block, lanes 32 .. 63 rows further down,
+// which take the same steps (column j: divided by the pivot's root, then out of
+// the later columns), so they cost nothing beyond the factor.  Column entries go
+// lane to lane by v_readlane.  1 / sqrt(pivot) is v_rsq_f64 (24 bits) and one
+// third-order step, within 2 ulp: a division and a square root a step, 60
+// dependent instructions, set the chain's length before.  r[k] = L[lane][k] on
+// return (k <= lane).  A pivot that is not positive and finite gives NaN and
+// sets *status to its 1-based column (first one only, when `report`).
 template <bool kFull>
-__device__ __forceinline__ void potrf_block(const double* __restrict__ A, int n, int k0, int nb, double (&r)[kNB],
-                                            int32_t* __restrict__ status, bool report) {
+__device__ __forceinline__ void potrf_rows(int k0, int nb, double (&r)[kNB], int32_t* __restrict__ status, bool report) {
   const int lane = threadIdx.x & 63;
   if (kFull) nb = kNB;
-#pragma unroll
-  for (int k = 0; k < kNB; ++k) r[k] = (lane < nb && k <= lane) ? A[(int64_t)(k0 + lane) * n + (k0 + k)] : 0.0;
   int bad = -1;
 #pragma unroll
   for (int j = 0; j < kNB; ++j) {
@@ -438,87 +483,51 @@ __device__ __forceinline__ void potrf_block(const double* __restrict__ A, int n,
       const double piv = lane_bcast(r[j], j);
       const bool ok = piv > 0.0 && isfinite(piv);
       bad = (!ok && bad < 0) ? j : bad;
-      const double d = ok ? sqrt(piv) : __builtin_nan("");
-      r[j] = lane == j ? d : (lane > j ? r[j] / d : r[j]);
+      const double p = ok ? piv : __builtin_nan("");
+      double y = __builtin_amdgcn_rsq(p);
+      const double e = fma(-p * y, y, 1.0);
+      y = fma(y * e, fma(0.375, e, 0.5), y);
+      double d = p * y;
+      d = fma(fma(-d, d, p), 0.5 * y, d);
+      r[j] = lane == j ? d : r[j] * y;
       // every lane updates every later column: entries above the diagonal
-      // (k > lane) and rows or columns past nb are never used, and only lower
-      // entries of columns before k feed a lower entry
+      // (k > lane) and columns past nb are never used, and only lower entries of
+      // columns before k feed a lower entry
 #pragma unroll
-      for (int k = j + 1; k < kNB; ++k) r[k] -= r[j] * lane_bcast(r[j], k);
+      for (int k = j + 1; k < kNB; ++k) r[k] = fma(-r[j], lane_bcast(r[j], k), r[k]);
     }
   }
   if (report && bad >= 0 && lane == 0 && status[0] == 0) status[0] = k0 + bad + 1;
 }
 
-// One panel: the diagonal block's factor and the rows below it,
-//   L[i][k0..k0+nb) = A[i][k0..) L_kk^-T  (one row a thread, 64 rows a
-// workgroup so that the panel's rows spread over many CUs).  Every workgroup
-// factors the 32 x 32 diagonal block itself (the same operations on the same
-// input, so the same bits) instead of waiting a launch for it; its rows are
-// loaded before that factor, which they do not depend on.  The block's lower
-// triangle is left as it is, since other workgroups may still be reading it;
-// workgroup 0 writes L^T into the block's strict upper triangle (read by the
-// forward solve along columns), and diag_writeback_kernel writes the lower
-// triangle and the diagonal once the whole factor is done.
-constexpr int kTrsmRows = 64;
-template <bool kFull>
-__global__ __launch_bounds__(kTrsmRows) void potrf_trsm_kernel(double* __restrict__ A, int n, int k0,
-                                                               int32_t* __restrict__ status) {
-  __shared__ double T[kNB][kNB + 1];
-  __shared__ double rT[kNB];
-  const int lane = threadIdx.x;
-  const int nb = kFull ? kNB : min(kNB, n - k0);
-  const int i = k0 + nb + blockIdx.x * kTrsmRows + lane;
-  double* row = A + (int64_t)i * n + k0;
-  double x[kNB];
+// 64 x 64 tile (ti, tj) of the update by panel p0 of the lower triangle from
+// row and column `base` on: A[i][j] -= sum_t L[i][p0 + t] L[j][p0 + t]
+__device__ __forceinline__ void trailing_tile(double* __restrict__ A, int n, int p0, int i0, int j0) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
+  const int r0 = i0 + 16 * w;
+  v4d c[4];
 #pragma unroll
-  for (int j = 0; j < kNB; ++j) x[j] = (i < n && j < nb) ? row[j] : 0.0;
-  {
-    double r[kNB];
-    potrf_block<kFull>(A, n, k0, nb, r, status, blockIdx.x == 0);
+  for (int q = 0; q < 4; ++q)
 #pragma unroll
-    for (int k = 0; k < kNB; ++k) {
-      if (lane < nb && k <= lane) {
-        T[lane][k] = r[k];
-        if (k == lane) rT[k] = 1.0 / r[k];
-        if (blockIdx.x == 0 && k < lane) A[(int64_t)(k0 + k) * n + (k0 + lane)] = r[k];
-      }
+    for (int r = 0; r < 4; ++r) {
+      const int i = r0 + 4 * r + lk, j = j0 + 16 * q + li;
+      c[q][r] = (i < n && j <= i) ? A[(int64_t)i * n + j] : 0.0;
     }
-  }
-  __syncthreads();
-  if (i >= n) return;
-  // column-oriented substitution with the pivots' reciprocals: once x_j is
-  // known it is taken out of every later entry at once, so the serial chain is
-  // one multiply and one FMA a column (the 31 - j updates of a step are
-  // independent); entry k receives its terms in the order t = 0, 1, ..., k - 1
+  double a[kSteps], b[4][kSteps];
+  panel_operand(A, n, r0, p0, a);
 #pragma unroll
-  for (int j = 0; j < kNB; ++j) {
-    if (kFull || j < nb) {
-      x[j] *= rT[j];
+  for (int q = 0; q < 4; ++q) panel_operand(A, n, j0 + 16 * q, p0, b[q]);
 #pragma unroll
-      for (int k = j + 1; k < kNB; ++k) x[k] -= x[j] * T[k][j];  // k >= nb: unused
+  for (int t = 0; t < kSteps; ++t)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) c[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[t], b[q][t], c[q], 0, 0, 0);
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = r0 + 4 * r + lk, j = j0 + 16 * q + li;
+      if (i < n && j <= i) A[(int64_t)i * n + j] = c[q][r];
     }
-  }
-#pragma unroll
-  for (int j = 0; j < kNB; ++j)
-    if (kFull || j < nb) {
-      row[j] = x[j];
-      A[(int64_t)(k0 + j) * n + i] = x[j];  // L^T in the upper triangle (coalesced over i)
-    }
-}
-
-// Lower triangle and diagonal of every diagonal block, one wave a block, after
-// the factor: each block still holds the input of its own factor (no later
-// panel's update reaches it), which is factored again to the same bits.
-__global__ __launch_bounds__(64) void diag_writeback_kernel(double* __restrict__ A, int n) {
-  const int lane = threadIdx.x;
-  const int k0 = blockIdx.x * kNB, nb = min(kNB, n - k0);
-  double r[kNB];
-  if (nb == kNB) potrf_block<true>(A, n, k0, nb, r, nullptr, false);
-  else potrf_block<false>(A, n, k0, nb, r, nullptr, false);
-#pragma unroll
-  for (int k = 0; k < kNB; ++k)
-    if (lane < nb && k <= lane) A[(int64_t)(k0 + lane) * n + (k0 + k)] = r[k];
 }
 
 // Envelope of the damped matrix: for each 32-row block, the first column
@@ -573,71 +582,90 @@ __device__ __forceinline__ int block_reach(const double* __restrict__ A, int n, 
   return *reinterpret_cast<const int*>(A + (int64_t)k0 * n + k0 + 1) / kNB;
 }
 
-// trailing update of the lower triangle: A[i][j] -= sum_t L[i][k0+t] L[j][k0+t]
-// for i >= j >= k0 + nb, one 64 x 64 tile per workgroup (lower tiles only)
-__global__ __launch_bounds__(256) void syrk_update_kernel(double* __restrict__ A, int n, int k0) {
-  __shared__ double PI[kUT][kNB + 1];
-  __shared__ double PJ[kUT][kNB + 1];
-  const int nb = min(kNB, n - k0);
-  const int base = k0 + nb;
-  // tile (ti, tj), tj <= ti, from the linear block index
-  const int b = blockIdx.x;
-  int ti = (int)((sqrt(8.0 * b + 1.0) - 1.0) * 0.5);
-  while ((ti + 1) * (ti + 2) / 2 <= b) ++ti;
-  while (ti * (ti + 1) / 2 > b) --ti;
-  const int tj = b - ti * (ti + 1) / 2;
-  const int i0 = base + ti * kUT, j0 = base + tj * kUT;
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  // A tile whose rows or whose columns have no nonzero entry in this panel (all
-  // their rows start past it) receives an exactly zero update and is skipped.
-  const int pk = k0 / kNB, bi = i0 / kNB, bj = j0 / kNB;
-  if (min(block_reach(A, n, bi), block_reach(A, n, bi + 1)) > pk ||
-      min(block_reach(A, n, bj), block_reach(A, n, bj + 1)) > pk)
-    return;
-  // the tile's own entries are read first, so their round trip overlaps the
-  // panel loads and the products
-  double a[4][4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int i = i0 + ty + 16 * r, j = j0 + tx + 16 * c;
-      a[r][c] = (i < n && j <= i) ? A[(int64_t)i * n + j] : 0.0;
+// Launch of panel k0: workgroups 0 .. row_wgs - 1 take the diagonal block and 32
+// rows below it each (every one factors the diagonal block itself, the same
+// operations on the same input, instead of waiting a launch for it); the others
+// take the tiles of the trailing update by the panel before, those whose rows
+// and columns all reach it: the update of the rest is exactly zero.  The
+// diagonal block's lower triangle is left as it is, since other workgroups may
+// still be reading it; workgroup 0 writes L^T into its strict upper triangle
+// (read by the forward solve along columns), and diag_writeback_kernel writes
+// the lower triangle and the diagonal once the whole factor is done.
+template <bool kFull>
+__global__ __launch_bounds__(256) void panel_kernel(double* __restrict__ A, int n, int k0, int row_wgs, int ntiles,
+                                                    int32_t* __restrict__ status) {
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int nb = kFull ? kNB : min(kNB, n - k0);
+  if ((int)blockIdx.x >= row_wgs) {
+    // tiles b0, b0 + step, ...: a lane looks at one, then the workgroup takes those that are reached
+    const int step = (int)gridDim.x - row_wgs, base = k0 + kNB, pk = k0 / kNB - 1;
+    for (int b0 = (int)blockIdx.x - row_wgs; b0 < ntiles; b0 += 64 * step) {
+      const int b = b0 + lane * step;
+      int ti = 0, tj = 0;
+      bool hit = false;
+      if (b < ntiles) {  // tile (ti, tj), tj <= ti, of the linear index
+        ti = (int)((sqrt(8.0 * b + 1.0) - 1.0) * 0.5);
+        while ((ti + 1) * (ti + 2) / 2 <= b) ++ti;
+        while (ti * (ti + 1) / 2 > b) --ti;
+        tj = b - ti * (ti + 1) / 2;
+        const int bi = (base + ti * kUT) / kNB, bj = (base + tj * kUT) / kNB;
+        hit = min(block_reach(A, n, bi), block_reach(A, n, bi + 1)) <= pk &&
+              min(block_reach(A, n, bj), block_reach(A, n, bj + 1)) <= pk;
+      }
+      for (uint64_t m = __ballot(hit); m; m &= m - 1) {
+        const int l = __ffsll((unsigned long long)m) - 1;
+        trailing_tile(A, n, k0 - kNB, base + __builtin_amdgcn_readlane(ti, l) * kUT,
+                      base + __builtin_amdgcn_readlane(tj, l) * kUT);
+      }
     }
-  for (int e = threadIdx.x; e < kUT * kNB; e += 256) {
-    const int r = e / kNB, t = e % kNB;
-    const int ii = i0 + r, jj = j0 + r;
-    PI[r][t] = (ii < n && t < nb) ? A[(int64_t)ii * n + k0 + t] : 0.0;
-    PJ[r][t] = (jj < n && t < nb) ? A[(int64_t)jj * n + k0 + t] : 0.0;
+    return;
+  }
+  __shared__ double T[2 * kNB][kNB + 1];
+  const int i0 = k0 + nb + (int)blockIdx.x * kNB;
+  panel_rows(A, n, k0, nb, w < 2 ? k0 + 16 * w : i0 + 16 * (w - 2), w, T);
+  __syncthreads();
+  if (w == 0) {
+    double r[kNB];
+#pragma unroll
+    for (int k = 0; k < kNB; ++k) r[k] = T[lane][k];
+    potrf_rows<kFull>(k0, nb, r, status, blockIdx.x == 0);
+#pragma unroll
+    for (int k = 0; k < kNB; ++k) T[lane][k] = r[k];
   }
   __syncthreads();
-  // thread: 4 rows (ty + 16 r) x 4 columns (tx + 16 c)
-  double acc[4][4];
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int c = 0; c < 4; ++c) acc[r][c] = 0.0;
-#pragma unroll 2
-  for (int t = 0; t < kNB; ++t) {
-    double pi[4], pj[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) pi[r] = PI[ty + 16 * r][t];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) pj[c] = PJ[tx + 16 * c][t];
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-      for (int c = 0; c < 4; ++c) acc[r][c] += pi[r] * pj[c];
+  for (int e = t; e < kNB * kNB; e += 256) {
+    const int p = e / kNB, q = e % kNB;
+    if (i0 + p < n && q < nb) A[(int64_t)(i0 + p) * n + k0 + q] = T[kNB + p][q];
+    if (i0 + q < n && p < nb) A[(int64_t)(k0 + p) * n + i0 + q] = T[kNB + q][p];  // L^T in the upper triangle
+    if (blockIdx.x == 0 && p < q && q < nb) A[(int64_t)(k0 + p) * n + k0 + q] = T[q][p];
   }
+}
+
+// Lower triangle and diagonal of every diagonal block, a workgroup of two waves
+// a block, after the factor: each block still holds what its own launch read
+// (no later panel's update reaches it), and is factored again to the same bits.
+__global__ __launch_bounds__(128) void diag_writeback_kernel(double* __restrict__ A, int n) {
+  __shared__ double T[kNB][kNB + 1];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int k0 = blockIdx.x * kNB, nb = min(kNB, n - k0);
+  panel_rows(A, n, k0, nb, k0 + 16 * w, w, T);
+  __syncthreads();
+  if (w == 0) {
+    double r[kNB];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int i = i0 + ty + 16 * r;
-    if (i >= n) continue;
+    for (int k = 0; k < kNB; ++k) r[k] = lane < kNB ? T[lane][k] : 0.0;
+    if (nb == kNB) potrf_rows<true>(k0, nb, r, nullptr, false);
+    else potrf_rows<false>(k0, nb, r, nullptr, false);
+    if (lane < kNB) {
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int j = j0 + tx + 16 * c;
-      if (j <= i) A[(int64_t)i * n + j] = a[r][c] - acc[r][c];
+      for (int k = 0; k < kNB; ++k) T[lane][k] = r[k];
     }
+  }
+  __syncthreads();
+  for (int e = t; e < kNB * kNB; e += 128) {
+    const int p = e / kNB, q = e % kNB;
+    if (q <= p && p < nb) A[(int64_t)(k0 + p) * n + k0 + q] = T[p][q];
   }
 }
 
@@ -955,15 +983,13 @@ int dense_damped_factor(int32_t n, const double* H, double L, double* A, int32_t
                      dim3(256), 0, stream, A, n);
   for (int k0 = 0; k0 < n; k0 += kNB) {
     const int nb = std::min(kNB, n - k0);
-    const int rest = n - k0 - nb;
-    const dim3 grid((unsigned)std::max(1, (rest + kTrsmRows - 1) / kTrsmRows));
-    if (nb == kNB) hipLaunchKernelGGL(potrf_trsm_kernel<true>, grid, dim3(kTrsmRows), 0, stream, A, n, k0, status);
-    else hipLaunchKernelGGL(potrf_trsm_kernel<false>, grid, dim3(kTrsmRows), 0, stream, A, n, k0, status);
-    if (rest <= 0) break;
-    const int T = (rest + kUT - 1) / kUT;
-    hipLaunchKernelGGL(syrk_update_kernel, dim3((unsigned)(T * (T + 1) / 2)), dim3(256), 0, stream, A, n, k0);
+    const int rest = n - k0 - nb, T = k0 > 0 ? (rest + kUT - 1) / kUT : 0, tiles = T * (T + 1) / 2;
+    const int rows = std::max(1, (rest + kNB - 1) / kNB);
+    const dim3 grid((unsigned)(rows + std::min(tiles, 1024)));
+    if (nb == kNB) hipLaunchKernelGGL(panel_kernel<true>, grid, dim3(256), 0, stream, A, n, k0, rows, tiles, status);
+    else hipLaunchKernelGGL(panel_kernel<false>, grid, dim3(256), 0, stream, A, n, k0, rows, tiles, status);
   }
-  hipLaunchKernelGGL(diag_writeback_kernel, dim3((unsigned)((n + kNB - 1) / kNB)), dim3(64), 0, stream, A, n);
+  hipLaunchKernelGGL(diag_writeback_kernel, dim3((unsigned)((n + kNB - 1) / kNB)), dim3(128), 0, stream, A, n);
   return check_launch("dense_factor");
 }
 

@@ -106,6 +106,35 @@ def test_dense_damped_cholesky_solve():
             assert np.abs(x.cpu().numpy() - ref).max() <= 1e-9 * np.abs(ref).max(), (n, band, Lval)
 
 
+@pytest.mark.parametrize("n", [1, 2, 31, 32, 33, 64, 65, 95, 96, 97, 129, 161, 517])
+def test_factor_and_solve_at_panel_edges(n):
+    """Partial panels, one and two panels, partial row groups and trailing tiles:
+    the factor (lower triangle, and its transpose above) and the solve against
+    numpy.  A is well conditioned (eigenvalues in [1, 4]), so both differ by a
+    few n 2^-53 only: 1e-12 covers n = 517.  A matrix that is not positive
+    definite reports the first bad column."""
+    lib = L.load()
+    rng = np.random.default_rng(n)
+    q, _ = np.linalg.qr(rng.normal(size=(n, n)))
+    Hm = (q * rng.uniform(1, 4, n)) @ q.T
+    Hm = 0.5 * (Hm + Hm.T)
+    Hd, b = torch.tensor(Hm, device="cuda"), torch.tensor(rng.normal(size=n), device="cuda")
+    fac, x = torch.empty((n, n), dtype=torch.float64, device="cuda"), torch.empty(n, dtype=torch.float64, device="cuda")
+    st = torch.zeros(1, dtype=torch.int32, device="cuda")
+    L.check(lib.apx_dense_damped_factor(n, L.ptr(Hd), 0.0, L.ptr(fac), L.ptr(st), L.stream()))
+    L.check(lib.apx_dense_cholesky_solve(n, L.ptr(fac), L.ptr(b), L.ptr(x), L.stream()))
+    ref = np.linalg.cholesky(Hm)
+    got = fac.cpu().numpy()
+    assert int(st.item()) == 0
+    assert np.abs(np.tril(got) - ref).max() <= 1e-12
+    assert np.abs(np.triu(got, 1) - np.tril(ref, -1).T).max() <= 1e-12
+    sol = np.linalg.solve(Hm, b.cpu().numpy())
+    assert np.abs(x.cpu().numpy() - sol).max() <= 1e-12 * max(1.0, np.abs(sol).max())
+    Hd[n // 2, n // 2] = -1.0
+    L.check(lib.apx_dense_damped_factor(n, L.ptr(Hd), 0.0, L.ptr(fac), L.ptr(st), L.stream()))
+    assert int(st.item()) == n // 2 + 1
+
+
 @pytest.mark.parametrize("masked", [False, True])
 @pytest.mark.parametrize("sky", [False, True])
 @pytest.mark.parametrize("nx,ny,wins", [
