@@ -420,7 +420,7 @@ __global__ __launch_bounds__(256) void damp_kernel(const double* __restrict__ H,
 // block column k and factors it (the first workgroups), and takes panel k - 1
 // out of the block columns after it (the others).  Two launches a panel, with
 // the rows solved after the diagonal factor and a division a step, took 20 + 11 us a
-// panel (n = 3501, a band 658 wide: 3.45 ms a factor); this one 11.8 us (1.29 ms).
+// panel (n = 3501, a band 658 wide: 3.45 ms a factor); this one 10.1 us (1.10 ms).
 typedef double v4d __attribute__((ext_vector_type(4)));
 
 // 16 x 16 blocks by v_mfma_f64_16x16x4_f64: lane l gives A[l % 16][l / 16] and
@@ -463,41 +463,82 @@ __device__ __forceinline__ void panel_rows(const double* __restrict__ A, int n, 
     for (int r = 0; r < 4; ++r) T[16 * w + 4 * r + lk][16 * q + li] = c[q][r];
 }
 
-// Cholesky of a diagonal block and the solve of rows below it on one wave:
-// lanes 0 .. 31 hold the rows of the block, lanes 32 .. 63 rows further down,
-// which take the same steps (column j: divided by the pivot's root, then out of
-// the later columns), so they cost nothing beyond the factor.  Column entries go
-// lane to lane by v_readlane.  1 / sqrt(pivot) is v_rsq_f64 (24 bits) and one
-// third-order step, within 2 ulp: a division and a square root a step, 60
-// dependent instructions, set the chain's length before.  r[k] = L[lane][k] on
-// return (k <= lane).  A pivot that is not positive and finite gives NaN and
-// sets *status to its 1-based column (first one only, when `report`).
+// Cholesky of a diagonal block and the solve of rows below it, in T (rows 0 ..
+// 31 the block, the others rows further down), by a workgroup whose wave w holds
+// T's rows 16 w ...  Wave 0 takes a row a lane: the rows below take the block's
+// own steps (column j: divided by the pivot's root, then out of the later
+// columns), so they cost nothing beyond the factor.  Column entries go lane to
+// lane by v_readlane, two a multiply-add, so only the steps within 16 columns go
+// this way; the first 16 columns leave the last 16 by MFMA, every wave its rows
+// (all 32 columns by lane reads: 11.8 us a panel; this way 10.1).
+// 1 / sqrt(pivot) is v_rsq_f64 (24 bits) and one third-order step, within 2 ulp:
+// a division and a square root a step, 60 dependent instructions, set the
+// chain's length before.  T[i][k] = L[i][k] on return (k <= i).  A pivot that is
+// not positive and finite gives NaN and sets *status to its 1-based column
+// (first one only, when `report`).
+constexpr int kHB = kNB / 2;
+
 template <bool kFull>
-__device__ __forceinline__ void potrf_rows(int k0, int nb, double (&r)[kNB], int32_t* __restrict__ status, bool report) {
+__device__ __forceinline__ int potrf_half(int nb, int j0, double (&r)[kHB]) {
   const int lane = threadIdx.x & 63;
-  if (kFull) nb = kNB;
   int bad = -1;
 #pragma unroll
-  for (int j = 0; j < kNB; ++j) {
-    if (kFull || j < nb) {  // uniform; constant trip counts keep r[] in registers
-      const double piv = lane_bcast(r[j], j);
+  for (int j = 0; j < kHB; ++j) {
+    if (kFull || j0 + j < nb) {  // uniform; constant trip counts keep r[] in registers
+      const double piv = lane_bcast(r[j], j0 + j);
       const bool ok = piv > 0.0 && isfinite(piv);
-      bad = (!ok && bad < 0) ? j : bad;
+      bad = (!ok && bad < 0) ? j0 + j : bad;
       const double p = ok ? piv : __builtin_nan("");
       double y = __builtin_amdgcn_rsq(p);
       const double e = fma(-p * y, y, 1.0);
       y = fma(y * e, fma(0.375, e, 0.5), y);
       double d = p * y;
       d = fma(fma(-d, d, p), 0.5 * y, d);
-      r[j] = lane == j ? d : r[j] * y;
+      r[j] = lane == j0 + j ? d : r[j] * y;
       // every lane updates every later column: entries above the diagonal
       // (k > lane) and columns past nb are never used, and only lower entries of
       // columns before k feed a lower entry
 #pragma unroll
-      for (int k = j + 1; k < kNB; ++k) r[k] = fma(-r[j], lane_bcast(r[j], k), r[k]);
+      for (int k = j + 1; k < kHB; ++k) r[k] = fma(-r[j], lane_bcast(r[j], j0 + k), r[k]);
     }
   }
-  if (report && bad >= 0 && lane == 0 && status[0] == 0) status[0] = k0 + bad + 1;
+  return bad;
+}
+
+template <bool kFull>
+__device__ __forceinline__ void factor_rows(double (*T)[kNB + 1], int rows, int k0, int nb, int32_t* __restrict__ status,
+                                            bool report) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
+  int bad = -1;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    __syncthreads();
+    if (h == 1) {
+      const double(*R)[kNB + 1] = T + 16 * w;
+      v4d c;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) c[q] = R[4 * q + lk][kHB + li];
+#pragma unroll
+      for (int t = 0; t < kHB / 4; ++t)
+        c = __builtin_amdgcn_mfma_f64_16x16x4f64(-R[li][4 * t + lk], T[kHB + li][4 * t + lk], c, 0, 0, 0);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) T[16 * w + 4 * q + lk][kHB + li] = c[q];
+      __syncthreads();
+    }
+    if (w == 0) {
+      double r[kHB];
+#pragma unroll
+      for (int k = 0; k < kHB; ++k) r[k] = lane < rows ? T[lane][kHB * h + k] : 0.0;
+      const int b = potrf_half<kFull>(nb, kHB * h, r);
+      bad = (b >= 0 && bad < 0) ? b : bad;
+      if (lane < rows) {
+#pragma unroll
+        for (int k = 0; k < kHB; ++k) T[lane][kHB * h + k] = r[k];
+      }
+    }
+  }
+  __syncthreads();
+  if (report && bad >= 0 && threadIdx.x == 0 && status[0] == 0) status[0] = k0 + bad + 1;
 }
 
 // 64 x 64 tile (ti, tj) of the update by panel p0 of the lower triangle from
@@ -623,16 +664,7 @@ __global__ __launch_bounds__(256) void panel_kernel(double* __restrict__ A, int 
   __shared__ double T[2 * kNB][kNB + 1];
   const int i0 = k0 + nb + (int)blockIdx.x * kNB;
   panel_rows(A, n, k0, nb, w < 2 ? k0 + 16 * w : i0 + 16 * (w - 2), w, T);
-  __syncthreads();
-  if (w == 0) {
-    double r[kNB];
-#pragma unroll
-    for (int k = 0; k < kNB; ++k) r[k] = T[lane][k];
-    potrf_rows<kFull>(k0, nb, r, status, blockIdx.x == 0);
-#pragma unroll
-    for (int k = 0; k < kNB; ++k) T[lane][k] = r[k];
-  }
-  __syncthreads();
+  factor_rows<kFull>(T, 2 * kNB, k0, nb, status, blockIdx.x == 0);
 #pragma unroll
   for (int e = t; e < kNB * kNB; e += 256) {
     const int p = e / kNB, q = e % kNB;
@@ -647,22 +679,11 @@ __global__ __launch_bounds__(256) void panel_kernel(double* __restrict__ A, int 
 // (no later panel's update reaches it), and is factored again to the same bits.
 __global__ __launch_bounds__(128) void diag_writeback_kernel(double* __restrict__ A, int n) {
   __shared__ double T[kNB][kNB + 1];
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int t = threadIdx.x, w = t >> 6;
   const int k0 = blockIdx.x * kNB, nb = min(kNB, n - k0);
   panel_rows(A, n, k0, nb, k0 + 16 * w, w, T);
-  __syncthreads();
-  if (w == 0) {
-    double r[kNB];
-#pragma unroll
-    for (int k = 0; k < kNB; ++k) r[k] = lane < kNB ? T[lane][k] : 0.0;
-    if (nb == kNB) potrf_rows<true>(k0, nb, r, nullptr, false);
-    else potrf_rows<false>(k0, nb, r, nullptr, false);
-    if (lane < kNB) {
-#pragma unroll
-      for (int k = 0; k < kNB; ++k) T[lane][k] = r[k];
-    }
-  }
-  __syncthreads();
+  if (nb == kNB) factor_rows<true>(T, kNB, k0, nb, nullptr, false);
+  else factor_rows<false>(T, kNB, k0, nb, nullptr, false);
   for (int e = t; e < kNB * kNB; e += 128) {
     const int p = e / kNB, q = e % kNB;
     if (q <= p && p < nb) A[(int64_t)(k0 + p) * n + k0 + q] = T[p][q];
@@ -676,14 +697,17 @@ __global__ __launch_bounds__(128) void diag_writeback_kernel(double* __restrict_
 // diagonal blocks on registers, lanes 0-31 the first and lanes 32-63 the
 // second.  Every entry receives the terms of the blocks one at a time, in
 // block order, each summed from its first column.  All loads of a launch are
-// issued before its first wait, and a diagonal solve multiplies by the
-// reciprocal of each pivot (taken once per lane before the serial chain), so a
-// step of the chain is one multiply, two lane reads and one FMA.
+// issued before its first wait.  A wave has at most 63 in flight, so the terms of
+// the first wave's own 64 rows are the second wave's work and reach it through
+// LDS: with them (128 loads) and a product and two choices a step of the
+// substitution, a launch took 8.4 us, n = 3501; now 5.4 (forward) and 6.0.
 
 // One half-wave's copy of the diagonal block [k0, k0 + nb): lane off + r holds
 // v[j] = A[(k0 + j) n + k0 + r], which is L[r][j] for j < r (the factor's
-// transposed copy in the upper triangle) and L[j][r] for j > r, and the
-// reciprocal of its diagonal entry.
+// transposed copy in the upper triangle) and L[j][r] for j > r, and its diagonal
+// entry.  diag_scale turns the entries a solve uses into v[j] / L[r][r], the
+// others into zero, and the diagonal into its reciprocal: a step of the solve is
+// then two lane reads and one FMA, without a product or a choice in the chain.
 struct DiagBlock {
   double v[kNB];
   double rdii;
@@ -697,34 +721,27 @@ __device__ __forceinline__ void diag_load(const double* __restrict__ A, int n, i
   d.rdii = in ? A[(int64_t)(k0 + r) * n + k0 + r] : 1.0;
 }
 
-// forward substitution of a diagonal block held by lanes off .. off + nb - 1:
-// lane off + r holds the right-hand side of row r on entry and x_r on return;
-// every other lane is left as it is
-__device__ __forceinline__ double diag_lower_solve(const DiagBlock& d, int off, int nb, double xi) {
-  const int r = (int)(threadIdx.x & 63) - off;
+// kLower: keeps v[j] for j < r; else for j > r
+template <bool kLower>
+__device__ __forceinline__ void diag_scale(DiagBlock& d, int r) {
+  d.rdii = 1.0 / d.rdii;
 #pragma unroll
-  for (int j = 0; j < kNB; ++j) {
-    if (j < nb) {
-      if (r == j) xi *= d.rdii;
-      const double xj = lane_bcast(xi, off + j);
-      if (r > j && r < nb) xi -= d.v[j] * xj;
-    }
-  }
-  return xi;
+  for (int j = 0; j < kNB; ++j) d.v[j] = (kLower ? j < r : j > r) ? d.v[j] * d.rdii : 0.0;
 }
 
-// back substitution with L_kk^T, j descending
-__device__ __forceinline__ double diag_upper_solve(const DiagBlock& d, int off, int nb, double xi) {
-  const int r = (int)(threadIdx.x & 63) - off;
+// substitution with the scaled diagonal block held by lanes off .. off + 31 (rows
+// and columns past the matrix are zero): lane off + r holds the right-hand side
+// of row r on entry and x_r on return; every other lane is left as it is
+template <bool kLower>
+__device__ __forceinline__ double diag_substitute(const DiagBlock& d, int off, double b) {
+  const bool mine = ((int)(threadIdx.x & 63) & ~(kNB - 1)) == off;
+  double xi = b * d.rdii;
 #pragma unroll
-  for (int j = kNB - 1; j >= 0; --j) {
-    if (j < nb) {
-      if (r == j) xi *= d.rdii;
-      const double xj = lane_bcast(xi, off + j);
-      if (r >= 0 && r < j) xi -= d.v[j] * xj;
-    }
+  for (int q = 0; q < kNB; ++q) {
+    const int j = kLower ? q : kNB - 1 - q;
+    xi = fma(-d.v[j], lane_bcast(xi, off + j), xi);
   }
-  return xi;
+  return mine ? xi : b;
 }
 
 template <bool kLower>
@@ -733,9 +750,9 @@ __global__ __launch_bounds__(64) void diag_solve_kernel(const double* __restrict
   DiagBlock d;
   const int lane = threadIdx.x, nb = min(kNB, n - k0);
   diag_load(A, n, k0, lane, d);
-  d.rdii = 1.0 / d.rdii;
+  diag_scale<kLower>(d, lane);
   const double b = lane < nb ? x[k0 + lane] : 0.0;
-  const double xi = kLower ? diag_lower_solve(d, 0, nb, b) : diag_upper_solve(d, 0, nb, b);
+  const double xi = diag_substitute<kLower>(d, 0, b);
   if (lane < nb) x[k0 + lane] = xi;
 }
 
@@ -747,7 +764,7 @@ __global__ __launch_bounds__(64) void diag_solve_kernel(const double* __restrict
 // Blocks b-1 and b are full, since rows follow them.
 __global__ __launch_bounds__(256) void trsv_lower_pair_kernel(const double* __restrict__ A, int n, int b,
                                                               double* __restrict__ x) {
-  __shared__ double xs[2 * kNB];
+  __shared__ double xs[2 * kNB], vs[2 * kNB];
   const int nblk = (n + kNB - 1) / kNB;
   const int first = b > 0 ? b - 1 : b;
   const int c0 = first * kNB, nblocks = b - first + 1;
@@ -755,14 +772,11 @@ __global__ __launch_bounds__(256) void trsv_lower_pair_kernel(const double* __re
   const bool lead = blockIdx.x == 0 && t < 64;
   const int b1 = b + 1, b2 = b + 2;
   const bool has2 = b2 < nblk;
-  const int i = b1 * kNB + blockIdx.x * 256 + t;
+  // this thread's row: 256 a workgroup from b1 kNB - 64 on; the lead's lanes hold the
+  // second wave's rows
+  const int i = b1 * kNB + (lead ? t : (int)blockIdx.x * 256 + t - 64);
   const bool row = i < n;
-  double c[2][kNB];
-#pragma unroll
-  for (int k = 0; k < 2; ++k)
-#pragma unroll
-    for (int u = 0; u < kNB; ++u)
-      c[k][u] = (row && k < nblocks) ? A[(int64_t)(c0 + k * kNB + u) * n + i] : 0.0;
+  double v = 0.0;
   DiagBlock d;
   double l21[kNB];  // lanes 32-63: L[i][b1 kNB + u], row i in block b2
   if (lead) {
@@ -770,32 +784,41 @@ __global__ __launch_bounds__(256) void trsv_lower_pair_kernel(const double* __re
     diag_load(A, n, second ? b2 * kNB : b1 * kNB, (second && !has2) ? -1 : (t & (kNB - 1)), d);
 #pragma unroll
     for (int u = 0; u < kNB; ++u) l21[u] = (second && row) ? A[(int64_t)(b1 * kNB + u) * n + i] : 0.0;
-  }
-  double v = row ? x[i] : 0.0;
-  if (t < nblocks * kNB) xs[t] = x[c0 + t];
-  __syncthreads();
+    diag_scale<true>(d, t & (kNB - 1));
+    __syncthreads();
+  } else {
+    double c[2][kNB];
 #pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    if (k < nblocks) {
-      double s = 0.0;
+    for (int k = 0; k < 2; ++k)
 #pragma unroll
-      for (int u = 0; u < kNB; ++u) s += c[k][u] * xs[k * kNB + u];
-      v -= s;
+      for (int u = 0; u < kNB; ++u)
+        c[k][u] = (row && k < nblocks) ? A[(int64_t)(c0 + k * kNB + u) * n + i] : 0.0;
+    v = row ? x[i] : 0.0;
+    const int e = t - 192;  // the last wave brings the solved entries
+    if (e >= 0 && e < nblocks * kNB) xs[e] = x[c0 + e];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      if (k < nblocks) {
+        double s = 0.0;
+#pragma unroll
+        for (int u = 0; u < kNB; ++u) s += c[k][u] * xs[k * kNB + u];
+        v -= s;
+      }
     }
+    if (blockIdx.x == 0 && t < 128) vs[t - 64] = v;
+    else if (row) x[i] = v;
   }
-  if (!lead) {
-    if (row) x[i] = v;
-    return;
-  }
-  d.rdii = 1.0 / d.rdii;
-  const int nb1 = min(kNB, n - b1 * kNB);
-  v = diag_lower_solve(d, 0, nb1, v);  // lanes 32-63 keep their right-hand sides
+  __syncthreads();
+  if (!lead) return;
+  v = vs[t];
+  v = diag_substitute<true>(d, 0, v);  // lanes 32-63 keep their right-hand sides
   if (has2) {
     double s = 0.0;
 #pragma unroll
     for (int u = 0; u < kNB; ++u) s += l21[u] * lane_bcast(v, u);
     if (t >= kNB) v -= s;
-    v = diag_lower_solve(d, kNB, min(kNB, n - b2 * kNB), v);
+    v = diag_substitute<true>(d, kNB, v);
   }
   if (row) x[i] = v;
 }
@@ -809,23 +832,19 @@ __global__ __launch_bounds__(256) void trsv_lower_pair_kernel(const double* __re
 // solves block b-1, takes its terms out of block b-2 and solves block b-2.
 __global__ __launch_bounds__(256) void trsv_upper_pair_kernel(const double* __restrict__ A, int n, int b,
                                                               double* __restrict__ x) {
-  __shared__ double xs[2 * kNB];
+  __shared__ double xs[2 * kNB], vs[2 * kNB];
   const int nblk = (n + kNB - 1) / kNB;
   const bool hi = b + 1 < nblk;
   const int kh = (b + 1) * kNB, nbh = hi ? min(kNB, n - kh) : 0;
   const int kb = b * kNB, nbb = min(kNB, n - kb);
   const int t = threadIdx.x;
-  const int g = blockIdx.x * 256 + t;
-  const bool lead = g < 64;
+  const bool lead = blockIdx.x == 0 && t < 64;
+  const int g = lead ? t : (int)blockIdx.x * 256 + t - 64;
   const int b1 = b - 1, b2 = b - 2;
   const bool has2 = b2 >= 0;
   const int i = g < kNB ? b1 * kNB + g : (g < 2 * kNB ? b2 * kNB + g - kNB : b2 * kNB + 2 * kNB - 1 - g);
   const bool row = i >= 0;
-  double c[2][kNB];
-#pragma unroll
-  for (int u = 0; u < kNB; ++u) c[0][u] = (row && u < nbh) ? A[(int64_t)(kh + u) * n + i] : 0.0;
-#pragma unroll
-  for (int u = 0; u < kNB; ++u) c[1][u] = (row && u < nbb) ? A[(int64_t)(kb + u) * n + i] : 0.0;
+  double v = 0.0;
   DiagBlock d;
   double l12[kNB];  // lanes 32-63: L[b1 kNB + u][i], row i in block b2
   if (lead) {
@@ -833,37 +852,45 @@ __global__ __launch_bounds__(256) void trsv_upper_pair_kernel(const double* __re
     diag_load(A, n, second ? b2 * kNB : b1 * kNB, (second && !has2) ? -1 : (t & (kNB - 1)), d);
 #pragma unroll
     for (int u = 0; u < kNB; ++u) l12[u] = (second && row) ? A[(int64_t)(b1 * kNB + u) * n + i] : 0.0;
+    diag_scale<false>(d, t & (kNB - 1));
+    __syncthreads();
+  } else {
+    double c[2][kNB];
+#pragma unroll
+    for (int u = 0; u < kNB; ++u) c[0][u] = (row && u < nbh) ? A[(int64_t)(kh + u) * n + i] : 0.0;
+#pragma unroll
+    for (int u = 0; u < kNB; ++u) c[1][u] = (row && u < nbb) ? A[(int64_t)(kb + u) * n + i] : 0.0;
+    v = row ? x[i] : 0.0;
+    const int e = t - 192;  // the last wave brings the solved entries
+    if (e >= 0) xs[e] = e < kNB ? (e < nbh ? x[kh + e] : 0.0) : (e - kNB < nbb ? x[kb + e - kNB] : 0.0);
+    __syncthreads();
+    if (hi) {
+      double s = 0.0;
+#pragma unroll
+      for (int u = 0; u < kNB; ++u)
+        if (u < nbh) s += c[0][u] * xs[u];
+      v -= s;
+    }
+    {
+      double s = 0.0;
+#pragma unroll
+      for (int u = 0; u < kNB; ++u)
+        if (u < nbb) s += c[1][u] * xs[kNB + u];
+      v -= s;
+    }
+    if (blockIdx.x == 0 && t < 128) vs[t - 64] = v;
+    else if (row) x[i] = v;
   }
-  double v = row ? x[i] : 0.0;
-  if (t < nbh) xs[t] = x[kh + t];
-  if (t >= kNB && t < kNB + nbb) xs[t] = x[kb + t - kNB];
   __syncthreads();
-  if (hi) {
-    double s = 0.0;
-#pragma unroll
-    for (int u = 0; u < kNB; ++u)
-      if (u < nbh) s += c[0][u] * xs[u];
-    v -= s;
-  }
-  {
-    double s = 0.0;
-#pragma unroll
-    for (int u = 0; u < kNB; ++u)
-      if (u < nbb) s += c[1][u] * xs[kNB + u];
-    v -= s;
-  }
-  if (!lead) {
-    if (row) x[i] = v;
-    return;
-  }
-  d.rdii = 1.0 / d.rdii;
-  v = diag_upper_solve(d, 0, kNB, v);  // lanes 32-63 keep their right-hand sides
+  if (!lead) return;
+  v = vs[t];
+  v = diag_substitute<false>(d, 0, v);  // lanes 32-63 keep their right-hand sides
   if (has2) {
     double s = 0.0;
 #pragma unroll
     for (int u = 0; u < kNB; ++u) s += l12[u] * lane_bcast(v, u);
     if (t >= kNB) v -= s;
-    v = diag_upper_solve(d, kNB, kNB, v);
+    v = diag_substitute<false>(d, kNB, v);
   }
   if (row) x[i] = v;
 }
@@ -1002,13 +1029,13 @@ int dense_cholesky_solve(int32_t n, const double* A, const double* b, double* x,
   hipLaunchKernelGGL(diag_solve_kernel<true>, dim3(1), dim3(64), 0, stream, A, n, 0, x);
   for (int blk = 0; blk + 1 < nblk; blk += 2) {
     const int rest = n - (blk + 1) * kNB;
-    hipLaunchKernelGGL(trsv_lower_pair_kernel, dim3((unsigned)((rest + 255) / 256)), dim3(256), 0, stream, A, n,
+    hipLaunchKernelGGL(trsv_lower_pair_kernel, dim3((unsigned)((rest + 64 + 255) / 256)), dim3(256), 0, stream, A, n,
                        blk, x);
   }
   // backward: the last block's diagonal solve, then two blocks a launch
   hipLaunchKernelGGL(diag_solve_kernel<false>, dim3(1), dim3(64), 0, stream, A, n, (nblk - 1) * kNB, x);
   for (int blk = nblk - 1; blk >= 1; blk -= 2)
-    hipLaunchKernelGGL(trsv_upper_pair_kernel, dim3((unsigned)((blk * kNB + 255) / 256)), dim3(256), 0, stream, A,
+    hipLaunchKernelGGL(trsv_upper_pair_kernel, dim3((unsigned)((blk * kNB + 64 + 255) / 256)), dim3(256), 0, stream, A,
                        n, blk, x);
   return check_launch("dense_solve");
 }
