@@ -40,36 +40,72 @@ struct ConcTable {
   float c[kNT];  // R80 / R20 of that index, increasing
 };
 
-__device__ __forceinline__ float block_sum(float v, float* red) {
-  v = wave_sum(v);
+// the workgroup's sums of N values, each its four waves' in order (red: 4 N)
+template <typename T, int N>
+__device__ __forceinline__ void block_sums(T (&v)[N], T* red) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] = wave_sum(v[k]);
   __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) red[4 * k + (threadIdx.x >> 6)] = v[k];
+  }
   __syncthreads();
-  return red[0] + red[1] + red[2] + red[3];
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] = red[4 * k] + red[4 * k + 1] + red[4 * k + 2] + red[4 * k + 3];
 }
 
-__device__ __forceinline__ double block_sumd(double v, double* red) {
-  v = wave_sum(v);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  return red[0] + red[1] + red[2] + red[3];
+// Coordinates along and across an angle, and a difference of two squares, with
+// every multiply-add written out: which of two products the compiler folds into
+// an addition depends on the code around it, and with it the last bit of the
+// estimates and the course of the fits that start from them.
+__device__ __forceinline__ float along(float c, float s, float X, float Y) { return fmaf(c, X, s * Y); }
+__device__ __forceinline__ float across(float c, float s, float X, float Y) { return fmaf(c, Y, -(s * X)); }
+__device__ __forceinline__ float diff(float xx, float yy) {
+#pragma clang fp contract(off)
+  return xx - yy;
 }
 
-__global__ __launch_bounds__(256) void moment_init_kernel(apx_batch b, ConcTable T, double* rep) {
-  __shared__ float redf[4];
-  __shared__ double redd[4];
+// column and row of this thread's pixel, and of the one 256 further on
+struct PixelWalk {
+  int i, j, di, dj, nx;
+  __device__ __forceinline__ explicit PixelWalk(int nx_) : nx(nx_) {
+    j = (int)threadIdx.x / nx;
+    i = (int)threadIdx.x - j * nx;
+    dj = 256 / nx;
+    di = 256 - dj * nx;
+  }
+  __device__ __forceinline__ void next() {
+    i += di;
+    j += dj;
+    if (i >= nx) {
+      i -= nx;
+      ++j;
+    }
+  }
+};
+
+// Bound by vector issue: 20,000 instructions a wave a 64 x 64 cutout, of 12 kB of
+// data.  So no pixel is divided into column and row, three passes over the pixels
+// take what five did, the bins' exponentials and logarithms and the indices' b_n
+// are taken a lane each (one thread took them bin after bin, and each point of
+// the (n, Re) grid its own b_n), and a centre window of up to 64 pixels is summed
+// by every wave for itself, without a barrier: 8,192 cutouts 784 -> 496 us (600 with
+// 98 registers, 4 waves a SIMD, in place of 64 and 8), the same bits.
+__global__ __launch_bounds__(256, 8) void moment_init_kernel(apx_batch b, ConcTable T, double* rep) {
+  __shared__ float redf[16];
+  __shared__ double redd[8];
   __shared__ float hist[kNB + 1], cnt[kNB + 1], yk[kNB + 1], lrk[kNB + 1];
+  __shared__ float rhi[kNB + 1];  // upper edges of the bins
   __shared__ unsigned long long hq[kNB + 1];  // fixed-point bin sums (two's complement)
   __shared__ float est[3], bres[4];
   __shared__ int bidx[4], nvalid;
-  __shared__ float cen[2];
-  __shared__ int stop;
   // the concentration table in LDS (read at run-time indices)
-  __shared__ float tn[kNT], tc[kNT];
+  __shared__ float tn[kNT], tc[kNT], tb[kNT];  // tb: b_n
   if (threadIdx.x < kNT) {
     tn[threadIdx.x] = T.n[threadIdx.x];
     tc[threadIdx.x] = T.c[threadIdx.x];
+    tb[threadIdx.x] = (float)sersic_b((double)T.n[threadIdx.x]);
   }
   __syncthreads();
   for (int g = blockIdx.x; g < b.ngal; g += gridDim.x) {
@@ -78,7 +114,7 @@ __global__ __launch_bounds__(256) void moment_init_kernel(apx_batch b, ConcTable
     const int nx = G.nx, ny = G.ny, n = nx * ny;
     // ---- edge level and scatter
     const int ne = nx > 1 && ny > 1 ? 2 * nx + 2 * (ny - 2) : n;
-    double s1 = 0.0, s2 = 0.0;
+    double s12[2] = {0.0, 0.0};
     for (int e = threadIdx.x; e < ne; e += 256) {
       int i, j;
       if (ne == n) {
@@ -92,91 +128,91 @@ __global__ __launch_bounds__(256) void moment_init_kernel(apx_batch b, ConcTable
         i = (k & 1) ? nx - 1 : 0, j = 1 + (k >> 1);
       }
       const double v = im[(int64_t)j * nx + i];
-      s1 += v;
-      s2 += v * v;
+      s12[0] += v;
+      s12[1] += v * v;
     }
-    s1 = block_sumd(s1, redd);
-    s2 = block_sumd(s2, redd);
+    block_sums(s12, redd);
+    const double s1 = s12[0], s2 = s12[1];
     const float edge = (float)(s1 / ne);
     const float scatter = (float)sqrt(fmax(s2 / ne - (s1 / ne) * (s1 / ne), 0.0));
     // ---- PSF second moment (per axis), for the moment corrections
     const float* K = b.psf + G.psf_off;
-    double k0 = 0.0, k2 = 0.0;
+    double k02[2] = {0.0, 0.0};
     for (int e = threadIdx.x; e < G.ph * G.pw; e += 256) {
       const double dx = e % G.pw - (G.pw - 1) / 2, dy = e / G.pw - (G.ph - 1) / 2;
-      k0 += K[e];
-      k2 += K[e] * (dx * dx + dy * dy);
+      k02[0] += K[e];
+      k02[1] += K[e] * (dx * dx + dy * dy);
     }
-    k0 = block_sumd(k0, redd);
-    k2 = block_sumd(k2, redd);
-    const float psf2 = (float)(0.5 * k2 / fmax(k0, 1e-30));  // sigma^2 per axis
+    block_sums(k02, redd);
+    const float psf2 = (float)(0.5 * k02[1] / fmax(k02[0], 1e-30));  // sigma^2 per axis
     // ---- centre: windowed centre of mass from the cutout centre (row, col)
     int win = max(min(min(nx, ny) / 10, 30), 6);
     win += win % 2;
-    if (threadIdx.x == 0) {
-      cen[0] = 0.5f * (ny - 1);  // row
-      cen[1] = 0.5f * (nx - 1);  // col
-      stop = 0;
-    }
-    __syncthreads();
-    const float init_r = cen[0], init_c = cen[1];
+    const float init_r = 0.5f * (ny - 1), init_c = 0.5f * (nx - 1);  // row, column
+    float pr = init_r, pc = init_c;  // pixel indices of the centre, the same in every thread
+    const bool one_wave = win * win <= 64;  // every wave sums the whole window
     for (int it = 0; it < 100; ++it) {
-      const int r0 = (int)rintf(cen[0]) - win / 2, c0 = (int)rintf(cen[1]) - win / 2;
+      const int r0 = (int)rintf(pr) - win / 2, c0 = (int)rintf(pc) - win / 2;
       if (r0 < 0 || c0 < 0 || r0 + win >= ny || c0 + win >= nx) {  // image edge: keep the start
-        __syncthreads();
-        if (threadIdx.x == 0) {
-          cen[0] = init_r;
-          cen[1] = init_c;
-        }
-        __syncthreads();
+        pr = init_r;
+        pc = init_c;
         break;
       }
-      float d = 0.0f, sr = 0.0f, sc = 0.0f;
-      for (int e = threadIdx.x; e < win * win; e += 256) {
+      float m[3] = {0.0f, 0.0f, 0.0f};
+      for (int e = one_wave ? (int)threadIdx.x & 63 : (int)threadIdx.x; e < win * win; e += 256) {
         const int rr = e / win, cc = e % win;
         const float v = im[(int64_t)(r0 + rr) * nx + c0 + cc];
-        d += v;
-        sr += v * rr;
-        sc += v * cc;
+        m[0] += v;
+        m[1] += v * rr;
+        m[2] += v * cc;
       }
-      d = block_sum(d, redf);
-      sr = block_sum(sr, redf);
-      sc = block_sum(sc, redf);
-      __syncthreads();
-      if (threadIdx.x == 0) {
-        const float nr = r0 + sr / d, nc = c0 + sc / d;
-        // converged: keep the previous centre, as center.py:45-49 does
-        if (!(fabsf(nr - cen[0]) + fabsf(nc - cen[1]) >= 0.1f)) {
-          stop = 1;
-          if (!isfinite(nr) || !isfinite(nc)) {
-            cen[0] = init_r;
-            cen[1] = init_c;
-          }
-        } else {
-          cen[0] = nr;
-          cen[1] = nc;
-        }
-      }
-      __syncthreads();
-      if (stop) break;
-    }
-    const float pr = cen[0], pc = cen[1];  // pixel indices of the centre
-    // ---- PA: angular centre of mass of (data - edge) about the centre
-    float cs = 0.0f, sn = 0.0f;
-    for (int p = threadIdx.x; p < n; p += 256) {
-      const float X = (p % nx) - pc, Y = (p / nx) - pr;
-      const float w = im[p] - edge;
-      const float r2 = X * X + Y * Y;
-      if (r2 > 0.0f) {
-        const float inv = 1.0f / r2;
-        cs += w * (X * X - Y * Y) * inv;  // cos 2 theta
-        sn += w * (2.0f * X * Y) * inv;   // sin 2 theta
+      if (one_wave) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) m[k] = wave_sum(m[k]);
       } else {
-        cs += w;  // a pixel on the centre: arctan2(0, 0) = 0 (angle_operations.py:52-55)
+        block_sums(m, redf);
+      }
+      const float nr = r0 + m[1] / m[0], nc = c0 + m[2] / m[0];
+      // converged: keep the previous centre, as center.py:45-49 does
+      if (!(fabsf(nr - pr) + fabsf(nc - pc) >= 0.1f)) {
+        if (!isfinite(nr) || !isfinite(nc)) {
+          pr = init_r;
+          pc = init_c;
+        }
+        break;
+      }
+      pr = nr;
+      pc = nc;
+    }
+    // ---- one pass: PA (angular centre of mass of (data - edge) about the
+    // centre), the rms radius of the pixels above 5 sigma (for q), and the sum of
+    // |data - edge| (for the growth curve)
+    float ps[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // cos, sin, light and r^2 light above 5 sigma
+    double sab[1] = {0.0};
+    {
+      PixelWalk at(nx);
+      for (int p = threadIdx.x; p < n; p += 256, at.next()) {
+        const float X = at.i - pc, Y = at.j - pr;
+        const float w = im[p] - edge;
+        const float xx = X * X, yy = Y * Y, r2 = fmaf(X, X, yy);
+        float c = w;  // a pixel on the centre: arctan2(0, 0) = 0 (angle_operations.py:52-55)
+        if (r2 > 0.0f) {
+          const float inv = 1.0f / r2;
+          c = w * diff(xx, yy) * inv;                      // cos 2 theta
+          ps[1] = fmaf(w * (2.0f * X * Y), inv, ps[1]);  // sin 2 theta
+        }
+        ps[0] += c;
+        if (w > 5.0f * scatter) {
+          ps[2] += w;
+          ps[3] = fmaf(w, r2, ps[3]);
+        }
+        sab[0] += fabs((double)w);
       }
     }
-    cs = block_sum(cs, redf);
-    sn = block_sum(sn, redf);
+    block_sums(ps, redf);
+    block_sums(sab, redd);
+    const float cs = ps[0], sn = ps[1], c0 = ps[2], c2 = ps[3];
+    const double sabs = sab[0];
     float ang = 0.5f * atan2f(sn, cs);  // angle of the light, mod pi
     // ---- q: second moments along / across that angle of the pixels above
     // 3 sigma within 4 core radii (+2 px) of the centre; the core radius is the
@@ -184,32 +220,24 @@ __global__ __launch_bounds__(256) void moment_init_kernel(apx_batch b, ConcTable
     // noise pixels far out, whose r^2 lever arm would otherwise round the light.
     const float ca = cosf(ang), sa = sinf(ang);
     const float thr = 3.0f * scatter;
-    float c0 = 0.0f, c2 = 0.0f;
-    for (int p = threadIdx.x; p < n; p += 256) {
-      const float w = im[p] - edge;
-      if (!(w > 5.0f * scatter)) continue;
-      const float X = (p % nx) - pc, Y = (p / nx) - pr;
-      c0 += w;
-      c2 += w * (X * X + Y * Y);
-    }
-    c0 = block_sum(c0, redf);
-    c2 = block_sum(c2, redf);
     const float rcore = c0 > 0.0f ? sqrtf(c2 / c0) : 0.125f * (float)min(nx, ny);
     const float rlim2 = (4.0f * rcore + 2.0f) * (4.0f * rcore + 2.0f);
-    float mu = 0.0f, mv = 0.0f, mw = 0.0f;
-    for (int p = threadIdx.x; p < n; p += 256) {
-      const float w = im[p] - edge;
-      if (!(w > thr)) continue;
-      const float X = (p % nx) - pc, Y = (p / nx) - pr;
-      if (X * X + Y * Y > rlim2) continue;
-      const float u = ca * X + sa * Y, v = -sa * X + ca * Y;
-      mu += w * u * u;
-      mv += w * v * v;
-      mw += w;
+    float ms[3] = {0.0f, 0.0f, 0.0f};
+    {
+      PixelWalk at(nx);
+      for (int p = threadIdx.x; p < n; p += 256, at.next()) {
+        const float w = im[p] - edge;
+        if (!(w > thr)) continue;
+        const float X = at.i - pc, Y = at.j - pr;
+        if (fmaf(X, X, Y * Y) > rlim2) continue;
+        const float u = along(ca, sa, X, Y), v = across(ca, sa, X, Y);
+        ms[0] = fmaf(u, w * u, ms[0]);
+        ms[1] = fmaf(v, w * v, ms[1]);
+        ms[2] += w;
+      }
     }
-    mu = block_sum(mu, redf);
-    mv = block_sum(mv, redf);
-    mw = block_sum(mw, redf);
+    block_sums(ms, redf);
+    const float mu = ms[0], mv = ms[1], mw = ms[2];
     // half the PSF second moment is removed: the thresholded moments see
     // only the part of the PSF wings above the threshold
     float q = 0.7f;
@@ -230,20 +258,19 @@ __global__ __launch_bounds__(256) void moment_init_kernel(apx_batch b, ConcTable
     // The bin sums are accumulated in 64-bit fixed point, so that they do not
     // depend on the order of the atomic adds: the scale puts sum |data - edge|
     // below 2^60, and each pixel is rounded to 2^-60 of that sum.
-    double sabs = 0.0;
-    for (int p = threadIdx.x; p < n; p += 256) sabs += fabs((double)(im[p] - edge));
-    sabs = block_sumd(sabs, redd);
     const bool fin = isfinite(sabs);  // else every bin takes the non-finite sum
     const double fx = sabs > 0.0 && fin ? ldexp(1.0, 60 - ilogb(sabs) - 1) : 1.0;
     for (int k = threadIdx.x; k <= kNB; k += 256) {
       cnt[k] = 0.0f;
       hq[k] = 0ull;
+      rhi[k] = kR0 * expf(lstep * k);
     }
     __syncthreads();
-    for (int p = threadIdx.x; p < n; p += 256) {
-      const float X = (p % nx) - pc, Y = (p / nx) - pr;
-      const float u = cu * X + su * Y, v = (-su * X + cu * Y) / q;
-      const float R = sqrtf(u * u + v * v);
+    PixelWalk at(nx);
+    for (int p = threadIdx.x; p < n; p += 256, at.next()) {
+      const float X = at.i - pc, Y = at.j - pr;
+      const float u = along(cu, su, X, Y), v = across(cu, su, X, Y) / q;
+      const float R = sqrtf(fmaf(u, u, v * v));
       const int k = R < kR0 ? 0 : min(kNB, 1 + (int)(logf(R / kR0) / lstep));
       const float w = im[p] - edge;
       if (fin) atomicAdd(&hq[k], (unsigned long long)(long long)rint((double)w * fx));
@@ -252,14 +279,36 @@ __global__ __launch_bounds__(256) void moment_init_kernel(apx_batch b, ConcTable
     __syncthreads();
     for (int k = threadIdx.x; k <= kNB; k += 256) hist[k] = fin ? (float)((double)(long long)hq[k] / fx) : (float)sabs;
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < 64) {
+      // radial profile bins for the fit below: mean surface brightness with
+      // S/N >= 3, outside the PSF core when enough such bins remain; lane k - 1
+      // looks at bin k and the kept ones close up in order
+      const int k = (int)threadIdx.x + 1;
+      const float rk = kR0 * expf(lstep * (k - 0.5f));
+      const float Ik = hist[k] / cnt[k];
+      const bool bright = !(cnt[k] < 4.0f) && Ik > 3.0f * scatter / sqrtf(cnt[k]);
+      const float y = log10f(Ik), lr = logf(rk);
+      int nv = 0;
+      for (int pass = 0; pass < 2 && nv < 4; ++pass) {
+        const float rcut = pass == 0 ? 1.5f * sqrtf(psf2) : 0.0f;
+        const bool keep = bright && !(rk < rcut);
+        const uint64_t bal = __ballot(keep);
+        nv = (int)__popcll(bal);
+        if (keep) {
+          const int at_k = (int)__popcll(bal & ((1ull << threadIdx.x) - 1));
+          yk[at_k] = y;
+          lrk[at_k] = lr;
+        }
+      }
+      if (threadIdx.x == 0) nvalid = nv;
+    } else if (threadIdx.x == 64) {
       float tot = 0.0f;
       for (int k = 0; k <= kNB; ++k) tot += hist[k];
       // radius (upper bin edge, linear within a bin) where the curve first reaches f * tot
       auto radius = [&](float f) {
         float cum = 0.0f, prev_r = 0.0f;
         for (int k = 0; k <= kNB; ++k) {
-          const float r_hi = kR0 * expf(lstep * k);
+          const float r_hi = rhi[k];
           const float nc = cum + hist[k];
           if (nc >= f * tot && hist[k] > 0.0f) return prev_r + (r_hi - prev_r) * (f * tot - cum) / hist[k];
           cum = nc;
@@ -287,23 +336,6 @@ __global__ __launch_bounds__(256) void moment_init_kernel(apx_batch b, ConcTable
       est[0] = re;
       est[1] = ns;
       est[2] = tot;
-      // radial profile bins for the fit below: mean surface brightness with
-      // S/N >= 3, outside the PSF core when enough such bins remain
-      int nv = 0;
-      for (int pass = 0; pass < 2 && nv < 4; ++pass) {
-        nv = 0;
-        const float rcut = pass == 0 ? 1.5f * sqrtf(psf2) : 0.0f;
-        for (int k = 1; k <= kNB; ++k) {
-          const float rk = kR0 * expf(lstep * (k - 0.5f));
-          if (cnt[k] < 4.0f || rk < rcut) continue;
-          const float Ik = hist[k] / cnt[k];
-          if (!(Ik > 3.0f * scatter / sqrtf(cnt[k]))) continue;
-          yk[nv] = log10f(Ik);
-          lrk[nv] = logf(rk);
-          ++nv;
-        }
-      }
-      nvalid = nv;
     }
     __syncthreads();
     // ---- Sersic profile fit of log10 I(R) over an (n, Re) grid, log10 Ie
@@ -319,7 +351,7 @@ __global__ __launch_bounds__(256) void moment_init_kernel(apx_batch b, ConcTable
         const float nn = tn[c / kNRe];
         if (nn < 0.4f || nn > 7.5f) continue;
         const float lre = lre0 + (lre1 - lre0) * (float)(c % kNRe) / (kNRe - 1);
-        const float bn = (float)sersic_b((double)nn), inv = 1.0f / nn;
+        const float bn = tb[c / kNRe], inv = 1.0f / nn;
         float s1 = 0.0f, s2 = 0.0f;
         for (int k = 0; k < nv; ++k) {
           const float m = -bn * (__expf((lrk[k] - lre) * inv) - 1.0f) * 0.43429448f;
@@ -362,7 +394,7 @@ __global__ __launch_bounds__(256) void moment_init_kernel(apx_batch b, ConcTable
         ns = tn[c / kNRe];
         const float lre0 = logf(0.5f), lre1 = logf(4.0f * rmax);
         re = expf(lre0 + (lre1 - lre0) * (float)(c % kNRe) / (kNRe - 1));
-        const float bn = (float)sersic_b((double)ns), inv = 1.0f / ns;
+        const float bn = tb[c / kNRe], inv = 1.0f / ns;
         float s1 = 0.0f;
         for (int k = 0; k < nv; ++k) s1 += yk[k] + bn * (__expf((lrk[k] - logf(re)) * inv) - 1.0f) * 0.43429448f;
         // log10 of the surface brightness at Re, per unit plane area
@@ -485,7 +517,7 @@ double sersic_light_fraction(double n, double r_over_re) {
 int batch_moment_init(const apx_batch* b, double* rep, hipStream_t stream) {
   if (!b || !b->gal || !b->data || !b->psf || !rep || b->ngal < 1)
     return set_error(APX_E_INVALID, "batch_moment_init: bad arguments");
-  hipLaunchKernelGGL(moment_init_kernel, dim3(std::min(b->ngal, 4096)), dim3(256), 0, stream, *b,
+  hipLaunchKernelGGL(moment_init_kernel, dim3(std::min(b->ngal, 16384)), dim3(256), 0, stream, *b,
                      conc_table(), rep);
   hipLaunchKernelGGL(moment_finish_kernel, dim3((b->ngal + 255) / 256), dim3(256), 0, stream, *b, rep);
   return check_launch("batch_moment_init");
