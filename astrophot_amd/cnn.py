@@ -49,6 +49,8 @@ SIGNATURES = {
     "apx_gate_colsum_bf16": (ctypes.c_int, [_p, _p, _i32, _i32, _p, _p, _p, _i64, _p]),
     "apx_adam": (ctypes.c_int, [_p, _p, _p, _p, _i64, _f32, _f32, _f32, _f32, _i32, _p, _p]),
     "apx_asinh_input": (ctypes.c_int, [_p, _p, _i32, _i32, _p, _p]),
+    "apx_init_features_workspace_bytes": (_i64, []),
+    "apx_init_features": (ctypes.c_int, [_p, _p, _i32, _p, _p, _p, _p, _i64, _p]),
 }
 L.register(SIGNATURES)
 
@@ -317,14 +319,35 @@ class InitNet:
                                  lay.b.numel(), lr, beta1, beta2, eps, self.step_count, None, L.stream()))
 
     # -- inference ---------------------------------------------------------
+    def _infer(self, images: torch.Tensor, sigma: torch.Tensor) -> torch.Tensor:
+        """The (B, 8) outputs of ``forward(input(images, sigma), B)``, without the
+        activations the gradients need: the convolutions of a cutout run in one
+        workgroup (apx_init_features)."""
+        lib = L.load()
+        B = images.shape[0]
+        f1, f2 = self.layers[4], self.layers[5]
+        dev = images.device
+        wsb = lib.apx_init_features_workspace_bytes()
+        ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
+        feat = torch.empty((B, f1.cin), dtype=torch.bfloat16, device=dev)
+        h = torch.empty((B, f1.cout), dtype=torch.float32, device=dev)
+        hb = torch.empty((B, f1.cout), dtype=torch.bfloat16, device=dev)
+        out = torch.empty((B, NOUT), dtype=torch.float32, device=dev)
+        conv = self.layers[:4]
+        w = (_p * 4)(*(lay.wb.data_ptr() for lay in conv))
+        b = (_p * 4)(*(lay.b.data_ptr() for lay in conv))
+        L.check(lib.apx_init_features(images.data_ptr(), sigma.data_ptr(), B, w, b, feat.data_ptr(), ws.data_ptr(),
+                                      wsb, L.stream()))
+        gemm(feat, f1.cin, 1, f1.wb, f1.cout, 1, h, B, f1.cout, f1.cin, bias=f1.b, relu=True, Cb=hb)
+        gemm(hb, f2.cin, 1, f2.wb, f2.cout, 1, out, B, f2.cout, f2.cin, bias=f2.b)
+        return out
+
     def predict(self, images: torch.Tensor, sigma: torch.Tensor, batch: int = 4096, on_device: bool = False):
         """[cx, cy, q, PA, n, Re, Ie] (cutout-relative) for every cutout: a host
         array, or with ``on_device`` a float64 tensor decoded on the device."""
         outs = []
         for s in range(0, images.shape[0], batch):
-            im, sg = images[s:s + batch], sigma[s:s + batch]
-            B = im.shape[0]
-            outs.append(self.forward(self.input(im, sg), B, keep_cols=False).clone())
+            outs.append(self._infer(images[s:s + batch].contiguous(), sigma[s:s + batch].contiguous()))
         if on_device:
             return decode_device(torch.cat(outs), sigma)
         # one device-to-host copy for every chunk

@@ -248,6 +248,13 @@ int apx_adam(float* w, const float* g, float* m, float* v, int64_t n, float lr, 
   return apx::adam(w, g, m, v, n, lr, beta1, beta2, eps, step, w_bf16, static_cast<hipStream_t>(stream));
 }
 
+int64_t apx_init_features_workspace_bytes(void) { return apx::init_features_workspace_bytes(); }
+
+int apx_init_features(const float* images, const float* sigma, int32_t B, const uint16_t* const* w, const float* const* b,
+                      uint16_t* out, void* workspace, int64_t workspace_bytes, void* stream) {
+  return apx::init_features(images, sigma, B, w, b, out, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
 int apx_asinh_input(const float* x, const float* sigma, int32_t B, int32_t npx, uint16_t* out,
                     void* stream) {
   return apx::asinh_input(x, sigma, B, npx, out, static_cast<hipStream_t>(stream));

@@ -88,6 +88,9 @@ int gate_colsum(const float* src, const float* mask, int M, int N, uint16_t* dst
 int adam(float* w, const float* g, float* m, float* v, int64_t n, float lr, float b1, float b2,
          float eps, int step, uint16_t* wb, hipStream_t stream);
 int asinh_input(const float* x, const float* sigma, int Bn, int npx, uint16_t* out, hipStream_t stream);
+int64_t init_features_workspace_bytes();
+int init_features(const float* images, const float* sigma, int Bn, const uint16_t* const* w, const float* const* b,
+                  uint16_t* out, void* ws, int64_t ws_bytes, hipStream_t stream);
 int batch_counters(const apx_batch* b, int32_t* out, hipStream_t stream);
 int batch_results(const apx_batch* b, double* rep, double* chi2, int32_t* status, int32_t* iters,
                   int32_t* fallback, int32_t* done, hipStream_t stream);

@@ -416,6 +416,240 @@ __global__ __launch_bounds__(256) void asinh_input_kernel(const float* x, const 
   }
 }
 
+// ---------------------------------------------------------------------------
+// The network's input and its four convolutions of one cutout in one workgroup:
+// asinh(x / sigma), 64 x 64 x 1 -> 32 x 32 x 32 -> 16 x 16 x 32 -> 8 x 8 x 64 ->
+// 4 x 4 x 64, every activation in LDS.  A launch a layer wrote each activation in
+// float32 (which only the gradients read) and bfloat16 and read it back, 3 GB for
+// 8,192 cutouts, bound by HBM at 1.42 ms with the input pass; here a cutout's
+// 16 kB come in and 2 kB go out: 0.25 ms, set by the waves' own instructions.
+//
+// A layer's products are those of gemm_bf16_kernel: K = (ky, kx, ci) in steps of
+// 32 through one accumulator, so the outputs have the same bits.  The weights are
+// the MFMA's A operand and the pixels its B, so a lane ends with 4 consecutive
+// channels of a pixel: one 8-byte write.  A row of an activation holds its even
+// columns, then its odd ones: the 16 pixels of an operand are neighbours in LDS
+// for each tap of the stride-2 kernel (without bank conflicts, 64 bytes apart).
+// LDS: 64 kB of layer 1 (then layer 3) and 16 kB of the input (then layer 2), so
+// that two workgroups of 8 waves fit a CU.
+constexpr int kFtWaves = 8, kFtThreads = 64 * kFtWaves;
+constexpr int kFtIn = 36;                 // dwords a row of the input: columns -1 .. 64 as pairs, whole 16 bytes
+constexpr int kFtBig = 32 * 1024;         // layer 1 (bf16 values)
+constexpr size_t kFtLds = 2 * (kFtBig + 8 * 1024);
+static_assert(65 * kFtIn * 4 <= 2 * 8 * 1024, "the input fits the second region");
+// packed weights: layer, k-step, 16 channels, lane, 8 values
+constexpr int kFtW[4] = {0, 32 * 32, 32 * 32 + 288 * 32, 32 * 32 + 288 * 32 + 288 * 64};
+constexpr int kFtWeights = 32 * 32 + 288 * 32 + 288 * 64 + 576 * 64;
+
+struct FeatureNet {
+  const uint16_t* w[4];  // (K, Cout) bf16 of each convolution, K padded to 32
+  const float* b[4];
+};
+
+// the four weight matrices in the order the lanes of a k-step read them: lane l
+// of step s and channel block t holds W[32 s + 8 (l / 16) + j][16 t + l % 16]
+__global__ __launch_bounds__(256) void pack_weights_kernel(FeatureNet net, uint16_t* __restrict__ out) {
+  const int e = blockIdx.x * 256 + threadIdx.x;
+  if (e >= kFtWeights) return;
+  const int layer = e < kFtW[1] ? 0 : e < kFtW[2] ? 1 : e < kFtW[3] ? 2 : 3;
+  const int N = layer < 2 ? 32 : 64;
+  int r = e - (layer == 0 ? kFtW[0] : layer == 1 ? kFtW[1] : layer == 2 ? kFtW[2] : kFtW[3]);
+  const int j = r & 7, l = (r >> 3) & 63;
+  r >>= 9;
+  const int t = r % (N / 16), s = r / (N / 16);
+  const uint16_t* W = layer == 0 ? net.w[0] : layer == 1 ? net.w[1] : layer == 2 ? net.w[2] : net.w[3];
+  out[e] = W[(int64_t)(32 * s + 8 * (l >> 4) + j) * N + 16 * t + (l & 15)];
+}
+
+__device__ __forceinline__ v8bf as_bf8(uint4 v) { return __builtin_bit_cast(v8bf, v); }
+
+// two values as bf16 pair (round to nearest even, the first in the low half): the
+// bits of to_bf16 but for a NaN's payload
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+  typedef float v2f __attribute__((ext_vector_type(2)));
+  typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(((v2f){a, b}), v2bf));
+}
+
+// bias, ReLU and bf16 of a lane's 4 channels, as 8 bytes
+__device__ __forceinline__ uint2 finish4(v4f acc, float4 b) {
+  return make_uint2(pack2(fmaxf(acc[0] + b.x, 0.0f), fmaxf(acc[1] + b.y, 0.0f)),
+                    pack2(fmaxf(acc[2] + b.z, 0.0f), fmaxf(acc[3] + b.w, 0.0f)));
+}
+
+// 8 channels of a tap's pixel, zero outside the image (`in` false).  The read goes
+// ahead all the same, at an address inside the activation: under a branch each
+// read would wait for itself.
+__device__ __forceinline__ v8bf tap8(const uint16_t* at, bool in) {
+  const uint4 v = *reinterpret_cast<const uint4*>(at);
+  const uint32_t m = in ? ~0u : 0u;
+  return as_bf8(make_uint4(v.x & m, v.y & m, v.z & m, v.w & m));
+}
+
+__device__ __forceinline__ float4 bias4(const float* b, int c) { return make_float4(b[c], b[c + 1], b[c + 2], b[c + 3]); }
+
+// asinh(z) to within kAsinhUlp of asinhf: the odd series below 1/4, log2 and sqrt
+// units above.  `sure`: its bf16 rounding is that of asinhf, since no float within
+// kAsinhMargin ulp rounds another way (the margin also covers z = x (1 / sigma)
+// for x / sigma, 3 ulp); a pixel in 1,000 is not sure and takes asinhf itself,
+// which is 230 instructions beside 25 here (20 us for 4,096 cutouts).
+constexpr int kAsinhUlp = 12, kAsinhMargin = 2 * kAsinhUlp;
+__device__ __forceinline__ float asinh_fast(float z, bool& sure) {
+  const float a = fabsf(z), t = a * a;
+  const float lo = fmaf(a * t, fmaf(t, fmaf(t, fmaf(t, 105.0f / 3456.0f, -15.0f / 336.0f), 3.0f / 40.0f), -1.0f / 6.0f), a);
+  const float hi = 0.693147180559945309f * __builtin_amdgcn_logf(a + __builtin_amdgcn_sqrtf(fmaf(a, a, 1.0f)));
+  const float y = a < 0.25f ? lo : hi;
+  const int off = (int)(__float_as_uint(y) & 0xffffu) - 0x8000;
+  sure = a >= 1e-30f && a <= 1e9f && (off > kAsinhMargin || off < -kAsinhMargin);
+  return copysignf(y, z);
+}
+
+__global__ __launch_bounds__(kFtThreads, 4) void features_kernel(const float* __restrict__ images,
+                                                                  const float* __restrict__ sigma, int B,
+                                                                  FeatureNet net, const uint16_t* __restrict__ wp,
+                                                                  uint16_t* __restrict__ out) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t sm[];
+  uint16_t* big = sm;             // layer 1 [y][x odd][x / 2][32], layer 3 [y][x odd][x / 2][64]
+  uint16_t* low = sm + kFtBig;    // layer 2 [y][x odd][x / 2][32]
+  uint32_t* in = reinterpret_cast<uint32_t*>(low);  // input: row y + 1, pair (x + 1) / 2
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6, p = lane & 15, kq = lane >> 4;
+  const uint4* w0 = reinterpret_cast<const uint4*>(wp);  // 64 x 16 bytes a block
+  const v8bf w1[2] = {as_bf8(w0[lane]), as_bf8(w0[64 + lane])};
+  const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
+  // this thread's pixels of a cutout: row y, columns 8 c ..
+  const int y = t >> 3, c = t & 7;
+  float px[8];
+  auto load = [&](int b) {
+    const float* src = images + (int64_t)b * 4096 + 8 * t;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) px[q] = src[q];
+  };
+  if ((int)blockIdx.x < B) load(blockIdx.x);
+  for (int b = blockIdx.x; b < B; b += gridDim.x) {
+    // the weights of layers 2 to 4 are read for each cutout (from L2): held across
+    // the loop, as the compiler would, they spill
+    int keep = 0;
+    asm volatile("" : "+s"(keep));
+    const uint4* w4 = w0 + keep + lane;
+    // ---- input
+    {
+      const float sg = sigma[b], rs = 1.0f / sg;
+      const bool range = fabsf(sg) >= 1e-30f && fabsf(sg) <= 1e30f;
+      float h[8];
+      uint32_t left = 0;  // the pixels that take asinhf
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        bool sure;
+        h[q] = asinh_fast(px[q] * rs, sure);
+        if (px[q] == 0.0f) {
+          h[q] = px[q] * copysignf(1.0f, sg);
+          sure = true;
+        }
+        left |= (sure && range) ? 0u : 1u << q;
+      }
+      const float before = __shfl_up(h[7], 1, 64);  // every lane takes part
+      uint32_t* row = in + (y + 1) * kFtIn + 4 * c;
+      *reinterpret_cast<uint4*>(row) =
+          make_uint4(pack2(c == 0 ? 0.0f : before, h[0]), pack2(h[1], h[2]), pack2(h[3], h[4]), pack2(h[5], h[6]));
+      if (c == 7) row[4] = pack2(h[7], 0.0f);
+      if (t < kFtIn) in[t] = 0u;  // the row above the image
+      while (__any(left != 0)) {
+        if (left) {
+          const int q = __ffs(left) - 1;
+          left &= left - 1;
+          reinterpret_cast<uint16_t*>(in)[(y + 1) * 2 * kFtIn + 1 + 8 * c + q] =
+              to_bf16(asinhf(images[(int64_t)b * 4096 + 8 * t + q] / sg));
+        }
+      }
+      if (b + (int)gridDim.x < B) load(b + gridDim.x);
+    }
+    __syncthreads();
+    // ---- layer 1: a tile is 16 pixels of a row; K = the 9 taps
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int oy = w + kFtWaves * (q >> 1), ox = 16 * (q & 1) + p;
+      const uint32_t* r0 = in + 2 * oy * kFtIn + ox;  // row 2 oy - 1, columns 2 ox - 1, 2 ox
+      const uint32_t d0 = r0[0], d1 = r0[1], e0 = r0[kFtIn], e1 = r0[kFtIn + 1], f0 = r0[2 * kFtIn], f1 = r0[2 * kFtIn + 1];
+      uint4 v = make_uint4(d0, (d1 & 0xffffu) | (e0 << 16), (e0 >> 16) | (e1 << 16), f0);
+      if (kq == 1) v = make_uint4(f1 & 0xffffu, 0u, 0u, 0u);
+      if (kq > 1) v = zero;
+      uint16_t* o = big + oy * 1024 + (ox & 1) * 512 + (ox >> 1) * 32 + 4 * kq;
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        const v4f acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1[n], as_bf8(v), (v4f){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+        *reinterpret_cast<uint2*>(o + 16 * n) = finish4(acc, bias4(net.b[0], 16 * n + 4 * kq));
+      }
+    }
+    __syncthreads();
+    // ---- layer 2: 16 channels and four rows of 16 pixels a wave
+    {
+      const int n = w & 1, oy0 = w >> 1;
+      v4f acc[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int tap = 0; tap < 9; ++tap) {
+        const int ky = tap / 3, kx = tap % 3;
+        const v8bf a = as_bf8(w4[kFtW[1] / 8 + (tap * 2 + n) * 64]);
+        const int col = (kx == 0 ? 512 - 32 : kx == 1 ? 0 : 512) + p * 32 + kq * 8;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int iy = 2 * (oy0 + 4 * i) + ky - 1;
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              a, tap8(big + max(iy, 0) * 1024 + col, !(i == 0 && ky == 0 && iy < 0) && !(kx == 0 && p == 0)), acc[i], 0, 0, 0);
+        }
+      }
+      const float4 bb = bias4(net.b[1], 16 * n + 4 * kq);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<uint2*>(low + (oy0 + 4 * i) * 512 + (p & 1) * 256 + (p >> 1) * 32 + 16 * n + 4 * kq) =
+            finish4(acc[i], bb);
+    }
+    __syncthreads();
+    // ---- layer 3: 16 channels and twice two rows of 8 pixels a wave
+    {
+      const int n = w & 3, m0 = w >> 2, ox = p & 7;
+      v4f acc[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) acc[i] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int tap = 0; tap < 9; ++tap) {
+        const int ky = tap / 3, kx = tap % 3;
+        const v8bf a = as_bf8(w4[kFtW[2] / 8 + (tap * 4 + n) * 64]);
+        const int col = (kx == 0 ? 256 - 32 : kx == 1 ? 0 : 256) + ox * 32 + kq * 8;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int iy = 2 * (2 * (m0 + 2 * i) + (p >> 3)) + ky - 1;
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              a, tap8(low + max(iy, 0) * 512 + col, !(i == 0 && ky == 0 && iy < 0) && !(kx == 0 && ox == 0)), acc[i], 0, 0, 0);
+        }
+      }
+      const float4 bb = bias4(net.b[2], 16 * n + 4 * kq);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        *reinterpret_cast<uint2*>(big + (2 * (m0 + 2 * i) + (p >> 3)) * 512 + (ox & 1) * 256 + (ox >> 1) * 64 + 16 * n +
+                                  4 * kq) = finish4(acc[i], bb);
+    }
+    __syncthreads();
+    // ---- layer 4: 16 channels of the 4 x 4 pixels a wave (the other waves go on
+    // to the next cutout's input)
+    if (w < 4) {
+      const int oy = p >> 2, ox = p & 3;
+      v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int s = 0; s < 18; ++s) {
+        const int ky = (s >> 1) / 3, kx = (s >> 1) % 3;
+        const v8bf a = as_bf8(w4[kFtW[3] / 8 + (s * 4 + w) * 64]);
+        const int iy = 2 * oy + ky - 1;
+        const uint16_t* at = big + max(iy, 0) * 512 + (kx == 0 ? 256 - 64 : kx == 1 ? 0 : 256) + ox * 64 + (s & 1) * 32 + kq * 8;
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, tap8(at, !(ky == 0 && iy < 0) && !(kx == 0 && ox == 0)), acc, 0, 0, 0);
+      }
+      *reinterpret_cast<uint2*>(out + (int64_t)b * 1024 + p * 64 + 16 * w + 4 * kq) =
+          finish4(acc, bias4(net.b[3], 16 * w + 4 * kq));
+    }
+  }
+}
+
 // The form of an operand with element (r, k) at X[r * sr + k * sk] (R rows,
 // depth K): 16-byte loads where one of the two strides is 1 and the other, the
 // contiguous extent and the base keep every load whole and on 16 bytes.
@@ -562,6 +796,32 @@ int adam(float* w, const float* g, float* m, float* v, int64_t n, float lr, floa
   hipLaunchKernelGGL(adam_kernel, grid_for(n), dim3(256), 0, stream, w, g, m, v, n, lr, b1, b2, eps, c1,
                      c2, wb);
   return check_launch("adam");
+}
+
+int64_t init_features_workspace_bytes() { return 2 * kFtWeights; }
+
+int init_features(const float* images, const float* sigma, int Bn, const uint16_t* const* w, const float* const* b,
+                  uint16_t* out, void* ws, int64_t ws_bytes, hipStream_t stream) {
+  if (!images || !sigma || !w || !b || !out || !ws || Bn < 1) return set_error(APX_E_INVALID, "init_features: bad arguments");
+  if (ws_bytes < init_features_workspace_bytes()) return set_error(APX_E_INVALID, "init_features: workspace too small");
+  if ((reinterpret_cast<uintptr_t>(ws) & 15) || (reinterpret_cast<uintptr_t>(out) & 7))
+    return set_error(APX_E_INVALID, "init_features: workspace not on 16 bytes or output not on 8");
+  FeatureNet net;
+  for (int k = 0; k < 4; ++k) {
+    if (!w[k] || !b[k]) return set_error(APX_E_INVALID, "init_features: bad arguments");
+    net.w[k] = w[k];
+    net.b[k] = b[k];
+  }
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&features_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                          (int)kFtLds) != hipSuccess)
+    return set_error(APX_E_HIP, "init_features: LDS size refused");
+  uint16_t* wp = static_cast<uint16_t*>(ws);
+  hipLaunchKernelGGL(pack_weights_kernel, dim3((kFtWeights + 255) / 256), dim3(256), 0, stream, net, wp);
+  // two workgroups a CU, each cutout after cutout: the weights of layer 1 and the
+  // next cutout's pixels stay in registers
+  hipLaunchKernelGGL(features_kernel, dim3(std::min(Bn, 512)), dim3(kFtThreads), kFtLds, stream, images, sigma, Bn, net,
+                     (const uint16_t*)wp, out);
+  return check_launch("init_features");
 }
 
 int asinh_input(const float* x, const float* sigma, int Bn, int npx, uint16_t* out, hipStream_t stream) {

@@ -561,6 +561,17 @@ int apx_adam(float* w, const float* g, float* m, float* v, int64_t n, float lr, 
 int apx_asinh_input(const float* x, const float* sigma, int32_t B, int32_t npx, uint16_t* out,
                     void* stream);
 
+/* The network's input and four convolutions of B cutouts (64 x 64 float32
+ * images, sigma (B,)) without the layers between in memory: out (B, 4, 4, 64)
+ * bf16, the bits of apx_asinh_input and four apx_conv_s2_bf16 with bias and
+ * ReLU.  w, b: host arrays of the four convolutions' device pointers, w[k]
+ * (K, Cout) bf16 with K padded to 32, b[k] (Cout,) float32.  workspace (on 16
+ * bytes): apx_init_features_workspace_bytes() bytes. */
+int64_t apx_init_features_workspace_bytes(void);
+int apx_init_features(const float* images, const float* sigma, int32_t B, const uint16_t* const* w,
+                      const float* const* b, uint16_t* out, void* workspace, int64_t workspace_bytes,
+                      void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -11,11 +11,14 @@ the CPU.
 * a short training run on renderer-generated cutouts lowers the loss.
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 import torch.nn.functional as F
 
+from astrophot_amd import _lib as L
 from astrophot_amd import cnn
 
 pytestmark = pytest.mark.gpu
@@ -178,3 +181,33 @@ def test_implicit_convolution_equals_im2col_gemm(B):
     for a, b in zip(acts_a, acts_b):
         assert torch.equal(a, b)
     assert torch.equal(out_a, out_b)
+
+
+@pytest.mark.parametrize("B,shift", [(1, 0), (3, 1), (511, 0), (513, 3), (1100, 0)])
+def test_fused_convolutions_equal_the_layers(B, shift):
+    """apx_init_features gives the bits of the input pass and the four
+    convolutions run one after another, whatever the number of cutouts a
+    workgroup takes (512 workgroups) and wherever the images start (shift floats
+    past 16 bytes), and so does the whole prediction; NaN and infinite pixels and
+    a zero sigma take the same way through."""
+    net = cnn.InitNet(seed=2)
+    for k, lay in enumerate(net.layers):
+        lay.b.copy_(0.1 * torch.randn(lay.b.shape, generator=torch.Generator().manual_seed(k)))
+    g = torch.Generator().manual_seed(B)
+    base = (3 * torch.randn(B * 4096 + 4, generator=g)).to(DEV)
+    images = base[shift:shift + B * 4096].view(B, 64, 64)
+    sigma = (0.2 + torch.rand(B, generator=g)).to(DEV)
+    images[0, 0, 0], images[-1, 63, 63], images[-1, 31, 32] = 1e30, float("inf"), -1e30
+    if B > 2:
+        images[1, 5, 7], sigma[2] = float("nan"), 0.0
+    lib = L.load()
+    wsb = lib.apx_init_features_workspace_bytes()
+    ws, feat = torch.empty(wsb, dtype=torch.uint8, device=DEV), torch.empty(B * 1024, dtype=torch.bfloat16, device=DEV)
+    w = (ctypes.c_void_p * 4)(*(lay.wb.data_ptr() for lay in net.layers[:4]))
+    b = (ctypes.c_void_p * 4)(*(lay.b.data_ptr() for lay in net.layers[:4]))
+    L.check(lib.apx_init_features(images.data_ptr(), sigma.data_ptr(), B, w, b, feat.data_ptr(), ws.data_ptr(), wsb,
+                                  L.stream()))
+    ref = net.forward(net.input(images, sigma), B, keep_cols=False).clone()
+    same = lambda a, b: torch.equal(torch.nan_to_num(a), torch.nan_to_num(b)) and torch.equal(a.isnan(), b.isnan())  # noqa: E731
+    assert same(feat.float(), net._buffers(B)["yb"][3].reshape(-1).float())
+    assert same(net._infer(images, sigma), ref)
