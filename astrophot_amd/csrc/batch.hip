@@ -813,16 +813,117 @@ __global__ __launch_bounds__(256) void pack_kernel(apx_batch b, Scratch s, int f
   }
 }
 
-// the pixels select_kernel left undecided, with float64 decisions
+// select_pixel<GRAD, true, 3> by a team of 16 lanes (every lane of the wave calls
+// it; `active` is the same in a team's lanes): the float64 samples of a decision
+// go to a lane each, 5 or 6 for the curvature and 9 for the level-1 test
+template <bool GRAD>
+__device__ __forceinline__ void select_team(const apx_batch& b, const Scratch& s, const QuadTab& t, bool active, int g,
+                                            int pix) {
+  const int tl = threadIdx.x & 15;
+  const apx_batch_galaxy G = b.gal[g];
+  const GalEval& E = s.ev[g];
+  const int nxw = E.nxw, i = pix % nxw, j = pix / nxw;
+  const int ii = min(max(i, 1), nxw - 2), jj = min(max(j, 1), E.nyw - 2);
+  const float* v = s.mid + G.work_off + (int64_t)jj * nxw + ii;
+  const float l = v[-1], r = v[1], u = v[-nxw], d = v[nxw], m = v[0];
+  const float metric = fabsf(l + r + u + d - 4.0f * m);
+  const float scale = fabsf(l) + fabsf(r) + fabsf(u) + fabsf(d) + 4.0f * fabsf(m);
+  const double band = 1.6e-5 * (double)scale + 2.0e-7 * E.thr;
+  bool sel = (double)metric > E.thr + band;
+  const bool close = active && !sel && (double)metric >= E.thr - band;
+  double X, Y, val = 0.0;
+  if (close && tl < 6) {  // the centre, its left, right, upper and lower neighbours, the pixel
+    const int a = tl == 1 ? ii - 1 : tl == 2 ? ii + 1 : tl == 5 ? i : ii;
+    const int c = tl == 3 ? jj - 1 : tl == 4 ? jj + 1 : tl == 5 ? j : jj;
+    pixel_xy(E.pd, E.ci, E.cj, a, c, X, Y);
+    val = eval_profile<double, false>(E.pd, X, Y, 1.0, nullptr);
+  }
+  double at[6];
+#pragma unroll
+  for (int q = 0; q < 6; ++q) at[q] = __shfl(val, q, 16);
+  if (close) {
+    const double curv = at[1] + at[2] + at[3] + at[4] - 4.0 * at[0];
+    const double mid = at[5];
+    sel = fabs(mid - (mid + curv)) > E.thr;
+  }
+  float* pl = b.planes + G.work_off + pix;
+  float X0, Y0, gs[APX_NSLOT], centre = 0.0f;
+  pixel_xy(E.pf, E.ci, E.cj, i, j, X0, Y0);
+  const float r1 = GRAD ? quad3_grad(E.pf, t, X0, Y0, 0.5f, 0.0f, gs, centre)
+                        : quad3_value(E.pf, t, X0, Y0, 0.5f, 0.0f, centre);
+  const int dec = t.max_depth > 1 ? band_test(r1, centre, E.thr) : 0;
+  const bool test = active && sel && dec < 0;
+  val = 0.0;
+  if (test && tl < 9) {
+    pixel_xy(E.pd, E.ci, E.cj, i, j, X, Y);
+    const double un = t.noded[tl % 3], vn = t.noded[tl / 3];
+    const double h00 = 0.5 * E.pd.P00, h01 = 0.5 * E.pd.P01, h10 = 0.5 * E.pd.P10, h11 = 0.5 * E.pd.P11;
+    val = eval_profile<double, false>(E.pd, X + h00 * un + h01 * vn, Y + h10 * un + h11 * vn, 1.0, nullptr);
+  }
+  double rd = 0.0, cd = 0.0;
+#pragma unroll
+  for (int q = 0; q < 9; ++q) {
+    const double x = __shfl(val, q, 16);
+    rd += t.w2d[q] * x;
+    if (q == 4) cd = x;
+  }
+  const bool deeper = test ? fabs(rd - cd) > E.thr : dec == 1;
+  if (!active || tl != 0) return;
+  if (!sel) {
+    pl[0] = s.mid[G.work_off + pix];
+  } else if (deeper) {
+    s.deep[G.work_off + atomicAdd(&s.gal_cnt[g], 1)] = pix;
+  } else {
+    pl[0] = r1;
+    if (GRAD) {
+#pragma unroll
+      for (int c = 1; c < kNChan; ++c) pl[c * b.nwork] = gs[c + 1] * (float)E.dvdr[c + 1];
+    }
+  }
+}
+
+// The pixels select_kernel left undecided, with float64 decisions: a lane each,
+// or 16 lanes each where the list is short enough that every team of the launch
+// has one at most.  One lane takes up to 15 float64 samples one after another
+// (11 -> 6 us with about 100 fits left); on a long list (125 scene sources, 0.3 ms)
+// the lanes are all busy.
 template <bool GRAD, int QN>
 __global__ __launch_bounds__(256) void select_redo_kernel(apx_batch b, Scratch s, QuadTab t) {
   const int total = s.cnt[4];
+  if (QN == 3 && total <= (int)gridDim.x * 16) {
+    const int k = blockIdx.x * 16 + (int)(threadIdx.x >> 4);
+    if ((k & ~3) >= total) return;  // none of the wave's four teams has a pixel
+    const int2 q = s.rq[min(k, total - 1)];
+    select_team<GRAD>(b, s, t, k < total, q.x, q.y);
+    return;
+  }
   for (int k = blockIdx.x * 256 + threadIdx.x; k < total; k += gridDim.x * 256) {
     const int2 q = s.rq[k];
     const int g = q.x, pix = q.y;
     const apx_batch_galaxy G = b.gal[g];
     if (select_pixel<GRAD, true, QN>(b, s, G, s.ev[g], t, pix) == PX_DEEPER)
       s.deep[G.work_off + atomicAdd(&s.gal_cnt[g], 1)] = pix;
+  }
+}
+
+// A lane's level-3 samples of one flagged sub-pixel at (xs, ys), summed in float32
+template <bool GRAD, int GS, int ITS>
+__device__ __forceinline__ void level3_lane(const Prof<float>& pf, float xs, float ys, const float (&l3x)[ITS],
+                                            const float (&l3y)[ITS], const float (&l3w)[ITS], int gl, int nq, float sc3,
+                                            float (&fs)[1 + APX_NSLOT]) {
+#pragma unroll
+  for (int q = 0; q <= APX_NSLOT; ++q) fs[q] = 0.0f;
+#pragma unroll
+  for (int it = 0; it < ITS; ++it) {
+    if (gl + GS * it < nq) {
+      float gv[APX_NSLOT];
+      const float val = sersic_f<GRAD>(pf, xs + l3x[it], ys + l3y[it], sc3, gv);
+      fs[0] = fmaf(l3w[it], val, fs[0]);
+      if (GRAD) {
+#pragma unroll
+        for (int q = 0; q < APX_NSLOT; ++q) fs[1 + q] = fmaf(l3w[it], gv[q], fs[1 + q]);
+      }
+    }
   }
 }
 
@@ -834,6 +935,17 @@ __global__ __launch_bounds__(256) void select_redo_kernel(apx_batch b, Scratch s
 // QN, QG: quadrature level and gridding when known at compile time (0: from
 // t).  With both known, each lane's level-3 sample offsets (plane units) and
 // weights are computed once per launch.
+//
+// A short list (at most two pixels a resident workgroup, kWideMax) is taken a
+// workgroup a pixel: its 8 groups of 32 lanes evaluate level 2 alike and take the
+// flagged sub-pixels in turn, and thread (channel, lane) adds that lane's level-2
+// value and sub-pixel sums in the order the one group adds them, so the bits do
+// not change.  One group walks up to 25 sub-pixels of 8 samples a lane one after
+// another, and a lane up to 9 float64 samples of an undecided one, which sets the
+// time of a launch with few fits left (about 100 of 4,096: Jacobian pass 30 -> 21
+// us, its float64 pass 28 -> 12, the value pass's 19 -> 10).
+// A long list keeps a group a pixel, which evaluates level 2 once.
+constexpr int kWideMax = 2048;
 template <bool GRAD, int GS, bool F64, int QN, int QG>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void integrate_kernel(apx_batch b, Scratch s,
                                                                                                 QuadTab t) {
@@ -868,8 +980,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void i
   }
   const uint64_t gmask = GS == 64 ? ~0ull : (((1ull << GS) - 1ull) << (grp * GS));
   int nsub3 = 0;  // level-3 sub-pixels this wave integrates (work counter, wave-uniform)
-  for (int k0 = wave * NG; k0 < total; k0 += nwaves * NG) {
-    const int k = k0 + grp;
+  constexpr bool CAN_WIDE = FIXED && GS == 32;
+  constexpr int NV = GRAD ? 1 + APX_NSLOT : 1;
+  __shared__ double sample[CAN_WIDE && F64 ? QG * QG : 1][9];  // wide: an undecided sub-pixel's float64 samples
+  __shared__ float subsum[CAN_WIDE ? QG * QG : 1][NV][32];  // wide: a lane's sum of a flagged sub-pixel
+  const bool wide = CAN_WIDE && total <= min(kWideMax, 2 * (int)gridDim.x);
+  const int team = threadIdx.x / GS;  // wide: group of the workgroup, and channel it adds up
+  for (int k0 = wide ? (int)blockIdx.x : wave * NG; k0 < total; k0 += wide ? (int)gridDim.x : nwaves * NG) {
+    const int k = wide ? k0 : k0 + grp;
     const bool active = k < total;
     int gal = 0, pix = 0;
     if (active) {
@@ -899,7 +1017,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void i
       if (t.max_depth > 2) {
         const double thr2 = E->thr * (double)gg;
         dec = band_test(r2, c2, thr2);
-        if (F64 && dec < 0) {
+        if (F64 && dec < 0 && !wide) {
           const double igd = 1.0 / (double)g_, sub0d = -(double)(g_ - 1) / (2.0 * g_);
           const double ad = sub0d + igd * (gl % g_), bd = sub0d + igd * (gl / g_);
           const Prof<double>& pd = E->pd;
@@ -908,6 +1026,37 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void i
           const double rd = quad_d(pd, t, X + pd.P00 * ad + pd.P01 * bd, Y + pd.P10 * ad + pd.P11 * bd,
                                    0.5 * igd, igd * igd, cd);
           dec = fabs(rd - cd) > thr2 ? 1 : 0;
+        }
+      }
+    }
+    if (F64 && wide) {
+      // the undecided sub-pixels' float64 samples, one a thread (25 x 9 at most),
+      // then each sub-pixel's sum in quad_d's order
+      const uint64_t und = (__ballot(dec < 0) & gmask) >> (grp * GS);
+      const int nu = (int)__popcll(und);
+      if (nu > 0) {
+        const int f = (int)threadIdx.x / 9, kk = (int)threadIdx.x % 9;
+        if (f < nu) {
+          uint64_t m = und;
+          for (int i = 0; i < f; ++i) m &= m - 1ull;
+          const int sp = __ffsll((unsigned long long)m) - 1;
+          const double igd = 1.0 / (double)g_, sub0d = -(double)(g_ - 1) / (2.0 * g_);
+          const double ad = sub0d + igd * (sp % g_), bd = sub0d + igd * (sp / g_), h = 0.5 * igd;
+          const Prof<double>& pd = E->pd;
+          double X, Y;
+          pixel_xy(pd, ci, cj, pi, pj, X, Y);
+          const double u = t.noded[kk % 3], v = t.noded[kk / 3];
+          sample[f][kk] = eval_profile<double, false>(pd, X + pd.P00 * ad + pd.P01 * bd + h * pd.P00 * u + h * pd.P01 * v,
+                                                      Y + pd.P10 * ad + pd.P11 * bd + h * pd.P10 * u + h * pd.P11 * v,
+                                                      igd * igd, nullptr);
+        }
+        __syncthreads();
+        if (dec < 0) {
+          const int f2 = (int)__popcll(und & ((1ull << gl) - 1ull));
+          double rd = 0.0;
+#pragma unroll
+          for (int q = 0; q < 9; ++q) rd += t.w2d[q] * sample[f2][q];
+          dec = fabs(rd - sample[f2][4]) > E->thr * (double)gg ? 1 : 0;
         }
       }
     }
@@ -922,8 +1071,50 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void i
     }
     // level 3: the group integrates each flagged sub-pixel in turn
     uint64_t todo = (__ballot(deeper) & gmask) >> (GS == 64 ? 0 : grp * GS);
-    nsub3 += (int)__popcll(__ballot(deeper));
     const float sc3 = ig * ig * ig * ig;
+    if (wide) {
+      const int nf = (int)__popcll(todo);
+      nsub3 += (threadIdx.x >> 6) == 0 ? nf : 0;
+      // sub-pixel f, f + 8, ... of the flagged ones
+      for (int f0 = 0; f0 < nf; f0 += 256 / GS) {
+        uint64_t m = todo;
+        const int f = f0 + team;
+        for (int i = 0; i < f; ++i) m &= m - 1ull;
+        const int sp = m ? __ffsll((unsigned long long)m) - 1 : 0;
+        const float xs = __shfl(x2, grp * GS + sp, 64), ys = __shfl(y2, grp * GS + sp, 64);
+        if (f < nf) {
+          float fs[1 + APX_NSLOT];
+          level3_lane<GRAD, GS, ITS>(pf, xs, ys, l3x, l3y, l3w, gl, nq, sc3, fs);
+#pragma unroll
+          for (int q = 0; q < NV; ++q) subsum[f][q][gl] = fs[q];
+        }
+      }
+      __syncthreads();
+      if (team < NV) {
+        float first = r2;  // this channel's level-2 value
+        if (GRAD) {
+#pragma unroll
+          for (int q = 0; q < APX_NSLOT; ++q) first = team == 1 + q ? gs[q] : first;
+        }
+        double a = (gl < gg && dec == 0 && !undecided) ? (double)first : 0.0;
+        for (int f = 0; f < nf; ++f) a += (double)subsum[f][team][gl];
+        a = half_sum(a);
+        if (gl == 0) {
+          const int64_t wo = b.gal[gal].work_off;
+          if (undecided) {
+            if (team == 0) s.redo[wo + atomicAdd(&s.gal_rcnt[gal], 1)] = pix;
+          } else {
+            // slots 2 .. 6 (channels 3 .. 7) go to planes 1 .. 5
+            float* pl = b.planes + wo + pix;
+            if (team == 0) pl[0] = (float)a;
+            else if (team >= 3 && team - 2 < kNChan) pl[(team - 2) * b.nwork] = (float)(a * E->dvdr[team - 1]);
+          }
+        }
+      }
+      __syncthreads();
+      continue;
+    }
+    nsub3 += (int)__popcll(__ballot(deeper));
     while (__ballot(todo != 0ull)) {
       int sp = -1;
       if (todo) {
@@ -937,20 +1128,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void i
           // this lane's at most ITS samples of the sub-pixel, summed in float32,
           // then into the float64 accumulators
           float fs[1 + APX_NSLOT];
-#pragma unroll
-          for (int q = 0; q <= APX_NSLOT; ++q) fs[q] = 0.0f;
-#pragma unroll
-          for (int it = 0; it < ITS; ++it) {
-            if (gl + GS * it < nq) {
-              float gv[APX_NSLOT];
-              const float val = sersic_f<GRAD>(pf, xs + l3x[it], ys + l3y[it], sc3, gv);
-              fs[0] = fmaf(l3w[it], val, fs[0]);
-              if (GRAD) {
-#pragma unroll
-                for (int q = 0; q < APX_NSLOT; ++q) fs[1 + q] = fmaf(l3w[it], gv[q], fs[1 + q]);
-              }
-            }
-          }
+          level3_lane<GRAD, GS, ITS>(pf, xs, ys, l3x, l3y, l3w, gl, nq, sc3, fs);
           acc[0] += (double)fs[0];
           if (GRAD) {
 #pragma unroll

@@ -110,6 +110,28 @@ def test_refined_pixel_lists_of_any_fit_count(n, quad_group):
             assert torch.equal(jm[k], jo[0])
 
 
+@pytest.mark.parametrize("quad_group", [32, 25])
+@pytest.mark.parametrize("n", [1, 40])
+def test_short_and_long_refined_lists_agree(n, quad_group):
+    """Few refined or undecided pixels get a workgroup or 16 lanes each, many a
+    group or a lane each, by the list's length against the launch's size
+    (quad_blocks): the same bits either way, with tolerances that leave many
+    pixels near a threshold and at every level."""
+    truths, shapes, _ = make_cutouts(n, seed=3, sizes=(24, 50))
+    cuts = [Cutout(np.zeros((s, s)), np.ones((s, s)), psf) for s, psf in shapes]
+    for tol in (1e-2, 1e-4):
+        bf = BatchFit(cuts, sampling_tolerance=tol)
+        bf.b.quad_group = quad_group
+        rep = values_to_rep(np.stack(truths))
+        out = []
+        for blocks in (1, 4096):
+            bf.b.quad_blocks = blocks
+            img, J = bf.jacobian(rep)
+            out.append((img.clone(), J.clone(), bf.render(rep).clone()))
+        for a, b in zip(*out):
+            assert torch.equal(a, b)
+
+
 def test_batch_jacobian_matches_single_model():
     """apx_batch_jacobian: every cutout's model and its 7 representation-space
     Jacobian columns equal the single-model jacobian(as_representation=True)
