@@ -180,8 +180,13 @@ __device__ inline void rep_to_values(const double* r, double* v, double* dvdr) {
   dvdr[5] = 0.5 + 0.5 * r[5] / sqrt(r[5] * r[5] + 4.0);
 }
 
-// render constants of fit g at its parameters (rep_override row g when given)
-__device__ void eval_fit(const apx_batch& b, const Scratch& s, int g, const double* rep_override, int stage) {
+// Render constants of fit g at its parameters (rep_override row g when given), in
+// parts that different waves take: the geometry, the profile in float64, the
+// profile in float32, and the threshold with the parameter derivatives.
+enum : int { EVAL_GEOMETRY = 0, EVAL_PROFD = 1, EVAL_PROFF = 2, EVAL_FLUX = 3 };
+
+__device__ __forceinline__ void eval_fit(const apx_batch& b, const Scratch& s, int g, const double* rep_override, int stage,
+                                         int part) {
   const apx_batch_galaxy G = b.gal[g];
   const double* rep = rep_override ? rep_override + (int64_t)g * NP
                                    : (stage == ST_TRIAL ? st_of(b, g)->ev2 : st_of(b, g)->ev);
@@ -190,30 +195,34 @@ __device__ void eval_fit(const apx_batch& b, const Scratch& s, int g, const doub
   const int bx = (G.pw + 1) / 2, by = (G.ph + 1) / 2;  // psf_image.py:71-93
   const int nxw = G.nx + 2 * bx, nyw = G.ny + 2 * by;
   const double det = b.P[0] * b.P[3] - b.P[1] * b.P[2];
-  const double Pi[4] = {b.P[3] / det, -b.P[1] / det, -b.P[2] / det, b.P[0] / det};
-  const double dx = v[0] - G.origin[0], dy = v[1] - G.origin[1];
-  const double pcx = Pi[0] * dx + Pi[1] * dy + (-0.5 + bx);
-  const double pcy = Pi[2] * dx + Pi[3] * dy + (-0.5 + by);
-  const double ci = rint(pcx), cj = rint(pcy);  // ties to even
   const double prm[3] = {v[4], v[5], v[6]};
   const double area = fabs(det);
-  GalEval e;
-  e.pf = make_prof<float>(APX_SERSIC, b.P, 0.0, 0.0, area, b.softening, v[2], v[3], prm);
-  e.pd = make_prof<double>(APX_SERSIC, b.P, 0.0, 0.0, area, b.softening, v[2], v[3], prm);
-  const double bn = sersic_b(v[4]);
-  const double flux = 2.0 * kPi * pow(10.0, v[6]) * v[5] * v[5] * v[2] * v[4] * exp(bn) *
-                      pow(bn, -2.0 * v[4]) * exp(lgamma(2.0 * v[4]));  // functions.py:168-190
-  e.thr = b.tolerance * flux / (G.ref_npix > 0 ? (double)G.ref_npix : (double)nxw * nyw);
-  for (int q = 0; q < NP; ++q) e.dvdr[q] = dvdr[q];
-  e.sx = pcx - ci;
-  e.sy = pcy - cj;
-  e.nxw = nxw;
-  e.nyw = nyw;
-  e.ci = (int)ci;
-  e.cj = (int)cj;
-  e.bx = bx;
-  e.by = by;
-  s.ev[g] = e;
+  GalEval* e = s.ev + g;
+  if (part == EVAL_GEOMETRY) {
+    const double Pi[4] = {b.P[3] / det, -b.P[1] / det, -b.P[2] / det, b.P[0] / det};
+    const double dx = v[0] - G.origin[0], dy = v[1] - G.origin[1];
+    const double pcx = Pi[0] * dx + Pi[1] * dy + (-0.5 + bx);
+    const double pcy = Pi[2] * dx + Pi[3] * dy + (-0.5 + by);
+    const double ci = rint(pcx), cj = rint(pcy);  // ties to even
+    e->sx = pcx - ci;
+    e->sy = pcy - cj;
+    e->nxw = nxw;
+    e->nyw = nyw;
+    e->ci = (int)ci;
+    e->cj = (int)cj;
+    e->bx = bx;
+    e->by = by;
+  } else if (part == EVAL_PROFD) {
+    e->pd = make_prof<double>(APX_SERSIC, b.P, 0.0, 0.0, area, b.softening, v[2], v[3], prm);
+  } else if (part == EVAL_PROFF) {
+    e->pf = make_prof<float>(APX_SERSIC, b.P, 0.0, 0.0, area, b.softening, v[2], v[3], prm);
+  } else {
+    const double bn = sersic_b(v[4]);
+    const double flux = 2.0 * kPi * pow(10.0, v[6]) * v[5] * v[5] * v[2] * v[4] * exp(bn) *
+                        pow(bn, -2.0 * v[4]) * exp(lgamma(2.0 * v[4]));  // functions.py:168-190
+    e->thr = b.tolerance * flux / (G.ref_npix > 0 ? (double)G.ref_npix : (double)nxw * nyw);
+    for (int q = 0; q < NP; ++q) e->dvdr[q] = dvdr[q];
+  }
 }
 
 // the exclusive prefix of n over the wave plus a base reserved on `counter`
@@ -231,18 +240,23 @@ __device__ __forceinline__ int wave_reserve(int n, int32_t* counter, int lane) {
   return __shfl(base, 63, 64) + x - n;
 }
 
-// work lists of the fits active in `stage` (one thread a fit): the fit, its
-// render chunks and its output tiles are appended (each fit's chunks and
-// tiles contiguous and in order), its per-fit counts cleared, and its render
-// constants evaluated
+// Work lists of the fits active in `stage`: the fit, its render chunks and its
+// output tiles are appended (each fit's chunks and tiles contiguous and in order),
+// its per-fit counts cleared, and its render constants evaluated.  Bound by one
+// fit's chain of float64 functions, so a workgroup takes 64 fits and its four
+// waves a part of their constants each; the first also writes the lists, the wave
+// together one fit after another (a thread a fit took 700 stores in series for a
+// 420 x 420 window): 256 uneven fits 33 -> 17 us, 125 windows of up to 420^2 48 -> 20.
 __global__ __launch_bounds__(256) void build_kernel(apx_batch b, Scratch s, int stage, const double* rep_override) {
-  const int g = blockIdx.x * 256 + threadIdx.x;
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63, part = threadIdx.x >> 6;
+  const int g = blockIdx.x * 64 + lane;
   bool active = false;
   int nch = 0, ntl = 0;
   if (g < b.ngal) {
-    s.gal_cnt[g] = 0;
-    s.gal_rcnt[g] = 0;
+    if (part == 0) {
+      s.gal_cnt[g] = 0;
+      s.gal_rcnt[g] = 0;
+    }
     const GalState* st = st_of(b, g);
     const int ph = st->phase;
     // the probe point's rpp only enters the step through the acceleration
@@ -258,14 +272,20 @@ __global__ __launch_bounds__(256) void build_kernel(apx_batch b, Scratch s, int 
       ntl = ((G.nx + 63) / 64) * ((G.ny + kTR - 1) / kTR);
     }
   }
-  const int slot = wave_reserve(active ? 1 : 0, &s.cnt[0], lane);
-  const int cb = wave_reserve(nch, &s.cnt[1], lane);
-  const int tb = wave_reserve(ntl, &s.cnt[2], lane);
-  if (!active) return;
-  s.gal_list[slot] = g;
-  for (int c = 0; c < nch; ++c) s.chunk_list[cb + c] = make_int2(g, c);
-  for (int t = 0; t < ntl; ++t) s.tile_list[tb + t] = make_int2(g, t);
-  eval_fit(b, s, g, rep_override, stage);
+  if (part == 0) {
+    const int slot = wave_reserve(active ? 1 : 0, &s.cnt[0], lane);
+    const int cb = wave_reserve(nch, &s.cnt[1], lane);
+    const int tb = wave_reserve(ntl, &s.cnt[2], lane);
+    if (active) s.gal_list[slot] = g;
+    for (uint64_t m = __ballot(active); m; m &= m - 1) {
+      const int l = __ffsll((unsigned long long)m) - 1, fit = blockIdx.x * 64 + l;
+      const int nc = __builtin_amdgcn_readlane(nch, l), c0 = __builtin_amdgcn_readlane(cb, l);
+      const int nt = __builtin_amdgcn_readlane(ntl, l), t0 = __builtin_amdgcn_readlane(tb, l);
+      for (int c = lane; c < nc; c += 64) s.chunk_list[c0 + c] = make_int2(fit, c);
+      for (int t = lane; t < nt; t += 64) s.tile_list[t0 + t] = make_int2(fit, t);
+    }
+  }
+  if (active) eval_fit(b, s, g, rep_override, stage, part);
 }
 
 // 1-D linear interpolation of the zero-padded factor f (n values, padded to
@@ -2580,9 +2600,8 @@ void quad_again(const apx_batch& b, const Scratch& s, bool jac, hipStream_t stre
 void render_part(const apx_batch& b, const Scratch& s, int stage, const double* rep_override,
                  hipStream_t stream, bool reset) {
   const bool jac = stage == ST_JAC || stage == ST_ALL_JAC;
-  const int gb = (b.ngal + 255) / 256;
   if (reset) hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(64), 0, stream, s.cnt);
-  hipLaunchKernelGGL(build_kernel, dim3(gb), dim3(256), 0, stream, b, s, stage, rep_override);
+  hipLaunchKernelGGL(build_kernel, dim3((b.ngal + 63) / 64), dim3(256), 0, stream, b, s, stage, rep_override);
   if (b.conv_impl == 3)
     hipLaunchKernelGGL(prepare_sep_kernel, dim3(std::min((b.ngal + 3) / 4, 16384)), dim3(256), 0, stream, b, s);
   else
