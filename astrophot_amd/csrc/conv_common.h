@@ -18,24 +18,45 @@ __host__ __device__ inline int fast_kts(int kh) { return 8 * fast_nt(kh) + 8; }
 
 // Bilinear sample of the 1-px zero-padded PSF at (c - sx, r - sy) with the
 // reference's clamped corners (utils/interpolate.py:282-329), and its
-// derivatives with respect to the shift.
-__device__ __forceinline__ void bilinear(const float* psf, int ph, int pw, int r, int c, double sx,
-                                         double sy, double& val, double& dsx, double& dsy) {
+// derivatives with respect to the shift; at(y, x) is the padded PSF's value.
+template <typename At>
+__device__ __forceinline__ void bilinear_of(At&& at, int ph, int pw, int r, int c, double sx, double sy, double& val,
+                                            double& dsx, double& dsy) {
   const int H2 = ph + 2, W2 = pw + 2;
   const double x = (double)c - sx, y = (double)r - sy;
   const int xf = (int)floor(x), yf = (int)floor(y);
   const int x0 = min(max(xf, 0), W2 - 2), x1 = min(max(xf + 1, 1), W2 - 1);
   const int y0 = min(max(yf, 0), H2 - 2), y1 = min(max(yf + 1, 1), H2 - 1);
-  auto at = [&](int yy, int xx) -> double {
-    return (yy >= 1 && yy <= ph && xx >= 1 && xx <= pw) ? (double)psf[(yy - 1) * pw + (xx - 1)]
-                                                        : 0.0;
-  };
   const double fa = at(y0, x0), fb = at(y1, x0), fc = at(y0, x1), fd = at(y1, x1);
   const double wx1 = (double)x1 - x, wx0 = x - (double)x0;
   const double wy1 = (double)y1 - y, wy0 = y - (double)y0;
   val = fa * wx1 * wy1 + fb * wx1 * wy0 + fc * wx0 * wy1 + fd * wx0 * wy0;
   dsx = -(-fa * wy1 - fb * wy0 + fc * wy1 + fd * wy0);  // d/ds_x = -d/dx
   dsy = -(-fa * wx1 + fb * wx1 - fc * wx0 + fd * wx0);  // d/ds_y = -d/dy
+}
+
+// the PSF in memory, without its border
+__device__ __forceinline__ void bilinear(const float* psf, int ph, int pw, int r, int c, double sx,
+                                         double sy, double& val, double& dsx, double& dsy) {
+  bilinear_of([&](int yy, int xx) -> double {
+    return (yy >= 1 && yy <= ph && xx >= 1 && xx <= pw) ? (double)psf[(yy - 1) * pw + (xx - 1)] : 0.0;
+  }, ph, pw, r, c, sx, sy, val, dsx, dsy);
+}
+
+// The padded PSF in LDS ((ph + 2) x (pw + 2) floats), by the whole workgroup.  A
+// sample reads four neighbours; from memory each is a conditional load that the
+// next waits for.
+__device__ __forceinline__ void pad_psf(const float* __restrict__ psf, int ph, int pw, float* lds) {
+  const int W2 = pw + 2, n = (ph + 2) * W2;
+  for (int e = threadIdx.x; e < n; e += blockDim.x) {
+    const int r = e / W2 - 1, c = e % W2 - 1;
+    lds[e] = (r >= 0 && r < ph && c >= 0 && c < pw) ? psf[r * pw + c] : 0.0f;
+  }
+}
+__device__ __forceinline__ void bilinear_lds(const float* lds, int ph, int pw, int r, int c, double sx, double sy,
+                                             double& val, double& dsx, double& dsy) {
+  bilinear_of([&](int yy, int xx) -> double { return (double)lds[yy * (pw + 2) + xx]; }, ph, pw, r, c, sx, sy, val, dsx,
+              dsy);
 }
 
 // One wavefront's share of a 64 x 8 output tile: input-row blocks j = wu,

@@ -539,3 +539,36 @@ def test_group_with_upscaled_psf():
     Jref = om.jacobian(rep)
     for k in range(J.shape[-1]):
         assert rel_err(J[..., k], Jref[..., k]) < JAC_TOL, k
+
+
+@pytest.mark.parametrize("ph,pw,sx,sy", [(1, 1, 0.3, -0.4), (3, 5, -0.5, 0.5), (51, 51, 0.25, 0.0), (123, 125, 0.1, 0.45),
+                                         (125, 123, -0.3, 0.2), (129, 129, 0.49, -0.49), (5, 129, 0.0, 0.0)])
+def test_psf_shift_of_any_side(ph, pw, sx, sy):
+    """The shifted, normalised PSF and its two shift derivatives against float64
+    numpy: padded sides up to 126 x 126 values go through LDS, larger ones do not.
+    Both take float64 steps and round once: 2^-24 of each plane's largest value,
+    taken as 1.2e-7."""
+    import ctypes
+    from astrophot_amd import _lib as L
+    rng = np.random.default_rng(ph * 131 + pw)
+    psf = (0.1 + rng.random((ph, pw))).astype(np.float32)
+    pad = np.zeros((ph + 2, pw + 2))
+    pad[1:-1, 1:-1] = psf
+    r, c = np.meshgrid(np.arange(ph + 2.0), np.arange(pw + 2.0), indexing="ij")
+    x, y = c - sx, r - sy
+    xf, yf = np.floor(x).astype(int), np.floor(y).astype(int)
+    x0, x1 = np.clip(xf, 0, pw), np.clip(xf + 1, 1, pw + 1)
+    y0, y1 = np.clip(yf, 0, ph), np.clip(yf + 1, 1, ph + 1)
+    fa, fb, fc, fd = pad[y0, x0], pad[y1, x0], pad[y0, x1], pad[y1, x1]
+    v = fa * (x1 - x) * (y1 - y) + fb * (x1 - x) * (y - y0) + fc * (x - x0) * (y1 - y) + fd * (x - x0) * (y - y0)
+    dx = -(-fa * (y1 - y) - fb * (y - y0) + fc * (y1 - y) + fd * (y - y0))
+    dy = -(-fa * (x1 - x) + fb * (x1 - x) - fc * (x - x0) + fd * (x - x0))
+    S = v.sum()
+    ref = [v / S, dx / S - v * dx.sum() / S ** 2, dy / S - v * dy.sum() / S ** 2]
+    out = torch.empty((3, ph + 2, pw + 2), dtype=torch.float32, device="cuda")
+    pinv = (ctypes.c_double * 4)(1.0, 0.0, 0.0, 1.0)
+    src = torch.tensor(psf, device="cuda")
+    L.check(L.load().apx_psf_shift(src.data_ptr(), ph, pw, sx, sy, ctypes.cast(pinv, ctypes.c_void_p), 1.0, 1.0,
+                                   out.data_ptr(), L.stream()))
+    for got, want in zip(out.cpu().numpy(), ref):
+        assert np.abs(got[::-1, ::-1] - want).max() <= 1.2e-7 * max(np.abs(want).max(), 1e-30)
