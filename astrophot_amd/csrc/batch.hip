@@ -45,7 +45,7 @@ constexpr int kConvChan = kNChan - 1;
 constexpr int kTR = 16;      // output rows of a batch tile (64 x kTR pixels)
 // separable-convolution tap vectors are zero-padded to a multiple of 4 taps
 __host__ __device__ inline int sp_k4(int k) { return (k + 3) & ~3; }
-constexpr int kMfmaMax = kMfmaWide;  // widest kernel the MFMA convolution takes (67, up to 73 KiB LDS)
+constexpr int kMfmaMax = kMfmaWide;  // widest kernel the MFMA convolution takes (67, up to 70 KiB LDS)
 
 enum : int32_t { PH_INIT = 0, PH_NEEDJ = 1, PH_SUB = 2, PH_DONE = 3 };
 enum : int32_t { ST_JAC = 0, ST_PROBE = 1, ST_TRIAL = 2, ST_ALL = 3, ST_ALL_JAC = 4 };
@@ -1657,6 +1657,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void c
     stage_rows(b.planes + (int64_t)c * b.nwork + G.work_off, nxw, nxw, nyw, ox0, oy0, rows, cols, tin, kMfLW);
     // tap-table row kx: dd -> Kf[dd - 15][kx] = KT[kk][kx][dd - 8], zero outside KT's row
     stage_rows(b.taps + G.tap_off + (int64_t)kk * kw * kts, kts, kts, kw, -8, 0, kw, DD, tab, DD);
+    if (threadIdx.x < 16) tab[kw * DD + threadIdx.x] = 0.0f;  // the last column's trailing zeros
     // this lane's 4 output pixels: x = 16 w + 4 lk + i, row lm
     const int oy = oy0 + lm;
     bool valid[4];

@@ -104,10 +104,11 @@ __device__ __forceinline__ void conv_accumulate(const float* smem, int LW, int l
 typedef __attribute__((address_space(3))) void* lds_ptr;
 constexpr int kBufWord3 = 0x00020000;  // buffer resource word 3 on gfx9: 32-bit data
 
+template <int NW = 4>  // waves of the workgroup
 __device__ __forceinline__ void stage_rows(const float* src, int64_t pitch, int nx, int ny, int gx0, int gy0, int rows,
                                            int cols, float* dst, int dpitch) {
   const int lane = threadIdx.x & 63;
-  for (int t = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); t < rows; t += 4) {
+  for (int t = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); t < rows; t += NW) {
     const int gy = gy0 + t;
     const bool in = gy >= 0 && gy < ny;
     // every field of the resource is uniform: read from lane 0 so that it stays in SGPRs
@@ -128,7 +129,8 @@ __device__ __forceinline__ void stage_rows(const float* src, int64_t pitch, int 
 //   A_kx[x][j] = in[j][x + kx],  B_kx[j][r] = Kf[j - r][kx] (zero outside the kernel),
 // j over the staged input rows in k-steps of 4.  A comes from the staged input
 // tile, B from a per-kernel tap table tab[kx][dd] = Kf[dd - 15][kx], both in
-// LDS.  Lane layout: A[l % 16][l / 16], B[l / 16][l % 16], and
+// LDS.  A table column is mf_dd long and is read 15 entries further, into the
+// next one's leading zeros.  Lane layout: A[l % 16][l / 16], B[l / 16][l % 16], and
 // D[4 (l / 16) + i][l % 16] in acc[i] (x = 4 (l / 16) + i, r = l % 16).
 // A kernel column needs kMfR + kh - 1 input rows, ceil of that / 4 k-steps
 // (a compile-time count dispatched on the kernel height); the staged rows and
@@ -144,12 +146,22 @@ __host__ __device__ inline int mf_rows(int kh) { return 4 * mf_nks(kh); }
 // columns of the widest kernel and put the 4 rows x 16 columns of an operand
 // (lanes l / 16, l % 16) in distinct LDS banks.
 constexpr int kMfLW = 144;
-__host__ __device__ inline int mf_dd(int kh) { return mf_rows(kh) + 15; }
-// LDS of one pass: the staged input and one tap table
-__host__ inline size_t mfma_lds_bytes(int kh, int kw) {
-  return sizeof(float) * ((size_t)mf_rows(kh) * kMfLW + (size_t)kw * mf_dd(kh));
+__host__ __device__ inline int mf_dd(int kh) { return mf_rows(kh) + 1; }
+__host__ __device__ inline int mf_tab(int kh, int kw) { return kw * mf_dd(kh) + 16; }  // the last column's zeros too
+// LDS of one pass: the staged input of `blocks` 16-row output blocks and one tap table
+__host__ inline size_t mfma_lds_bytes(int kh, int kw, int blocks = 1) {
+  return sizeof(float) * ((size_t)(mf_rows(kh) + kMfR * (blocks - 1)) * kMfLW + (size_t)mf_tab(kh, kw));
 }
 __host__ inline size_t mfma_lds_bytes(int kmax) { return mfma_lds_bytes(kmax, kmax); }
+// The single-image convolution gives two 16-row blocks to a workgroup of 8 waves,
+// which share the halo rows and the tap table: two such workgroups fit a CU
+// (kernels to 67: 80.4 kB of 80 KiB), with 4 waves a SIMD in place of 2 and half
+// the staging an output.  512^2, 53 x 53, Jacobian of 7 columns: 122 -> 115 us;
+// 1537 x 1201, 67 x 67, four planes: 861 -> 792.  Where the launch has fewer than
+// kMfTallMin of them (two a CU) a block a workgroup spreads better.  (The batched
+// convolution keeps one tile a workgroup: its tile pairs took 0.82 -> 0.88 ms over
+// 256 uneven cutouts, where many last pairs are half empty.)
+constexpr int kMfTallMin = 512;
 
 // All kernel columns of one output block: column kx needs NKS k-steps.  The
 // operands of the next column are loaded between the MFMAs of the current one

@@ -310,8 +310,8 @@ __global__ __launch_bounds__(256) void convolve_fast_kernel(apx_conv_job job,
 }
 
 // MFMA convolution of one job (kernels of kMfmaMin .. kMfmaWide rows): a
-// 64 x kMfR output tile per workgroup, each wave one 16 x 16 block
-// (mfma_block, conv_common.h).  A workgroup does one pass, one render plane
+// 64 x kMfR output tile per workgroup (64 x 2 kMfR where there are enough of them,
+// TALL), each wave one 16 x 16 block (mfma_block, conv_common.h).  A workgroup does one pass, one render plane
 // with one kernel: its staged rows (stage_rows) and its tap table leave room for
 // a second workgroup on the CU, which multiplies while this one loads, and a
 // small image's passes spread over the CUs instead of following one another.
@@ -330,7 +330,8 @@ struct ConvPasses {
   int8_t plane[kMaxPass], kernel[kMaxPass];
 };
 
-__global__ __launch_bounds__(256) void convolve_mfma_kernel(apx_conv_job job, const float* __restrict__ planes,
+template <bool TALL>
+__global__ __launch_bounds__(TALL ? 512 : 256) void convolve_mfma_kernel(apx_conv_job job, const float* __restrict__ planes,
                                                             const float* __restrict__ kernels, ConvPasses passes,
                                                             int ntx, int ntile) {
   extern __shared__ float smem[];
@@ -338,30 +339,32 @@ __global__ __launch_bounds__(256) void convolve_mfma_kernel(apx_conv_job job, co
   const int pass = blockIdx.x / padded, tile = blockIdx.x - pass * padded;
   if (tile >= ntile) return;
   const int c = passes.plane[pass], k = passes.kernel[pass];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  constexpr int NW = TALL ? 8 : 4;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, w = wave & 3, half = wave >> 2;
   const int lm = lane & 15, lk = lane >> 4;
-  const int ox0 = (tile % ntx) * 64, oy0 = (tile / ntx) * kMfR;
+  const int ox0 = (tile % ntx) * 64, oy0 = (tile / ntx) * (NW / 4 * kMfR);
   const int kh = job.kh, kw = job.kw, ch = (kh - 1) / 2, cw = (kw - 1) / 2;
-  const int rows = mf_rows(kh), DD = mf_dd(kh);
+  const int rows = mf_rows(kh) + (NW / 4 - 1) * kMfR, DD = mf_dd(kh);
   float* tin = smem;             // rows x kMfLW
   float* tab = smem + rows * kMfLW; // [kx][dd] = Kf[dd - 15][kx]
-  stage_rows(planes + (int64_t)c * job.nx * job.ny, job.nx, job.nx, job.ny, job.x0 + ox0 - cw, job.y0 + oy0 - ch, rows,
+  stage_rows<NW>(planes + (int64_t)c * job.nx * job.ny, job.nx, job.nx, job.ny, job.x0 + ox0 - cw, job.y0 + oy0 - ch, rows,
              64 + kw - 1, tin, kMfLW);
   // the tap table: kernel rows read coalesced, stored DD (odd) apart; its first
   // 15 and last columns stay zero
   const float* K = kernels + (int64_t)k * kh * kw;
   for (int kx = lane; kx < kw; kx += 64) {
 #pragma unroll 6
-    for (int a = w; a < kh; a += 4) tab[kx * DD + 15 + a] = K[a * kw + kx];
-    for (int dd = w; dd < DD; dd += 4)
-      if (dd < 15 || dd >= 15 + kh) tab[kx * DD + dd] = 0.0f;
+    for (int a = wave; a < kh; a += NW) tab[kx * DD + 15 + a] = K[a * kw + kx];
+    // up to the next column's taps
+    for (int dd = 15 + kh + wave; dd < DD + 15; dd += NW) tab[kx * DD + dd] = 0.0f;
   }
+  if (threadIdx.x < 15) tab[threadIdx.x] = 0.0f;
   __builtin_amdgcn_s_waitcnt(0);  // this wave's rows have landed in LDS
   __syncthreads();
   if (ox0 + 16 * w >= job.ow) return;
-  const v4f acc = mfma_block(mf_nks(kh), tin + lk * kMfLW + 16 * w + lm, tab + lk - lm + 15, kw, DD);
-  // this lane's 4 outputs: x = 16 w + 4 lk + i, row lm
-  const int oy = oy0 + lm, ox = ox0 + 16 * w + 4 * lk;
+  const v4f acc = mfma_block(mf_nks(kh), tin + (kMfR * half + lk) * kMfLW + 16 * w + lm, tab + lk - lm + 15, kw, DD);
+  // this lane's 4 outputs: x = 16 w + 4 lk + i, row lm of the wave's block
+  const int oy = oy0 + kMfR * half + lm, ox = ox0 + 16 * w + 4 * lk;
   if (oy >= job.oh) return;
   const int n = min(4, job.ow - ox);
   if (c == 0 && k == 0) {
@@ -500,7 +503,6 @@ int convolve(const apx_conv_job* jp, const float* planes, const float* kernels, 
   const int nk0 = dk ? 3 : 1;
   if (job.kh >= kMfmaMin && job.kh <= kMfmaWide && job.kw >= kMfmaMin && job.kw <= kMfmaWide &&
       job.nx < (1 << 29) /* a row's bytes fit the range check of its buffer resource */) {
-    const size_t lds = mfma_lds_bytes(job.kh, job.kw);
     ConvPasses ps = {};
     auto add = [&](int plane, int kernel) {
       ps.plane[ps.n] = (int8_t)plane;
@@ -517,12 +519,17 @@ int convolve(const apx_conv_job* jp, const float* planes, const float* kernels, 
     for (int p = job.img ? 1 : 0; p < ps.n; ++p)
       for (int q = job.img ? 1 : 0; q < p; ++q) own = own && column(p) != column(q);
     const int ntx = (job.ow + 63) / 64;
-    const int64_t ntile = (int64_t)ntx * ((job.oh + kMfR - 1) / kMfR), blocks = ((ntile + 7) & ~(int64_t)7) * ps.n;
-    if (own && blocks <= (int64_t)INT32_MAX / 256) {
-      if (lds > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(&convolve_mfma_kernel),
+    auto blocks_of = [&](int64_t ntile) { return ((ntile + 7) & ~(int64_t)7) * ps.n; };
+    const int64_t tall = (int64_t)ntx * ((job.oh + 2 * kMfR - 1) / (2 * kMfR));
+    const bool two = tall * ps.n >= kMfTallMin;
+    const int64_t ntile = two ? tall : (int64_t)ntx * ((job.oh + kMfR - 1) / kMfR), blocks = blocks_of(ntile);
+    if (own && blocks <= (int64_t)INT32_MAX / 512) {
+      auto* kernel = two ? &convolve_mfma_kernel<true> : &convolve_mfma_kernel<false>;
+      const size_t lds = mfma_lds_bytes(job.kh, job.kw, two ? 2 : 1);
+      if (lds > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
         return set_error(APX_E_HIP, "convolve: LDS size refused");
-      hipLaunchKernelGGL(convolve_mfma_kernel, dim3((unsigned)blocks), dim3(256), lds, stream, job, planes, kernels, ps, ntx,
+      hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(two ? 512 : 256), lds, stream, job, planes, kernels, ps, ntx,
                          (int)ntile);
       return check_launch("convolve (MFMA)");
     }

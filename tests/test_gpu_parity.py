@@ -572,3 +572,12 @@ def test_psf_shift_of_any_side(ph, pw, sx, sy):
                                    out.data_ptr(), L.stream()))
     for got, want in zip(out.cpu().numpy(), ref):
         assert np.abs(got[::-1, ::-1] - want).max() <= 1.2e-7 * max(np.abs(want).max(), 1e-30)
+
+
+@pytest.mark.parametrize("kh,kw,ow,oh,nchan", [(21, 67, 513, 321, 4), (67, 21, 449, 352, 5), (67, 67, 640, 337, 3),
+                                               (33, 35, 1985, 513, 1)])
+def test_convolve_two_blocks_a_workgroup(kh, kw, ow, oh, nchan):
+    """apx_convolve where its launch has 512 workgroups of two 16-row blocks or
+    more: whole and half last blocks, one-column last tiles, zero outside."""
+    test_convolve_shapes(kh, kw, ow, oh, nchan, 0, False)
+    test_convolve_shapes(kh, kw, ow, oh, nchan, 1, False)
