@@ -252,6 +252,24 @@ __global__ __launch_bounds__(256) void im2col_kernel(const uint16_t* X, int Bn, 
   }
 }
 
+// im2col_kernel 8 columns a thread: one 16-byte store, and one 16-byte load where
+// they are 8 channels of one tap (Cin a multiple of 8).  Bound by the store of
+// col; an element a thread spent its time on 64-bit divisions (the four layers of
+// 256 cutouts: 128 -> 41 us).
+__global__ __launch_bounds__(256) void im2col8_kernel(const uint16_t* __restrict__ X, int H, int W, int Cin, int Kp,
+                                                      uint32_t total, uint16_t* __restrict__ col) {
+  const int Ho = (H + 1) / 2, Wo = (W + 1) / 2;
+  const uint32_t K8 = (uint32_t)Kp / 8;
+  for (uint32_t e = blockIdx.x * 256u + threadIdx.x; e < total; e += gridDim.x * 256u) {
+    const uint32_t m = e / K8, q = m / (uint32_t)Wo;
+    const int k = 8 * (int)(e - m * K8), ox = (int)(m - q * (uint32_t)Wo);
+    const uint32_t b = q / (uint32_t)Ho;
+    const ConvA cv{X, H, W, Cin, Ho, Wo};
+    *reinterpret_cast<uint4*>(col + (int64_t)e * 8) =
+        load_patch(cv, true, (int)b, (int)(q - b * (uint32_t)Ho), ox, k, 9 * Cin);
+  }
+}
+
 // dX (B, H, W, Cin) float32 = col2im(dcol (B * Ho * Wo, Kp)): each input
 // element gathers the (oy, ky) x (ox, kx) pairs that read it
 __global__ __launch_bounds__(256) void col2im_kernel(const float* dcol, int Bn, int H, int W, int Cin,
@@ -276,6 +294,36 @@ __global__ __launch_bounds__(256) void col2im_kernel(const float* dcol, int Bn, 
       }
     }
     dX[e] = s;
+  }
+}
+
+// col2im_kernel 4 channels a thread (16-byte loads, 32-bit divisions): the three
+// layers of 256 cutouts 83 -> 32 us
+__global__ __launch_bounds__(256) void col2im4_kernel(const float* __restrict__ dcol, int H, int W, int Cin, int Kp,
+                                                      uint32_t total, float* __restrict__ dX) {
+  const int Ho = (H + 1) / 2, Wo = (W + 1) / 2;
+  const uint32_t C4 = (uint32_t)Cin / 4;
+  for (uint32_t e = blockIdx.x * 256u + threadIdx.x; e < total; e += gridDim.x * 256u) {
+    const uint32_t pix = e / C4, q = pix / (uint32_t)W, b = q / (uint32_t)H;
+    const int ci = 4 * (int)(e - pix * C4), ix = (int)(pix - q * (uint32_t)W), iy = (int)(q - b * (uint32_t)H);
+    float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+    for (int ky = 0; ky < 3; ++ky) {
+      const int ty = iy + 1 - ky;  // = 2 oy
+      if (ty < 0 || (ty & 1) || ty / 2 >= Ho) continue;
+#pragma unroll
+      for (int kx = 0; kx < 3; ++kx) {
+        const int tx = ix + 1 - kx;
+        if (tx < 0 || (tx & 1) || tx / 2 >= Wo) continue;
+        const int64_t m = ((int64_t)b * Ho + ty / 2) * Wo + tx / 2;
+        const float4 v = *reinterpret_cast<const float4*>(dcol + m * Kp + (ky * 3 + kx) * Cin + ci);
+        s.x += v.x;
+        s.y += v.y;
+        s.z += v.z;
+        s.w += v.w;
+      }
+    }
+    *reinterpret_cast<float4*>(dX + (int64_t)e * 4) = s;
   }
 }
 
@@ -742,7 +790,13 @@ int im2col_s2(const uint16_t* X, int Bn, int H, int W, int Cin, int Kp, uint16_t
   if (!X || !col || Bn < 1 || H < 1 || W < 1 || Cin < 1 || Kp < 9 * Cin)
     return set_error(APX_E_INVALID, "im2col: bad arguments");
   const int64_t n = (int64_t)Bn * ((H + 1) / 2) * ((W + 1) / 2) * Kp;
-  hipLaunchKernelGGL(im2col_kernel, grid_for(n), dim3(256), 0, stream, X, Bn, H, W, Cin, Kp, col);
+  // 8 columns a thread where every row starts on 16 bytes (and so does each tap's
+  // group of 8 channels); their count fits 32 bits with a grid's stride to spare
+  const uintptr_t at = reinterpret_cast<uintptr_t>(col) | (Cin % 8 == 0 ? reinterpret_cast<uintptr_t>(X) : 0);
+  if (Kp % 8 == 0 && (at & 15) == 0 && n / 8 < (int64_t)1 << 31)
+    hipLaunchKernelGGL(im2col8_kernel, grid_for(n / 8), dim3(256), 0, stream, X, H, W, Cin, Kp, (uint32_t)(n / 8), col);
+  else
+    hipLaunchKernelGGL(im2col_kernel, grid_for(n), dim3(256), 0, stream, X, Bn, H, W, Cin, Kp, col);
   return check_launch("im2col");
 }
 
@@ -750,7 +804,12 @@ int col2im_s2(const float* dcol, int Bn, int H, int W, int Cin, int Kp, float* d
   if (!dcol || !dX || Bn < 1 || H < 1 || W < 1 || Cin < 1 || Kp < 9 * Cin)
     return set_error(APX_E_INVALID, "col2im: bad arguments");
   const int64_t n = (int64_t)Bn * H * W * Cin;
-  hipLaunchKernelGGL(col2im_kernel, grid_for(n), dim3(256), 0, stream, dcol, Bn, H, W, Cin, Kp, dX);
+  // 4 channels a thread where every row of dcol and of dX keeps them on 16 bytes
+  if (Cin % 4 == 0 && Kp % 4 == 0 && ((reinterpret_cast<uintptr_t>(dcol) | reinterpret_cast<uintptr_t>(dX)) & 15) == 0 &&
+      n / 4 < (int64_t)1 << 31)
+    hipLaunchKernelGGL(col2im4_kernel, grid_for(n / 4), dim3(256), 0, stream, dcol, H, W, Cin, Kp, (uint32_t)(n / 4), dX);
+  else
+    hipLaunchKernelGGL(col2im_kernel, grid_for(n), dim3(256), 0, stream, dcol, Bn, H, W, Cin, Kp, dX);
   return check_launch("col2im");
 }
 

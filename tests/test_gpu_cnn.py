@@ -211,3 +211,41 @@ def test_fused_convolutions_equal_the_layers(B, shift):
     same = lambda a, b: torch.equal(torch.nan_to_num(a), torch.nan_to_num(b)) and torch.equal(a.isnan(), b.isnan())  # noqa: E731
     assert same(feat.float(), net._buffers(B)["yb"][3].reshape(-1).float())
     assert same(net._infer(images, sigma), ref)
+
+
+@pytest.mark.parametrize("B,H,W,C,Kp", [(2, 64, 64, 1, 32), (3, 7, 5, 8, 72), (2, 9, 16, 32, 288), (1, 1, 1, 4, 36),
+                                        (2, 6, 7, 12, 112), (2, 5, 5, 3, 27), (3, 4, 4, 64, 584), (2, 8, 3, 8, 76)])
+def test_im2col_and_its_adjoint_any_shape(B, H, W, C, Kp):
+    """Both widths of im2col and col2im (8 columns and 4 channels a thread where
+    rows stay on 16 bytes, one otherwise, and with operands 2 or 4 bytes past it)
+    against the definition: im2col moves bits, col2im adds at most 4 float32
+    values in a fixed order (4 x 2^-24 of their magnitudes)."""
+    lib = L.load()
+    g = torch.Generator().manual_seed(B * 100 + H)
+    Ho, Wo = (H + 1) // 2, (W + 1) // 2
+    M = B * Ho * Wo
+    x = torch.randn(B, H, W, C, generator=g).to(torch.bfloat16)
+    d = torch.randn(M, Kp, generator=g)
+    pad = torch.nn.functional.pad(x.float(), (0, 0, 1, 2, 1, 2))
+    ref = torch.zeros(B, Ho, Wo, Kp)
+    back, mag = torch.zeros(B, H + 3, W + 3, C, dtype=torch.float64), torch.zeros(B, H + 3, W + 3, C, dtype=torch.float64)
+    for t in range(9):
+        ky, kx = divmod(t, 3)
+        ref[..., t * C:(t + 1) * C] = pad[:, ky:ky + 2 * Ho:2, kx:kx + 2 * Wo:2]
+        part = d.view(B, Ho, Wo, Kp)[..., t * C:(t + 1) * C].double()
+        back[:, ky:ky + 2 * Ho:2, kx:kx + 2 * Wo:2] += part
+        mag[:, ky:ky + 2 * Ho:2, kx:kx + 2 * Wo:2] += part.abs()
+    for shift in (0, 1):
+        xd = torch.zeros(x.numel() + 8, dtype=torch.bfloat16, device=DEV)
+        xd[shift:shift + x.numel()] = x.reshape(-1).to(DEV)
+        col = torch.full((M * Kp + 8,), 7.0, dtype=torch.bfloat16, device=DEV)
+        L.check(lib.apx_im2col_s2(xd[shift:].data_ptr(), B, H, W, C, Kp, col[shift:].data_ptr(), L.stream()))
+        assert torch.equal(col[shift:shift + M * Kp].float().cpu(), ref.reshape(-1))
+        assert (col[shift + M * Kp:].float() == 7.0).all()
+        dd = torch.zeros(M * Kp + 8, device=DEV)
+        dd[shift:shift + M * Kp] = d.reshape(-1).to(DEV)
+        dx = torch.full((x.numel() + 8,), 7.0, device=DEV)
+        L.check(lib.apx_col2im_s2(dd[shift:].data_ptr(), B, H, W, C, Kp, dx[shift:].data_ptr(), L.stream()))
+        got = dx[shift:shift + x.numel()].view(B, H, W, C).double().cpu()
+        assert ((got - back[:, 1:H + 1, 1:W + 1]).abs() <= 4 * 2.0 ** -24 * mag[:, 1:H + 1, 1:W + 1]).all()
+        assert (dx[shift + x.numel():] == 7.0).all()
