@@ -601,6 +601,8 @@ __global__ __launch_bounds__(kFtThreads, 4) void features_kernel(const float* __
           make_uint4(pack2(c == 0 ? 0.0f : before, h[0]), pack2(h[1], h[2]), pack2(h[3], h[4]), pack2(h[5], h[6]));
       if (c == 7) row[4] = pack2(h[7], 0.0f);
       if (t < kFtIn) in[t] = 0u;  // the row above the image
+      // the 2-byte writes below come after the 16-byte ones above (one wave's rows)
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       while (__any(left != 0)) {
         if (left) {
           const int q = __ffs(left) - 1;

@@ -320,8 +320,7 @@ __global__ __launch_bounds__(256) void convolve_fast_kernel(apx_conv_job job,
 // take the workgroups round robin).  Bound by the FP32 matrix pipe.  With all
 // passes of a tile in one workgroup, rows copied through registers a load at a
 // time, 512^2 with 53 x 53 kernels took 41 us (value) and 244 us (Jacobian of 7
-// columns); so 24.5 and 122 us
-// (100^2 with 27 x 27: 19 and 110 us, 12 and 14 us).
+// columns); so 24.5 and 115 us (100^2 with 27 x 27: 19 and 110 us, 12 and 14 us).
 constexpr int kMfmaMin = 21;  // shorter kernels waste over half of each MFMA on the band's zeros
 constexpr int kMaxPass = APX_MAX_CHAN + 2;
 

@@ -581,3 +581,36 @@ def test_convolve_two_blocks_a_workgroup(kh, kw, ow, oh, nchan):
     more: whole and half last blocks, one-column last tiles, zero outside."""
     test_convolve_shapes(kh, kw, ow, oh, nchan, 0, False)
     test_convolve_shapes(kh, kw, ow, oh, nchan, 1, False)
+
+
+@pytest.mark.parametrize("mode", ["midpoint", "trapezoid"])
+@pytest.mark.parametrize("px,py", [(22, 18), (16, 21), (0, 0)])
+def test_selection_at_its_threshold(mode, px, py):
+    """A pixel whose curvature sits at the selection threshold is decided in
+    float64 whichever side it falls: the tolerance at which the oracle's pixel
+    switches between its sample and its quadrature is found by bisection, and
+    the image agrees with the oracle's a part in 1e8 to either side of it (the
+    float32 test cannot tell), at the repository's bar of 1e-5 of the max.  Last,
+    a Gaussian wide enough (sigma 300 px) that no pixel of a wave is decided in
+    float32."""
+    p = dict(GAL["sersic"], center=[20.0, 18.0], q=0.98, n=1.5, Re=3.0)
+    knobs = dict(sampling_mode=mode, integrate_max_depth=1)
+
+    def at(tol):
+        om, m = single("sersic", p, sampling_tolerance=tol, **knobs)
+        return om.forward(om.vector_representation()).reshape(36, 40), m
+
+    lo, hi = 1e-9, 1e6  # selected, not selected
+    v_lo, v_hi = float(at(lo)[0][py, px]), float(at(hi)[0][py, px])
+    assert v_lo != v_hi
+    for _ in range(60):
+        mid = math.sqrt(lo * hi)
+        if float(at(mid)[0][py, px]) == v_hi:
+            hi = mid
+        else:
+            lo = mid
+    for tol in (lo * (1 - 1e-8), hi * (1 + 1e-8)):
+        ref, m = at(tol)
+        assert rel_err(m().data, ref) < 1e-5
+    om, m = single("gaussian", dict(GAL["gaussian"], sigma=300.0, flux=6.0), sampling_tolerance=1e-12, **knobs)
+    assert rel_err(m().data, om.forward(om.vector_representation()).reshape(36, 40)) < 1e-5
