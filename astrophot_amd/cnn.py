@@ -73,7 +73,9 @@ def gemm(A, sam, sak, B, sbk, sbn, C, M, N, K, ldc=None, bias=None, relu=False, 
     tiles = ((M + 63) // 64) * ((N + 63) // 64)
     splits = 1
     if K >= 4096 and tiles < 128 and ws is not None:
-        splits = int(min(max(1, K // 2048), 256, ws.numel() // max(M * N, 1)))
+        # 512 deep a workgroup: each k-step of 32 waits for its operands, and the weight gradients of 256
+        # cutouts have 1 to 9 tiles (six gradients: 258 us at 2,048 deep, 121 so)
+        splits = int(min(max(1, K // 512), 256, ws.numel() // max(M * N, 1)))
     L.check(lib.apx_gemm_bf16(M, N, K, A.data_ptr(), sam, sak, B.data_ptr(), sbk, sbn, C.data_ptr(), ldc,
                               _ptr(bias), int(relu), _ptr(Cb), int(accumulate), splits,
                               _ptr(ws) if splits > 1 else None, ws.numel() if ws is not None else 0,
