@@ -68,8 +68,8 @@ __global__ __launch_bounds__(256) void sum_partials_kernel(const double* __restr
 //   A[r][k] = J[p_k][r], B[k][c] = W_p J[p_k][c], D[4(l/16)+i][l%16] (reg i).
 // Bound by HBM (J, model, data and weight read once).  A wave has the loads of
 // kStep steps in flight: with one step's it waited out a memory round trip
-// every 4 pixels, 308 us for 2048^2 x 13 (268 MB), 102 us now.
-constexpr int kStep = 8;  // divides 64, the steps between two flushes
+// every 4 pixels, 308 us for 2048^2 x 13 (268 MB); with 8 steps' 102 us, with 16 97.
+constexpr int kStep = 16;  // divides 64, the steps between two flushes
 __global__ __launch_bounds__(256) void normal_eq_kernel(const float* __restrict__ J,
                                                         const float* __restrict__ model,
                                                         const float* __restrict__ data,
