@@ -420,7 +420,7 @@ __global__ __launch_bounds__(256) void damp_kernel(const double* __restrict__ H,
 // block column k and factors it (the first workgroups), and takes panel k - 1
 // out of the block columns after it (the others).  Two launches a panel, with
 // the rows solved after the diagonal factor and a division a step, took 20 + 11 us a
-// panel (n = 3501, a band 658 wide: 3.45 ms a factor); this one 10.1 us (1.10 ms).
+// panel (n = 3501, a band 658 wide: 3.45 ms a factor); this one 10.2 us (1.13 ms).
 typedef double v4d __attribute__((ext_vector_type(4)));
 
 // 16 x 16 blocks by v_mfma_f64_16x16x4_f64: lane l gives A[l % 16][l / 16] and
@@ -435,7 +435,11 @@ __device__ __forceinline__ void panel_operand(const double* __restrict__ A, int 
 }
 
 // Rows of block column k0 with panel k0 - kNB taken out, into T: a wave's 16
-// rows r0 .. (T rows 16 w ..) by the block's 32 columns.
+// rows r0 .. (T rows 16 w ..) by the block's 32 columns.  Here and in
+// trailing_tile a panel's 32 products are summed from zero and subtracted once:
+// added into the entry itself, each would round at the entry's size, and
+// |L L^T - A| grew with sqrt(n) in place of sqrt(n / 32) (dense, n = 701: 7.6e-16
+// of |A| in place of 2.0e-16).
 __device__ __forceinline__ void panel_rows(const double* __restrict__ A, int n, int k0, int nb, int r0, int w,
                                            double (*T)[kNB + 1]) {
   const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
@@ -452,10 +456,13 @@ __device__ __forceinline__ void panel_rows(const double* __restrict__ A, int n, 
     panel_operand(A, n, r0, k0 - kNB, a);
     panel_operand(A, n, k0, k0 - kNB, b[0]);
     panel_operand(A, n, k0 + 16, k0 - kNB, b[1]);
+    v4d sum[2] = {};
 #pragma unroll
     for (int t = 0; t < kSteps; ++t)
 #pragma unroll
-      for (int q = 0; q < 2; ++q) c[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[t], b[q][t], c[q], 0, 0, 0);
+      for (int q = 0; q < 2; ++q) sum[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t], b[q][t], sum[q], 0, 0, 0);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) c[q] -= sum[q];
   }
 #pragma unroll
   for (int q = 0; q < 2; ++q)
@@ -470,10 +477,12 @@ __device__ __forceinline__ void panel_rows(const double* __restrict__ A, int n, 
 // columns), so they cost nothing beyond the factor.  Column entries go lane to
 // lane by v_readlane, two a multiply-add, so only the steps within 16 columns go
 // this way; the first 16 columns leave the last 16 by MFMA, every wave its rows
-// (all 32 columns by lane reads: 11.8 us a panel; this way 10.1).
-// 1 / sqrt(pivot) is v_rsq_f64 (24 bits) and one third-order step, within 2 ulp:
-// a division and a square root a step, 60 dependent instructions, set the
-// chain's length before.  T[i][k] = L[i][k] on return (k <= i).  A pivot that is
+// (all 32 columns by lane reads: 11.8 us a panel; this way 10.2).
+// 1 / sqrt(pivot) is v_rsq_f64 (24 bits) and one third-order step, within 2 ulp,
+// and a quotient takes one more step from it (rounded as a division's: without
+// it |L L^T - A| of systems up to 16 wide is 4 to 10 % larger; it takes 1 % of
+// the factor's time): a division and a square root a step, 60 dependent
+// instructions, set the chain's length before.  T[i][k] = L[i][k] on return (k <= i).  A pivot that is
 // not positive and finite gives NaN and sets *status to its 1-based column
 // (first one only, when `report`).
 constexpr int kHB = kNB / 2;
@@ -494,7 +503,8 @@ __device__ __forceinline__ int potrf_half(int nb, int j0, double (&r)[kHB]) {
       y = fma(y * e, fma(0.375, e, 0.5), y);
       double d = p * y;
       d = fma(fma(-d, d, p), 0.5 * y, d);
-      r[j] = lane == j0 + j ? d : r[j] * y;
+      const double q = r[j] * y;
+      r[j] = lane == j0 + j ? d : fma(fma(-q, d, r[j]), y, q);
       // every lane updates every later column: entries above the diagonal
       // (k > lane) and columns past nb are never used, and only lower entries of
       // columns before k feed a lower entry
@@ -515,14 +525,14 @@ __device__ __forceinline__ void factor_rows(double (*T)[kNB + 1], int rows, int 
     __syncthreads();
     if (h == 1) {
       const double(*R)[kNB + 1] = T + 16 * w;
-      v4d c;
+      v4d c, sum = {};
 #pragma unroll
       for (int q = 0; q < 4; ++q) c[q] = R[4 * q + lk][kHB + li];
 #pragma unroll
       for (int t = 0; t < kHB / 4; ++t)
-        c = __builtin_amdgcn_mfma_f64_16x16x4f64(-R[li][4 * t + lk], T[kHB + li][4 * t + lk], c, 0, 0, 0);
+        sum = __builtin_amdgcn_mfma_f64_16x16x4f64(R[li][4 * t + lk], T[kHB + li][4 * t + lk], sum, 0, 0, 0);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) T[16 * w + 4 * q + lk][kHB + li] = c[q];
+      for (int q = 0; q < 4; ++q) T[16 * w + 4 * q + lk][kHB + li] = c[q] - sum[q];
       __syncthreads();
     }
     if (w == 0) {
@@ -558,16 +568,17 @@ __device__ __forceinline__ void trailing_tile(double* __restrict__ A, int n, int
   panel_operand(A, n, r0, p0, a);
 #pragma unroll
   for (int q = 0; q < 4; ++q) panel_operand(A, n, j0 + 16 * q, p0, b[q]);
+  v4d sum[4] = {};
 #pragma unroll
   for (int t = 0; t < kSteps; ++t)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) c[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[t], b[q][t], c[q], 0, 0, 0);
+    for (int q = 0; q < 4; ++q) sum[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t], b[q][t], sum[q], 0, 0, 0);
 #pragma unroll
   for (int q = 0; q < 4; ++q)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = r0 + 4 * r + lk, j = j0 + 16 * q + li;
-      if (i < n && j <= i) A[(int64_t)i * n + j] = c[q][r];
+      if (i < n && j <= i) A[(int64_t)i * n + j] = c[q][r] - sum[q][r];
     }
 }
 
@@ -705,9 +716,11 @@ __global__ __launch_bounds__(128) void diag_writeback_kernel(double* __restrict_
 // One half-wave's copy of the diagonal block [k0, k0 + nb): lane off + r holds
 // v[j] = A[(k0 + j) n + k0 + r], which is L[r][j] for j < r (the factor's
 // transposed copy in the upper triangle) and L[j][r] for j > r, and its diagonal
-// entry.  diag_scale turns the entries a solve uses into v[j] / L[r][r], the
-// others into zero, and the diagonal into its reciprocal: a step of the solve is
-// then two lane reads and one FMA, without a product or a choice in the chain.
+// entry.  diag_ready clears the entries a solve does not use and takes the
+// diagonal's reciprocal, so that a step of the solve is a product, two lane reads
+// and an FMA, without a choice in the chain.  (Rows scaled by the reciprocal
+// beforehand save the product of the chain, and round every entry of L once
+// more: badly scaled 16 x 16 systems came out with twice the error.)
 struct DiagBlock {
   double v[kNB];
   double rdii;
@@ -723,25 +736,25 @@ __device__ __forceinline__ void diag_load(const double* __restrict__ A, int n, i
 
 // kLower: keeps v[j] for j < r; else for j > r
 template <bool kLower>
-__device__ __forceinline__ void diag_scale(DiagBlock& d, int r) {
+__device__ __forceinline__ void diag_ready(DiagBlock& d, int r) {
   d.rdii = 1.0 / d.rdii;
 #pragma unroll
-  for (int j = 0; j < kNB; ++j) d.v[j] = (kLower ? j < r : j > r) ? d.v[j] * d.rdii : 0.0;
+  for (int j = 0; j < kNB; ++j) d.v[j] = (kLower ? j < r : j > r) ? d.v[j] : 0.0;
 }
 
-// substitution with the scaled diagonal block held by lanes off .. off + 31 (rows
-// and columns past the matrix are zero): lane off + r holds the right-hand side
-// of row r on entry and x_r on return; every other lane is left as it is
+// substitution with the diagonal block held by lanes off .. off + 31 (rows and
+// columns past the matrix are zero): lane off + r holds the right-hand side of
+// row r on entry and x_r on return; every other lane is left as it is
 template <bool kLower>
 __device__ __forceinline__ double diag_substitute(const DiagBlock& d, int off, double b) {
   const bool mine = ((int)(threadIdx.x & 63) & ~(kNB - 1)) == off;
-  double xi = b * d.rdii;
+  double xi = b;
 #pragma unroll
   for (int q = 0; q < kNB; ++q) {
     const int j = kLower ? q : kNB - 1 - q;
-    xi = fma(-d.v[j], lane_bcast(xi, off + j), xi);
+    xi = fma(-d.v[j], lane_bcast(xi * d.rdii, off + j), xi);
   }
-  return mine ? xi : b;
+  return mine ? xi * d.rdii : b;
 }
 
 template <bool kLower>
@@ -750,7 +763,7 @@ __global__ __launch_bounds__(64) void diag_solve_kernel(const double* __restrict
   DiagBlock d;
   const int lane = threadIdx.x, nb = min(kNB, n - k0);
   diag_load(A, n, k0, lane, d);
-  diag_scale<kLower>(d, lane);
+  diag_ready<kLower>(d, lane);
   const double b = lane < nb ? x[k0 + lane] : 0.0;
   const double xi = diag_substitute<kLower>(d, 0, b);
   if (lane < nb) x[k0 + lane] = xi;
@@ -784,7 +797,7 @@ __global__ __launch_bounds__(256) void trsv_lower_pair_kernel(const double* __re
     diag_load(A, n, second ? b2 * kNB : b1 * kNB, (second && !has2) ? -1 : (t & (kNB - 1)), d);
 #pragma unroll
     for (int u = 0; u < kNB; ++u) l21[u] = (second && row) ? A[(int64_t)(b1 * kNB + u) * n + i] : 0.0;
-    diag_scale<true>(d, t & (kNB - 1));
+    diag_ready<true>(d, t & (kNB - 1));
     __syncthreads();
   } else {
     double c[2][kNB];
@@ -852,7 +865,7 @@ __global__ __launch_bounds__(256) void trsv_upper_pair_kernel(const double* __re
     diag_load(A, n, second ? b2 * kNB : b1 * kNB, (second && !has2) ? -1 : (t & (kNB - 1)), d);
 #pragma unroll
     for (int u = 0; u < kNB; ++u) l12[u] = (second && row) ? A[(int64_t)(b1 * kNB + u) * n + i] : 0.0;
-    diag_scale<false>(d, t & (kNB - 1));
+    diag_ready<false>(d, t & (kNB - 1));
     __syncthreads();
   } else {
     double c[2][kNB];

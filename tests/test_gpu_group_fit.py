@@ -135,6 +135,24 @@ def test_factor_and_solve_at_panel_edges(n):
     assert int(st.item()) == n // 2 + 1
 
 
+def test_factor_rounds_once_a_panel():
+    """|L L^T - A| of a dense 417 x 417 system, in extended precision: every entry
+    has 13 panels taken out of it and is written once more, 14 roundings of at
+    most 2^-53 of its size in random directions, so sqrt(14) 2^-53 of |A| covers
+    it.  (The panels' products added into the entry one by one round at its size
+    32 times a panel and come out at 5.9e-16.)"""
+    lib, n = L.load(), 417
+    B = np.random.default_rng(n).normal(size=(2 * n, n))
+    Hm = B.T @ B
+    Hd, fac = torch.tensor(Hm, device="cuda"), torch.empty((n, n), dtype=torch.float64, device="cuda")
+    st = torch.zeros(1, dtype=torch.int32, device="cuda")
+    L.check(lib.apx_dense_damped_factor(n, L.ptr(Hd), 0.0, L.ptr(fac), L.ptr(st), L.stream()))
+    low = np.tril(fac.cpu().numpy()).astype(np.longdouble)
+    err = (low @ low.T - Hm).astype(np.float64)
+    assert int(st.item()) == 0
+    assert np.linalg.norm(err) <= math.sqrt(14) * 2.0 ** -53 * np.linalg.norm(Hm)
+
+
 @pytest.mark.parametrize("masked", [False, True])
 @pytest.mark.parametrize("sky", [False, True])
 @pytest.mark.parametrize("nx,ny,wins", [
