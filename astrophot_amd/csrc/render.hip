@@ -269,14 +269,43 @@ __device__ __forceinline__ void vjp_part(const apx_component& cp, const double* 
 // sample and its sum.  A wave a pixel kept 9 lanes of 64 busy, and carried the
 // pixel's deeper levels in the same wave (render_deep_kernel): 51 us for a 100^2
 // cutout, 71 us for 1537 x 1201 (adjoint 114); 17 and 35 us (42) the two passes.
-template <int MODE>
+// ROW: lanes a pixel, summed by a butterfly, for rules of more than 9 nodes, whose
+// many lane reads would take longer than their samples (level1_row).
+template <int MODE, int ROW>
 __global__ __launch_bounds__(256) void render_level1_kernel(apx_component cp, RenderConst rc, float* planes,
                                                             const float* __restrict__ B, RenderWs ws) {
   constexpr bool GRAD = MODE != Q_VALUE;
   const int lane = threadIdx.x & 63;
-  const int n = cp.quad_level, nn = n * n, per = 64 / nn;
-  const int grp = lane / nn, node = lane - grp * nn, first = grp * nn;
-  const int wave = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), nwaves = (int)(gridDim.x * 4);
+  const int n = cp.quad_level, nn = n * n, width = ROW ? ROW : nn, per = 64 / width;
+  const int grp = lane / width, at = lane - grp * width, first = grp * width;
+  const bool has = ROW == 0 || at < nn;  // this lane holds a node
+  const int node = has ? at : 0;
+  auto sum = [&](double v) {
+    if constexpr (ROW == 64) return wave_sum(v);
+    else if constexpr (ROW == 32) return half_sum(v);
+    else if constexpr (ROW == 16) return row_sum(v);
+    double r = 0.0;
+    for (int j = 0; j < nn; ++j) r += __shfl(v, first + j, 64);
+    return r;
+  };
+  const int wv = threadIdx.x >> 6, wave = (int)blockIdx.x * 4 + wv, nwaves = (int)(gridDim.x * 4);
+  // The wave's refined pixels, appended to the list 64 at a time: where most pixels
+  // are refined, an atomic a step on the one counter sets the time (512^2, 4 x 4
+  // nodes, depth 2, tolerance 1e-4: 341 us, so 170).
+  __shared__ int32_t pend[4][64];
+  int npend = 0;
+  auto flush = [&]() {
+    if (npend == 0) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    int base = 0;
+    if (lane == 0) base = atomicAdd(ws.count + 1, npend);
+    base = __shfl(base, 0, 64);
+    if (lane < npend) ws.deep[base + lane] = pend[wv][lane];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    npend = 0;
+  };
   const int count = ws.count[0];
   const int64_t npix = (int64_t)cp.nx * cp.ny;
   const Prof<double>& p = rc.d;
@@ -291,7 +320,7 @@ __global__ __launch_bounds__(256) void render_level1_kernel(apx_component cp, Re
     const int k = k0 + grp;
     const bool on = grp < per && k < count;
     const int32_t pix = on ? ws.list[k] : 0;
-    if (MODE == Q_VJP && (!on || ws.flags[pix] == 2)) continue;  // no lane reads below
+    if (MODE == Q_VJP && (!on || !has || ws.flags[pix] == 2)) continue;  // no lane reads below
     double X0, Y0, gl[APX_NSLOT];
     pixel_xy(p, cp, pix % cp.nx, pix / cp.nx, X0, Y0);
     const double v1 = eval_profile<double, GRAD>(p, X0 + ox, Y0 + oy, 1.0, gl);
@@ -301,21 +330,15 @@ __global__ __launch_bounds__(256) void render_level1_kernel(apx_component cp, Re
       for (int s = 0; s < APX_NSLOT; ++s) adj[s] += wb * gl[s];
       continue;
     }
-    const double t = w * v1;
-    double res = 0.0;
-    for (int j = 0; j < nn; ++j) res += __shfl(t, first + j, 64);
+    const double res = sum(has ? w * v1 : 0.0);
     const double centre = __shfl(v1, first + nn / 2, 64);
     const bool refine = on && cp.max_depth > 1 && fabs(res - centre) > thr1;
     double gs[APX_NSLOT];
     if (GRAD) {
 #pragma unroll
-      for (int s = 0; s < APX_NSLOT; ++s) {
-        const double tg = w * gl[s];
-        gs[s] = 0.0;
-        for (int j = 0; j < nn; ++j) gs[s] += __shfl(tg, first + j, 64);
-      }
+      for (int s = 0; s < APX_NSLOT; ++s) gs[s] = sum(has ? w * gl[s] : 0.0);
     }
-    const bool lead = on && node == 0;
+    const bool lead = on && at == 0;
     if (lead && !refine) {
       planes[pix] = (float)res;
       if (GRAD)
@@ -326,15 +349,16 @@ __global__ __launch_bounds__(256) void render_level1_kernel(apx_component cp, Re
     }
     const uint64_t ballot = __ballot(lead && refine);
     if (ballot) {
-      int base = 0;
-      if (lane == 0) base = atomicAdd(ws.count + 1, (int)__popcll(ballot));
-      base = __shfl(base, 0, 64);
+      const int c = (int)__popcll(ballot);
+      if (npend + c > 64) flush();
       if (lead && refine) {
-        ws.deep[base + (int)__popcll(ballot & ((lane == 0) ? 0ull : (~0ull >> (64 - lane))))] = pix;
+        pend[wv][npend + (int)__popcll(ballot & ((1ull << lane) - 1ull))] = pix;
         ws.flags[pix] = 2;
       }
+      npend += c;
     }
   }
+  if (MODE != Q_VJP) flush();
   if (MODE == Q_VJP) vjp_part(cp, adj, ws.vpart + 8 * blockIdx.x);
 }
 
@@ -345,19 +369,26 @@ __global__ __launch_bounds__(256) void render_level1_kernel(apx_component cp, Re
 // of every flagged sub-pixel form one run that the 256 threads share, so that a
 // cuspy centre pixel, up to 25 x 225 samples, is not one wave's serial chain.
 // FAST: the default 3 x 3 rule on 5 x 5 sub-pixels, whose 225 level-2 samples
-// take a thread each (summed per sub-pixel in node order); else a thread a
-// sub-pixel.
+// take a thread each (summed per sub-pixel in node order); else each sub-pixel's
+// nodes are dealt out to `slices` threads, as many as fit, whose partial sums one
+// thread adds; and where more pixels are listed than workgroups were launched (a
+// rule without a central node refines every selected pixel) a workgroup takes four
+// at once, level 2 of each by a wave of its own: 512^2, 4 x 4 nodes, depth 2,
+// tolerance 1e-4, Jacobian 761 us a pixel at a time, 265 so (with the
+// list of render_level1_kernel).
 template <int MODE, bool FAST>
 __global__ __launch_bounds__(256) void render_deep_kernel(apx_component cp, RenderConst rc, float* planes,
                                                           const float* __restrict__ B, RenderWs ws, int voff) {
   constexpr bool GRAD = MODE != Q_VALUE;
   constexpr int NV = GRAD ? 1 + APX_NSLOT : 1;
-  constexpr int NS = FAST ? 225 : 1;
-  __shared__ float sample[NV][NS];
-  __shared__ double sx[64], sy[64];   // flagged sub-pixels
+  constexpr int NS = FAST ? 225 : 1, NG = FAST ? 1 : 64;
+  __shared__ float sample[NV][FAST ? NS : 256], middle[NG];
+  __shared__ double sx[4 * 64], sy[4 * 64];  // flagged sub-pixels (of up to four pixels)
   __shared__ double ox3[NS], oy3[NS], w3[NS];
+  __shared__ double nodeu[NG], nodev[NG], nodew[NG], suba[NG], subb[NG];  // node q; sub-pixel's place in its pixel
   __shared__ double red[4][NV];
-  __shared__ int nflag;
+  __shared__ double red3[FAST ? 1 : 4][4][NV];
+  __shared__ int nflag, nflags[4], pixel[4];
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const int n = FAST ? 3 : cp.quad_level, nn = n * n, g = FAST ? 5 : cp.gridding, gg = g * g;
   const int64_t npix = (int64_t)cp.nx * cp.ny;
@@ -370,24 +401,172 @@ __global__ __launch_bounds__(256) void render_deep_kernel(apx_component cp, Rend
   // offset and weight of level-3 sample e of a sub-pixel: sub-sub-pixel e / nn, node e % nn
   auto offset3 = [&](int e, double& x, double& y, double& w) {
     const int q = e / nn, kk = e - q * nn;
-    const double a = (sub0 + subd * (q % g)) * ig, b = (sub0 + subd * (q / g)) * ig;
-    const double hu = a + 0.5 * ig * ig * cp.gl_node[kk % n], hv = b + 0.5 * ig * ig * cp.gl_node[kk / n];
+    const double a = (FAST ? sub0 + subd * (q % g) : suba[q]) * ig, b = (FAST ? sub0 + subd * (q / g) : subb[q]) * ig;
+    const double hu = a + 0.5 * ig * ig * (FAST ? cp.gl_node[kk % n] : nodeu[kk]);
+    const double hv = b + 0.5 * ig * ig * (FAST ? cp.gl_node[kk / n] : nodev[kk]);
     x = p.P00 * hu + p.P01 * hv;
     y = p.P10 * hu + p.P11 * hv;
-    w = cp.gl_weight[kk % n] * cp.gl_weight[kk / n] * 0.25;
+    w = FAST ? cp.gl_weight[kk % n] * cp.gl_weight[kk / n] * 0.25 : nodew[kk];
   };
-  if (FAST && t < NS) offset3(t, ox3[t], oy3[t], w3[t]);
-  // sub-pixel and node of this thread at level 2
-  const int sub = FAST ? t / 9 : t, k2 = FAST ? t - 9 * sub : 0;
-  const double sa = sub0 + subd * (sub % g), sb = sub0 + subd * (sub / g);
-  const double sdx = p.P00 * sa + p.P01 * sb, sdy = p.P10 * sa + p.P11 * sb;
-  const float nu = (float)cp.gl_node[k2 % n], nv = (float)cp.gl_node[k2 / n];
-  auto weight2 = [&](int q) { return (float)(cp.gl_weight[q % 3] * cp.gl_weight[q / 3] * 0.25); };
   const int count = ws.count[1];
   double adj[APX_NSLOT];
 #pragma unroll
   for (int s = 0; s < APX_NSLOT; ++s) adj[s] = 0.0;
-  for (int k = blockIdx.x; k < count; k += gridDim.x) {
+  if ((int)blockIdx.x >= count) {  // no pixel for this workgroup
+    if (MODE == Q_VJP) vjp_part(cp, adj, ws.vpart + 8 * (voff + blockIdx.x));
+    return;
+  }
+  if (FAST) {
+    if (t < NS) offset3(t, ox3[t], oy3[t], w3[t]);
+  } else {
+    if (t < nn) {
+      nodeu[t] = cp.gl_node[t % n];
+      nodev[t] = cp.gl_node[t / n];
+      nodew[t] = cp.gl_weight[t % n] * cp.gl_weight[t / n] * 0.25;
+    }
+    if (t < gg) {
+      suba[t] = sub0 + subd * (t % g);
+      subb[t] = sub0 + subd * (t / g);
+    }
+    __syncthreads();
+  }
+  // sub-pixel and (first) node of this thread at level 2
+  const int slices = FAST ? 9 : min(nn, 256 / gg);
+  const int sub = FAST ? t / 9 : t % gg, k2 = FAST ? t - 9 * sub : t / gg;
+  const double sa = sub0 + subd * (sub % g), sb = sub0 + subd * (sub / g);
+  const double sdx = p.P00 * sa + p.P01 * sb, sdy = p.P10 * sa + p.P11 * sb;
+  const float nu = FAST ? (float)cp.gl_node[k2 % 3] : 0.0f, nv = FAST ? (float)cp.gl_node[k2 / 3] : 0.0f;
+  auto weight2 = [&](int q) { return (float)(cp.gl_weight[q % 3] * cp.gl_weight[q / 3] * 0.25); };
+  // does float64 arithmetic refine the sub-pixel at (x2, y2) with float32 value r2, centre node `centre`
+  auto refine = [&](double x2, double y2, float r2, float centre) {
+    const double D = fabs((double)r2 - (double)centre);
+    const double band = kSampleBand * (fabs((double)r2) + fabs((double)centre)) + 1e-7 * thr2;
+    if (D > thr2 + band) return true;
+    if (!(D >= thr2 - band)) return false;
+    double cd = 0.0;
+    const double rd = quad_sample<double, false>(p, cp, x2, y2, n, cp.gl_node, cp.gl_weight, sc2, 0.5 * ig * p.P00,
+                                                 0.5 * ig * p.P01, 0.5 * ig * p.P10, 0.5 * ig * p.P11, nullptr, cd);
+    return fabs(rd - cd) > thr2;
+  };
+  // weighted level-2 samples of nodes q0, q0 + step, .. of the sub-pixel at (x2, y2), added to part
+  auto nodes2 = [&](float x2, float y2, int q0, int step, float (&part)[NV], float& centre) {
+    for (int q = q0; q < nn; q += step) {
+      const float u = (float)nodeu[q], v = (float)nodev[q], w = (float)nodew[q];
+      float gl[APX_NSLOT];
+      const float val = eval_profile<float, GRAD>(pf, x2 + h * pf.P00 * u + h * pf.P01 * v,
+                                                  y2 + h * pf.P10 * u + h * pf.P11 * v, (float)sc2, gl);
+      part[0] += w * val;
+      if (q == nn / 2) centre = val;
+      if (GRAD) {
+#pragma unroll
+        for (int s = 0; s < APX_NSLOT; ++s) part[1 + s] += w * gl[s];
+      }
+    }
+  };
+  // level 3: the samples of nf flagged sub-pixels, one run over the workgroup, added to acc
+  auto level3 = [&](const double* xs, const double* ys, int nf, double (&acc)[NV]) {
+    const int per3 = gg * nn, total3 = nf * per3;
+    for (int e = t; e < total3; e += 256) {
+      const int f = e / per3, q = e - f * per3;
+      double dx, dy, w;
+      if (FAST) {
+        dx = ox3[q];
+        dy = oy3[q];
+        w = w3[q];
+      } else {
+        offset3(q, dx, dy, w);
+      }
+      float gl[APX_NSLOT];
+      const float val = eval_profile<float, GRAD>(pf, (float)(xs[f] + dx), (float)(ys[f] + dy), (float)sc3, gl);
+      acc[0] += w * (double)val;
+      if (GRAD) {
+#pragma unroll
+        for (int s = 0; s < APX_NSLOT; ++s) acc[1 + s] += w * (double)gl[s];
+      }
+    }
+  };
+  const bool many = !FAST && count > (int)gridDim.x;
+  if (many) {
+    const int deal = min(nn, 64 / gg), mine = lane % gg, q0 = lane / gg;
+    for (int k0 = blockIdx.x; k0 < count; k0 += 4 * (int)gridDim.x) {
+      const int k = k0 + wv * (int)gridDim.x;
+      const bool on = k < count;
+      const int32_t pix = on ? ws.deep[k] : 0;
+      double X0, Y0;
+      pixel_xy(p, cp, pix % cp.nx, pix / cp.nx, X0, Y0);
+      const double x2 = X0 + p.P00 * suba[mine] + p.P01 * subb[mine], y2 = Y0 + p.P10 * suba[mine] + p.P11 * subb[mine];
+      float part[NV], own = 0.0f;
+#pragma unroll
+      for (int s = 0; s < NV; ++s) part[s] = 0.0f;
+      if (on && q0 < deal) nodes2((float)x2, (float)y2, q0, deal, part, own);
+      const float centre = __shfl(own, (nn / 2) % deal * gg + mine, 64);
+      float r2 = 0.0f;
+      double acc[NV];
+#pragma unroll
+      for (int s = 0; s < NV; ++s) {
+        float v = 0.0f;
+        for (int j = 0; j < deal; ++j) v += __shfl(part[s], j * gg + mine, 64);
+        if (s == 0) r2 = v;
+        acc[s] = (double)v;
+      }
+      const bool deeper = on && lane < gg && cp.max_depth > 2 && refine(x2, y2, r2, centre);
+      if (lane >= gg || deeper) {
+#pragma unroll
+        for (int s = 0; s < NV; ++s) acc[s] = 0.0;
+      }
+      const uint64_t flags = __ballot(deeper);
+      if (deeper) {
+        const int at = 64 * wv + (int)__popcll(flags & ((1ull << lane) - 1ull));
+        sx[at] = x2;
+        sy[at] = y2;
+      }
+      if (lane == 0) {
+        nflags[wv] = (int)__popcll(flags);
+        pixel[wv] = pix;
+      }
+      if (MODE == Q_VJP) {
+        const double wb = on ? (double)B[pix] : 0.0;
+#pragma unroll
+        for (int s = 0; s < APX_NSLOT; ++s) adj[s] += wb * acc[1 + s];
+      } else {
+#pragma unroll
+        for (int s = 0; s < NV; ++s) {
+          const double a = wave_sum(acc[s]);
+          if (lane == 0) red[wv][s] = a;
+        }
+      }
+      __syncthreads();
+      // level 3 of each wave's pixel by the whole workgroup
+      for (int j = 0; j < 4; ++j) {
+        const int nf = nflags[j];
+        if (nf == 0) continue;
+        double a3[NV];
+#pragma unroll
+        for (int s = 0; s < NV; ++s) a3[s] = 0.0;
+        level3(sx + 64 * j, sy + 64 * j, nf, a3);
+        if (MODE == Q_VJP) {
+          const double wb = (double)B[pixel[j]];
+#pragma unroll
+          for (int s = 0; s < APX_NSLOT; ++s) adj[s] += wb * a3[1 + s];
+        } else {
+#pragma unroll
+          for (int s = 0; s < NV; ++s) {
+            const double a = wave_sum(a3[s]);
+            if (lane == 0) red3[j][wv][s] = a;
+          }
+        }
+      }
+      __syncthreads();
+      if (MODE != Q_VJP && on && lane < cp.nchan && (GRAD || lane == 0)) {
+        const int s = lane == 0 ? 0 : 1 + cp.chan_slot[lane];
+        double a = red[wv][s];
+        if (nflags[wv] > 0) a += red3[wv][0][s] + red3[wv][1][s] + red3[wv][2][s] + red3[wv][3][s];
+        planes[lane * npix + pix] = (float)(lane == 0 ? a : a * cp.dvdr[s - 1]);
+      }
+      __syncthreads();  // the next pixels write sx, sy, red and red3 again
+    }
+  }
+  for (int k = many ? count : (int)blockIdx.x; k < count; k += gridDim.x) {
     const int32_t pix = ws.deep[k];
     double X0, Y0;
     pixel_xy(p, cp, pix % cp.nx, pix / cp.nx, X0, Y0);
@@ -405,8 +584,16 @@ __global__ __launch_bounds__(256) void render_deep_kernel(apx_component cp, Rend
           for (int s = 0; s < APX_NSLOT; ++s) sample[1 + s][t] = gl[s];
         }
       }
-      __syncthreads();
+    } else if (k2 < slices) {
+      float part[NV], centre = 0.0f;
+#pragma unroll
+      for (int s = 0; s < NV; ++s) part[s] = 0.0f;
+      nodes2((float)(X0 + sdx), (float)(Y0 + sdy), k2, slices, part, centre);
+      if (k2 == (nn / 2) % slices) middle[sub] = centre;
+#pragma unroll
+      for (int s = 0; s < NV; ++s) sample[s][t] = part[s];
     }
+    __syncthreads();
     // level 2: thread t < gg sums sub-pixel t and tests it
     if (t < 64) {
       bool deeper = false;
@@ -429,22 +616,17 @@ __global__ __launch_bounds__(256) void render_deep_kernel(apx_component cp, Rend
             }
           }
         } else {
-          r2 = quad_sample<float, GRAD>(pf, cp, (float)x2, (float)y2, n, cp.gl_node, cp.gl_weight, (float)sc2, h * pf.P00,
-                                        h * pf.P01, h * pf.P10, h * pf.P11, gs, centre);
-        }
-        if (cp.max_depth > 2) {
-          const double D = fabs((double)r2 - (double)centre);
-          const double band = kSampleBand * (fabs((double)r2) + fabs((double)centre)) + 1e-7 * thr2;
-          if (D > thr2 + band) {
-            deeper = true;
-          } else if (D >= thr2 - band) {
-            double cd = 0.0;
-            const double rd = quad_sample<double, false>(p, cp, x2, y2, n, cp.gl_node, cp.gl_weight, sc2,
-                                                         0.5 * ig * p.P00, 0.5 * ig * p.P01, 0.5 * ig * p.P10,
-                                                         0.5 * ig * p.P11, nullptr, cd);
-            deeper = fabs(rd - cd) > thr2;
+          for (int q = 0; q < slices; ++q) r2 += sample[0][q * gg + t];
+          centre = middle[t];
+          if (GRAD) {
+#pragma unroll
+            for (int s = 0; s < APX_NSLOT; ++s) {
+              gs[s] = 0.0f;
+              for (int q = 0; q < slices; ++q) gs[s] += sample[1 + s][q * gg + t];
+            }
           }
         }
+        if (cp.max_depth > 2) deeper = refine(x2, y2, r2, centre);
         if (!deeper) {
           acc[0] = (double)r2;
           if (GRAD) {
@@ -462,26 +644,7 @@ __global__ __launch_bounds__(256) void render_deep_kernel(apx_component cp, Rend
       if (t == 0) nflag = (int)__popcll(flags);
     }
     __syncthreads();
-    // level 3: the samples of the flagged sub-pixels, one run over the workgroup
-    const int per3 = gg * nn, total3 = nflag * per3;
-    for (int e = t; e < total3; e += 256) {
-      const int f = e / per3, q = e - f * per3;
-      double dx, dy, w;
-      if (FAST) {
-        dx = ox3[q];
-        dy = oy3[q];
-        w = w3[q];
-      } else {
-        offset3(q, dx, dy, w);
-      }
-      float gl[APX_NSLOT];
-      const float val = eval_profile<float, GRAD>(pf, (float)(sx[f] + dx), (float)(sy[f] + dy), (float)sc3, gl);
-      acc[0] += w * (double)val;
-      if (GRAD) {
-#pragma unroll
-        for (int s = 0; s < APX_NSLOT; ++s) acc[1 + s] += w * (double)gl[s];
-      }
-    }
+    level3(sx, sy, nflag, acc);
     if (MODE == Q_VJP) {
       const double wb = (double)B[pix];
 #pragma unroll
@@ -559,9 +722,17 @@ __global__ __launch_bounds__(256) void render_vjp_final_kernel(apx_component cp,
   if (threadIdx.x == 0) grad[c - 1] = (red[0] + red[1] + red[2] + red[3]) * cp.dvdr[cp.chan_slot[c]];
 }
 
+// Lanes a pixel of the level-1 pass whose terms a butterfly adds; 0: nn lanes, added
+// in node order by nn lane reads a channel.  The reads take 20 instructions a pixel
+// and channel for the 3 x 3 rule (7 pixels a wave) and 784 for 7 x 7, a butterfly 5
+// to 18.  512^2, tolerance 1e-4, Jacobian without the deeper levels: 5 x 5 nodes by
+// lane reads 229 us, so 73; 7 x 7 751 and 119.
+int level1_row(int nn) { return nn <= 9 ? 0 : nn <= 16 ? 16 : nn <= 32 ? 32 : 64; }
+
 // workgroups of the two passes over npix pixels: no more than could find work
 int level_blocks(const apx_component& cp, int64_t npix) {
-  const int per = 4 * (64 / (cp.quad_level * cp.quad_level));
+  const int nn = cp.quad_level * cp.quad_level, row = level1_row(nn);
+  const int per = 4 * (64 / (row ? row : nn));
   return (int)std::min<int64_t>(kLevelBlocks, (npix + per - 1) / per);
 }
 int deep_blocks(const apx_component& cp, int64_t npix) {
@@ -574,7 +745,15 @@ void integrate(const apx_component& cp, const RenderConst& rc, float* planes, co
                hipStream_t stream) {
   const int64_t npix = (int64_t)cp.nx * cp.ny;
   const int nl = level_blocks(cp, npix), nd = deep_blocks(cp, npix);
-  hipLaunchKernelGGL((render_level1_kernel<MODE>), dim3(nl), dim3(256), 0, stream, cp, rc, planes, B, ws);
+#define APX_LEVEL1(ROW) \
+  hipLaunchKernelGGL((render_level1_kernel<MODE, ROW>), dim3(nl), dim3(256), 0, stream, cp, rc, planes, B, ws)
+  switch (level1_row(cp.quad_level * cp.quad_level)) {
+    case 64: APX_LEVEL1(64); break;
+    case 32: APX_LEVEL1(32); break;
+    case 16: APX_LEVEL1(16); break;
+    default: APX_LEVEL1(0);
+  }
+#undef APX_LEVEL1
   if (nd == 0) return;
   if (cp.quad_level == 3 && cp.gridding == 5)
     hipLaunchKernelGGL((render_deep_kernel<MODE, true>), dim3(nd), dim3(256), 0, stream, cp, rc, planes, B, ws, nl);

@@ -310,6 +310,33 @@ def test_integration_settings(level, gridding, depth):
     assert bool(((g.cpu() - gref).abs() <= 2e-4 * scale).all())
 
 
+@pytest.mark.parametrize("level,gridding,depth,tol,many", [
+    (2, 5, 2, 1e-4, True), (4, 2, 3, 1e-4, True), (4, 5, 2, 1e-2, False), (6, 2, 3, 1e-2, False), (6, 3, 2, 1e-4, True),
+    (5, 3, 3, 1e-4, True), (5, 1, 3, 1e-8, True), (7, 4, 2, 1e-8, True), (7, 8, 2, 1e-3, False)])
+def test_integration_orders_and_list_lengths(level, gridding, depth, tol, many):
+    """Every way the level-1 terms are added (by lane reads, over 16, 32 and 64
+    lanes), and the deep pass with more listed pixels than its 1,024 workgroups
+    (four pixels a workgroup) and with fewer (one), rules without a central node
+    among them: image, Jacobian and adjoint at the bars of
+    test_integration_settings."""
+    p = dict(GAL["sersic"], n=4.5, Re=5.0)
+    om, m = single("sersic", p, psf=PSF11, psf_mode="full", integrate_quad_level=level, integrate_gridding=gridding,
+                   integrate_max_depth=depth, sampling_tolerance=tol)
+    rep = om.vector_representation()
+    assert rel_err(m().data, om.forward(rep).reshape(36, 40)) < 1e-5
+    refined = int(m._apx_buffers["render_ws"].view(torch.int32)[1])
+    assert refined > 0 and (refined > 1024) == many
+    J = m.jacobian(parameters=rep.clone(), as_representation=True).data
+    ref = om.jacobian(rep).reshape(36, 40, -1)
+    for k in range(7):
+        assert rel_err(J[..., k], ref[..., k]) < 2e-4, k
+    G = torch.randn(36, 40, generator=torch.Generator().manual_seed(level), dtype=torch.float64)
+    g = m.vjp(G, parameters=rep.clone())
+    gref = (ref * G[..., None]).sum(dim=(0, 1))
+    scale = (ref * G[..., None]).abs().sum(dim=(0, 1))
+    assert bool(((g.cpu() - gref).abs() <= 2e-4 * scale).all())
+
+
 @pytest.mark.parametrize("kh,kw,ow,oh,nchan,zero,shared", [
     (1, 1, 70, 33, 1, 0, False), (19, 19, 64, 16, 2, 0, False), (21, 21, 65, 17, 3, 0, False), (53, 21, 130, 31, 2, 0, False),
     (23, 67, 63, 48, 2, 1, False), (67, 67, 100, 40, 4, 1, False), (69, 69, 64, 24, 2, 0, False), (27, 27, 66, 20, 3, 0, True),
