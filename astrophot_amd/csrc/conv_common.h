@@ -97,10 +97,11 @@ __device__ __forceinline__ void conv_accumulate(const float* smem, int LW, int l
 // Rows from HBM straight into LDS: row t of dst (rows x cols, pitch dpitch) gets
 // src[(gy0 + t) * pitch + gx0 ..], zero where that lies outside nx x ny.  The
 // workgroup's waves take the rows in turn, 64 floats a load, through a buffer
-// resource of one source row: its range check gives the zeros (a column before
-// the row is a huge unsigned offset, a row outside has an empty resource), so no
-// register holds the data, nothing is divided and every load of the tile is in
-// flight at once.  Completion: vmcnt, then a barrier.
+// resource of one source row from the tile's first column on: its range check gives
+// the zeros (a column before the row is a huge unsigned offset, a row outside has an
+// empty resource), so no register holds the data, nothing is divided and every load
+// of the tile is in flight at once.  A resource has 32 bits of bytes: the rest of a
+// longer row, which no tile reaches, is cut off.  Completion: vmcnt, then a barrier.
 typedef __attribute__((address_space(3))) void* lds_ptr;
 constexpr int kBufWord3 = 0x00020000;  // buffer resource word 3 on gfx9: 32-bit data
 
@@ -108,17 +109,18 @@ template <int NW = 4>  // waves of the workgroup
 __device__ __forceinline__ void stage_rows(const float* src, int64_t pitch, int nx, int ny, int gx0, int gy0, int rows,
                                            int cols, float* dst, int dpitch) {
   const int lane = threadIdx.x & 63;
+  const int bx = max(gx0, 0), bytes = min(max(nx - bx, 0), 1 << 28) * 4;
   for (int t = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); t < rows; t += NW) {
     const int gy = gy0 + t;
     const bool in = gy >= 0 && gy < ny;
     // every field of the resource is uniform: read from lane 0 so that it stays in SGPRs
-    const uint64_t a = (uint64_t)(src + (int64_t)(in ? gy : 0) * pitch);
+    const uint64_t a = (uint64_t)(src + (int64_t)(in ? gy : 0) * pitch + bx);
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-        reinterpret_cast<void*>(((uint64_t)hi << 32) | lo), (short)0, __builtin_amdgcn_readfirstlane(in ? nx * 4 : 0), kBufWord3);
+        reinterpret_cast<void*>(((uint64_t)hi << 32) | lo), (short)0, __builtin_amdgcn_readfirstlane(in ? bytes : 0), kBufWord3);
     for (int c = 0; c < cols; c += 64)
       if (c + lane < cols)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr)(dst + t * dpitch + c), 4, (gx0 + c + lane) * 4, 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr)(dst + t * dpitch + c), 4, (gx0 - bx + c + lane) * 4, 0, 0, 0);
   }
 }
 

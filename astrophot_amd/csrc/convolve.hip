@@ -332,16 +332,17 @@ struct ConvPasses {
 template <bool TALL>
 __global__ __launch_bounds__(TALL ? 512 : 256) void convolve_mfma_kernel(apx_conv_job job, const float* __restrict__ planes,
                                                             const float* __restrict__ kernels, ConvPasses passes,
-                                                            int ntx, int ntile) {
+                                                            int ntx, uint32_t tile0, int count) {
   extern __shared__ float smem[];
-  const int padded = (ntile + 7) & ~7;
-  const int pass = blockIdx.x / padded, tile = blockIdx.x - pass * padded;
-  if (tile >= ntile) return;
+  const int padded = (count + 7) & ~7;
+  const int pass = blockIdx.x / padded, local = blockIdx.x - pass * padded;
+  if (local >= count) return;
+  const uint32_t tile = tile0 + (uint32_t)local;
   const int c = passes.plane[pass], k = passes.kernel[pass];
   constexpr int NW = TALL ? 8 : 4;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, w = wave & 3, half = wave >> 2;
   const int lm = lane & 15, lk = lane >> 4;
-  const int ox0 = (tile % ntx) * 64, oy0 = (tile / ntx) * (NW / 4 * kMfR);
+  const int ty = (int)(tile / (uint32_t)ntx), ox0 = ((int)tile - ty * ntx) * 64, oy0 = ty * (NW / 4 * kMfR);
   const int kh = job.kh, kw = job.kw, ch = (kh - 1) / 2, cw = (kw - 1) / 2;
   const int rows = mf_rows(kh) + (NW / 4 - 1) * kMfR, DD = mf_dd(kh);
   float* tin = smem;             // rows x kMfLW
@@ -459,6 +460,49 @@ int64_t convolve_workspace_bytes(int32_t kh, int32_t kw) {
   return (int64_t)sizeof(float) * 3 * kw * fast_kts(kh) + 256;
 }
 
+// The passes of a launch run side by side, so each has a Jacobian column of its
+// own: passes that add to one column go to launches after one another, in their
+// order.  A launch stays below 2^31 threads; one that would not is cut by tiles.
+static int convolve_mfma(const apx_conv_job& job, const float* planes, const float* kernels, hipStream_t stream) {
+  ConvPasses turn[kMaxPass] = {};
+  auto add = [&](int plane, int kernel, int col) {
+    int k = 0;
+    for (;; ++k) {
+      bool taken = false;
+      for (int p = 0; p < turn[k].n; ++p)
+        taken = taken || col == (turn[k].plane[p] > 0 ? job.chan_col[turn[k].plane[p]]
+                                 : turn[k].kernel[p] > 0 ? job.dk_col[turn[k].kernel[p] - 1] : -1);
+      if (!taken) break;
+    }
+    ConvPasses& t = turn[k];
+    t.plane[t.n] = (int8_t)plane;
+    t.kernel[t.n++] = (int8_t)kernel;
+  };
+  int n = 0;
+  if (job.img) add(0, 0, -1), ++n;
+  for (int k = 0; k < 2; ++k)
+    if (job.dk_col[k] >= 0) add(0, 1 + k, job.dk_col[k]), ++n;
+  for (int c = 1; c < job.nchan; ++c) add(c, 0, job.chan_col[c]), ++n;
+  const int ntx = (job.ow + 63) / 64;
+  const int64_t tall = (int64_t)ntx * ((job.oh + (int64_t)2 * kMfR - 1) / (2 * kMfR));
+  const bool two = tall * n >= kMfTallMin;
+  const int64_t ntile = two ? tall : (int64_t)ntx * ((job.oh + kMfR - 1) / kMfR);
+  auto* kernel = two ? &convolve_mfma_kernel<true> : &convolve_mfma_kernel<false>;
+  const size_t lds = mfma_lds_bytes(job.kh, job.kw, two ? 2 : 1);
+  if (lds > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+    return set_error(APX_E_HIP, "convolve: LDS size refused");
+  for (int k = 0; k < kMaxPass && turn[k].n > 0; ++k) {
+    const int64_t most = ((int64_t)INT32_MAX / 512 / turn[k].n) & ~(int64_t)7;
+    for (int64_t tile0 = 0; tile0 < ntile; tile0 += most) {
+      const int count = (int)std::min(most, ntile - tile0);
+      hipLaunchKernelGGL(kernel, dim3((unsigned)(((count + 7) & ~7) * turn[k].n)), dim3(two ? 512 : 256), lds, stream, job,
+                         planes, kernels, turn[k], ntx, (uint32_t)tile0, count);
+    }
+  }
+  return check_launch("convolve (MFMA)");
+}
+
 int convolve(const apx_conv_job* jp, const float* planes, const float* kernels, void* workspace,
              int64_t ws_bytes, hipStream_t stream) {
   if (!jp || !planes || !kernels) return set_error(APX_E_INVALID, "convolve: null pointer");
@@ -500,39 +544,8 @@ int convolve(const apx_conv_job* jp, const float* planes, const float* kernels, 
         return set_error(APX_E_INVALID, "convolve: centre column out of range");
   }
   const int nk0 = dk ? 3 : 1;
-  if (job.kh >= kMfmaMin && job.kh <= kMfmaWide && job.kw >= kMfmaMin && job.kw <= kMfmaWide &&
-      job.nx < (1 << 29) /* a row's bytes fit the range check of its buffer resource */) {
-    ConvPasses ps = {};
-    auto add = [&](int plane, int kernel) {
-      ps.plane[ps.n] = (int8_t)plane;
-      ps.kernel[ps.n++] = (int8_t)kernel;
-    };
-    if (job.img) add(0, 0);
-    for (int k = 0; k < 2; ++k)
-      if (job.dk_col[k] >= 0) add(0, 1 + k);
-    for (int c = 1; c < job.nchan; ++c) add(c, 0);
-    if (ps.n == 0) return APX_OK;
-    // the passes run side by side, so each needs a column of its own
-    bool own = true;
-    auto column = [&](int p) { return ps.plane[p] == 0 ? job.dk_col[ps.kernel[p] - 1] : job.chan_col[ps.plane[p]]; };
-    for (int p = job.img ? 1 : 0; p < ps.n; ++p)
-      for (int q = job.img ? 1 : 0; q < p; ++q) own = own && column(p) != column(q);
-    const int ntx = (job.ow + 63) / 64;
-    auto blocks_of = [&](int64_t ntile) { return ((ntile + 7) & ~(int64_t)7) * ps.n; };
-    const int64_t tall = (int64_t)ntx * ((job.oh + 2 * kMfR - 1) / (2 * kMfR));
-    const bool two = tall * ps.n >= kMfTallMin;
-    const int64_t ntile = two ? tall : (int64_t)ntx * ((job.oh + kMfR - 1) / kMfR), blocks = blocks_of(ntile);
-    if (own && blocks <= (int64_t)INT32_MAX / 512) {
-      auto* kernel = two ? &convolve_mfma_kernel<true> : &convolve_mfma_kernel<false>;
-      const size_t lds = mfma_lds_bytes(job.kh, job.kw, two ? 2 : 1);
-      if (lds > 65536 && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-        return set_error(APX_E_HIP, "convolve: LDS size refused");
-      hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(two ? 512 : 256), lds, stream, job, planes, kernels, ps, ntx,
-                         (int)ntile);
-      return check_launch("convolve (MFMA)");
-    }
-  }
+  if (job.kh >= kMfmaMin && job.kh <= kMfmaWide && job.kw >= kMfmaMin && job.kw <= kMfmaWide)
+    return convolve_mfma(job, planes, kernels, stream);
   if (job.kh <= kFastMax && job.kw <= kFastMax) {
     if (!workspace || ws_bytes < convolve_workspace_bytes(job.kh, job.kw))
       return set_error(APX_E_INVALID, "convolve: workspace too small");

@@ -381,6 +381,87 @@ def test_convolve_shapes(kh, kw, ow, oh, nchan, zero, shared):
     assert float((jac.double() - ref_j).abs().max()) <= tol
 
 
+def conv_job(planes, kern, img=None, jac=None, x0=0, y0=0, ow=0, oh=0):
+    """An apx_conv_job on every output pixel of img or jac, zero outside the planes."""
+    job = ap._lib.ConvJob()
+    job.nchan, job.ny, job.nx = planes.shape
+    job.kh, job.kw = kern.shape[1:]
+    job.x0, job.y0, job.ow, job.oh, job.zero_outside = x0, y0, ow, oh, 1
+    job.chan_col[:], job.dk_col[:] = [-1] * 8, [-1] * 2
+    if img is not None:
+        job.img, job.img_row, job.img_w, job.img_h = img.data_ptr(), ow, ow, oh
+    if jac is not None:
+        job.jac, job.jac_np, job.jac_row, job.jac_w, job.jac_h = jac.data_ptr(), jac.shape[2], ow * jac.shape[2], ow, oh
+    return job
+
+
+def conv_float64(box, kern):
+    """Full convolution of the rows and columns around a box that the kernel covers."""
+    return torch.nn.functional.conv2d(box.double().cpu()[None, None], kern.double().cpu()[None, None])[0, 0].cuda()
+
+
+@pytest.mark.parametrize("side,ow,cols,dk", [(21, 70, [2, 2, 2], [2, -1]), (27, 40, [0, 1, 0], [1, 1]), (67, 130, [1, 1, 0], [0, 1])])
+def test_convolve_shared_columns_without_workspace(side, ow, cols, dk):
+    """Passes that add to one Jacobian column, and kernels of 21 to 67 rows, need
+    no workspace: the columns' sums against float64, 1e-5 of the sum of the
+    magnitudes as test_convolve_shapes."""
+    g = torch.Generator().manual_seed(side)
+    planes, kern = torch.randn(4, ow, ow, generator=g).cuda(), torch.randn(3, side, side, generator=g).cuda()
+    jac = torch.randn(ow, ow, 3, generator=g).cuda()
+    ref, tol = jac.double(), 0.0
+    pad = torch.nn.functional.pad(planes, (side // 2,) * 4)
+    for p, k, c in [(0, 1, dk[0]), (0, 2, dk[1]), (1, 0, cols[0]), (2, 0, cols[1]), (3, 0, cols[2])]:
+        if c >= 0:
+            ref[..., c] += conv_float64(pad[p], kern[k])
+            tol += 1e-5 * float(conv_float64(pad[p].abs(), kern[k].abs()).max())
+    job = conv_job(planes, kern, jac=jac, ow=ow, oh=ow)
+    job.chan_col[1], job.chan_col[2], job.chan_col[3] = cols
+    job.dk_col[0], job.dk_col[1] = dk
+    ap._lib.check(ap._lib.load().apx_convolve(ctypes.byref(job), planes.data_ptr(), kern.data_ptr(), None, 0, ap._lib.stream()))
+    assert float((jac.double() - ref).abs().max()) <= tol
+
+
+def test_convolve_rows_of_half_a_billion_pixels():
+    """A plane row of more than 2^29 pixels, whose bytes exceed a buffer resource:
+    the last columns and the first ones, zero beyond either end."""
+    g = torch.Generator().manual_seed(1)
+    nx, ow, side = 2 ** 29 + 77, 150, 21
+    plane, kern = torch.zeros(1, 1, nx, device="cuda"), torch.randn(1, side, side, generator=g).cuda()
+    plane[0, 0, :400], plane[0, 0, -400:] = torch.randn(400, generator=g).cuda(), torch.randn(400, generator=g).cuda()
+    lib = ap._lib.load()
+    for x0 in (0, nx - ow):
+        img = torch.zeros(1, ow, device="cuda")
+        job = conv_job(plane, kern, img=img, x0=x0, ow=ow, oh=1)
+        ap._lib.check(lib.apx_convolve(ctypes.byref(job), plane.data_ptr(), kern.data_ptr(), None, 0, ap._lib.stream()))
+        row = torch.nn.functional.pad(plane[0, 0, :ow + 10] if x0 == 0 else plane[0, 0, -(ow + 10):],
+                                      (10, 0) if x0 == 0 else (0, 10))
+        box = torch.nn.functional.pad(row[None], (0, 0, 10, 10))
+        want = conv_float64(box, kern[0])
+        assert float((img.double() - want).abs().max()) <= 1e-5 * float(conv_float64(box.abs(), kern[0].abs()).max())
+
+
+def test_convolve_of_more_tiles_than_a_launch():
+    """A one-column image of 4.2 million tiles, past the 2^31 threads a launch is
+    kept below: the rows around the cut, the first and the last."""
+    g = torch.Generator().manual_seed(2)
+    side = 21
+    cut = ((2 ** 31 - 1) // 512 // 8) * 8 * 32
+    ny = cut + 100
+    plane, kern = torch.zeros(1, ny, 1, device="cuda"), torch.randn(1, side, side, generator=g).cuda()
+    where = [0, cut - 100, ny - 200]
+    for y in where:
+        plane[0, y:y + 200, 0] = torch.randn(200, generator=g).cuda()
+    img = torch.zeros(ny, 1, device="cuda")
+    job = conv_job(plane, kern, img=img, ow=1, oh=ny)
+    ap._lib.check(ap._lib.load().apx_convolve(ctypes.byref(job), plane.data_ptr(), kern.data_ptr(), None, 0, ap._lib.stream()))
+    for y in where:
+        lo, hi = max(y - 50, 0), min(y + 250, ny)
+        rows = plane[0, max(lo - 10, 0):min(hi + 10, ny)]
+        box = torch.nn.functional.pad(rows, (10, 10, 10 if lo == 0 else 0, 10 if hi == ny else 0))
+        want = conv_float64(box, kern[0])
+        assert float((img[lo:hi].double() - want).abs().max()) <= 1e-5 * float(conv_float64(box.abs(), kern[0].abs()).max())
+
+
 @pytest.mark.parametrize("npar", [1, 2, 13, 15, 16, 17, 64])
 def test_lm_solve_sizes_and_bad_pivots(npar):
     """The one-wave solve (up to 16) and the workgroup one at the edges of
