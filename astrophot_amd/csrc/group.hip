@@ -100,11 +100,12 @@ __global__ __launch_bounds__(256) void group_rpp_weights_kernel(apx_group g, con
   }
 }
 
-// A window (or an overlap of two) of n pixels goes to several workgroups: at
-// most S pieces, of at least kPiece pixels, so that the largest (400 x 400 beside
-// a median overlap of 4,500 pixels) does not set the pass's time.  One workgroup
-// a window: pairs, sources and J^T v of 500 sources on 2048^2 (3,051 pairs, 35 M
-// pair pixels) took 0.94, 0.73 and 0.43 ms; in pieces 0.33, 0.16 and 0.12 ms.
+// A window (or an overlap of two) of n pixels goes to several workgroups: pieces
+// of up to kPiece pixels, larger only where there would be more than S of them, so
+// that the largest (400 x 400 beside a median overlap of 4,500 pixels) does not set
+// the pass's time.  One workgroup a window: pairs, sources and J^T v of 500 sources
+// on 2048^2 (3,051 pairs, 35 M pair pixels) took 0.94, 0.73 and 0.43 ms; in pieces
+// 0.33, 0.16 and 0.12 ms.
 constexpr int kPiece = 4096;
 
 struct Piece {
@@ -139,13 +140,21 @@ struct Piece {
 __device__ __forceinline__ int pieces_of(int64_t n, int S) {
   return (int)min((int64_t)S, max((int64_t)1, (n + kPiece - 1) / kPiece));
 }
-// the most pieces a window gets when `count` of them share the chip
-inline int max_pieces(int count) { return std::max(1, std::min(16, 32768 / std::max(1, count))); }
+// The most pieces a window (or an overlap) gets when `count` of them share the
+// chip.  Every one is launched, also those that small windows do not have, so a
+// group of small windows gets fewer: as many as one of four times the mean window
+// has (1,000 windows of 30 x 30: normal equations 362 us with 16, 142 with 1).  With
+// one, the kernels write the result itself in place of a partial sum.
+inline int max_pieces(const apx_group& g, int count) {
+  const int64_t mean = g.nsrcpix / std::max(1, g.nsrc);
+  return (int)std::max<int64_t>(1, std::min<int64_t>({16, 32768 / std::max(1, count), 4 * mean / kPiece}));
+}
 
-// part[s S + piece][k] = sum over the piece of the window of J_k * v (v a double image)
+// part[s S + piece][k] = sum over the piece of the window of J_k * v (v a double
+// image); with S = 1 out[col0 + k] itself
 __global__ __launch_bounds__(256) void group_jtv_kernel(apx_group g, const float* __restrict__ J,
                                                         const double* __restrict__ v, int S,
-                                                        double* __restrict__ part) {
+                                                        double* __restrict__ part, double* __restrict__ out) {
   __shared__ double red[4][APX_BATCH_NP];
   const int s = blockIdx.x / S;
   const int* w = g.win + 4 * s;
@@ -165,7 +174,8 @@ __global__ __launch_bounds__(256) void group_jtv_kernel(apx_group g, const float
   __syncthreads();
   if (threadIdx.x < APX_BATCH_NP) {
     const int k = threadIdx.x;
-    part[(int64_t)blockIdx.x * APX_BATCH_NP + k] = red[0][k] + red[1][k] + red[2][k] + red[3][k];
+    double* to = S == 1 ? out + g.col0[s] : part + (int64_t)blockIdx.x * APX_BATCH_NP;
+    to[k] = red[0][k] + red[1][k] + red[2][k] + red[3][k];
   }
 }
 
@@ -244,13 +254,29 @@ __global__ __launch_bounds__(256) void fill_kernel(double* __restrict__ a, int64
   for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) a[e] = v;
 }
 
-// Per piece of a source's window: the sums of J_k w (data - model) and J_k w.
+// Entry k of a source: grad[col0 + k] = v, and from k = NP on the sky column
+// H[col0 + k - NP][sky] = H[sky][col0 + k - NP] = c v.
+__device__ __forceinline__ void source_entry(const apx_group& g, int s, int k, double c, double v, double* H, double* grad) {
+  constexpr int NP = APX_BATCH_NP;
+  if (k < NP) {
+    grad[g.col0[s] + k] = v;
+  } else if (g.sky_col >= 0) {
+    const int col = g.col0[s] + k - NP;
+    H[(int64_t)col * g.np + g.sky_col] = c * v;
+    H[(int64_t)g.sky_col * g.np + col] = c * v;
+  }
+}
+
+// Per piece of a source's window: the sums of J_k w (data - model) and J_k w; kOne
+// (S is 1): the entries themselves.
+template <bool kOne>
 __global__ __launch_bounds__(256) void group_source_kernel(apx_group g, const float* __restrict__ J,
                                                            const float* __restrict__ model,
                                                            const float* __restrict__ data,
                                                            const float* __restrict__ weight,
                                                            const uint8_t* __restrict__ mask, int S,
-                                                           double* __restrict__ part) {
+                                                           double* __restrict__ part, double c,
+                                                           double* __restrict__ H, double* __restrict__ grad) {
   constexpr int NP = APX_BATCH_NP;
   __shared__ double red[4][2 * NP];
   const int s = blockIdx.x / S;
@@ -278,12 +304,13 @@ __global__ __launch_bounds__(256) void group_source_kernel(apx_group g, const fl
   __syncthreads();
   if (threadIdx.x < 2 * NP) {
     const int k = threadIdx.x;
-    part[(int64_t)blockIdx.x * 2 * NP + k] = red[0][k] + red[1][k] + red[2][k] + red[3][k];
+    const double v = red[0][k] + red[1][k] + red[2][k] + red[3][k];
+    if (kOne) source_entry(g, s, k, c, v, H, grad);
+    else part[(int64_t)blockIdx.x * 2 * NP + k] = v;
   }
 }
 
-// grad[col0 + k] = sum J_k w (data - model) over the window, and the sky column
-// H[col0 + k][sky] = H[sky][col0 + k] = c sum J_k w: the source's pieces in order.
+// the entries from the source's pieces, in order
 __global__ __launch_bounds__(256) void group_source_final_kernel(apx_group g, int S, double c,
                                                                  const double* __restrict__ part,
                                                                  double* __restrict__ H,
@@ -292,17 +319,10 @@ __global__ __launch_bounds__(256) void group_source_final_kernel(apx_group g, in
   const int e = blockIdx.x * 256 + threadIdx.x;
   if (e >= g.nsrc * 2 * NP) return;
   const int s = e / (2 * NP), k = e % (2 * NP);
-  if (k >= NP && g.sky_col < 0) return;
   const int np = pieces_of((int64_t)g.win[4 * s + 2] * g.win[4 * s + 3], S);
   double v = 0.0;
   for (int q = 0; q < np; ++q) v += part[((int64_t)s * S + q) * 2 * NP + k];
-  if (k < NP) {
-    grad[g.col0[s] + k] = v;
-  } else {
-    const int col = g.col0[s] + k - NP;
-    H[(int64_t)col * g.np + g.sky_col] = c * v;
-    H[(int64_t)g.sky_col * g.np + col] = c * v;
-  }
+  source_entry(g, s, k, c, v, H, grad);
 }
 
 // the overlap of windows a and b: corner (x0, y0), size ow x oh (not positive: none)
@@ -316,14 +336,22 @@ struct Overlap {
   }
 };
 
+// entry e of the pair's 7 x 7 block, at (a, b) and (b, a)
+__device__ __forceinline__ void pair_entry(const apx_group& g, int a, int b, int e, double v, double* H) {
+  const int ra = g.col0[a] + e / APX_BATCH_NP, rb = g.col0[b] + e % APX_BATCH_NP;
+  H[(int64_t)ra * g.np + rb] = v;
+  H[(int64_t)rb * g.np + ra] = v;
+}
+
 // One 7 x 7 block of J^T W J per pair of overlapping windows (a <= b): sum
-// over the overlap of w J_a J_b^T, a piece a workgroup.  Bound by the J values of
+// over the overlap of w J_a J_b^T, a piece a workgroup (kOne: S is 1, the block itself).  Bound by the J values of
 // the pair pixels (56 bytes a pixel, most of them from the caches): the next
 // pixel's loads are issued before the 49 multiply-adds of the current one.
+template <bool kOne>
 __global__ __launch_bounds__(256) void group_pair_kernel(apx_group g, const float* __restrict__ J,
                                                          const float* __restrict__ weight,
                                                          const uint8_t* __restrict__ mask, int S,
-                                                         double* __restrict__ part) {
+                                                         double* __restrict__ part, double* __restrict__ H) {
   constexpr int NP = APX_BATCH_NP, NN = NP * NP;
   __shared__ double red[4][NN];
   const int pr = blockIdx.x / S;
@@ -377,12 +405,15 @@ __global__ __launch_bounds__(256) void group_pair_kernel(apx_group g, const floa
   }
   wave_sums(acc, red[threadIdx.x >> 6]);
   __syncthreads();
-  if (threadIdx.x < NN)
-    part[(int64_t)blockIdx.x * NN + threadIdx.x] =
-        red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
+  if (threadIdx.x < NN) {
+    const int k = threadIdx.x;
+    const double v = red[0][k] + red[1][k] + red[2][k] + red[3][k];
+    if (kOne) pair_entry(g, a, b, k, v, H);
+    else part[(int64_t)blockIdx.x * NN + k] = v;
+  }
 }
 
-// the pair's pieces in order, written at (a, b) and (b, a)
+// the pair's pieces, in order
 __global__ __launch_bounds__(64) void group_pair_final_kernel(apx_group g, int S, const double* __restrict__ part,
                                                               double* __restrict__ H) {
   constexpr int NP = APX_BATCH_NP, NN = NP * NP;
@@ -392,10 +423,7 @@ __global__ __launch_bounds__(64) void group_pair_final_kernel(apx_group g, int S
   const int np = pieces_of((int64_t)o.ow * o.oh, S);
   double v = 0.0;
   for (int q = 0; q < np; ++q) v += part[((int64_t)blockIdx.x * S + q) * NN + threadIdx.x];
-  const int k = threadIdx.x / NP, l = threadIdx.x % NP;
-  const int ca = g.col0[a], cb = g.col0[b];
-  H[(int64_t)(ca + k) * g.np + (cb + l)] = v;
-  H[(int64_t)(cb + l) * g.np + (ca + k)] = v;
+  pair_entry(g, a, b, threadIdx.x, v, H);
 }
 
 // ---------------------------------------------------------------------------
@@ -941,13 +969,14 @@ int group_image(const apx_group* g, const float* src, double sky, float* out, hi
 
 static int64_t group_part_bytes(const apx_group* g) {
   const int64_t npix = (int64_t)g->nx * g->ny;
-  return 8 * std::max(npix, (int64_t)g->npair * max_pieces(g->npair) * APX_BATCH_NP * APX_BATCH_NP);
+  const int S = max_pieces(*g, g->npair);
+  return 8 * std::max(npix, S == 1 ? 0 : (int64_t)g->npair * S * APX_BATCH_NP * APX_BATCH_NP);
 }
 
 int64_t group_workspace_bytes(const apx_group* g) {
   if (!g) return 0;
   // [u of group_rpp, or the pair partials | image partials | source partials]
-  return group_part_bytes(g) + 8 * 2 * 4096 + 8 * 2 * APX_BATCH_NP * (int64_t)g->nsrc * max_pieces(g->nsrc) + 256;
+  return group_part_bytes(g) + 8 * 2 * 4096 + 8 * 2 * APX_BATCH_NP * (int64_t)g->nsrc * max_pieces(*g, g->nsrc) + 256;
 }
 
 int group_normal(const apx_group* g, const float* J, const float* model, const float* data,
@@ -962,18 +991,21 @@ int group_normal(const apx_group* g, const float* J, const float* model, const f
   double* part = reinterpret_cast<double*>(static_cast<char*>(ws) + group_part_bytes(g));
   double* spart = part + 2 * 4096;
   if (g->npair > 0) {
-    const int S = max_pieces(g->npair);
+    const int S = max_pieces(*g, g->npair);
     double* pp = static_cast<double*>(ws);
-    hipLaunchKernelGGL(group_pair_kernel, dim3((unsigned)g->npair * S), dim3(256), 0, stream, *g, J, weight, mask, S,
-                       pp);
-    hipLaunchKernelGGL(group_pair_final_kernel, dim3((unsigned)g->npair), dim3(64), 0, stream, *g, S,
-                       (const double*)pp, H);
+    auto* kernel = S == 1 ? &group_pair_kernel<true> : &group_pair_kernel<false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)g->npair * S), dim3(256), 0, stream, *g, J, weight, mask, S, pp, H);
+    if (S > 1)
+      hipLaunchKernelGGL(group_pair_final_kernel, dim3((unsigned)g->npair), dim3(64), 0, stream, *g, S,
+                         (const double*)pp, H);
   }
-  const int S = max_pieces(g->nsrc);
-  hipLaunchKernelGGL(group_source_kernel, dim3((unsigned)g->nsrc * S), dim3(256), 0, stream, *g, J, model, data,
-                     weight, mask, S, spart);
-  hipLaunchKernelGGL(group_source_final_kernel, dim3((unsigned)((2 * APX_BATCH_NP * g->nsrc + 255) / 256)), dim3(256),
-                     0, stream, *g, S, sky_dcol, (const double*)spart, H, grad);
+  const int S = max_pieces(*g, g->nsrc);
+  auto* kernel = S == 1 ? &group_source_kernel<true> : &group_source_kernel<false>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)g->nsrc * S), dim3(256), 0, stream, *g, J, model, data, weight, mask, S, spart,
+                     sky_dcol, H, grad);
+  if (S > 1)
+    hipLaunchKernelGGL(group_source_final_kernel, dim3((unsigned)((2 * APX_BATCH_NP * g->nsrc + 255) / 256)), dim3(256),
+                       0, stream, *g, S, sky_dcol, (const double*)spart, H, grad);
   if (g->sky_col >= 0) {
     const int64_t npix = (int64_t)g->nx * g->ny;
     const int nb = std::min(grid_for(npix), 512);
@@ -997,11 +1029,12 @@ int group_rpp(const apx_group* g, const float* J, const float* m0, const float* 
   double* spart = part + 2 * 4096;
   hipLaunchKernelGGL(group_rpp_weights_kernel, dim3((unsigned)(g->ntx * g->nty)), dim3(256), 0, stream, *g, J,
                      m0, m1, weight, mask, h, d, sky_dcol, u);
-  const int S = max_pieces(g->nsrc);
+  const int S = max_pieces(*g, g->nsrc);
   hipLaunchKernelGGL(group_jtv_kernel, dim3((unsigned)g->nsrc * S), dim3(256), 0, stream, *g, J, (const double*)u,
-                     S, spart);
-  hipLaunchKernelGGL(group_jtv_final_kernel, dim3((unsigned)((APX_BATCH_NP * g->nsrc + 255) / 256)), dim3(256), 0,
-                     stream, *g, S, (const double*)spart, out);
+                     S, spart, out);
+  if (S > 1)
+    hipLaunchKernelGGL(group_jtv_final_kernel, dim3((unsigned)((APX_BATCH_NP * g->nsrc + 255) / 256)), dim3(256), 0,
+                       stream, *g, S, (const double*)spart, out);
   if (g->sky_col >= 0) {
     const int nb = std::min(grid_for(npix), 512);
     hipLaunchKernelGGL(group_image_sums_kernel, dim3(nb), dim3(256), 0, stream, npix, 1, (const float*)nullptr,
