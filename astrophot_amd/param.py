@@ -75,20 +75,24 @@ def _inv(x):
     return 1.0 / x if x != 0.0 else math.copysign(math.inf, x)
 
 
+def _wrap(x, lo, hi):
+    return lo + (x - lo) % (hi - lo) if hi != lo else math.nan
+
+
 def _val_to_rep1(v, lo, hi, cyclic):
     if cyclic:
-        return lo + (v - lo) % (hi - lo)
+        return _wrap(v, lo, hi)
     if lo is None:
         return v if hi is None else v - _inv(v - hi)
     if hi is None:
         return v - _inv(v - lo)
-    x = (v - lo) * math.pi / (hi - lo) - math.pi / 2
+    x = (v - lo) * math.pi / (hi - lo) - math.pi / 2 if hi != lo else math.nan
     return math.tan(x) if math.isfinite(x) else math.nan
 
 
 def _rep_to_val1(r, lo, hi, cyclic):
     if cyclic:
-        return lo + (r - lo) % (hi - lo)
+        return _wrap(r, lo, hi)
     if lo is None:
         return r if hi is None else (r + hi - math.sqrt((r - hi) * (r - hi) + 4)) * 0.5
     if hi is None:

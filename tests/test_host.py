@@ -363,3 +363,17 @@ def test_plain_vectors_equal_the_tensor_path():
         a.vector_set_values(a.vector_values() * 1.001)
     with pytest.raises((InvalidParameter, RuntimeError)):
         a.vector_set_values(torch.ones(9, dtype=torch.float64))
+
+
+@pytest.mark.parametrize("limits,cyclic", [((2.0, 2.0), False), ((2.0, 2.0), True), ((3.0, 1.0), True), ((-0.0, 0.0), True)])
+def test_float_parameter_maps_of_degenerate_limits(limits, cyclic):
+    """Equal or crossed limits: the float maps give what the tensor maps do, NaN
+    where those divide by zero, and raise nothing."""
+    from astrophot_amd import param as PM
+    n = PM.Parameter_Node("p", limits=limits, cyclic=cyclic)
+    for x in (2.0, 0.5, -3.25, 0.0, math.inf, math.nan):
+        t = torch.tensor(x, dtype=torch.float64)
+        for tensor_map, float_map in ((n._leaf_rep_to_val, PM._rep_to_val1), (n._leaf_val_to_rep, PM._val_to_rep1),
+                                      (n._leaf_dval_drep, PM._dval_drep1)):
+            a, b = float(tensor_map(t)), float_map(x, *limits, cyclic)
+            assert (math.isnan(a) and math.isnan(b)) or a == b or abs(a - b) <= 4 * 2.3e-16 * abs(a), (x, a, b)
