@@ -110,14 +110,11 @@ def _dval_drep1(r, lo, hi, cyclic):
     return (hi - lo) / (math.pi * (r * r + 1))
 
 
-def _floats(v):
-    """The elements of a plain tensor as Python floats; None for one that
+def _plain(v):
+    """Whether Python floats can stand in for the tensor: not for one that
     carries a graph, a tangent or a transform, which the tensor operations keep."""
-    if type(v) is not torch.Tensor or v.requires_grad or torch._C._are_functorch_transforms_active():
-        return None
-    if torch.autograd.forward_ad._current_level >= 0 or v.dtype.is_complex:
-        return None
-    return v.to(AP_config.ap_dtype).reshape(-1).tolist()
+    return not (type(v) is not torch.Tensor or v.requires_grad or torch._C._are_functorch_transforms_active()
+                or torch.autograd.forward_ad._current_level >= 0 or v.dtype.is_complex)
 
 
 class Parameter_Node:
@@ -263,25 +260,30 @@ class Parameter_Node:
         """(leaf, its number of free elements) in the order of the flat vector."""
         return [(n, n._value.numel() if n._mask is None else int(n._mask.sum())) for n in self._leaves()]
 
+    def _plain_leaves(self):
+        """The leaves of the flat vector; None when the tensor operations have to
+        keep a value as it is: one that is not plain, or whose type is not the
+        present one (it was set under another)."""
+        leaves = self._leaves()
+        for n in leaves:
+            if n._mask is not None or n._value.dtype != AP_config.ap_dtype or not _plain(n._value):
+                return None
+        return leaves
+
     def _plain_values(self):
         """The flat vector as Python floats (None when a tensor has to be kept)."""
-        out = []
-        for n in self._leaves():
-            v = None if n._mask is not None else _floats(n._value)
-            if v is None:
-                return None
-            out += v
-        return out
+        leaves = self._plain_leaves()
+        return None if leaves is None else [x for n in leaves for x in n._value.reshape(-1).tolist()]
 
     def _plain_set(self, vec, to_value):
         """Set every free element from a plain vector, each mapped by
         ``to_value(leaf, element)``; False when the tensor path has to do it."""
-        v = _floats(vec)
-        leaves = None if v is None else self._free_leaves()
-        if v is None or sum(m for _, m in leaves) != len(v) or any(n._mask is not None for n, _ in leaves):
+        leaves = self._plain_leaves() if _plain(vec) else None
+        if leaves is None or sum(n._value.numel() for n in leaves) != vec.numel():
             return False
-        k = 0
-        for n, m in leaves:
+        v, k = vec.to(AP_config.ap_dtype).reshape(-1).tolist(), 0
+        for n in leaves:
+            m = n._value.numel()
             n._value = torch.tensor([to_value(n, x) for x in v[k:k + m]], dtype=AP_config.ap_dtype).reshape(n._value.shape)
             k += m
         return True

@@ -377,3 +377,25 @@ def test_float_parameter_maps_of_degenerate_limits(limits, cyclic):
                                       (n._leaf_dval_drep, PM._dval_drep1)):
             a, b = float(tensor_map(t)), float_map(x, *limits, cyclic)
             assert (math.isnan(a) and math.isnan(b)) or a == b or abs(a - b) <= 4 * 2.3e-16 * abs(a), (x, a, b)
+
+
+def test_values_set_under_another_type_or_with_a_graph_are_kept():
+    """Values of another type than the present one (set before it changed) are
+    read as they are, not rounded to it, and a vector of the present type is not
+    taken for them; a value that carries a graph keeps taking part in it."""
+    from astrophot_amd import AP_config
+    from astrophot_amd.param import Parameter_Node
+    top = Parameter_Node("top")
+    for k in range(2):
+        top.link(Parameter_Node(f"p{k}", value=[1.1 + k, 1.6 + k]))
+    old = AP_config.ap_dtype
+    AP_config.ap_dtype = torch.float32
+    try:
+        assert torch.equal(top.vector_values(), torch.tensor([1.1, 1.6, 2.1, 2.6], dtype=torch.float64))
+        with pytest.raises(RuntimeError):
+            top.vector_set_values(torch.ones(4))
+    finally:
+        AP_config.ap_dtype = old
+    top.vector_set_values(torch.ones(4, dtype=torch.float64, requires_grad=True))
+    top.vector_set_values(torch.arange(4, dtype=torch.float64))
+    assert top.vector_values().requires_grad and top.vector_values().tolist() == [0.0, 1.0, 2.0, 3.0]
