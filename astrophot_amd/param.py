@@ -110,11 +110,20 @@ def _dval_drep1(r, lo, hi, cyclic):
     return (hi - lo) / (math.pi * (r * r + 1))
 
 
+def _watched() -> bool:
+    """Whether something follows the tensor operations: a functorch transform,
+    forward-mode differentiation, a trace or a dispatch mode.  torch has no public
+    question for most of these; where one of its private ones is missing, the
+    answer is yes."""
+    transforms = getattr(torch._C, "_are_functorch_transforms_active", None)
+    modes = getattr(torch._C, "_len_torch_dispatch_stack", None)
+    return (transforms is None or transforms() or modes is None or modes() > 0 or torch.jit.is_tracing()
+            or getattr(torch.autograd.forward_ad, "_current_level", 0) >= 0)
+
+
 def _plain(v):
-    """Whether Python floats can stand in for the tensor: not for one that
-    carries a graph, a tangent or a transform, which the tensor operations keep."""
-    return not (type(v) is not torch.Tensor or v.requires_grad or torch._C._are_functorch_transforms_active()
-                or torch.autograd.forward_ad._current_level >= 0 or v.dtype.is_complex)
+    """Whether Python floats can stand in for the tensor: not for one that carries a graph."""
+    return type(v) is torch.Tensor and not v.requires_grad and not v.dtype.is_complex
 
 
 class Parameter_Node:
@@ -262,8 +271,10 @@ class Parameter_Node:
 
     def _plain_leaves(self):
         """The leaves of the flat vector; None when the tensor operations have to
-        keep a value as it is: one that is not plain, or whose type is not the
-        present one (it was set under another)."""
+        keep a value as it is (one that is not plain, or whose type is not the
+        present one, as it was set under another), or are followed."""
+        if _watched():
+            return None
         leaves = self._leaves()
         for n in leaves:
             if n._mask is not None or n._value.dtype != AP_config.ap_dtype or not _plain(n._value):

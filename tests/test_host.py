@@ -399,3 +399,51 @@ def test_values_set_under_another_type_or_with_a_graph_are_kept():
     top.vector_set_values(torch.ones(4, dtype=torch.float64, requires_grad=True))
     top.vector_set_values(torch.arange(4, dtype=torch.float64))
     assert top.vector_values().requires_grad and top.vector_values().tolist() == [0.0, 1.0, 2.0, 3.0]
+
+
+def _pair():
+    from astrophot_amd.param import Parameter_Node
+    top = Parameter_Node("top")
+    top.link(Parameter_Node("a", value=1.1, limits=(0.0, None)))
+    top.link(Parameter_Node("b", value=2.1))
+    return top
+
+
+def test_vector_operations_are_followed_by_traces_and_transforms(monkeypatch):
+    """A trace, a dispatch mode, a functorch transform and a tangent see the
+    vector's operations, so the result follows the input; and where torch's
+    private questions about them are gone, everything stays on the tensor path."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from astrophot_amd import param as PM
+
+    class Count(TorchDispatchMode):
+        seen = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            Count.seen += func is torch.ops.aten.sqrt.default
+            return func(*args, **(kwargs or {}))
+
+    top, v = _pair(), torch.tensor([0.7, 1.9], dtype=torch.float64)
+
+    def run(x):
+        top.vector_set_representation(x)
+        return top.vector_values()
+
+    want = run(v + 0.25)
+    assert not want.requires_grad and PM._plain(v) and top._plain_leaves() is not None
+    traced = torch.jit.trace(run, (v,), check_trace=False)
+    assert torch.allclose(traced(v + 0.25), want, rtol=1e-15, atol=0)
+    top.vector_set_values(v.clone())
+    with Count():
+        run(v)
+    assert Count.seen == 1
+    d = torch.func.jvp(run, (v,), (torch.ones_like(v),))[1]
+    assert torch.allclose(d, top.vector_dval_drep(v).detach(), rtol=1e-15, atol=0)
+    for owner, name in ((torch._C, "_are_functorch_transforms_active"), (torch._C, "_len_torch_dispatch_stack"),
+                        (torch.autograd.forward_ad, "_current_level")):
+        top = _pair()
+        with monkeypatch.context() as m:
+            m.delattr(owner, name)
+            assert top._plain_leaves() is None
+            if owner is torch._C:
+                assert torch.allclose(run(v + 0.25), want, rtol=1e-15, atol=0)
