@@ -295,7 +295,8 @@ class Parameter_Node:
         v, k = vec.to(AP_config.ap_dtype).reshape(-1).tolist(), 0
         for n in leaves:
             m = n._value.numel()
-            n._value = torch.tensor([to_value(n, x) for x in v[k:k + m]], dtype=AP_config.ap_dtype).reshape(n._value.shape)
+            n._value = torch.tensor([to_value(n, x) for x in v[k:k + m]], dtype=AP_config.ap_dtype,
+                                    device="cpu").reshape(n._value.shape)
             k += m
         return True
 
@@ -305,7 +306,7 @@ class Parameter_Node:
             return self._value.reshape(-1)[self.mask]
         plain = self._plain_values()
         if plain is not None:
-            return torch.tensor(plain, dtype=AP_config.ap_dtype)
+            return torch.tensor(plain, dtype=AP_config.ap_dtype, device="cpu")
         vec = [n.vector_values() for n in self._leaves()]
         return torch.cat(vec) if vec else torch.zeros(0, dtype=AP_config.ap_dtype)
 

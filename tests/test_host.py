@@ -447,3 +447,13 @@ def test_vector_operations_are_followed_by_traces_and_transforms(monkeypatch):
             assert top._plain_leaves() is None
             if owner is torch._C:
                 assert torch.allclose(run(v + 0.25), want, rtol=1e-15, atol=0)
+
+
+def test_vectors_stay_on_the_host_under_a_default_device():
+    """Values live on the host whatever torch's default device is."""
+    top = _pair()
+    with torch.device("meta"):
+        assert top.vector_values().device.type == "cpu"
+        top.vector_set_representation(torch.tensor([0.7, 1.9], dtype=torch.float64, device="cpu"))
+        top.vector_set_values(top.vector_values())
+    assert all(n.value.device.type == "cpu" for n in top._leaves())
