@@ -19,6 +19,7 @@ from __future__ import annotations
 import math
 from collections import OrderedDict
 from contextlib import contextmanager
+from itertools import compress
 from typing import Optional
 
 import numpy as np
@@ -270,34 +271,42 @@ class Parameter_Node:
         return [(n, n._value.numel() if n._mask is None else int(n._mask.sum())) for n in self._leaves()]
 
     def _plain_leaves(self):
-        """The leaves of the flat vector; None when the tensor operations have to
-        keep a value as it is (one that is not plain, or whose type is not the
-        present one, as it was set under another), or are followed."""
+        """(leaf, its mask as a list or None) of the flat vector; None when the
+        tensor operations have to keep a value as it is (one that is not plain, or
+        whose type is not the present one, as it was set under another), or are
+        followed."""
         if _watched():
             return None
-        leaves = self._leaves()
-        for n in leaves:
-            if n._mask is not None or n._value.dtype != AP_config.ap_dtype or not _plain(n._value):
+        out = []
+        for n in self._leaves():
+            keep = None if n._mask is None else n._mask.tolist()
+            if n._value.dtype != AP_config.ap_dtype or not _plain(n._value) or \
+                    (keep is not None and len(keep) != n._value.numel()):
                 return None
-        return leaves
+            out.append((n, keep))
+        return out
 
     def _plain_values(self):
         """The flat vector as Python floats (None when a tensor has to be kept)."""
         leaves = self._plain_leaves()
-        return None if leaves is None else [x for n in leaves for x in n._value.reshape(-1).tolist()]
+        if leaves is None:
+            return None
+        return [x for n, keep in leaves for x in (n._value.reshape(-1).tolist() if keep is None else
+                                                  compress(n._value.reshape(-1).tolist(), keep))]
 
     def _plain_set(self, vec, to_value):
         """Set every free element from a plain vector, each mapped by
         ``to_value(leaf, element)``; False when the tensor path has to do it."""
         leaves = self._plain_leaves() if _plain(vec) else None
-        if leaves is None or sum(n._value.numel() for n in leaves) != vec.numel():
+        if leaves is None or sum(n._value.numel() if keep is None else sum(keep) for n, keep in leaves) != vec.numel():
             return False
-        v, k = vec.to(AP_config.ap_dtype).reshape(-1).tolist(), 0
-        for n in leaves:
-            m = n._value.numel()
-            n._value = torch.tensor([to_value(n, x) for x in v[k:k + m]], dtype=AP_config.ap_dtype,
-                                    device="cpu").reshape(n._value.shape)
-            k += m
+        new = iter(vec.to(AP_config.ap_dtype).reshape(-1).tolist())
+        for n, keep in leaves:
+            if keep is None:
+                v = [to_value(n, next(new)) for _ in range(n._value.numel())]
+            else:
+                v = [to_value(n, next(new)) if k else old for k, old in zip(keep, n._value.reshape(-1).tolist())]
+            n._value = torch.tensor(v, dtype=AP_config.ap_dtype, device="cpu").reshape(n._value.shape)
         return True
 
     # -- vector API (param/parameter.py:169-420) ---------------------------

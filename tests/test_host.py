@@ -457,3 +457,24 @@ def test_vectors_stay_on_the_host_under_a_default_device():
         top.vector_set_representation(torch.tensor([0.7, 1.9], dtype=torch.float64, device="cpu"))
         top.vector_set_values(top.vector_values())
     assert all(n.value.device.type == "cpu" for n in top._leaves())
+
+
+@pytest.mark.parametrize("mask", [[True] * 5, [True, False, True, True, False], [False] * 5])
+def test_masked_vectors_on_floats_equal_the_tensor_path(mask):
+    """Under a mask, and after one, the vector is read and set by floats as
+    without: the same values, masked ones untouched."""
+    from astrophot_amd.param import Param_Mask, Parameter_Node
+    made = []
+    for graph in (False, True):
+        top = Parameter_Node("top")
+        for k, (lim, cyc) in enumerate(LIMITS[:4]):
+            top.link(Parameter_Node(f"p{k}", value=[1.1, 2.1] if k == 1 else 1.3 + 0.1 * k, limits=lim, cyclic=cyc))
+        with Param_Mask(top, torch.tensor(mask)):
+            assert top._plain_leaves() is not None
+            rep = top.vector_representation() * 1.01 + 0.01
+            assert len(rep) == sum(mask)
+            top.vector_set_representation(rep.requires_grad_(graph))
+            made.append(top.vector_values().detach())
+        assert top._plain_leaves() is not None or graph
+        made.append(top.vector_values().detach())
+    assert torch.allclose(made[0], made[2], rtol=1e-15, atol=0) and torch.allclose(made[1], made[3], rtol=1e-15, atol=0)
