@@ -163,6 +163,8 @@ def ptr(t) -> int:
 
 
 def stream() -> int:
-    """The current stream of the current device (its handle alone: a Stream object costs 3 us)."""
-    torch.cuda._lazy_init()
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    """The current stream of the current device (its handle alone, by torch's own
+    private question where it has one: a Stream object costs 3 us)."""
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    device = torch.cuda.current_device()
+    return torch.cuda.current_stream(device).cuda_stream if raw is None else raw(device)

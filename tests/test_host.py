@@ -478,3 +478,18 @@ def test_masked_vectors_on_floats_equal_the_tensor_path(mask):
         assert top._plain_leaves() is not None or graph
         made.append(top.vector_values().detach())
     assert torch.allclose(made[0], made[2], rtol=1e-15, atol=0) and torch.allclose(made[1], made[3], rtol=1e-15, atol=0)
+
+
+def test_stream_handle_without_the_private_interface(monkeypatch):
+    """The current stream's handle comes from the public Stream object where torch
+    has no raw one to give."""
+    class Stream:
+        cuda_stream = 77
+
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: Stream() if device == 3 else None)
+    monkeypatch.delattr(torch._C, "_cuda_getDevice", raising=False)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda device: 78 + device, raising=False)
+    assert L.stream() == 81
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
+    assert L.stream() == 77
