@@ -132,6 +132,34 @@ def test_short_and_long_refined_lists_agree(n, quad_group):
             assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("quad_group", [32, 25])
+def test_both_branches_of_the_list_passes_are_taken(quad_group):
+    """Three copies of a nearly round, centred galaxy, whose pixels come to a
+    threshold by eights: the lengths of the three lists (refined pixels, undecided
+    selections, pixels redone in float64) are on the long side of every rule for a
+    launch of one workgroup and on the short side for one of 4,096, and the bits
+    are the same."""
+    v = np.array([16.5, 16.5, 0.999999, 0.3, 3.0, 3.0, 0.5])
+    bf = BatchFit([Cutout(np.zeros((33, 33)), np.ones((33, 33)), H.gaussian_psf(1.0, 9, 1.0))] * 3)
+    bf.b.quad_group = quad_group
+    rep = values_to_rep(np.stack([v] * 3))
+    for tol in (8.36e-4, 6.52e-4, 6.03e-4):
+        bf.b.tolerance = tol
+        out = []
+        for blocks in (1, 4096):
+            bf.b.quad_blocks = blocks
+            img, J = bf.jacobian(rep)
+            counts = [bf.counters()]
+            out.append((img.clone(), J.clone(), bf.render(rep).clone()))
+            counts.append(bf.counters())
+            for c in counts:
+                assert 2 < c["refined"] <= 2048
+                assert 16 < c["undecided_select"] <= 16 * 4096
+                assert 2 < c["redone"] <= 2048
+        for a, b in zip(*out):
+            assert torch.equal(a, b)
+
+
 def test_batch_jacobian_matches_single_model():
     """apx_batch_jacobian: every cutout's model and its 7 representation-space
     Jacobian columns equal the single-model jacobian(as_representation=True)
