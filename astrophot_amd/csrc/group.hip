@@ -141,13 +141,16 @@ __device__ __forceinline__ int pieces_of(int64_t n, int S) {
   return (int)min((int64_t)S, max((int64_t)1, (n + kPiece - 1) / kPiece));
 }
 // The most pieces a window (or an overlap) gets when `count` of them share the
-// chip.  Every one is launched, also those that small windows do not have, so a
-// group of small windows gets fewer: as many as one of four times the mean window
-// has (1,000 windows of 30 x 30: normal equations 362 us with 16, 142 with 1).  With
-// one, the kernels write the result itself in place of a partial sum.
+// chip.  Every one is launched, also those that small windows do not have, at some
+// 10 ns each, so the launch is kept to 8,192 workgroups where that leaves 5 pieces
+// or more (normal equations of 250 sources, 1,182 pairs: 372 us with 16, 285 with
+// 8; of 30 sources, 185 pairs: 108 with 16, 127 with 8), and a group of small
+// windows gets fewer: as many as one of three times the mean window has (1,000
+// windows of 30 x 30: 362 us with 16, 142 with 1).  With one, the kernels write the
+// result itself in place of a partial sum.
 inline int max_pieces(const apx_group& g, int count) {
-  const int64_t mean = g.nsrcpix / std::max(1, g.nsrc);
-  return (int)std::max<int64_t>(1, std::min<int64_t>({16, 32768 / std::max(1, count), 4 * mean / kPiece}));
+  const int64_t mean = g.nsrcpix / std::max(1, g.nsrc), n = std::max(1, count);
+  return (int)std::max<int64_t>(1, std::min<int64_t>({16, std::max(8192 / n, std::min<int64_t>(5, 32768 / n)), 3 * mean / kPiece}));
 }
 
 // part[s S + piece][k] = sum over the piece of the window of J_k * v (v a double
