@@ -155,15 +155,20 @@ __host__ inline size_t mfma_lds_bytes(int kh, int kw, int blocks = 1) {
   return sizeof(float) * ((size_t)(mf_rows(kh) + kMfR * (blocks - 1)) * kMfLW + (size_t)mf_tab(kh, kw));
 }
 __host__ inline size_t mfma_lds_bytes(int kmax) { return mfma_lds_bytes(kmax, kmax); }
-// The single-image convolution gives two 16-row blocks to a workgroup of 8 waves,
+// The single-image convolution may give two 16-row blocks to a workgroup of 8 waves,
 // which share the halo rows and the tap table: two such workgroups fit a CU
-// (kernels to 67: 80.4 kB of 80 KiB), with 4 waves a SIMD in place of 2 and half
-// the staging an output.  512^2, 53 x 53, Jacobian of 7 columns: 122 -> 115 us;
-// 1537 x 1201, 67 x 67, four planes: 861 -> 792.  Where the launch has fewer than
-// kMfTallMin of them (two a CU) a block a workgroup spreads better.  (The batched
-// convolution keeps one tile a workgroup: its tile pairs took 0.82 -> 0.88 ms over
-// 256 uneven cutouts, where many last pairs are half empty.)
-constexpr int kMfTallMin = 512;
+// (kernels to 67: 80.4 kB of 80 KiB), 512 the chip, with 4 waves a SIMD in place of 2
+// and half the staging an output.  For the value plane this is faster from one full
+// round on (kMfTallMin): 512 workgroups, 1024^2: 21 rows 19.9 -> 19.2 us, 53 rows 64.6
+// -> 59.0; 288: 15.9 -> 18.5 and 51.0 -> 58.7.  Columns of a Jacobian add to
+// interleaved memory, which more, smaller workgroups hide better: there from two
+// rounds and a half on, whose last one weighs less, and from kMfTallRows rows on,
+// with enough products a row.  Seven columns: 1024^2 (3,584) 21 rows 113 -> 134 us, 31
+// rows 199 -> 204, 39 rows 286 -> 261, 67 rows 699 -> 614; 640^2 (1,400) 53 rows 182
+// -> 175; 512^2 (896) 114 -> 121.  (The batched convolution keeps one tile a
+// workgroup: its tile pairs took 0.82 -> 0.88 ms over 256 uneven cutouts, where many
+// last pairs are half empty.)
+constexpr int kMfTallMin = 512, kMfTallMinColumns = 1280, kMfTallRows = 37;
 
 // All kernel columns of one output block: column kx needs NKS k-steps.  The
 // operands of the next column are loaded between the MFMAs of the current one
