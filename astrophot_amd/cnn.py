@@ -73,8 +73,12 @@ def gemm(A, sam, sak, B, sbk, sbn, C, M, N, K, ldc=None, bias=None, relu=False, 
     tiles = ((M + 63) // 64) * ((N + 63) // 64)
     splits = 1
     if K >= 4096 and tiles < 128 and ws is not None:
-        # 512 deep a workgroup: each k-step of 32 waits for its operands, and the weight gradients of 256
-        # cutouts have 1 to 9 tiles (six gradients: 258 us at 2,048 deep, 121 so)
+        # 512 deep a workgroup where 256 splits reach: each k-step of 32 waits for its operands, and the
+        # convolutions' weight gradients have 1 to 9 tiles.  At 256 cutouts the first one's K is 262,144,
+        # so its workgroups are 1,024 deep; the dense layers' K is the batch and stays whole.  Training
+        # steps at depths 256 / 512 / 1,024 / 2,048: 16 cutouts 255 / 274 / 296 / 351 us, 256 cutouts
+        # 451 / 458 / 491 / 584, 1,024 cutouts 1,153 / 1,154 / 1,168 / 1,228; 512 has half the partial
+        # sums of 256 to hold
         splits = int(min(max(1, K // 512), 256, ws.numel() // max(M * N, 1)))
     L.check(lib.apx_gemm_bf16(M, N, K, A.data_ptr(), sam, sak, B.data_ptr(), sbk, sbn, C.data_ptr(), ldc,
                               _ptr(bias), int(relu), _ptr(Cb), int(accumulate), splits,
@@ -249,7 +253,8 @@ class InitNet:
         """x: bf16 input of B cutouts (NHWC, C = 1) -> (B, 8) float32 outputs.
         keep_cols: write each convolution's im2col matrix (the weight
         gradients of training read it); without, each convolution reads its
-        input directly (apx_conv_s2_bf16), with the same result."""
+        input directly (apx_conv_s2_bf16), with the same result: layer by layer what
+        ``predict`` does in one kernel, whose outputs are checked against it."""
         lib = L.load()
         buf = self._buffers(B)
         cur = x

@@ -967,7 +967,10 @@ __device__ __forceinline__ void level3_lane(const Prof<float>& pf, float xs, flo
 // another, and a lane up to 9 float64 samples of an undecided one, which sets the
 // time of a launch with few fits left (about 100 of 4,096: Jacobian pass 30 -> 21
 // us, its float64 pass 28 -> 12, the value pass's 19 -> 10).
-// A long list keeps a group a pixel, which evaluates level 2 once.
+// A long list keeps a group a pixel, which evaluates level 2 once.  The two cross
+// between 2,000 and 10,000 pixels, by how many sub-pixels are flagged: renders of
+// 3,100 refined pixels of small cutouts 57 us so and 61 wide, of 3,000 of larger
+// windows 77 and 76 (Jacobians 61 and 65, 98 and 84), of 12,000 75 and 91.
 constexpr int kWideMax = 2048;
 template <bool GRAD, int GS, bool F64, int QN, int QG>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void integrate_kernel(apx_batch b, Scratch s,
@@ -2519,8 +2522,10 @@ QuadTab quad_table(const apx_batch& b) {
   return t;
 }
 
-// the packed list of the segments `seg` with counts `cnt`; few fits go a workgroup
-// each, their runs are the longer for it (125 scene sources: 100^2 to 420^2 pixels)
+// The packed list of the segments `seg` with counts `cnt`.  Few fits go a workgroup
+// each, since few are often large (125 windows of 100^2 to 420^2: renders 285 us so,
+// 303 with 8 fits a workgroup); many fits share them (48^2 cutouts: 4,096 fits 596 us
+// with a workgroup each, 421 with 8; 512 fits 134 and 125).
 inline void pack_list(const apx_batch& b, const Scratch& s, int32_t* cnt, const int32_t* seg, int2* out, int32_t* len,
                       int clear, hipStream_t stream) {
   const int fits = std::max(1, std::min(kPackFits, b.ngal / 512));
@@ -2712,9 +2717,9 @@ int batch_plan(apx_batch_galaxy* gal, int32_t ngal, apx_batch* b) {
     kmax = std::max(kmax, std::max(G.ph, G.pw) + 2);
   }
   // the VALU convolution is every batch's fallback and must fit 64 KiB; the MFMA
-  // one (kmax <= kMfmaMax) takes up to 73 KiB of the 160 KiB a workgroup has
-  if (conv_lds_bytes(kmax) + kConvStaticLds > 65536 ||
-      (kmax <= kMfmaMax && mfma_lds_bytes(kmax) + kConvStaticLds > 160 * 1024))
+  // one (kmax <= kMfmaMax) takes up to 70 KiB of the 160 KiB a workgroup has
+  static_assert(mfma_lds_bytes(kMfmaMax) + kConvStaticLds <= 70 * 1024, "two workgroups a CU");
+  if (conv_lds_bytes(kmax) + kConvStaticLds > 65536)
     return set_error(APX_E_LIMIT, "batch_plan: psf too large for the batched Jacobian convolution");
   if (work > (int64_t)INT32_MAX || chunk > (int64_t)INT32_MAX || tile > (int64_t)INT32_MAX)
     return set_error(APX_E_LIMIT, "batch_plan: batch too large");

@@ -367,8 +367,8 @@ __global__ __launch_bounds__(256) void colsum_kernel(const float* X, int M, int 
 // Bound by HBM: 4 B (8 with a mask) read and 2 B written an element.  It stands
 // in for a gate pass that also wrote v in float32 and a column sum of that copy
 // on one workgroup per 64 columns, whose rows were read one after another: the
-// six layers of a training step on 256 cutouts took 21.05 ms, and take 73 us
-// (46 here, 27 in column_final_kernel).
+// six layers of a training step on 256 cutouts took 21.05 ms, and take 64 us
+// (43 here, 20 in column_final_kernel).
 // VEC: 4 consecutive columns a thread (16-byte loads); a workgroup covers
 // 1024 / N whole rows a step, so a thread's columns never change.  Else: 64
 // columns (blockIdx.y) x 4 rows a step, for any N.

@@ -142,19 +142,19 @@ constexpr int kMfR = 16;       // output rows of an MFMA block
 constexpr int kMfmaWide = 67;  // tallest kernel mfma_block dispatches (21 k-steps)
 
 __host__ __device__ constexpr int mf_nks(int kh) { return (kMfR + kh - 1 + 3) / 4; }  // k-steps per kx
-__host__ __device__ inline int mf_rows(int kh) { return 4 * mf_nks(kh); }
+__host__ __device__ constexpr int mf_rows(int kh) { return 4 * mf_nks(kh); }
 // Row pitch of the staged input, one for every kernel width, so that an A
 // operand's k-steps lie at immediate offsets.  144 floats hold the 64 + 67 - 1
 // columns of the widest kernel and put the 4 rows x 16 columns of an operand
 // (lanes l / 16, l % 16) in distinct LDS banks.
 constexpr int kMfLW = 144;
-__host__ __device__ inline int mf_dd(int kh) { return mf_rows(kh) + 1; }
-__host__ __device__ inline int mf_tab(int kh, int kw) { return kw * mf_dd(kh) + 16; }  // the last column's zeros too
+__host__ __device__ constexpr int mf_dd(int kh) { return mf_rows(kh) + 1; }
+__host__ __device__ constexpr int mf_tab(int kh, int kw) { return kw * mf_dd(kh) + 16; }  // the last column's zeros too
 // LDS of one pass: the staged input of `blocks` 16-row output blocks and one tap table
-__host__ inline size_t mfma_lds_bytes(int kh, int kw, int blocks = 1) {
+__host__ constexpr size_t mfma_lds_bytes(int kh, int kw, int blocks = 1) {
   return sizeof(float) * ((size_t)(mf_rows(kh) + kMfR * (blocks - 1)) * kMfLW + (size_t)mf_tab(kh, kw));
 }
-__host__ inline size_t mfma_lds_bytes(int kmax) { return mfma_lds_bytes(kmax, kmax); }
+__host__ constexpr size_t mfma_lds_bytes(int kmax) { return mfma_lds_bytes(kmax, kmax); }
 // The single-image convolution may give two 16-row blocks to a workgroup of 8 waves,
 // which share the halo rows and the tap table: two such workgroups fit a CU
 // (kernels to 67: 80.4 kB of 80 KiB), 512 the chip, with 4 waves a SIMD in place of 2

@@ -92,6 +92,22 @@ def test_gate_colsum(M, N, masked, off):
     assert bool((err <= 64 * 2.0 ** -24 * ref.double().abs().sum(0)).all())
 
 
+@pytest.mark.parametrize("M,N", [(1, 1), (7, 64), (130, 65), (1001, 8)])
+def test_separate_gate_and_column_sums(M, N):
+    """apx_cast_gate_bf16 with a gate and a float32 copy, and apx_colsum of that
+    copy, the C entry points that gate_colsum does in one: a column is four chains
+    of M / 4 additions."""
+    g = torch.Generator().manual_seed(M)
+    src, mask = torch.randn(M, N, generator=g).to(DEV), torch.randn(M, N, generator=g).to(DEV)
+    dst, dstf, out = torch.zeros((M, N), dtype=torch.bfloat16, device=DEV), torch.zeros_like(src), torch.zeros(N, device=DEV)
+    cnn.cast_bf16(src, dst, mask=mask, dstf=dstf)
+    cnn.L.check(cnn.L.load().apx_colsum(dstf.data_ptr(), M, N, out.data_ptr(), cnn.L.stream()))
+    ref = torch.where(mask > 0, src, torch.zeros_like(src))
+    assert torch.equal(dst, ref.to(torch.bfloat16)) and torch.equal(dstf, ref)
+    err = (out.double() - ref.double().sum(0)).abs()
+    assert bool((err <= (M // 4 + 4) * 2.0 ** -24 * ref.double().abs().sum(0)).all())
+
+
 def torch_reference(net, x, dout_seed=3):
     """The same network in torch on the CPU (float32), bf16 rounding where the kernels round."""
     params = []
