@@ -153,6 +153,13 @@ def rep_to_values(r: np.ndarray) -> np.ndarray:
     return v
 
 
+def conv_grids(ntile: int, impl: int) -> List[int]:
+    """Workgroup counts to time for a convolution: no more than it has work items, a
+    tile each, or for the MFMA kernel (2) one of the 7 passes of a tile."""
+    items = ntile * (7 if impl == 2 else 1)
+    return sorted({min(c, items) for c in (1024, 2048, 4096, 8192, 16384)})
+
+
 class BatchFit:
     """All cutouts resident on the GPU; ``fit(rep0)`` runs every LM to the end."""
 
@@ -305,9 +312,8 @@ class BatchFit:
         self.jacobian(rep, out=out, parts=1)
         impls = [1] + ([2] if b.max_kernel <= 67 else []) + ([3] if self.sep_all and b.max_kernel <= 61 else [])
         best = None
-        conv_grid = sorted({min(c, int(b.ntile)) for c in (1024, 2048, 4096, 8192, 16384)})  # launches clamp to ntile
         for impl in impls:
-            for blocks in conv_grid:
+            for blocks in conv_grids(int(b.ntile), impl):
                 b.conv_impl, b.conv_blocks = impl, blocks
                 ms = self._time(lambda: self.jacobian(rep, out=out, parts=2))
                 log["conv"][f"{CONV_IMPL[impl]}:{blocks}"] = ms

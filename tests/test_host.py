@@ -493,3 +493,13 @@ def test_stream_handle_without_the_private_interface(monkeypatch):
     assert L.stream() == 81
     monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
     assert L.stream() == 77
+
+
+def test_convolution_grids_reach_every_work_item():
+    """The MFMA convolution's items are the 7 passes of a tile: a small batch's
+    tuned launch can have a workgroup for each, and none has more."""
+    from astrophot_amd.batch import conv_grids
+    for ntile in (1, 4, 146, 147, 420, 5000):
+        assert max(conv_grids(ntile, 2)) == min(7 * ntile, 16384)
+        for impl in (1, 3):
+            assert max(conv_grids(ntile, impl)) == min(ntile, 16384)
