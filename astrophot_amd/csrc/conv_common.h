@@ -158,17 +158,16 @@ __host__ constexpr size_t mfma_lds_bytes(int kmax) { return mfma_lds_bytes(kmax,
 // The single-image convolution may give two 16-row blocks to a workgroup of 8 waves,
 // which share the halo rows and the tap table: two such workgroups fit a CU
 // (kernels to 67: 80.4 kB of 80 KiB), 512 the chip, with 4 waves a SIMD in place of 2
-// and half the staging an output.  For the value plane this is faster from one full
-// round on (kMfTallMin): 512 workgroups, 1024^2: 21 rows 19.9 -> 19.2 us, 53 rows 64.6
-// -> 59.0; 288: 15.9 -> 18.5 and 51.0 -> 58.7.  Columns of a Jacobian add to
-// interleaved memory, which more, smaller workgroups hide better: there from two
-// rounds and a half on, whose last one weighs less, and from kMfTallRows rows on,
-// with enough products a row.  Seven columns: 1024^2 (3,584) 21 rows 113 -> 134 us, 31
-// rows 199 -> 204, 39 rows 286 -> 261, 67 rows 699 -> 614; 640^2 (1,400) 53 rows 182
-// -> 175; 512^2 (896) 114 -> 121.  (The batched convolution keeps one tile a
-// workgroup: its tile pairs took 0.82 -> 0.88 ms over 256 uneven cutouts, where many
-// last pairs are half empty.)
-constexpr int kMfTallMin = 512, kMfTallMinColumns = 1280, kMfTallRows = 37;
+// and half the staging an output.  It takes a full round of them (kMfTallMin): value
+// plane, 768^2 (288 workgroups) 53 rows 51.0 -> 58.7 us, 1024^2 (512) 64.6 -> 59.0 and
+// 21 rows 19.9 -> 19.2.  A Jacobian's columns also take kMfTallRows kernel rows: with
+// fewer products a row their additions to interleaved memory weigh more, which more,
+// smaller workgroups hide better.  Seven of 13 columns, 1024^2: 31 rows 201 -> 221 us,
+// 39 rows 301 -> 276, 67 rows 723 -> 632; 512^2 (896): 31 rows 52.0 -> 58.4, 39 rows
+// 80.5 -> 76.7, 53 rows 115.5 -> 116.8, and within a Jacobian of two components
+// 112.5 -> 107.5.  (The batched convolution keeps one tile a workgroup: its tile pairs
+// took 0.82 -> 0.88 ms over 256 uneven cutouts, where many last pairs are half empty.)
+constexpr int kMfTallMin = 512, kMfTallRows = 37;
 
 // All kernel columns of one output block: column kx needs NKS k-steps.  The
 // operands of the next column are loaded between the MFMAs of the current one

@@ -320,7 +320,7 @@ __global__ __launch_bounds__(256) void convolve_fast_kernel(apx_conv_job job,
 // take the workgroups round robin).  Bound by the FP32 matrix pipe.  With all
 // passes of a tile in one workgroup, rows copied through registers a load at a
 // time, 512^2 with 53 x 53 kernels took 41 us (value) and 244 us (Jacobian of 7
-// columns); so 24.5 and 114 us (100^2 with 27 x 27: 19 and 110 us, 12 and 14 us).
+// columns); so 24.5 and 115 us (100^2 with 27 x 27: 19 and 110 us, 12 and 14 us).
 constexpr int kMfmaMin = 21;  // shorter kernels waste over half of each MFMA on the band's zeros
 constexpr int kMaxPass = APX_MAX_CHAN + 2;
 
@@ -485,7 +485,7 @@ static int convolve_mfma(const apx_conv_job& job, const float* planes, const flo
   for (int c = 1; c < job.nchan; ++c) add(c, 0, job.chan_col[c]), ++n;
   const int ntx = (job.ow + 63) / 64;
   const int64_t tall = (int64_t)ntx * ((job.oh + (int64_t)2 * kMfR - 1) / (2 * kMfR));
-  const bool two = tall * n >= (n == 1 ? kMfTallMin : kMfTallMinColumns) && (n == 1 || job.kh >= kMfTallRows);
+  const bool two = tall * n >= kMfTallMin && (n == 1 || job.kh >= kMfTallRows);
   const int64_t ntile = two ? tall : (int64_t)ntx * ((job.oh + kMfR - 1) / kMfR);
   auto* kernel = two ? &convolve_mfma_kernel<true> : &convolve_mfma_kernel<false>;
   const size_t lds = mfma_lds_bytes(job.kh, job.kw, two ? 2 : 1);
