@@ -383,7 +383,7 @@ __global__ __launch_bounds__(256) void render_deep_kernel(apx_component cp, Rend
   constexpr int NV = GRAD ? 1 + APX_NSLOT : 1;
   constexpr int NS = FAST ? 225 : 1, NG = FAST ? 1 : 64;
   __shared__ float sample[NV][FAST ? NS : 256], middle[NG];
-  __shared__ double sx[4 * 64], sy[4 * 64];  // flagged sub-pixels (of up to four pixels)
+  __shared__ double sx[(FAST ? 1 : 4) * 64], sy[(FAST ? 1 : 4) * 64];  // flagged sub-pixels (of up to four pixels)
   __shared__ double ox3[NS], oy3[NS], w3[NS];
   __shared__ double nodeu[NG], nodev[NG], nodew[NG], suba[NG], subb[NG];  // node q; sub-pixel's place in its pixel
   __shared__ double red[4][NV];
@@ -412,11 +412,7 @@ __global__ __launch_bounds__(256) void render_deep_kernel(apx_component cp, Rend
   double adj[APX_NSLOT];
 #pragma unroll
   for (int s = 0; s < APX_NSLOT; ++s) adj[s] = 0.0;
-  if ((int)blockIdx.x >= count) {  // no pixel for this workgroup
-    if (MODE == Q_VJP) vjp_part(cp, adj, ws.vpart + 8 * (voff + blockIdx.x));
-    return;
-  }
-  if (FAST) {
+  if (FAST) {  // ahead of the first use of count, which is on its way
     if (t < NS) offset3(t, ox3[t], oy3[t], w3[t]);
   } else {
     if (t < nn) {
@@ -429,6 +425,10 @@ __global__ __launch_bounds__(256) void render_deep_kernel(apx_component cp, Rend
       subb[t] = sub0 + subd * (t / g);
     }
     __syncthreads();
+  }
+  if ((int)blockIdx.x >= count) {  // no pixel for this workgroup
+    if (MODE == Q_VJP) vjp_part(cp, adj, ws.vpart + 8 * (voff + blockIdx.x));
+    return;
   }
   // sub-pixel and (first) node of this thread at level 2
   const int slices = FAST ? 9 : min(nn, 256 / gg);
