@@ -271,19 +271,24 @@ class Parameter_Node:
         return [(n, n._value.numel() if n._mask is None else int(n._mask.sum())) for n in self._leaves()]
 
     def _plain_leaves(self):
-        """(leaf, its mask as a list or None) of the flat vector; None when the
-        tensor operations have to keep a value as it is (one that is not plain, or
-        whose type is not the present one, as it was set under another), or are
-        followed."""
+        """(leaf, its mask as a list or None, its number of free elements) of the
+        flat vector; None when the tensor operations have to keep a value as it is
+        (one that is not plain, or whose type is not the present one, as it was set
+        under another), or are followed."""
         if _watched():
             return None
-        out = []
+        out, dtype = [], AP_config.ap_dtype
         for n in self._leaves():
-            keep = None if n._mask is None else n._mask.tolist()
-            if n._value.dtype != AP_config.ap_dtype or not _plain(n._value) or \
-                    (keep is not None and len(keep) != n._value.numel()):
+            v = n._value
+            if v.dtype != dtype or not _plain(v):
                 return None
-            out.append((n, keep))
+            if n._mask is None:
+                out.append((n, None, v.numel()))
+            else:
+                keep = n._mask.tolist()
+                if len(keep) != v.numel():
+                    return None
+                out.append((n, keep, sum(keep)))
         return out
 
     def _plain_values(self):
@@ -291,22 +296,27 @@ class Parameter_Node:
         leaves = self._plain_leaves()
         if leaves is None:
             return None
-        return [x for n, keep in leaves for x in (n._value.reshape(-1).tolist() if keep is None else
-                                                  compress(n._value.reshape(-1).tolist(), keep))]
+        out = []
+        for n, keep, _ in leaves:
+            v = n._value.reshape(-1).tolist()
+            out += v if keep is None else compress(v, keep)
+        return out
 
     def _plain_set(self, vec, to_value):
         """Set every free element from a plain vector, each mapped by
         ``to_value(leaf, element)``; False when the tensor path has to do it."""
         leaves = self._plain_leaves() if _plain(vec) else None
-        if leaves is None or sum(n._value.numel() if keep is None else sum(keep) for n, keep in leaves) != vec.numel():
+        if leaves is None or sum(m for _, _, m in leaves) != vec.numel():
             return False
-        new = iter(vec.to(AP_config.ap_dtype).reshape(-1).tolist())
-        for n, keep in leaves:
-            if keep is None:
-                v = [to_value(n, next(new)) for _ in range(n._value.numel())]
-            else:
-                v = [to_value(n, next(new)) if k else old for k, old in zip(keep, n._value.reshape(-1).tolist())]
-            n._value = torch.tensor(v, dtype=AP_config.ap_dtype, device="cpu").reshape(n._value.shape)
+        dtype, k = AP_config.ap_dtype, 0
+        new = vec.to(dtype).reshape(-1).tolist()
+        for n, keep, m in leaves:
+            v = [to_value(n, x) for x in new[k:k + m]]
+            k += m
+            if keep is not None:
+                free, old = iter(v), n._value.reshape(-1).tolist()
+                v = [next(free) if f else x for f, x in zip(keep, old)]
+            n._value = torch.tensor(v, dtype=dtype, device="cpu").reshape(n._value.shape)
         return True
 
     # -- vector API (param/parameter.py:169-420) ---------------------------
