@@ -127,6 +127,12 @@ def _plain(v):
     return type(v) is torch.Tensor and not v.requires_grad and not v.dtype.is_complex
 
 
+def _from_floats(v, shape):
+    """A host tensor of Python floats (by way of numpy: a third of torch.tensor's
+    time, and torch's default device has no say in it)."""
+    return torch.from_numpy(np.array(v, dtype=np.float64).reshape(shape)).to(AP_config.ap_dtype)
+
+
 class Parameter_Node:
     """A leaf parameter or a group of nodes (param/parameter.py:18-742)."""
 
@@ -308,15 +314,14 @@ class Parameter_Node:
         leaves = self._plain_leaves() if _plain(vec) else None
         if leaves is None or sum(m for _, _, m in leaves) != vec.numel():
             return False
-        dtype, k = AP_config.ap_dtype, 0
-        new = vec.to(dtype).reshape(-1).tolist()
+        new, k = vec.to(AP_config.ap_dtype).reshape(-1).tolist(), 0
         for n, keep, m in leaves:
             v = [to_value(n, x) for x in new[k:k + m]]
             k += m
             if keep is not None:
                 free, old = iter(v), n._value.reshape(-1).tolist()
                 v = [next(free) if f else x for f, x in zip(keep, old)]
-            n._value = torch.tensor(v, dtype=dtype, device="cpu").reshape(n._value.shape)
+            n._value = _from_floats(v, n._value.shape)
         return True
 
     # -- vector API (param/parameter.py:169-420) ---------------------------
@@ -325,7 +330,7 @@ class Parameter_Node:
             return self._value.reshape(-1)[self.mask]
         plain = self._plain_values()
         if plain is not None:
-            return torch.tensor(plain, dtype=AP_config.ap_dtype, device="cpu")
+            return _from_floats(plain, (len(plain),))
         vec = [n.vector_values() for n in self._leaves()]
         return torch.cat(vec) if vec else torch.zeros(0, dtype=AP_config.ap_dtype)
 
