@@ -480,7 +480,8 @@ __device__ __forceinline__ void panel_rows(const double* __restrict__ A, int n, 
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = r0 + 4 * r + lk, col = 16 * q + li;
-      c[q][r] = (row < n && col < nb) ? A[(int64_t)row * n + k0 + col] : 0.0;
+      // lower triangle: workgroup 0 of the launch writes the block's upper one
+      c[q][r] = (row < n && col < nb && k0 + col <= row) ? A[(int64_t)row * n + k0 + col] : 0.0;
     }
   if (k0 > 0) {
     double a[kSteps], b[2][kSteps];

@@ -135,6 +135,25 @@ def test_factor_and_solve_at_panel_edges(n):
     assert int(st.item()) == n // 2 + 1
 
 
+@pytest.mark.parametrize("n", [2, 33, 100])
+def test_factor_reads_the_lower_triangle_only(n):
+    """The strict upper triangle of the matrix takes no part (the factor's transpose
+    is written there while other workgroups still read the block): NaN there leaves
+    the same bits."""
+    lib = L.load()
+    B = np.random.default_rng(n).normal(size=(2 * n, n))
+    Hm = B.T @ B
+    made = []
+    for fill in (0.0, np.nan):
+        M = np.tril(Hm) + np.triu(np.full((n, n), fill), 1)
+        Hd, fac = torch.tensor(M, device="cuda"), torch.empty((n, n), dtype=torch.float64, device="cuda")
+        st = torch.zeros(1, dtype=torch.int32, device="cuda")
+        L.check(lib.apx_dense_damped_factor(n, L.ptr(Hd), 0.5, L.ptr(fac), L.ptr(st), L.stream()))
+        assert int(st.item()) == 0
+        made.append(fac)
+    assert torch.equal(*made)
+
+
 def test_factor_rounds_once_a_panel():
     """|L L^T - A| of a dense 417 x 417 system, in extended precision: every entry
     has 13 panels taken out of it and is written once more, 14 roundings of at
